@@ -9,6 +9,8 @@
 #include <vector>
 
 #include "nyl_ctx.h"
+#include "nyl_march.h"
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 
@@ -51,12 +53,6 @@ namespace {
 }  // namespace
 
 namespace {
-
-// prolongation fused into the first post-smoothing sweep of tiled levels
-#ifndef NYL_FUSE_PROLONG
-#define NYL_FUSE_PROLONG 0
-#endif
-
 
 uint64_t align256(uint64_t v) { return (v + 255) & ~uint64_t(255); }
 
@@ -149,6 +145,8 @@ void build_layout(nyl_ctx *c) {
     }
     c->partials = take(NYL_RED_BLOCKS * sizeof(double));
     c->result = take(8 * sizeof(double));
+    c->ctl = take(sizeof(MGCtl));
+    c->ent = take(sizeof(c->cyc_ent));
     c->cs_tab = c->exact ? take(coarse_table_doubles() * sizeof(double)) : 0;
     for (int q = 0; q < c->ntr; q++) {
         c->tst[0][q] = take(fb);
@@ -244,16 +242,9 @@ void arm_publish(nyl_ctx *c, int n) {
     r.consumed = 0;
 }
 
-int read_results(nyl_ctx *c, double *out, int n) {
-    const double *src = reinterpret_cast<const double *>(c->ws + c->result);
-    Publish &r = g_publish;
-    const bool armed = r.consumed && r.dst && r.dst == c->host_dev && r.src == src && r.n == n;
-    const uint32_t seq = armed ? r.seq : ++c->pub_seq;
-    r = Publish{};
+// wait until the results with sequence number seq are in host memory
+int wait_published(nyl_ctx *c, uint32_t seq) {
     volatile uint32_t *flag = reinterpret_cast<volatile uint32_t *>(c->host_out + 8);
-    if (!armed)
-        HIPCHK(launch_publish(src, n, c->host_dev, reinterpret_cast<uint32_t *>(c->host_dev + 8),
-                              seq, c->stream));
     const auto t0 = std::chrono::steady_clock::now();
     for (uint64_t it = 1; *flag != seq; it++) {
         if ((it & 1023) == 0 &&
@@ -264,6 +255,20 @@ int read_results(nyl_ctx *c, double *out, int n) {
         }
     }
     std::atomic_thread_fence(std::memory_order_acquire);
+    return NYL_OK;
+}
+
+int read_results(nyl_ctx *c, double *out, int n) {
+    const double *src = reinterpret_cast<const double *>(c->ws + c->result);
+    Publish &r = g_publish;
+    const bool armed = r.consumed && r.dst && r.dst == c->host_dev && r.src == src && r.n == n;
+    const uint32_t seq = armed ? r.seq : ++c->pub_seq;
+    r = Publish{};
+    if (!armed)
+        HIPCHK(launch_publish(src, n, c->host_dev, reinterpret_cast<uint32_t *>(c->host_dev + 8),
+                              seq, c->stream));
+    int rc = wait_published(c, seq);
+    if (rc) return rc;
     const volatile double *v = c->host_out;
     for (int q = 0; q < n; q++) out[q] = v[q];
     return NYL_OK;
@@ -306,248 +311,192 @@ void set_tendency_out(nyl_ctx *c, StageArgs<T> &a, int slot) {
     a.tv = F<T>(c, c->ds[slot][2]); a.tw = F<T>(c, c->ds[slot][3]);
 }
 
-// One smooth() of level l: the two fsmoother3d sweeps x -> y -> x.
-// xc_level >= 0 first adds the prolongation from that coarse level.
-// pre_done: the first sweep already ran into y (speculatively, with the
-// convergence test of the previous V-cycle, or from e = 0 in the outer
-// residual of the mixed solve).
-// addx (level 0 of the mixed solve): the last sweep adds its result to the
-// FP64 solution instead of storing it (tiled levels), or an add follows.
-// Post-smoothing of the tiled levels as one two-sweep pass after the
-// prolongation into y: src and b are read once for two sweeps (256^3:
-// 37.8 us FP32 and 93.4 us FP64 against 2 x 31.6 and 2 x 80 us).  The pass
-// can also add the second sweep's result to an FP64 solution.
-#ifndef NYL_SWEEP2
-#define NYL_SWEEP2 1
-#endif
-
-// Levels 1 .. nlev-2 run the fused level kernels (down: second pre-sweep +
-// restriction; up: prolongation + both post-sweeps), whose up-leg leaves the
-// level's correction in y.
-#ifndef NYL_FUSED_LEVELS
-#define NYL_FUSED_LEVELS 1
-#endif
+// ---- the levels of a V-cycle ------------------------------------------------
+// How the passes of a level run:
+//   cycle   from the first level whose whole remainder fits one workgroup
+//           (cells <= CYC_CELLS and the LDS): k_mg_cycle, one launch
+//   fused   other levels of at most NYL_FUSED_MAX_CELLS cells: k_mg_down and
+//           k_mg_up, 4^3 tiles (32^3: 5.9 us each, where a march takes 7.5
+//           and 10.4)
+//   tiled   nx % 64 == 0, ny % 8 == 0 and one type with the level below:
+//           k_mg_sweep25 + k_mg_restrict25, k_mg_prolong25 + k_mg_sweep2t
+//   march   any other level: k_mg_march down and up
+// Every level's first sweep is written by the restriction from the level
+// above.  The correction of a level ends in its y, of a tiled level and of a
+// coarsest level in its x.
 #ifndef NYL_FUSED_MAX_CELLS
 #define NYL_FUSED_MAX_CELLS 32768
 #endif
+// cells of the largest level of the cycle
+#ifndef CYC_CELLS
+#define CYC_CELLS 4096
+#endif
+
 bool fused_level(const nyl_ctx *c, int l) {
-    return NYL_FUSED_LEVELS && l >= 1 && l <= c->nlev - 2 &&
-           cells(c->lev[l].g) <= NYL_FUSED_MAX_CELLS &&
+    return l >= 1 && l <= c->nlev - 2 && cells(c->lev[l].g) <= NYL_FUSED_MAX_CELLS &&
            fused_fits(c->lev[l].g, c->lev[l + 1].g);
 }
 
-// offset of the buffer that holds level l's correction after its up-leg
+bool tiled_level(const nyl_ctx *c, int l) {
+    return l <= c->nlev - 2 && restrict25_fits(c->lev[l].g) && lev64(c, l) == lev64(c, l + 1) &&
+           sweep2x_blocks(c->lev[l].g, lev64(c, l) ? 8 : 4) <= NYL_RED_BLOCKS;
+}
+
+// offset of the buffer that holds level l's correction (l >= 1)
 uint64_t sol_off(const nyl_ctx *c, int l) {
-    return fused_level(c, l) ? c->lev[l].y : c->lev[l].x;
+    if (l == c->nlev - 1) return c->lev[l].x;
+    if (l >= c->t0 || fused_level(c, l)) return c->lev[l].y;
+    return tiled_level(c, l) ? c->lev[l].x : c->lev[l].y;
 }
 
-template <typename Tf>
-int smooth_level_t(nyl_ctx *c, int l, int xc_level, bool pre_done, double *addx,
-                   bool sol_in_y) {
-    Level &f = c->lev[l];
-    const double om = c->d.mg_omega;
-    Tf *x = F<Tf>(c, f.x), *b = F<Tf>(c, f.b), *y = F<Tf>(c, f.y);
-    const int SWC = NYL_K_MG_SWEEP | (l == 0 ? kFineLevel : 0);
-    const double by = 3 * cells(f.g) * sizeof(Tf);
-    const bool tiled = sweep25_fits(f.g);
-    if (xc_level >= 0) {
-        Level &q = c->lev[xc_level];
-        const uint64_t qx = sol_off(c, xc_level);
-        const bool same = lev64(c, xc_level) == std::is_same<Tf, double>::value;
-        if (sol_in_y) {
-            // the level's solution is in y (both pre-sweeps in one pass):
-            // y += P(xc) in place, then both post-sweeps y -> x
-            if (!(NYL_SWEEP2 && same && restrict25_fits(f.g) && tiled))
-                return fail(NYL_E_STATE, "level solution in y without the two-sweep pass");
-            Tf *yv = F<Tf>(c, f.y);
-            LAUNCH(NYL_K_MG_PROLONG, 2.125 * cells(f.g) * sizeof(Tf),
-                   launch_mg_prolong25<Tf, Tf>(f.g, q.g, yv, F<Tf>(c, qx), c->tabs, c->stream));
-            const double b2 = addx ? (2 * sizeof(Tf) + 2 * sizeof(double)) * cells(f.g) : by;
-            LAUNCH(NYL_K_MG_SWEEP2 | (l == 0 ? kFineLevel : 0), b2,
-                   launch_mg_sweep2x25<Tf>(f.g, yv, x, b, om, c->tabs, c->stream, addx));
-            return NYL_OK;
-        }
-        if (NYL_FUSE_PROLONG && tiled && same) {
-            // prolongation fused into the first sweep: x + P(xc) -> y, then y -> x
-            const double bp = (3 + 0.125) * cells(f.g) * sizeof(Tf);
-            LAUNCH(SWC, bp,
-                   launch_mg_sweep25<Tf>(f.g, x, y, b, om, c->tabs, nullptr, nullptr, c->stream,
-                                         &q.g, F<Tf>(c, qx)));
-            LAUNCH(SWC, by, launch_mg_sweep25<Tf>(f.g, y, x, b, om, c->tabs, nullptr,
-                                                              nullptr, c->stream));
-            return NYL_OK;
-        }
-        const double bp = 2.125 * cells(f.g) * sizeof(Tf);
-        if (NYL_SWEEP2 && same && restrict25_fits(f.g) && tiled && !pre_done) {
-            // y = x + P(xc), then both post-smoothing sweeps y -> x in one
-            // pass (with addx: the second sweep's result added to the FP64 x)
-            Tf *yv = F<Tf>(c, f.y);
-            LAUNCH(NYL_K_MG_PROLONG, bp,
-                   launch_mg_prolong25<Tf, Tf>(f.g, q.g, x, F<Tf>(c, qx), c->tabs, c->stream, yv));
-            const double b2 = addx ? (2 * sizeof(Tf) + 2 * sizeof(double)) * cells(f.g) : by;
-            LAUNCH(NYL_K_MG_SWEEP2 | (l == 0 ? kFineLevel : 0), b2,
-                   launch_mg_sweep2x25<Tf>(f.g, yv, x, b, om, c->tabs, c->stream, addx));
-            return NYL_OK;
-        }
-        if (same && restrict25_fits(f.g)) {
-            LAUNCH(NYL_K_MG_PROLONG, bp,
-                   launch_mg_prolong25<Tf, Tf>(f.g, q.g, x, F<Tf>(c, qx), c->tabs, c->stream));
-        } else if (lev64(c, xc_level)) {
-            LAUNCH(NYL_K_MG_PROLONG, bp,
-                   launch_mg_prolong<Tf, double>(f.g, q.g, x, F<double>(c, qx), c->tabs,
-                                                 c->stream));
-        } else if constexpr (std::is_same<Tf, float>::value) {
-            LAUNCH(NYL_K_MG_PROLONG, bp,
-                   launch_mg_prolong<float, float>(f.g, q.g, x, F<float>(c, qx), c->tabs,
-                                                   c->stream));
-        } else {
-            return fail(NYL_E_STATE, "FP64 level above an FP32 level");
-        }
+// first level of the cycle: the largest that fits (never the finest); its
+// position table is uploaded when the workspace is bound
+int cycle_first(nyl_ctx *c) {
+    Geo g[kMaxLevels];
+    for (int l = 0; l < c->nlev; l++) g[l] = c->lev[l].g;
+    int t0 = c->nlev;
+    for (int l = c->nlev - 1; l >= 1; l--) {
+        CycleArgs a;
+        CycleEnt ent[CYC_ENT];
+        // a direct solve alone pays only while it is small: 25x15x7 takes 21 us
+        // in one workgroup, 13 us in its own three launches
+        if (l == c->nlev - 1 && c->exact && cells(g[l]) > 1024) break;
+        if (cells(g[l]) > CYC_CELLS ||
+            !cycle_layout(a, ent, g, l, c->nlev, lev64(c, l) ? 8 : 4, c->exact != 0,
+                          c->d.mg_omega, c->tabs))
+            break;
+        t0 = l;
+        c->cyc = a;
+        memcpy(c->cyc_ent, ent, sizeof(ent));
     }
-    if (tiled) {
-        if (!pre_done)
-            LAUNCH(SWC, by, launch_mg_sweep25<Tf>(f.g, x, y, b, om, c->tabs, nullptr,
-                                                              nullptr, c->stream));
-        if (addx) {
-            const double bx = (2 * sizeof(Tf) + 2 * sizeof(double)) * cells(f.g);
-            LAUNCH(SWC, bx, launch_mg_sweep25<Tf>(f.g, y, x, b, om, c->tabs, nullptr,
-                                                              nullptr, c->stream, nullptr,
-                                                              nullptr, addx));
-        } else {
-            LAUNCH(SWC, by, launch_mg_sweep25<Tf>(f.g, y, x, b, om, c->tabs, nullptr,
-                                                              nullptr, c->stream));
-        }
-        return NYL_OK;
-    }
-    if (!pre_done)
-        LAUNCH(SWC, by, launch_mg_sweep<Tf>(f.g, x, y, b, om, c->tabs, c->stream));
-    LAUNCH(SWC, by, launch_mg_sweep<Tf>(f.g, y, x, b, om, c->tabs, c->stream));
-    if (addx) {
-        if constexpr (std::is_same<Tf, float>::value) {
-            LAUNCH(NYL_K_MG_UPDATE, (2 * sizeof(double) + sizeof(float)) * cells(f.g),
-                   launch_add_correction<float>(f.g, addx, x, c->stream));
-        } else {
-            return fail(NYL_E_STATE, "FP64 inner level");
-        }
-    }
-    return NYL_OK;
+    return t0;
 }
 
-int smooth_level(nyl_ctx *c, int l, int xc_level, bool pre_done = false,
-                 double *addx = nullptr, bool sol_in_y = false) {
-    return lev64(c, l) ? smooth_level_t<double>(c, l, xc_level, pre_done, addx, sol_in_y)
-                       : smooth_level_t<float>(c, l, xc_level, pre_done, addx, sol_in_y);
+template <typename T, typename TC>
+MarchArgs<T, TC> march_args(nyl_ctx *c, int l, uint64_t src, uint64_t dst) {
+    MarchArgs<T, TC> a = {};
+    const Level &f = c->lev[l], &q = c->lev[l + 1 < c->nlev ? l + 1 : l];
+    a.g = f.g;
+    a.gc = q.g;
+    a.src = F<T>(c, src);
+    a.dst = F<T>(c, dst);
+    a.b = F<T>(c, f.b);
+    a.omega = c->d.mg_omega;
+    a.tab = c->tabs;
+    return a;
 }
 
-// residual of level l restricted into level l + 1, with level l+1's first
-// smoothing sweep from x = 0 written to its y (from_y: level l's solution is
-// in its y)
-int restrict_level(nyl_ctx *c, int l, bool from_y = false) {
-    Level &f = c->lev[l], &q = c->lev[l + 1];
-    const uint64_t fx = from_y ? f.y : f.x;   // the level's solution
+// calls fn(T, TC) with values of the types of levels l and l + 1
+template <typename Fn>
+int with_types(const nyl_ctx *c, int l, Fn fn) {
     const bool f64 = lev64(c, l), c64 = lev64(c, l + 1);
-    const double om = c->d.mg_omega;
-    const double bytes = 2.25 * cells(f.g) * (f64 ? sizeof(double) : sizeof(float));
-    if (f64 == c64 && restrict25_fits(f.g)) {
-        if (f64)
-            LAUNCH(NYL_K_MG_RESTRICT, bytes,
-                   launch_mg_restrict25<double, double>(f.g, q.g, F<double>(c, fx),
-                                                        F<double>(c, f.b), F<double>(c, q.b),
-                                                        F<double>(c, q.x), c->tabs, c->stream,
-                                                        F<double>(c, q.y), om));
-        else
-            LAUNCH(NYL_K_MG_RESTRICT, bytes,
-                   launch_mg_restrict25<float, float>(f.g, q.g, F<float>(c, fx),
-                                                      F<float>(c, f.b), F<float>(c, q.b),
-                                                      F<float>(c, q.x), c->tabs, c->stream,
-                                                      F<float>(c, q.y), om));
-    } else if (f64 && c64) {
-        LAUNCH(NYL_K_MG_RESTRICT, bytes,
-               launch_mg_resid_restrict<double, double>(f.g, q.g, F<double>(c, fx),
-                                                        F<double>(c, f.b), F<double>(c, q.b),
-                                                        F<double>(c, q.x), c->tabs, c->stream,
-                                                        F<double>(c, q.y), om));
-    } else if (!f64 && c64) {
-        LAUNCH(NYL_K_MG_RESTRICT, bytes,
-               launch_mg_resid_restrict<float, double>(f.g, q.g, F<float>(c, fx),
-                                                       F<float>(c, f.b), F<double>(c, q.b),
-                                                       F<double>(c, q.x), c->tabs, c->stream,
-                                                       F<double>(c, q.y), om));
-    } else if (!f64 && !c64) {
-        LAUNCH(NYL_K_MG_RESTRICT, bytes,
-               launch_mg_resid_restrict<float, float>(f.g, q.g, F<float>(c, fx),
-                                                      F<float>(c, f.b), F<float>(c, q.b),
-                                                      F<float>(c, q.x), c->tabs, c->stream,
-                                                      F<float>(c, q.y), om));
-    } else {
-        return fail(NYL_E_STATE, "FP64 level above an FP32 level");
-    }
-    return NYL_OK;
+    if (f64 && c64) return fn(double(), double());
+    if (!f64 && c64) return fn(float(), double());
+    if (!f64) return fn(float(), float());
+    return fail(NYL_E_STATE, "FP64 level above an FP32 level");
 }
+
+double elem(const nyl_ctx *c, int l) { return lev64(c, l) ? sizeof(double) : sizeof(float); }
 
 // level l's second pre-sweep (y -> x) and the restriction into level l + 1
-// (b and the first sweep from zero into y) in one launch
-int fused_down(nyl_ctx *c, int l) {
-    Level &f = c->lev[l], &q = c->lev[l + 1];
-    const bool f64 = lev64(c, l), c64 = lev64(c, l + 1);
-    const double om = c->d.mg_omega;
-    const double es = f64 ? sizeof(double) : sizeof(float);
-    const double bytes = 3 * cells(f.g) * es + 2 * cells(q.g) * (c64 ? 8.0 : 4.0);
-    if (f64 && c64)
-        LAUNCH(NYL_K_MG_SWEEP, bytes,
-               launch_mg_down<double, double>(f.g, q.g, F<double>(c, f.y), F<double>(c, f.b),
-                                              F<double>(c, f.x), F<double>(c, q.b),
-                                              F<double>(c, q.y), om, c->tabs, c->stream));
-    else if (!f64 && c64)
-        LAUNCH(NYL_K_MG_SWEEP, bytes,
-               launch_mg_down<float, double>(f.g, q.g, F<float>(c, f.y), F<float>(c, f.b),
-                                             F<float>(c, f.x), F<double>(c, q.b),
-                                             F<double>(c, q.y), om, c->tabs, c->stream));
-    else if (!f64 && !c64)
-        LAUNCH(NYL_K_MG_SWEEP, bytes,
-               launch_mg_down<float, float>(f.g, q.g, F<float>(c, f.y), F<float>(c, f.b),
-                                            F<float>(c, f.x), F<float>(c, q.b),
-                                            F<float>(c, q.y), om, c->tabs, c->stream));
-    else
-        return fail(NYL_E_STATE, "FP64 level above an FP32 level");
-    return NYL_OK;
+int level_down(nyl_ctx *c, int l) {
+    const Level &f = c->lev[l], &q = c->lev[l + 1];
+    const double om = c->d.mg_omega, n = cells(f.g) * elem(c, l);
+    return with_types(c, l, [&](auto t, auto tc) -> int {
+        using T = decltype(t);
+        using TC = decltype(tc);
+        if (fused_level(c, l)) {
+            LAUNCH(NYL_K_MG_SWEEP, 3 * n + 2 * cells(q.g) * sizeof(TC),
+                   launch_mg_down<T, TC>(f.g, q.g, F<T>(c, f.y), F<T>(c, f.b), F<T>(c, f.x),
+                                         F<TC>(c, q.b), F<TC>(c, q.y), om, c->tabs, c->stream));
+            return NYL_OK;
+        }
+        if constexpr (std::is_same<T, TC>::value) {
+            if (tiled_level(c, l)) {
+                LAUNCH(NYL_K_MG_SWEEP, 3 * n,
+                       launch_mg_sweep25<T>(f.g, F<T>(c, f.y), F<T>(c, f.x), F<T>(c, f.b), om,
+                                            c->tabs, nullptr, nullptr, c->stream));
+                LAUNCH(NYL_K_MG_RESTRICT, 2.25 * n,
+                       launch_mg_restrict25<T, T>(f.g, q.g, F<T>(c, f.x), F<T>(c, f.b),
+                                                  F<T>(c, q.b), F<T>(c, q.x), c->tabs, c->stream,
+                                                  F<T>(c, q.y), om));
+                return NYL_OK;
+            }
+        }
+        MarchArgs<T, TC> a = march_args<T, TC>(c, l, f.y, f.x);
+        a.bc = F<TC>(c, q.b);
+        a.yc = F<TC>(c, q.y);
+        LAUNCH(NYL_K_MG_SWEEP, 3 * n + 2 * cells(q.g) * sizeof(TC),
+               (launch_march_down<T, TC>(a, c->stream)));
+        return NYL_OK;
+    });
 }
 
-// level l's prolongation from level l + 1 and both post-sweeps, x -> y
-int fused_up(nyl_ctx *c, int l) {
-    Level &f = c->lev[l], &q = c->lev[l + 1];
-    const bool f64 = lev64(c, l), c64 = lev64(c, l + 1);
-    const double om = c->d.mg_omega;
+// level l's prolongation from level l + 1 and both post-sweeps.  Level 0:
+// from y (both pre-sweeps were done there) into x, unless the solve has
+// stopped (gate).
+// The march reads x and b once and writes once; the tiled form's
+// prolongation writes and its two-sweep pass reads the level once more.
+// At 256^3 the march takes 57 us in FP32 and 113 us in FP64 where the tiled
+// launches take 68 and 148; at 128^3 they are even (18 and 17, 22 and 23),
+// and below that the tiled kernels' shorter prologues win (64x32x32: 8.3
+// against 10.8 us).
+#ifndef NYL_UP_MARCH_CELLS
+#define NYL_UP_MARCH_CELLS (1 << 22)
+#endif
+int level_up(nyl_ctx *c, int l, const int *gate = nullptr) {
+    const Level &f = c->lev[l], &q = c->lev[l + 1];
+    const double om = c->d.mg_omega, n = cells(f.g) * elem(c, l);
     const uint64_t qx = sol_off(c, l + 1);
-    const double es = f64 ? sizeof(double) : sizeof(float);
-    const double bytes = 3 * cells(f.g) * es + cells(q.g) * (c64 ? 8.0 : 4.0);
-    if (f64 && c64)
-        LAUNCH(NYL_K_MG_PROLONG, bytes,
-               launch_mg_up<double, double>(f.g, q.g, F<double>(c, f.x), F<double>(c, qx),
-                                            F<double>(c, f.b), F<double>(c, f.y), om, c->tabs,
-                                            c->stream));
-    else if (!f64 && c64)
-        LAUNCH(NYL_K_MG_PROLONG, bytes,
-               launch_mg_up<float, double>(f.g, q.g, F<float>(c, f.x), F<double>(c, qx),
-                                           F<float>(c, f.b), F<float>(c, f.y), om, c->tabs,
-                                           c->stream));
-    else if (!f64 && !c64)
-        LAUNCH(NYL_K_MG_PROLONG, bytes,
-               launch_mg_up<float, float>(f.g, q.g, F<float>(c, f.x), F<float>(c, qx),
-                                          F<float>(c, f.b), F<float>(c, f.y), om, c->tabs,
-                                          c->stream));
-    else
-        return fail(NYL_E_STATE, "FP64 level above an FP32 level");
-    return NYL_OK;
+    return with_types(c, l, [&](auto t, auto tc) -> int {
+        using T = decltype(t);
+        using TC = decltype(tc);
+        if (l > 0 && fused_level(c, l)) {
+            LAUNCH(NYL_K_MG_PROLONG, 3 * n + cells(q.g) * sizeof(TC),
+                   launch_mg_up<T, TC>(f.g, q.g, F<T>(c, f.x), F<TC>(c, qx), F<T>(c, f.b),
+                                       F<T>(c, f.y), om, c->tabs, c->stream));
+            return NYL_OK;
+        }
+        const bool tiled = tiled_level(c, l);
+        if constexpr (std::is_same<T, TC>::value) {
+            if (tiled && (l > 0 || cells(f.g) < NYL_UP_MARCH_CELLS)) {
+                // level 0: y += P(xc) in place; else y = x + P(xc)
+                T *x = F<T>(c, f.x), *y = F<T>(c, f.y);
+                LAUNCH(NYL_K_MG_PROLONG, 2.125 * n,
+                       launch_mg_prolong25<T, T>(f.g, q.g, l > 0 ? x : y, F<T>(c, qx), c->tabs,
+                                                 c->stream, l > 0 ? y : nullptr));
+                LAUNCH(NYL_K_MG_SWEEP2 | (l == 0 ? kFineLevel : 0), 3 * n,
+                       launch_mg_sweep2x25<T>(f.g, y, x, F<T>(c, f.b), om, c->tabs, c->stream,
+                                              nullptr, nullptr, gate));
+                return NYL_OK;
+            }
+        }
+        MarchArgs<T, TC> a = march_args<T, TC>(c, l, l > 0 ? f.x : f.y, l > 0 ? f.y : f.x);
+        a.xc = F<TC>(c, qx);
+        a.gate = gate;
+        LAUNCH(NYL_K_MG_PROLONG, 3 * n + cells(q.g) * sizeof(TC),
+               (launch_march_up<T, TC>(a, c->stream)));
+        return NYL_OK;
+    });
 }
 
-// the coarsest level's step of a V-cycle: mgfor's smooth() (two sweeps, the
-// first already written by the restriction), or the direct solve of a level
-// with an odd size
+// the coarsest level's step of a V-cycle outside the cycle: mgfor's smooth()
+// (its second sweep, the first was written by the restriction), or the
+// direct solve of a level with an odd size
 int coarsest(nyl_ctx *c) {
     const int L = c->nlev - 1;
-    if (!c->exact) return smooth_level(c, L, -1, true);
-    Level &f = c->lev[L];
+    const Level &f = c->lev[L];
+    if (!c->exact) {
+        if (lev64(c, L))
+            LAUNCH(NYL_K_MG_SWEEP, 3 * cells(f.g) * sizeof(double),
+                   launch_mg_sweep<double>(f.g, F<double>(c, f.y), F<double>(c, f.x),
+                                           F<double>(c, f.b), c->d.mg_omega, c->tabs, c->stream));
+        else
+            LAUNCH(NYL_K_MG_SWEEP, 3 * cells(f.g) * sizeof(float),
+                   launch_mg_sweep<float>(f.g, F<float>(c, f.y), F<float>(c, f.x),
+                                          F<float>(c, f.b), c->d.mg_omega, c->tabs, c->stream));
+        return NYL_OK;
+    }
     CoarseArgs a;
     a.g = f.g;
     a.b = F<double>(c, f.b);
@@ -558,157 +507,119 @@ int coarsest(nyl_ctx *c) {
     return NYL_OK;
 }
 
-// The smallest levels (fused, one type, at most NYL_TAIL_MAX_CELLS cells,
-// all of them with the coarsest level within the tail kernel's LDS) and the
-// coarsest level run in one single-workgroup launch (k_mg_tail): below a
-// few hundred cells a level's launches cost more than its work, while one
-// workgroup's issue rate makes a larger level cheaper as separate launches.
-#ifndef NYL_TAIL
-#define NYL_TAIL 1
-#endif
-#ifndef NYL_TAIL_MAX_CELLS
-#define NYL_TAIL_MAX_CELLS TAIL_T
-#endif
-// first level of the tail, -1 when there is none
-int tail_level(const nyl_ctx *c) {
-    const int L = c->nlev;
-    if (!NYL_TAIL || c->exact || L < 3 || L > NYL_TAIL_MAXLEV) return -1;
-    auto lds = [&](int l) {
-        const int64_t n = (int64_t)cells(c->lev[l].g) * (lev64(c, l) ? 8 : 4);
-        return 3.0 * (double)((n + 15) / 16 * 16);
-    };
-    double used = lds(L - 1);
-    int t0 = -1;
-    for (int l = L - 2; l >= 1; l--) {
-        used += lds(l);
-        if (!fused_level(c, l) || used > NYL_TAIL_LDS || cells(c->lev[l].g) > NYL_TAIL_MAX_CELLS ||
-            lev64(c, l) != lev64(c, L - 2))
-            break;
-        t0 = l;
-    }
-    return t0;
-}
-
-int tail(nyl_ctx *c, int t0) {
-    const int L = c->nlev;
-    TailArgs a;
-    memset(&a, 0, sizeof(a));
-    a.ws = c->ws;
-    double bytes = 0.0;
-    for (int l = 0; l < L; l++) {
-        const Level &v = c->lev[l];
-        a.lev[l].g = v.g;
-        a.lev[l].x = v.x;
-        a.lev[l].b = v.b;
-        a.lev[l].y = v.y;
-        if (l >= t0) bytes += 3.0 * cells(v.g) * (lev64(c, l) ? 8.0 : 4.0);
-    }
-    a.l0 = t0;
-    a.nlev = L;
-    a.omega = c->d.mg_omega;
-    a.tab = c->tabs;
-    const bool t64 = lev64(c, t0), c64 = lev64(c, L - 1);
-    if (t64 && c64) LAUNCH(NYL_K_MG_COARSE, bytes, (launch_mg_tail<double, double>(a, c->stream)));
-    else if (!t64 && c64) LAUNCH(NYL_K_MG_COARSE, bytes, (launch_mg_tail<float, double>(a, c->stream)));
-    else if (!t64 && !c64) LAUNCH(NYL_K_MG_COARSE, bytes, (launch_mg_tail<float, float>(a, c->stream)));
-    else return fail(NYL_E_STATE, "FP64 level above an FP32 level");
-    return NYL_OK;
-}
-
-// the part of a V-cycle below level 1: from level 2's smoothing (its first
-// sweep written by the restriction from level 1) down to the coarsest level
-// and back up to level 2's post-smoothing
-int coarse_cycle(nyl_ctx *c) {
-    const int L = c->nlev;
-    const int t0 = tail_level(c);
-    const int down_end = t0 >= 0 ? t0 : L - 1;   // levels [1, down_end) run here
+// Levels 1 and below of a V-cycle (core/mgfor/solvers.f90:35-55), from the
+// right-hand side and first sweep of level 1.  fin: the test that is waiting
+// for its sum, run beside the cycle (or before, where there is no cycle).
+int coarse_levels(nyl_ctx *c, const CtlArgs *fin) {
+    const int L = c->nlev, t0 = c->t0;
+    const int last = t0 < L ? t0 : L - 1;   // levels [1, last) run here
     int rc;
-    for (int l = 1; l < down_end; l++) {
-        if (fused_level(c, l)) {
-            if ((rc = fused_down(c, l))) return rc;
-            continue;
-        }
-        if ((rc = smooth_level(c, l, -1, true))) return rc;
-        if ((rc = restrict_level(c, l))) return rc;
-    }
-    if (t0 >= 0) {
-        if ((rc = tail(c, t0))) return rc;
+    if (fin && t0 >= L) HIPCHK(launch_ctl(*fin, c->stream));
+    for (int l = 1; l < last; l++)
+        if ((rc = level_down(c, l))) return rc;
+    if (t0 < L) {
+        const Level &f = c->lev[t0];
+        double bytes = 0.0;
+        for (int l = t0; l < L; l++) bytes += 3.0 * cells(c->lev[l].g) * elem(c, l);
+        if (lev64(c, t0))
+            LAUNCH(NYL_K_MG_COARSE, bytes,
+                   launch_mg_cycle<double>(c->cyc, F<double>(c, f.b), F<double>(c, f.y),
+                                           F<double>(c, f.x), fin, c->stream));
+        else
+            LAUNCH(NYL_K_MG_COARSE, bytes,
+                   launch_mg_cycle<float>(c->cyc, F<float>(c, f.b), F<float>(c, f.y),
+                                          F<float>(c, f.x), fin, c->stream));
     } else if ((rc = coarsest(c))) {
         return rc;
     }
-    for (int l = down_end - 1; l >= 1; l--) {
-        if (fused_level(c, l)) {
-            if ((rc = fused_up(c, l))) return rc;
-            continue;
+    for (int l = last - 1; l >= 1; l--)
+        if ((rc = level_up(c, l))) return rc;
+    return NYL_OK;
+}
+
+// Both pre-smoothing sweeps of level 0 into its y and the restriction into
+// level 1.  zero: from a zero solution; else from x, with the block sums of
+// its residual norm in the partials (their number in *np).
+// A level that does not tile runs the march; up to 1M cells with the
+// restriction in the same pass (96^3 FP64: 19.4 us against 12.9 + 7.0), above
+// that its wider rings cost more than the second pass reads (192x128x96: 39
+// against 20.7 + 11.6).
+int pre_smooth(nyl_ctx *c, bool zero, int *np) {
+    const Level &f = c->lev[0], &q = c->lev[1];
+    const double om = c->d.mg_omega, n = cells(f.g) * elem(c, 0);
+    double *part = F<double>(c, c->partials);
+    return with_types(c, 0, [&](auto t, auto tc) -> int {
+        using T = decltype(t);
+        using TC = decltype(tc);
+        if constexpr (std::is_same<T, TC>::value) {
+            if (tiled_level(c, 0)) {
+                if (zero) {
+                    // (not in the fine-level class of the roofline: it reads one field)
+                    LAUNCH(NYL_K_MG_SWEEP2, 2 * n,
+                           launch_mg_sweep2x25<T>(f.g, nullptr, F<T>(c, f.y), F<T>(c, f.b), om,
+                                                  c->tabs, c->stream));
+                } else {
+                    LAUNCH(NYL_K_MG_SWEEP2 | kFineLevel, 3 * n,
+                           launch_mg_sweep2x25<T>(f.g, F<T>(c, f.x), F<T>(c, f.y), F<T>(c, f.b),
+                                                  om, c->tabs, c->stream, part));
+                    *np = sweep2x_blocks(f.g, (int)sizeof(T));
+                }
+                LAUNCH(NYL_K_MG_RESTRICT, 2.25 * n,
+                       launch_mg_restrict25<T, T>(f.g, q.g, F<T>(c, f.y), F<T>(c, f.b),
+                                                  F<T>(c, q.b), F<T>(c, q.x), c->tabs, c->stream,
+                                                  F<T>(c, q.y), om));
+                return NYL_OK;
+            }
         }
-        if ((rc = smooth_level(c, l, l + 1))) return rc;
-    }
-    return NYL_OK;
+        MarchArgs<T, TC> a = march_args<T, TC>(c, 0, f.x, f.y);
+        const bool one = cells(f.g) <= (1 << 20);
+        if (zero) a.src = nullptr;
+        else a.partials = part;
+        if (one) {
+            a.bc = F<TC>(c, q.b);
+            a.yc = F<TC>(c, q.y);
+        }
+        if (!zero) {
+            *np = march_grid(f.g, (int)sizeof(T), one).blocks();
+            if (*np > NYL_RED_BLOCKS) {   // too wide for one partial sum per block
+                if constexpr (std::is_same<T, double>::value) {
+                    LAUNCH(NYL_K_RESNORM, 2 * n,
+                           launch_resnorm2<double>(f.g, a.src, a.b, c->tabs, part, nullptr,
+                                                   c->stream));
+                    *np = red_blocks((int64_t)cells(f.g));
+                    a.partials = nullptr;
+                } else {
+                    return fail(NYL_E_SIZE, "level 1 is too wide for the residual norm");
+                }
+            }
+        }
+        LAUNCH(NYL_K_MG_SWEEP2 | (zero ? 0 : kFineLevel), (zero ? 2 : 3) * n,
+               (launch_march_pre<T, TC>(a, c->stream)));
+        if (!one) {
+            MarchArgs<T, TC> r = march_args<T, TC>(c, 0, f.y, f.x);
+            r.bc = F<TC>(c, q.b);
+            r.yc = F<TC>(c, q.y);
+            LAUNCH(NYL_K_MG_RESTRICT, 2.25 * n, (launch_march_restrict<T, TC>(r, c->stream)));
+        }
+        return NYL_OK;
+    });
 }
 
-void drop_graphs(nyl_ctx *c) {
-    if (c->g_coarse) {
-        (void)hipGraphExecDestroy(c->g_coarse);
-        c->g_coarse = nullptr;
-    }
-}
-
-// The coarse part is the same launch sequence every V-cycle: it is captured
-// once into a hipGraph and replayed (the per-launch overhead dominates these
-// small levels).  Direct launches are used on the null stream, and while a
-// kernel class that includes coarse-level launches is being timed.
-int coarse_cycle_run(nyl_ctx *c) {
-    const int pc = c->prof_cls;
-    const bool timed = pc == NYL_K_MG_SWEEP || pc == NYL_K_MG_RESTRICT || pc == NYL_K_MG_PROLONG ||
-                       pc == NYL_K_MG_SWEEP2 || pc == NYL_K_MG_COARSE ||
-                       pc == NYL_K_MG_SWEEP2_FINE;
-    if (!c->use_graphs || !c->stream || timed) return coarse_cycle(c);
-    if (!c->g_coarse) {
-        hipGraph_t graph;
-        HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        const int prof = c->prof_cls;
-        c->prof_cls = 0;                 // no event records inside the graph
-        int rc = coarse_cycle(c);
-        c->prof_cls = prof;
-        hipError_t e = hipStreamEndCapture(c->stream, &graph);
-        if (rc) return rc;
-        HIPCHK(e);
-        HIPCHK(hipGraphInstantiate(&c->g_coarse, graph, nullptr, nullptr, 0));
-        HIPCHK(hipGraphDestroy(graph));
-    }
-    HIPCHK(hipGraphLaunch(c->g_coarse, c->stream));
-    return NYL_OK;
-}
-
-// core/mgfor/solvers.f90:35-55.  pre_done: the level-1 pre-smooth already
-// ran into the spare buffer.  addx: the mixed solve's x, which receives the
-// level-1 result (x += e).  Below level 1 the first sweep of each level is
-// written by the restriction.
-// pre: the level-1 pre-smoothing done before the call, 0 none, 1 the first
-// sweep (in y), 2 both (in y, by the two-sweep pass of the convergence
-// test): then the restriction reads y, the prolongation adds to y in place
-// and the post-smoothing pass writes x.
-int vcycle(nyl_ctx *c, int pre, double *addx = nullptr) {
-    int rc;
-    if (pre < 2 && (rc = smooth_level(c, 0, -1, pre == 1))) return rc;
-    if ((rc = restrict_level(c, 0, pre == 2))) return rc;
-    if (c->nlev > 2) {
-        if ((rc = coarse_cycle_run(c))) return rc;
-    } else {
-        if ((rc = coarsest(c))) return rc;
-    }
-    return smooth_level(c, 0, 1, false, addx, pre == 2);
-}
-
-// The convergence test's residual norm can come with both pre-smoothing
-// sweeps of the next V-cycle (k_mg_sweep2t, solution into y): level 1 tiled
-// for the two-sweep pass and level 2 of the same type (the post-smoothing
-// that follows uses the pass too)
-bool spec2_fits(const nyl_ctx *c) {
+// the residual norm of level 0's x alone, block sums in the partials
+template <typename T>
+int resid_norm(nyl_ctx *c, int *np) {
     const Level &f = c->lev[0];
-    return NYL_SWEEP2 && c->nlev >= 2 && sweep25_fits(f.g) && restrict25_fits(f.g) &&
-           lev64(c, 0) == lev64(c, 1) &&
-           sweep2x_blocks(f.g, lev64(c, 0) ? 8 : 4) <= NYL_RED_BLOCKS;
+    MarchArgs<T, T> a = march_args<T, T>(c, 0, f.x, f.y);
+    a.partials = F<double>(c, c->partials);
+    *np = march_grid(f.g, (int)sizeof(T), false).blocks();
+    if (*np > NYL_RED_BLOCKS) {
+        *np = red_blocks((int64_t)cells(f.g));
+        LAUNCH(NYL_K_RESNORM, 2 * cells(f.g) * sizeof(T),
+               launch_resnorm2<T>(f.g, a.src, a.b, c->tabs, a.partials, nullptr, c->stream));
+        return NYL_OK;
+    }
+    LAUNCH(NYL_K_RESNORM, 2 * cells(f.g) * sizeof(T), launch_march_norm<T>(a, c->stream));
+    return NYL_OK;
 }
 
 void fill_stats(nyl_ctx *c, nyl_mg_stats *st, int nite, double res, double normb) {
@@ -721,61 +632,121 @@ void fill_stats(nyl_ctx *c, nyl_mg_stats *st, int nite, double res, double normb
     }
 }
 
-// core/mgfor/solvers.f90:8-33 with normresidual (core/mgfor/operators.f90:81-96).
-// When level 1 uses the tiled sweeps, the residual norm of x is computed by
-// the pre-smoothing of the next V-cycle, launched before the test (both
-// sweeps in the two-sweep pass, or the first one): if the test stops the
-// solve, that output (in y) is unused and x is untouched.
-int mg_solve_fp64(nyl_ctx *c, nyl_mg_stats *st) {
+// ---- the solve loops ---------------------------------------------------------
+// mgfor tests the residual after every V-cycle (core/mgfor/solvers.f90:8-33).
+// Waiting for each test on the host left the GPU idle for 10 to 20 us per
+// V-cycle.  Here the tests run on the device (CtlArgs): the V-cycles that the
+// last solve at the same place of a step needed are enqueued without a wait,
+// and one that follows the stopping test leaves the solution as it is (its
+// last pass is gated), so the result does not depend on the guess; the host
+// reads the sums of all tests once and takes the same decisions from them.
+// When the guess was too low, V-cycles follow one at a time.
+
+// mixed: squared reduction of one inner solve, its most V-cycles (see mg_solve_mixed)
+constexpr double kInnerRed2 = 1e-6;
+constexpr int kInnerMax = 8;
+
+CtlArgs ctl_args(nyl_ctx *c, int kind, int np) {
+    CtlArgs a = {};
+    a.ctl = F<MGCtl>(c, c->ctl);
+    a.partials = F<double>(c, c->partials);
+    a.np = np;
+    a.kind = kind;
+    a.slot = -1;
+    a.tol = c->d.mg_tol;
+    a.ncell = cells(c->lev[0].g);
+    a.inner_red = kInnerRed2;
+    a.inner_max = kInnerMax;
+    return a;
+}
+
+// publish the first n sums of the tests with this launch
+void ctl_publish(nyl_ctx *c, CtlArgs &a, int n) {
+    a.dst = c->host_dev + kHostCtl;
+    a.flag = reinterpret_cast<uint32_t *>(c->host_dev + 8);
+    a.seq = ++c->pub_seq;
+    a.nhist = n;
+}
+
+// the published results: normb and the sums of the tests
+int ctl_read(nyl_ctx *c, double *normb, double *hist, int n) {
+    int rc = wait_published(c, c->pub_seq);
+    if (rc) return rc;
+    const volatile double *v = c->host_out + kHostCtl;
+    *normb = v[0];
+    for (int q = 0; q < n; q++) hist[q] = v[2 + q];
+    return NYL_OK;
+}
+
+// most tests between two reads
+constexpr int kMaxAhead = CTL_HIST - 8;
+
+int known(int pred, int other) { return pred >= 0 ? pred : other; }
+
+// core/mgfor/solvers.f90:8-33 with normresidual (core/mgfor/operators.f90:81-96)
+int mg_solve_fp64(nyl_ctx *c, nyl_mg_stats *st, int site) {
     Level &f = c->lev[0];
-    double *part = F<double>(c, c->partials), *res_dev = F<double>(c, c->result);
-    const bool spec = sweep25_fits(f.g) && sweep25_blocks(f.g) <= NYL_RED_BLOCKS;
-    const bool spec2 = spec2_fits(c);
+    const int maxite = c->d.mg_maxite > 1 ? c->d.mg_maxite : 1;   // one V-cycle at least
+    const int *gate = &F<MGCtl>(c, c->ctl)->stop;
     int rc;
-    double normb, rn, res;
-    arm_publish(c, 1);
-    HIPCHK(launch_norm2<double>(f.g, F<double>(c, f.b), part, res_dev, c->stream));
-    if ((rc = read_result(c, &normb))) return rc;
-    int pending = 0;   // pre-smoothing sweeps of the next V-cycle already done
-    auto normresidual = [&](double *out) -> int {
-        pending = 0;
-        if (normb > 0.0) {
-            arm_publish(c, 1);
-            if (spec2) {
-                LAUNCH(NYL_K_MG_SWEEP2 | kFineLevel, 3 * cells(f.g) * sizeof(double),
-                       launch_mg_sweep2x25<double>(f.g, F<double>(c, f.x), F<double>(c, f.y),
-                                                   F<double>(c, f.b), c->d.mg_omega, c->tabs,
-                                                   c->stream, nullptr, part, res_dev));
-                pending = 2;
-            } else if (spec) {
-                LAUNCH(NYL_K_MG_SWEEP | kFineLevel, 3 * cells(f.g) * sizeof(double),
-                       launch_mg_sweep25<double>(f.g, F<double>(c, f.x), F<double>(c, f.y),
-                                                 F<double>(c, f.b), c->d.mg_omega, c->tabs,
-                                                 part, res_dev, c->stream));
-                pending = 1;
-            } else {
-                LAUNCH(NYL_K_RESNORM, 2 * cells(f.g) * sizeof(double),
-                       launch_resnorm2<double>(f.g, F<double>(c, f.x), F<double>(c, f.b), c->tabs,
-                                               part, res_dev, c->stream));
-            }
-            int r2 = read_result(c, &rn);
-            if (r2) return r2;
-            *out = rn / normb;
-        } else {
-            *out = 0.0;
-        }
-        return NYL_OK;
-    };
-    if ((rc = normresidual(&res))) return rc;
-    int nite = 0;
+    HIPCHK(launch_norm2<double>(f.g, F<double>(c, f.b), F<double>(c, c->partials), nullptr,
+                                c->stream));
+    HIPCHK(launch_ctl(ctl_args(c, CTL_NORMB, red_blocks((int64_t)cells(f.g))), c->stream));
+    double normb = 0.0, res = 0.0, hist[CTL_HIST];
+    int done = 0;    // V-cycles enqueued
+    int guess = known(c->pred[site][0], known(c->pred[0][0], 0));
+    bool pre = false;   // the sweeps (and test) of V-cycle done + 1 are enqueued
     for (;;) {
-        if (res < c->d.mg_tol) break;
-        if ((rc = vcycle(c, pending))) return rc;
-        nite = nite + 1;
-        if (nite >= c->d.mg_maxite) break;
-        if ((rc = normresidual(&res))) return rc;
+        const int first = done;   // V-cycles before the first test of this round
+        int nt = 0;               // tests of this round
+        const int to = std::min(std::min(guess, maxite), first + kMaxAhead);
+        while (done < to) {
+            CtlArgs t;
+            if (!pre) {
+                int np = 0;
+                if ((rc = pre_smooth(c, false, &np))) return rc;
+                t = ctl_args(c, CTL_TEST, np);
+                t.slot = nt++;
+            }
+            if ((rc = coarse_levels(c, pre ? nullptr : &t))) return rc;
+            if ((rc = level_up(c, 0, gate))) return rc;
+            pre = false;
+            done++;
+        }
+        CtlArgs t = ctl_args(c, CTL_NONE, 0);
+        if (done < maxite) {
+            // the test after the last V-cycle: the norm alone where the solve
+            // is expected to stop, else with the next V-cycle's sweeps
+            int np = 0;
+            const bool ends = first == 0 && done > 0;
+            if (ends) rc = resid_norm<double>(c, &np);
+            else rc = pre_smooth(c, false, &np);
+            if (rc) return rc;
+            pre = !ends;
+            t = ctl_args(c, CTL_TEST, np);
+            t.slot = nt++;
+        }
+        ctl_publish(c, t, nt);
+        HIPCHK(launch_ctl(t, c->stream));
+        if ((rc = ctl_read(c, &normb, hist, nt))) return rc;
+        // the tests in order: test q follows V-cycle first + q (the first round
+        // and those after a norm), or first + 1 + q when the round began with
+        // the V-cycle of a test already read
+        const int tests_from = done < maxite ? done - (nt - 1) : done - nt;
+        int stop = -1;
+        for (int q = 0; q < nt && stop < 0; q++) {
+            res = normb > 0.0 ? hist[q] / normb : 0.0;
+            if (res < c->d.mg_tol) stop = tests_from + q;
+        }
+        if (stop >= 0) {
+            done = stop;
+            break;
+        }
+        if (done >= maxite) break;
+        guess = done + 1;
     }
-    fill_stats(c, st, nite, res, normb);
+    c->pred[site][0] = done;
+    fill_stats(c, st, done, res, normb);
     return NYL_OK;
 }
 
@@ -799,101 +770,160 @@ int mg_solve_fp64(nyl_ctx *c, nyl_mg_stats *st) {
 // residual against kInnerRed2*|r|^2 instead and runs at most kInnerMax
 // V-cycles; the FP64 residual decides.  At mgfor's tolerance (1e-6) the
 // tolerance is the target and the V-cycle count is that of the FP64 solve.
-constexpr double kInnerRed2 = 1e-6;   // squared reduction of one inner solve
-constexpr int kInnerMax = 8;
-int mg_solve_mixed(nyl_ctx *c, nyl_mg_stats *st) {
+// Each outer step is enqueued whole, its V-cycles as guessed, with the add
+// and the next FP64 residual: the add is gated by the inner loop's stop, so
+// that a guess that was too low leaves x, and the next residual, as they
+// were.
+int mg_solve_mixed(nyl_ctx *c, nyl_mg_stats *st, int site) {
     Level &f = c->lev[0];
-    double *part = F<double>(c, c->partials), *res_dev = F<double>(c, c->result);
+    const int maxite = c->d.mg_maxite > 1 ? c->d.mg_maxite : 1;
+    MGCtl *ctl = F<MGCtl>(c, c->ctl);
     double *xo = F<double>(c, c->mgx), *bo = F<double>(c, c->mgb);
-    float *e = F<float>(c, f.x), *r = F<float>(c, f.b), *y = F<float>(c, f.y);
-    const bool spec = sweep25_fits(f.g) && sweep25_blocks(f.g) <= NYL_RED_BLOCKS;
-    const bool spec2 = spec2_fits(c);
+    float *e = F<float>(c, f.x);
+    const double ncell = cells(f.g), tol = c->d.mg_tol;
     int rc;
-    double rn, res;
-    // sum of b and of b**2 in FP64: the mean to remove and the norm of b - mean
-    double s2[2];
-    arm_publish(c, 2);
-    HIPCHK(launch_sum_sumsq(f.g, bo, part, res_dev, c->stream));
-    if ((rc = read_results(c, s2, 2))) return rc;
-    const double ncell = cells(f.g);
-    const double shift = s2[0] / ncell;
-    double normb = s2[1] - ncell * shift * shift;
-    if (normb < 0.0) normb = 0.0;
-    // FP64 residual of x into r (and the first sweep from e = 0 into y)
-    auto outer = [&](double *out) -> int {
-        if (normb > 0.0) {
-            arm_publish(c, 1);
-            LAUNCH(NYL_K_RESNORM, (2 * sizeof(double) + 2 * sizeof(float)) * cells(f.g),
-                   launch_mg_outer_resid<float>(f.g, xo, bo, shift, r, spec2 ? nullptr : y,
-                                                c->d.mg_omega, c->tabs, part, res_dev,
-                                                c->stream, false));
-            int r2 = read_result(c, &rn);
-            if (r2) return r2;
-            *out = rn / normb;
-        } else {
-            *out = 0.0;
-        }
+    HIPCHK(launch_sum_sumsq(f.g, bo, F<double>(c, c->partials), c->stream));
+    HIPCHK(launch_ctl(ctl_args(c, CTL_SHIFT, sumsq_blocks((int64_t)ncell)), c->stream));
+    // FP64 residual of x into r, its test into hist[slot]
+    auto outer = [&](int slot, bool publish) -> int {
+        MarchArgs<double, double> a = {};
+        a.g = a.gc = f.g;
+        a.src = xo;
+        a.b = bo;
+        a.tab = c->tabs;
+        a.partials = F<double>(c, c->partials);
+        a.rout = F<float>(c, f.b);
+        a.shift = &ctl->shift;
+        LAUNCH(NYL_K_RESNORM, (2 * sizeof(double) + sizeof(float)) * ncell,
+               launch_march_outer(a, c->stream));
+        CtlArgs t = ctl_args(c, CTL_OUTER, march_grid(f.g, sizeof(double), false).blocks());
+        t.slot = slot;
+        if (publish) ctl_publish(c, t, slot + 1);
+        HIPCHK(launch_ctl(t, c->stream));
         return NYL_OK;
     };
-    // FP32 residual r - A e (speculative pre-smoothing of the next V-cycle:
-    // both sweeps into y, or the first)
-    auto inner = [&](double *out) -> int {
-        arm_publish(c, 1);
-        if (spec2) {
-            LAUNCH(NYL_K_MG_SWEEP2 | kFineLevel, 3 * cells(f.g) * sizeof(float),
-                   launch_mg_sweep2x25<float>(f.g, e, y, r, c->d.mg_omega, c->tabs, c->stream,
-                                              nullptr, part, res_dev));
-        } else if (spec) {
-            LAUNCH(NYL_K_MG_SWEEP | kFineLevel, 3 * cells(f.g) * sizeof(float),
-                   launch_mg_sweep25<float>(f.g, e, y, r, c->d.mg_omega, c->tabs, part, res_dev,
-                                            c->stream));
-        } else {
-            LAUNCH(NYL_K_RESNORM, 2 * cells(f.g) * sizeof(float),
-                   launch_resnorm2<float>(f.g, e, r, c->tabs, part, res_dev, c->stream));
-        }
-        int r2 = read_result(c, &rn);
-        if (r2) return r2;
-        *out = rn / normb;
+    auto add = [&](const int *gate) -> int {
+        LAUNCH(NYL_K_MG_UPDATE, (2 * sizeof(double) + sizeof(float)) * ncell,
+               launch_add_correction<float>(f.g, xo, e, gate, c->stream));
         return NYL_OK;
     };
-    if ((rc = outer(&res))) return rc;
-    // mgfor's loop shape (core/mgfor/solvers.f90:22-29): test, V-cycle,
-    // count, stop at maxite (so maxite = 0 still runs one V-cycle)
+    double normb = 0.0, res = 0.0, hist[CTL_HIST];
+    auto relative = [&](double s) { return normb > 0.0 ? s / normb : 0.0; };
+    // the first outer residual is read with the first outer step's tests,
+    // unless the solve is expected to stop at it
+    const int g0 = known(c->pred[site][0], known(c->pred[0][0], 1));
+    bool have_res = g0 == 0;
+    if ((rc = outer(0, have_res))) return rc;
+    if (have_res) {
+        if ((rc = ctl_read(c, &normb, hist, 1))) return rc;
+        res = relative(hist[0]);
+    }
     int nite = 0;
     bool at_max = false;
-    while (!(res < c->d.mg_tol) && !at_max) {
-        // both pre-smoothing sweeps from e = 0 in one pass into y, or the first
-        // one (written by the outer residual)
-        int pending = 1;
-        if (spec2) {
-            // (not in the fine-level class of the roofline: it reads one field)
-            LAUNCH(NYL_K_MG_SWEEP2, 2 * cells(f.g) * sizeof(float),
-                   launch_mg_sweep2x25<float>(f.g, nullptr, y, r, c->d.mg_omega, c->tabs,
-                                              c->stream));
-            pending = 2;
+    for (int j = 0;; j++) {
+        if (have_res && (res < tol || at_max)) {
+            if (j < kPredOuter) c->pred[site][j] = 0;
+            break;
         }
-        const bool rel = res * kInnerRed2 > c->d.mg_tol;
-        const double target = rel ? res * kInnerRed2 : c->d.mg_tol;
-        for (int k = 1;; k++) {
-            if ((rc = vcycle(c, pending))) return rc;
-            nite = nite + 1;
-            at_max = nite >= c->d.mg_maxite;
-            if (at_max || (rel && k >= kInnerMax)) break;
-            double rin;
-            if ((rc = inner(&rin))) return rc;
-            pending = spec2 ? 2 : spec ? 1 : 0;
-            if (rin < target) break;
+        const int jp = std::min(j, kPredOuter - 1);
+        int guess = known(c->pred[site][jp], known(c->pred[0][jp], 1));
+        if (guess < 1) guess = 1;
+        const bool sure = c->pred[site][jp] > 0 || c->pred[0][jp] > 0;
+        int k = 0;            // V-cycles of this inner loop enqueued
+        bool open = true;     // the inner loop has not stopped
+        bool pre = false;     // the sweeps (and test) of V-cycle k + 1 are enqueued
+        bool first = true, added = false;
+        while (open) {
+            int nt = j == 0 && !have_res ? 1 : 0;   // hist[0] is the first outer residual
+            const int in0 = nt;
+            int kq[CTL_HIST];                       // V-cycles before each test
+            const int to = std::min(std::min(std::max(guess, k + 1), maxite - nite), k + kMaxAhead);
+            while (k < to) {
+                CtlArgs t;
+                bool test = false;
+                if (!pre) {
+                    int np = 0;
+                    if ((rc = pre_smooth(c, k == 0, &np))) return rc;
+                    if (k > 0) {
+                        test = true;
+                        t = ctl_args(c, CTL_INNER, np);
+                        t.k = k;
+                        kq[nt] = k;
+                        t.slot = nt++;
+                    }
+                }
+                if ((rc = coarse_levels(c, test ? &t : nullptr))) return rc;
+                if ((rc = level_up(c, 0, &ctl->stop))) return rc;
+                pre = false;
+                k++;
+            }
+            const bool max_now = nite + k >= maxite;
+            const bool ends = max_now || (first && sure);   // expected to stop here
+            if (!max_now) {
+                int np = 0;
+                if (ends) rc = resid_norm<float>(c, &np);
+                else rc = pre_smooth(c, false, &np);
+                if (rc) return rc;
+                pre = !ends;
+                CtlArgs t = ctl_args(c, CTL_INNER, np);
+                t.k = k;
+                kq[nt] = k;
+                t.slot = nt++;
+                if (!ends) ctl_publish(c, t, nt);
+                HIPCHK(launch_ctl(t, c->stream));
+            }
+            int last = -1;   // hist entry of the next outer residual
+            if (ends) {
+                if ((rc = add(max_now ? &ctl->outer_stop : &ctl->no_add))) return rc;
+                last = nt++;
+                if ((rc = outer(last, true))) return rc;
+            }
+            if ((rc = ctl_read(c, &normb, hist, nt))) return rc;
+            if (!have_res) {
+                res = relative(hist[0]);
+                have_res = true;
+                if (res < tol) {   // nothing was to be done
+                    k = 0;
+                    open = false;
+                    break;
+                }
+            }
+            const bool rel = res * kInnerRed2 > tol;
+            const double target = rel ? res * kInnerRed2 : tol;
+            for (int q = in0; q < (last >= 0 ? last : nt) && open; q++) {
+                const double rin = relative(hist[q]);
+                if (rin < target || (rel && kq[q] >= kInnerMax)) {
+                    k = kq[q];
+                    open = false;
+                }
+            }
+            if (max_now) open = false;
+            if (!open && last >= 0) {
+                added = true;
+                res = relative(hist[last]);
+            }
+            first = false;
         }
-        LAUNCH(NYL_K_MG_UPDATE, (2 * sizeof(double) + sizeof(float)) * cells(f.g),
-               launch_add_correction<float>(f.g, xo, e, c->stream));
-        if ((rc = outer(&res))) return rc;
+        if (k == 0) {   // the first outer residual was below the tolerance
+            c->pred[site][0] = 0;
+            break;
+        }
+        nite += k;
+        at_max = nite >= maxite;
+        if (j < kPredOuter) c->pred[site][j] = k;
+        if (!added) {
+            if ((rc = add(nullptr)) || (rc = outer(0, true))) return rc;
+            if ((rc = ctl_read(c, &normb, hist, 1))) return rc;
+            res = relative(hist[0]);
+        }
     }
     fill_stats(c, st, nite, res, normb);
     return NYL_OK;
 }
 
-int mg_solve(nyl_ctx *c, nyl_mg_stats *st) {
-    return c->mixed ? mg_solve_mixed(c, st) : mg_solve_fp64(c, st);
+// site: the place of the solve in a step (1..3), 0 outside a step
+int mg_solve(nyl_ctx *c, nyl_mg_stats *st, int site) {
+    return c->mixed ? mg_solve_mixed(c, st, site) : mg_solve_fp64(c, st, site);
 }
 
 template <typename T>
@@ -950,10 +980,10 @@ int apply_op(nyl_ctx *c, int op) {
 
 // core/model_les.py:97-127 (halo fills are implicit in the wrapped reads)
 template <typename T>
-int diagnose_t(nyl_ctx *c, nyl_mg_stats *st) {
+int diagnose_t(nyl_ctx *c, nyl_mg_stats *st, int site) {
     int rc;
     if ((rc = apply_op_t<T>(c, NYL_OP_DIV))) return rc;
-    if ((rc = mg_solve(c, st))) return rc;
+    if ((rc = mg_solve(c, st, site))) return rc;
     if ((rc = apply_op_t<T>(c, NYL_OP_CORRECT))) return rc;
     // vorticity and ke (not in the linear model, core/model_les.py:122-127);
     // U is not stored (the stage kernel recomputes it, NYL_OP_U_FROM_U fills
@@ -964,8 +994,8 @@ int diagnose_t(nyl_ctx *c, nyl_mg_stats *st) {
     return NYL_OK;
 }
 
-int diagnose(nyl_ctx *c, nyl_mg_stats *st) {
-    return c->mixed ? diagnose_t<float>(c, st) : diagnose_t<double>(c, st);
+int diagnose(nyl_ctx *c, nyl_mg_stats *st, int site) {
+    return c->mixed ? diagnose_t<float>(c, st, site) : diagnose_t<double>(c, st, site);
 }
 
 // words of HBM traffic per cell of each stage-kernel mode: reads b,u,v,w,
@@ -1174,16 +1204,16 @@ int nyl_ctx_create(const nyl_desc *desc, nyl_ctx **out) {
     if (rc) { delete c; return rc; }
     build_tabs(c->tabs);
     build_layout(c);
+    c->t0 = cycle_first(c);
+    for (int q = 0; q < kSites; q++)
+        for (int j = 0; j < kPredOuter; j++) c->pred[q][j] = -1;
     c->stream = nullptr;
-    c->use_graphs = 1;
-    c->g_coarse = nullptr;
     *out = c;
     return NYL_OK;
 }
 
 int nyl_ctx_destroy(nyl_ctx *c) {
     if (!c) return NYL_OK;
-    drop_graphs(c);
     for (int q = 0; q < c->prof_nev; q++) (void)hipEventDestroy(c->prof_ev[q]);
     if (c->host_out) (void)hipHostFree(c->host_out);
     delete c;
@@ -1203,21 +1233,19 @@ int nyl_set_stream(nyl_ctx *c, void *stream) {
 }
 
 int nyl_set_graphs(nyl_ctx *c, int on) {
+    (void)on;   // a step enqueues its launches ahead of the GPU: nothing is replayed
     if (!c) return fail(NYL_E_ARG, "null context");
-    c->use_graphs = on ? 1 : 0;
-    if (!on) drop_graphs(c);
     return NYL_OK;
 }
 
 int nyl_bind_workspace(nyl_ctx *c, void *dptr, uint64_t bytes) {
     if (!c || !dptr) return fail(NYL_E_ARG, "null argument");
-    drop_graphs(c);
     if (bytes < c->ws_bytes)
         return fail(NYL_E_ARG, "workspace of %llu bytes is smaller than the %llu needed",
                     (unsigned long long)bytes, (unsigned long long)c->ws_bytes);
     if (((uintptr_t)dptr) & 255) return fail(NYL_E_ARG, "workspace must be 256-byte aligned");
     if (!c->host_out) {
-        HIPCHK(hipHostMalloc((void **)&c->host_out, 16 * sizeof(double),
+        HIPCHK(hipHostMalloc((void **)&c->host_out, (kHostCtl + 2 + CTL_HIST) * sizeof(double),
                              hipHostMallocMapped | hipHostMallocCoherent));
         HIPCHK(hipHostGetDevicePointer((void **)&c->host_dev, c->host_out, 0));
         *reinterpret_cast<volatile uint32_t *>(c->host_out + 8) = 0;
@@ -1225,11 +1253,15 @@ int nyl_bind_workspace(nyl_ctx *c, void *dptr, uint64_t bytes) {
     }
     c->ws = (char *)dptr;
     HIPCHK(launch_fill((double *)c->ws, (int64_t)(c->ws_bytes / sizeof(double)), 0.0, c->stream));
+    HIPCHK(hipMemcpyAsync(c->ws + c->ent, c->cyc_ent, sizeof(c->cyc_ent), hipMemcpyHostToDevice,
+                          c->stream));
+    c->cyc.ent = F<CycleEnt>(c, c->ent);
     if (c->exact) {
         std::vector<double> tab(coarse_table_doubles());
         coarse_tables(c->lev[c->nlev - 1].g, tab.data());
         HIPCHK(hipMemcpyAsync(c->ws + c->cs_tab, tab.data(), tab.size() * sizeof(double),
                               hipMemcpyHostToDevice, c->stream));
+        c->cyc.etab = F<double>(c, c->cs_tab);
     }
     HIPCHK(hipStreamSynchronize(c->stream));
     c->cur = 0;
@@ -1318,7 +1350,7 @@ int nyl_rk3_stage(nyl_ctx *c, int st, double coef) {
 int nyl_diagnose(nyl_ctx *c, nyl_mg_stats *st) {
     int rc = check_ready(c);
     if (rc) return rc;
-    return diagnose(c, st);
+    return diagnose(c, st, 0);
 }
 
 int nyl_step_rk3(nyl_ctx *c, double dt, nyl_mg_stats *st) {
@@ -1329,7 +1361,7 @@ int nyl_step_rk3(nyl_ctx *c, double dt, nyl_mg_stats *st) {
     const double coef[3] = {dt, dt / 4., dt / 12.};
     for (int k = 1; k <= 3; k++) {
         if ((rc = stage(c, k, coef[k - 1], 0.0, k == 3))) return rc;
-        if ((rc = diagnose(c, &s1))) return rc;
+        if ((rc = diagnose(c, &s1, k))) return rc;
         acc.nite += s1.nite;
         acc.res = s1.res;
         acc.normb = s1.normb;
@@ -1343,7 +1375,7 @@ int nyl_step_ef(nyl_ctx *c, double dt, nyl_mg_stats *st) {
     int rc = check_ready(c);
     if (rc) return rc;
     if ((rc = stage(c, 1, dt, 0.0, true))) return rc;
-    return diagnose(c, st);
+    return diagnose(c, st, 1);
 }
 
 int nyl_step_lfam3(nyl_ctx *c, double dt, nyl_mg_stats *st) {
@@ -1352,16 +1384,16 @@ int nyl_step_lfam3(nyl_ctx *c, double dt, nyl_mg_stats *st) {
     if (c->lf_first) {
         if ((rc = stage(c, 6, dt, 0.0, false))) return rc;
         c->lf_first = 0;
-        return diagnose(c, st);
+        return diagnose(c, st, 1);
     }
     nyl_mg_stats s1, s2;
     // predictor: the current buffer keeps sn, the next one receives s
     if ((rc = stage(c, 4, 0.0, 2. * dt, false))) return rc;
-    if ((rc = diagnose(c, &s1))) return rc;
+    if ((rc = diagnose(c, &s1, 1))) return rc;
     // corrector: rhs at n+1/2, then s = sn + dt*ds written over sn
     if ((rc = stage(c, 5, dt, 0.0, true))) return rc;
     c->cur = 1 - c->cur;
-    if ((rc = diagnose(c, &s2))) return rc;
+    if ((rc = diagnose(c, &s2, 2))) return rc;
     if (st) {
         *st = s2;
         st->nite = s1.nite + s2.nite;
@@ -1378,7 +1410,7 @@ int nyl_lfam3_reset(nyl_ctx *c) {
 int nyl_mg_solve(nyl_ctx *c, nyl_mg_stats *st) {
     int rc = check_ready(c);
     if (rc) return rc;
-    return mg_solve(c, st);
+    return mg_solve(c, st, 0);
 }
 
 int nyl_apply(nyl_ctx *c, int op) {
@@ -1449,8 +1481,7 @@ int nyl_debug_mg(nyl_ctx *c, int what) {
         if (what == 5 && sweep2x_blocks(f.g, 8) > NYL_RED_BLOCKS)
             return fail(NYL_E_SIZE, "too many blocks for the residual norm");
         HIPCHK(launch_mg_sweep2x25<double>(f.g, what == 6 ? nullptr : x, y, b, c->d.mg_omega,
-                                           c->tabs, c->stream, nullptr,
-                                           what == 5 ? part : nullptr,
+                                           c->tabs, c->stream, what == 5 ? part : nullptr,
                                            what == 5 ? res_dev : nullptr));
         break;
     default:

@@ -1,12 +1,15 @@
 // nyl_ctx.h -- the model context shared by the translation units of
 // libnyles_hip.so (not part of the public ABI).
 #pragma once
+#include "nyl_cycle.h"
 #include "nyl_internal.h"
 #include "../../include/nyles_hip.h"
 
 namespace nyl {
 
 constexpr int kMaxLevels = 32;
+constexpr int kSites = 4, kPredOuter = 8;
+constexpr int kHostCtl = 16;   // doubles of host_out before the solve's results
 
 struct Level {
     Geo g;
@@ -36,17 +39,24 @@ struct nyl_ctx {
     uint64_t ke, vor[3], uc[3], p;
     uint64_t mgx, mgb;       // FP64 solution and right-hand side of the projection
     uint64_t partials, result;
+    uint64_t ctl;            // MGCtl: the stop rule of a solve on the device
     uint64_t ws_bytes;
     int cur;                 // which state buffer is current
     char *ws;
     hipStream_t stream;
-    double *host_out;        // pinned host memory, coherent: 8 result doubles + a sequence flag
+    double *host_out;        // pinned host memory, coherent: 8 result doubles, a sequence flag,
+                             // and from kHostCtl on the published results of a solve
     double *host_dev;        // host_out as the device addresses it
     uint32_t pub_seq;        // last published result sequence number
     int total_cycles;
-    // the V-cycle below level 1, replayed from a hipGraph (captured on first use)
-    int use_graphs;
-    hipGraphExec_t g_coarse;
+    // V-cycles the last solves needed, by the place of the solve in a step
+    // (0: outside a step) and, in mixed precision, by outer step: how many
+    // the next one enqueues before it reads their tests (-1: not known yet)
+    int pred[nyl::kSites][nyl::kPredOuter];
+    int t0;                  // first level of the single-workgroup cycle (nlev: none)
+    nyl::CycleArgs cyc;
+    nyl::CycleEnt cyc_ent[CYC_ENT];
+    uint64_t ent;            // cyc_ent in the workspace
     // HIP-event timing of one kernel class (nyl_prof_start / nyl_prof_stop)
     int prof_cls;
     int prof_used;

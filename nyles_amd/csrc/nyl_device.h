@@ -243,6 +243,23 @@ __device__ __forceinline__ void store_stream(T *p, T v) {
 }
 
 // ---------------------------------------------------------------------------
+// Block sums of the deterministic reductions.
+#define RED_T 256
+
+// Fixed-order tree over the RED_T threads of a block; tid is the linear
+// thread index (blocks may be 2-D).
+__device__ __forceinline__ void block_sum_store(double v, double *out, int tid) {
+    __shared__ double sh[RED_T];
+    sh[tid] = v;
+    __syncthreads();
+    for (int s = RED_T / 2; s > 0; s >>= 1) {
+        if (tid < s) sh[tid] = sh[tid] + sh[tid + s];
+        __syncthreads();
+    }
+    if (tid == 0) *out = sh[0];
+}
+
+// ---------------------------------------------------------------------------
 // Ensemble batches: the item (one per member) owning flattened block `blk`
 // (items sorted by h.start, h.start of the first item is 0).
 template <typename I>

@@ -193,21 +193,15 @@ template <typename Tf, typename Tc>
 hipError_t launch_mg_prolong(const Geo &gf, const Geo &gc, Tf *xf, const Tc *xc,
                              const MGTabs &tab, hipStream_t s);
 
-// mixed precision defect correction: outer FP64 residual of x (b - shift)
-// into the inner right-hand side r and the inner first sweep y, with the sum
-// of r**2 in dev_out[0] and, with_bsq (only where outer_bsq_fits), the sum of
-// b**2 in dev_out[1]; x += e
+// whether the mixed solve takes a level-1 grid of this width
 bool outer_resid_fits(const Geo &g);
-bool outer_bsq_fits(const Geo &g);
+// x += e, unless *gate is non-zero (gate null: always)
 template <typename TI>
-hipError_t launch_mg_outer_resid(const Geo &g, const double *x, const double *b, double shift,
-                                 TI *r, TI *y, double omega, const MGTabs &tab, double *partials,
-                                 double *dev_out, hipStream_t s, bool with_bsq);
-template <typename TI>
-hipError_t launch_add_correction(const Geo &g, double *x, const TI *e, hipStream_t s);
-// dev_out[0] = sum v, dev_out[1] = sum v**2
-hipError_t launch_sum_sumsq(const Geo &g, const double *v, double *partials, double *dev_out,
-                            hipStream_t s);
+hipError_t launch_add_correction(const Geo &g, double *x, const TI *e, const int *gate,
+                                 hipStream_t s);
+// partial sums of v (sumsq_blocks of them) and of v**2 (as many, after them)
+int sumsq_blocks(int64_t ncell);
+hipError_t launch_sum_sumsq(const Geo &g, const double *v, double *partials, hipStream_t s);
 // dev_out[0] = sum of the FP64 kinetic-energy field of u, v, w
 template <typename T>
 hipError_t launch_kesum(const Geo &g, const T *u, const T *v, const T *w, double idx2,
@@ -219,14 +213,10 @@ hipError_t launch_kesum(const Geo &g, const T *u, const T *v, const T *w, double
 // dev_out (needs sweep25_blocks(g) <= NYL_RED_BLOCKS partials).
 bool sweep25_fits(const Geo &g);
 int sweep25_blocks(const Geo &g);
-// gc/xc non-null: the sweep reads src + prolongation of xc (level gc) in
-// place of src (fused k_mg_prolong; src itself is not modified).
-// addx non-null: the result is added to the FP64 addx instead of stored.
 template <typename T>
 hipError_t launch_mg_sweep25(const Geo &g, const T *src, T *dst, const T *b, double omega,
                              const MGTabs &tab, double *partials, double *dev_out,
-                             hipStream_t s, const Geo *gc = nullptr, const T *xc = nullptr,
-                             double *addx = nullptr);
+                             hipStream_t s);
 // residual + restriction and prolongation with 2.5-D tiling (fine level
 // with sweep25_fits and even nz)
 bool restrict25_fits(const Geo &g);
@@ -268,17 +258,15 @@ inline uint64_t tail_layout(TailArgs &a, int es, int esc) {
     }
     return o;
 }
-template <typename T, typename TC>
-hipError_t launch_mg_tail(const TailArgs &a, hipStream_t s);
-
 // two consecutive tiled sweeps src -> (tmp) -> dst in one pass (src != dst;
-// src null: from src = 0, nothing read); addx: the result added to that
-// FP64 field instead of stored; partials: also the residual norm of src into
-// dev_out (needs sweep2x_blocks(g, es) <= NYL_RED_BLOCKS partials)
+// src null: from src = 0, nothing read); partials: also the block sums of the
+// squared residual of src (sweep2x_blocks(g, es) <= NYL_RED_BLOCKS of them),
+// summed into dev_out when that is given; gate: nothing is done when *gate
+// is non-zero
 template <typename T>
 hipError_t launch_mg_sweep2x25(const Geo &g, const T *src, T *dst, const T *b, double omega,
-                               const MGTabs &tab, hipStream_t s, double *addx = nullptr,
-                               double *partials = nullptr, double *dev_out = nullptr);
+                               const MGTabs &tab, hipStream_t s, double *partials = nullptr,
+                               double *dev_out = nullptr, const int *gate = nullptr);
 int sweep2x_blocks(const Geo &g, int es);
 template <typename Tf, typename Tc>
 hipError_t launch_mg_restrict25(const Geo &gf, const Geo &gc, const Tf *x, const Tf *b, Tc *bc,
@@ -386,8 +374,11 @@ hipError_t launch_b_coarse(const CoarseItem *items, int n, int64_t nblk, int pas
 // mode 0: acc = 0; mode 1: acc += nite
 hipError_t launch_b_acc(int n, const BMG &mg, int mode, hipStream_t s);
 
-// reductions: partials then one final block; result written to dev_out[0]
+// reductions: partials (red_blocks of them) then one final block; result
+// written to dev_out[0] (launch_norm2, launch_resnorm2: dev_out null leaves
+// the partials)
 #define NYL_RED_BLOCKS 16384
+int red_blocks(int64_t ncell);
 template <typename T>
 hipError_t launch_norm2(const Geo &g, const T *v, double *partials, double *dev_out,
                         hipStream_t s);

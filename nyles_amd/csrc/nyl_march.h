@@ -1,0 +1,59 @@
+// nyl_march.h -- one pass over a multigrid level (k_mg_march): arguments and
+// launchers shared by nyl_march.hip and the host code.
+#pragma once
+#include "nyl_internal.h"
+
+namespace nyl {
+
+// what a pass reads as the solution of its level
+enum MarchSrc {
+    MS_FIELD = 0,   // src
+    MS_ZERO = 1,    // zero (src is not read)
+    MS_PROLONG = 2  // src + the prolongation of the coarse level's xc
+};
+
+template <typename T, typename TC>
+struct MarchArgs {
+    Geo g, gc;              // the level, the next coarser one
+    const T *src, *b;
+    T *dst;                 // the result of the last sweep (src != dst)
+    const TC *xc;           // MS_PROLONG: the coarse correction
+    TC *bc, *yc;            // restriction: coarse right-hand side, its first sweep from zero
+    double omega;
+    MGTabs tab;
+    double *partials;       // one per block: sum of the input's squared residuals
+    float *rout;            // outer residual: r of the input, in the inner precision
+    const double *shift;    // outer residual: subtracted from b (null: 0)
+    const int *gate;        // the pass does nothing when *gate != 0 (null: always runs)
+    int kz;                 // planes per block
+};
+
+// Blocks of a pass over a level, and their march length.  even: the march
+// works on plane pairs (restriction or prolongation).
+struct MarchGrid {
+    int tx, bx, by, bz, kz;
+    int blocks() const { return bx * by * bz; }
+};
+MarchGrid march_grid(const Geo &g, int es, bool even);
+
+// two sweeps src + P(xc) -> dst
+template <typename T, typename TC>
+hipError_t launch_march_up(const MarchArgs<T, TC> &a, hipStream_t s);
+// one sweep src -> dst, then residual and restriction of dst into bc and yc
+template <typename T, typename TC>
+hipError_t launch_march_down(const MarchArgs<T, TC> &a, hipStream_t s);
+// two sweeps src (null: zero) -> dst; partials non-null: the residual norm of
+// src; bc, yc non-null: also the residual and restriction of dst
+template <typename T, typename TC>
+hipError_t launch_march_pre(const MarchArgs<T, TC> &a, hipStream_t s);
+// residual and restriction of src into bc and yc
+template <typename T, typename TC>
+hipError_t launch_march_restrict(const MarchArgs<T, TC> &a, hipStream_t s);
+// the residual norm of src alone
+template <typename T>
+hipError_t launch_march_norm(const MarchArgs<T, T> &a, hipStream_t s);
+// the mixed solve's FP64 residual (b - shift) - A src: its norm, and its
+// values in FP32 into rout
+hipError_t launch_march_outer(const MarchArgs<double, double> &a, hipStream_t s);
+
+}  // namespace nyl

@@ -1,0 +1,518 @@
+// nyl_march.hip -- the passes of a multigrid V-cycle over one level: sweeps,
+// prolongation, residual and restriction fused into one 2.5-D march, for
+// levels of any size.
+#include "nyl_march.h"
+
+#include <type_traits>
+
+namespace nyl {
+
+// periodic wrap of any offset
+__device__ __forceinline__ int wrap_any(int m, int n) {
+    const int r = m % n;
+    return r < 0 ? r + n : r;
+}
+
+// A block owns a TX x TY tile of columns (TY = 512 / TX) and marches up kz
+// planes.  Thread (tx, ty) owns rows 2 ty and 2 ty + 1 of column tx, and one
+// cell of each of the R rings around the tile (R = the number of in-plane
+// stencils applied one after another: sweeps, and the residual of a
+// restriction).  Stage 0 is the input, stage s the s-th sweep; stage s is
+// evaluated on the tile and its first R - s rings.  A position keeps the
+// planes m-1, m, m+1 of a stage in registers (z neighbours) and its in-plane
+// neighbours come from LDS, two slots per stage: in step p the block stores
+// plane p of stage 0, passes one barrier, evaluates stage 1 of plane p, stage
+// 2 of plane p-1 (whose neighbours were stored in step p-1) and the residual
+// one plane later still.  A slot is written again two steps after it was
+// read, with a barrier between.  Loads are issued two steps ahead of their
+// use, from valid addresses (clamped or wrapped), and values outside a wall
+// are replaced by zero when they enter the window.
+// PROLONG: the input is src + P(xc); a coarse plane is staged in LDS every
+// second step and every position keeps the planar sums (9,3,3,1) of the two
+// latest ones, so each is evaluated once for the two fine planes that use it.
+// Every value is the per-cell kernel's expression (sweep_cell, residual_at,
+// restrict_cell, prolong_term) in its order, so the results are bitwise those
+// of the separate launches.
+template <typename T, typename TC, int TX, int SRC, int NSW, bool RESN, bool RESTR, bool OUTER>
+__global__ __launch_bounds__(256) void k_mg_march(MarchArgs<T, TC> a) {
+    constexpr int TY = 512 / TX;
+    constexpr int R = RESTR ? NSW + 1 : (NSW > 0 ? NSW : 1);
+    constexpr int NP = 2 + R;                       // own cells, then one per ring
+    constexpr int N1 = NSW > 0 ? 1 + R : 0;         // positions of stage 1
+    constexpr int N2 = NSW == 2 ? R : 0;            // ... and of stage 2
+    constexpr int NB = NSW > 0 ? N1 : 2;            // positions that read b
+    constexpr int W0 = TX + 2 * R, H0 = TY + 2 * R;
+    constexpr int W1 = W0 - 2, H1 = H0 - 2, W2 = W0 - 4, H2 = H0 - 4;
+    constexpr bool LDS1 = NSW == 2 || (RESTR && NSW == 1), LDS2 = NSW == 2 && RESTR;
+    constexpr int CW = TX / 2 + 4, CH = TY / 2 + 4, NC = CW * CH;   // coarse footprint (R = 2)
+    constexpr int CR = (NC + 255) / 256;
+    __shared__ T s0[SRC == MS_ZERO ? 1 : 2 * W0 * H0];
+    __shared__ T s1[LDS1 ? 2 * W1 * H1 : 1];
+    __shared__ T s2[LDS2 ? 2 * W2 * H2 : 1];
+    __shared__ T sc[SRC == MS_PROLONG ? 3 * NC : 1];
+    __shared__ T sid[8], spc[8];
+    if (a.gate && *a.gate) return;
+    const Geo &g = a.g, &gc = a.gc;
+    const int tid = threadIdx.x, tx = tid % TX, ty = tid / TX;
+    const Blk3 bk = xcd_block();
+    const int i0 = bk.x * TX, j0 = bk.y * TY, k0 = bk.z * a.kz;
+    const int nz = g.nz, k1 = k0 + a.kz < nz ? k0 + a.kz : nz;
+    const bool pz = g.pz != 0;
+    const T om = T(a.omega), cff1 = T(1.0 - a.omega);
+    if (tid < 7) sid[tid] = T(a.tab.idiag[tid]);
+    if (tid < 8) spc[tid] = T(a.tab.pcoef[tid]);
+
+    // positions: in-plane offset, domain test, in-plane neighbour count, place
+    // in the stage-0 plane; own cells: also whether the cell is stored
+    int off[NP], nxy[NP], at[NP], ay[NP];
+    bool in[NP], has[NP], st[2];
+    int cb[NP], cdx[NP], cdy[NP], mxy[NP];          // PROLONG: coarse cell, its neighbours
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+        int lx, ly;
+        has[p] = true;
+        if (p < 2) {
+            lx = tx + R;
+            ly = 2 * ty + p + R;
+        } else {
+            const int q = p - 1, W = TX + 2 * q, H = TY + 2 * q;
+            // rings 1 and 3 belong to the first threads, ring 2 to the last
+            const int t = q == 2 ? 255 - tid : tid;
+            has[p] = t < 2 * W + 2 * (H - 2);
+            const int u = t - 2 * W;
+            lx = t < W ? t : (t < 2 * W ? t - W : ((u & 1) ? W - 1 : 0));
+            ly = t < W ? 0 : (t < 2 * W ? H - 1 : 1 + (u >> 1));
+            lx += R - q;
+            ly += R - q;
+            if (!has[p]) lx = ly = 0;
+        }
+        at[p] = ly * W0 + lx;
+        ay[p] = ly;
+        const int ui = i0 - R + lx, uj = j0 - R + ly;   // unwrapped
+        int gi = ui, gj = uj;
+        bool ok = has[p];
+        if (g.px) gi = wrap_any(ui, g.nx); else ok = ok && ui >= 0 && ui < g.nx;
+        if (g.py) gj = wrap_any(uj, g.ny); else ok = ok && uj >= 0 && uj < g.ny;
+        in[p] = ok;
+        off[p] = ok ? gj * (int)g.sy + gi : 0;
+        nxy[p] = (g.px || gi > 0) + (g.px || gi < g.nx - 1) + (g.py || gj > 0) +
+                 (g.py || gj < g.ny - 1);
+        if (!ok) nxy[p] = 0;
+        if (p < 2) st[p] = ok && ui < g.nx && uj < g.ny;
+        if (SRC == MS_PROLONG) {
+            const int ic = ui >> 1, jc = uj >> 1;
+            cdx[p] = (ui & 1) ? 1 : -1;
+            cdy[p] = (uj & 1) ? CW : -CW;
+            const int icn = ic + cdx[p], jcn = jc + ((uj & 1) ? 1 : -1);
+            mxy[p] = ((gc.px || (icn >= 0 && icn < gc.nx)) ? 1 : 0) +
+                     ((gc.py || (jcn >= 0 && jcn < gc.ny)) ? 2 : 0);
+            cb[p] = (jc - ((j0 >> 1) - 2)) * CW + ic - ((i0 >> 1) - 2);
+        }
+    }
+    __syncthreads();   // sid, spc
+    T id2[NP], pc1[NP];   // the coefficients of planes with both z neighbours
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+        id2[p] = sid[nxy[p] + 2];
+        if (SRC == MS_PROLONG) pc1[p] = spc[mxy[p] + 4];
+    }
+
+    auto zin = [&](int m) { return pz || (m >= 0 && m < nz); };
+    auto nzw = [&](int m) { return pz ? 2 : (m > 0) + (m < nz - 1); };
+    // a plane that can be loaded for plane m: the wrapped one, or the nearest
+    auto pl = [&](int m, int n, bool per) {
+        return per ? wrap_any(m, n) : (m < 0 ? 0 : (m < n ? m : n - 1));
+    };
+    auto next = [&](int q, int m, int n, bool per) {   // pl(m + 1) from q = pl(m)
+        return per ? (q + 1 == n ? 0 : q + 1) : (m + 1 < 0 ? 0 : (m + 1 < n ? m + 1 : n - 1));
+    };
+    auto ldx = [&](int q, T (&v)[NP]) {
+        if (SRC == MS_ZERO) return;
+        const T *s = a.src + (int64_t)q * g.sz;
+#pragma unroll
+        for (int p = 0; p < NP; p++) v[p] = s[off[p]];
+    };
+    auto ldb = [&](int q, T (&v)[NB]) {
+        const T *s = a.b + (int64_t)q * g.sz;
+#pragma unroll
+        for (int p = 0; p < NB; p++) v[p] = s[off[p]];
+    };
+
+    // ---- coarse planes (PROLONG)
+    int coff[CR];
+    bool cin[CR];
+    T A0[NP] = {}, A1[NP] = {}, craw[CR] = {};
+    if (SRC == MS_PROLONG) {
+#pragma unroll
+        for (int r = 0; r < CR; r++) {
+            const int t = tid + 256 * r;
+            const int lx = t % CW, ly = t / CW;
+            int gi = (i0 >> 1) - 2 + lx, gj = (j0 >> 1) - 2 + ly;
+            bool ok = t < NC;
+            if (gc.px) gi = wrap_any(gi, gc.nx); else ok = ok && gi >= 0 && gi < gc.nx;
+            if (gc.py) gj = wrap_any(gj, gc.ny); else ok = ok && gj >= 0 && gj < gc.ny;
+            cin[r] = ok;
+            coff[r] = ok ? gj * (int)gc.sy + gi : 0;
+        }
+    }
+    auto czin = [&](int m) { return pz || (m >= 0 && m < gc.nz); };
+    auto ldc = [&](int m) {
+        const TC *s = a.xc + (int64_t)pl(m, gc.nz, pz) * gc.sz;
+#pragma unroll
+        for (int r = 0; r < CR; r++) craw[r] = T(s[coff[r]]);
+    };
+    auto putc = [&](int m, int slot) {   // zero outside the domain
+        const bool zi = czin(m);
+#pragma unroll
+        for (int r = 0; r < CR; r++)
+            if (tid + 256 * r < NC) sc[slot * NC + tid + 256 * r] = (zi && cin[r]) ? craw[r] : T(0);
+    };
+    auto planar = [&](int slot, T (&A)[NP]) {
+        const T *c = sc + slot * NC;
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+            if (p >= 2 && !has[p]) continue;
+            A[p] = T(9) * c[cb[p]] + T(3) * c[cb[p] + cdx[p]] + T(3) * c[cb[p] + cdy[p]] +
+                   c[cb[p] + cdx[p] + cdy[p]];
+        }
+    };
+    // stage-0 values of plane m from the raw loads; PROLONG: lo, hi the planar
+    // sums of the coarse planes around it (lo the lower one), par the parity of m
+    auto enter = [&](auto par, int m, const T (&v)[NP], const T (&lo)[NP], const T (&hi)[NP],
+                     T (&out)[NP]) {
+        constexpr bool odd = decltype(par)::value != 0;
+        const bool zi = zin(m);
+        const bool mz = SRC == MS_PROLONG && czin(odd ? (m >> 1) + 1 : (m >> 1) - 1);
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+            T t = v[p];
+            if (SRC == MS_PROLONG) {
+                const T bmid = odd ? lo[p] : hi[p], aside = odd ? hi[p] : lo[p];
+                T pc = pc1[p];
+                if (!mz) pc = spc[mxy[p]];
+                t = t + pc * (T(3) * bmid + aside);
+            }
+            out[p] = (zi && in[p]) ? t : T(0);
+        }
+    };
+    using Even = std::integral_constant<int, 0>;
+    using Odd = std::integral_constant<int, 1>;
+
+    const int p0 = k0 - (R - 1), p1 = k1 - 1 + (R - 1);
+    // windows: stage 0 planes p-1, p, p+1; stage 1 planes p-2, p-1, p; stage 2
+    // planes p-3, p-2, p-1; b of planes p, p-1, p-2
+    T I0[NP] = {}, I1[NP] = {}, I2[NP] = {};
+    T M0[N1 > 0 ? N1 : 2] = {}, M1[N1 > 0 ? N1 : 2] = {}, M2[N1 > 0 ? N1 : 2] = {};
+    T K0[2] = {}, K1[2] = {}, K2[N2 > 0 ? N2 : 2] = {};
+    T B0[NB] = {}, B1[NB] = {}, B2[2] = {};
+    T xa[NP] = {}, xb[NP] = {}, ba[NB] = {}, bb[NB] = {};
+    T racc = T(0);
+    double acc = 0.0;
+    const double shift = OUTER && a.shift ? *a.shift : 0.0;
+    {
+        T x0[NP] = {}, x1[NP] = {}, x2[NP] = {};
+        ldx(pl(p0 - 1, nz, pz), x0);
+        ldx(pl(p0, nz, pz), x1);
+        ldx(pl(p0 + 1, nz, pz), x2);
+        ldx(pl(p0 + 2, nz, pz), xa);
+        ldb(pl(p0, nz, pz), B0);
+        ldb(pl(p0 + 1, nz, pz), ba);
+        if (SRC == MS_PROLONG) {
+            // p0 - 1 = 2 kc, so the three planes use the coarse planes kc-1, kc, kc+1
+            const int kc = (p0 - 1) >> 1;
+            ldc(kc - 1);
+            putc(kc - 1, 0);
+            ldc(kc);
+            putc(kc, 1);
+            ldc(kc + 1);
+            putc(kc + 1, 2);
+            __syncthreads();
+            T Am[NP] = {};
+            planar(0, Am);
+            planar(1, A0);
+            planar(2, A1);
+            enter(Even(), p0 - 1, x0, Am, A0, I0);
+            enter(Odd(), p0, x1, A0, A1, I1);
+            enter(Even(), p0 + 1, x2, A0, A1, I2);
+            ldc(kc + 2);
+            __syncthreads();   // slot 0 is written again in the first step
+        } else if (SRC == MS_FIELD) {
+            enter(Even(), p0 - 1, x0, A0, A1, I0);
+            enter(Even(), p0, x1, A0, A1, I1);
+            enter(Even(), p0 + 1, x2, A0, A1, I2);
+        }
+    }
+    int qx = pl(p0 + 3, nz, pz), qb = pl(p0 + 2, nz, pz);
+
+    // place of position p in the plane of stage e
+    auto place = [&](int p, int e) { return at[p] - e * (W0 + 1) - 2 * e * (ay[p] - e); };
+    // sum of the x-, x+, y-, y+, z-, z+ neighbours of position p in the plane P
+    // of stage e; the two own cells are each other's y neighbours
+    auto six = [&](const T *P, int e, int p, const T (&c)[2], T zm, T zp) -> T {
+        const int q = place(p, e), W = W0 - 2 * e;
+        const T xm = P[q - 1], xp = P[q + 1];
+        const T ym = p == 1 ? c[0] : P[q - W];
+        const T yp = p == 0 ? c[1] : P[q + W];
+        return xm + xp + ym + yp + zm + zp;
+    };
+
+    // One step; ph alternates 0, 1 from the first one.  The march of a
+    // restriction or prolongation starts on an even plane k0, so there ph = 0
+    // is an odd p of a prolongation (p0 = k0 - 1) and an even residual plane.
+    auto step = [&](auto ph, int p, T (&xu)[NP], T (&xn)[NP], T (&bu)[NB], T (&bn)[NB]) {
+        constexpr int A = decltype(ph)::value, B = 1 - A;   // slots of planes p, p - 1
+        constexpr bool pair = SRC == MS_PROLONG && A == 0;  // a new coarse plane this step
+        if (SRC != MS_ZERO) {
+            T *P = s0 + A * (W0 * H0);
+#pragma unroll
+            for (int q = 0; q < NP; q++)
+                if (q < 2 || has[q]) P[at[q]] = I1[q];
+        }
+        if (pair) {
+            putc((p + 3) >> 1, 0);
+            if (p + 2 <= p1 + 1) ldc(((p + 3) >> 1) + 1);
+        }
+        if (p + 3 <= p1 + 1) ldx(qx, xn);
+        if (p + 2 <= p1) ldb(qb, bn);
+        __syncthreads();
+        // residual of the input, and stage 1 of plane p
+        const T *P0 = s0 + A * (W0 * H0);
+        const bool z0 = zin(p);
+        const int n0 = nzw(p);
+        T *P1 = s1 + A * (W1 * H1);
+#pragma unroll
+        for (int q = 0; q < (NSW > 0 ? N1 : 2); q++) {
+            if (q >= 2 && !has[q]) continue;
+            T S = T(0);
+            if (SRC != MS_ZERO) {
+                const T own[2] = {I1[0], I1[1]};
+                S = six(P0, 0, q, own, I0[q], I2[q]);
+            }
+            if (RESN && q < 2 && p >= k0 && p < k1 && st[q]) {
+                const T d = T(nxy[q] + n0);
+                if constexpr (OUTER) {
+                    const double rr = (B0[q] - shift) + d * I1[q] - S;
+                    acc = acc + rr * rr;
+                    if (a.rout) a.rout[(int64_t)p * g.sz + off[q]] = float(rr);
+                } else {
+                    const double rr = (double)(B0[q] + d * I1[q] - S);
+                    acc = acc + rr * rr;
+                }
+            }
+            if constexpr (NSW > 0) {
+                T id = id2[q];
+                if (n0 != 2) id = sid[nxy[q] + n0];
+                const T v = cff1 * I1[q] + om * (S - B0[q]) * id;
+                M2[q] = (z0 && in[q]) ? v : T(0);
+                if (LDS1) P1[place(q, 1)] = M2[q];
+                if (NSW == 1 && q < 2 && p >= k0 && p < k1 && st[q])
+                    a.dst[(int64_t)p * g.sz + off[q]] = M2[q];
+            }
+        }
+        // stage 2 of plane p - 1
+        const int m = p - 1;
+        const T *Q1 = s1 + B * (W1 * H1);
+        const int n1 = nzw(m);
+        const bool z1 = zin(m);
+        if constexpr (NSW == 2) {
+            if (m >= p0 && m >= k0 - (R - 2)) {
+                T *P2 = s2 + B * (W2 * H2);
+#pragma unroll
+                for (int q = 0; q < N2; q++) {
+                    if (q >= 2 && !has[q]) continue;
+                    const T own[2] = {M1[0], M1[1]};
+                    const T S = six(Q1, 1, q, own, M0[q], M2[q]);
+                    T id = id2[q];
+                    if (n1 != 2) id = sid[nxy[q] + n1];
+                    const T v = cff1 * M1[q] + om * (S - B1[q]) * id;
+                    if (RESTR) {
+                        K2[q] = (z1 && in[q]) ? v : T(0);
+                        P2[place(q, 2)] = K2[q];
+                    }
+                    if (q < 2 && m >= k0 && m < k1 && st[q])
+                        a.dst[(int64_t)m * g.sz + off[q]] = v;
+                }
+            }
+        }
+        // residual of the last stage and its restriction
+        if constexpr (RESTR) {
+            const int k = p - NSW;
+            if (k >= k0 && k < k1) {
+                const T *Q = NSW == 2 ? s2 + A * (W2 * H2) : (NSW == 1 ? Q1 : P0);
+                const int nk = nzw(k);
+                T r[2];
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    const T own[2] = {NSW == 2 ? K1[0] : (NSW == 1 ? M1[0] : I1[0]),
+                                      NSW == 2 ? K1[1] : (NSW == 1 ? M1[1] : I1[1])};
+                    const T zm = NSW == 2 ? K0[q] : (NSW == 1 ? M0[q] : I0[q]);
+                    const T zp = NSW == 2 ? K2[q] : (NSW == 1 ? M2[q] : I2[q]);
+                    const T S = six(Q, NSW, q, own, zm, zp);
+                    const T bv = NSW == 2 ? B2[q] : (NSW == 1 ? B1[q] : B0[q]);
+                    r[q] = bv + T(nxy[q] + nk) * own[q] - S;
+                }
+                const T rx0 = __shfl_down(r[0], 1), rx1 = __shfl_down(r[1], 1);
+                if constexpr (A == 0) {
+                    racc = ((r[0] + rx0) + r[1]) + rx1;
+                } else {
+                    racc = (((racc + r[0]) + rx0) + r[1]) + rx1;
+                    const int ic = (i0 + tx) >> 1, jc = (j0 >> 1) + ty, kc = k >> 1;
+                    if ((tx & 1) == 0 && ic < gc.nx && jc < gc.ny) {
+                        const int64_t cc = (int64_t)kc * gc.sz + (int64_t)jc * gc.sy + ic;
+                        const TC bv = TC(T(0.5) * racc);
+                        const int nw = (gc.px || ic > 0) + (gc.px || ic < gc.nx - 1) +
+                                       (gc.py || jc > 0) + (gc.py || jc < gc.ny - 1) +
+                                       (gc.pz || kc > 0) + (gc.pz || kc < gc.nz - 1);
+                        a.bc[cc] = bv;
+                        // the coarse level's first sweep from x = 0
+                        const TC omc = TC(a.omega), c1 = TC(1.0 - a.omega);
+                        a.yc[cc] = c1 * TC(0) + omc * (TC(0) - bv) * TC(a.tab.idiag[nw]);
+                    }
+                }
+            }
+        }
+        // the next plane
+        if (pair) {
+#pragma unroll
+            for (int q = 0; q < NP; q++) A0[q] = A1[q];
+            planar(0, A1);
+        }
+        T In[NP];
+        // (p + 2 is odd in the steps that bring a coarse plane)
+        if (SRC != MS_ZERO)
+            enter(std::integral_constant<int, B>(), p + 2, xu, A0, A1, In);
+#pragma unroll
+        for (int q = 0; q < NP; q++) {
+            I0[q] = I1[q];
+            I1[q] = I2[q];
+            if (SRC != MS_ZERO) I2[q] = In[q];
+        }
+#pragma unroll
+        for (int q = 0; q < N1; q++) {
+            M0[q] = M1[q];
+            M1[q] = M2[q];
+        }
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            if (NSW == 2 && RESTR) {
+                K0[q] = K1[q];
+                K1[q] = K2[q];
+            }
+            B2[q] = B1[q];
+        }
+#pragma unroll
+        for (int q = 0; q < NB; q++) {
+            B1[q] = B0[q];
+            B0[q] = bu[q];
+        }
+        qx = next(qx, p + 3, nz, pz);
+        qb = next(qb, p + 2, nz, pz);
+    };
+    for (int p = p0; p <= p1; p += 2) {
+        step(Even(), p, xa, xb, ba, bb);
+        if (p + 1 <= p1) step(Odd(), p + 1, xb, xa, bb, ba);
+    }
+    if (RESN) {
+        __syncthreads();
+        const int nb = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+        block_sum_store(acc, a.partials + nb, tid);
+    }
+}
+
+// Tile width and march length of a level.  The width (64 or 32 columns, rows
+// to match) is the one that pads the level less; the march is the longest
+// that still gives the chip `want` blocks (each block evaluates R extra
+// planes, so long marches save work and short ones latency), and at least
+// long enough to keep within the partial sums of a residual norm.
+MarchGrid march_grid(const Geo &g, int es, bool even) {
+    auto up = [](int n, int t) { return (n + t - 1) / t; };
+    MarchGrid m;
+    const int64_t a64 = (int64_t)up(g.nx, 64) * up(g.ny, 8), a32 = (int64_t)up(g.nx, 32) * up(g.ny, 16);
+    m.tx = a32 < a64 ? 32 : 64;
+    m.bx = up(g.nx, m.tx);
+    m.by = up(g.ny, 512 / m.tx);
+    const int64_t cols = (int64_t)m.bx * m.by;
+    const int64_t want = 1024;
+    int kz = es == 4 ? 16 : 32;
+    const int least = even ? 2 : 1;
+    while (kz > least && cols * up(g.nz, kz) < want) kz >>= 1;
+    while (cols * up(g.nz, kz) > NYL_RED_BLOCKS && kz < g.nz) kz <<= 1;
+    m.kz = kz;
+    m.bz = up(g.nz, kz);
+    return m;
+}
+
+#define MARCH_GO(T, TC, SRC, NSW, RESN, RESTR, OUTER)                                          \
+    do {                                                                                      \
+        MarchArgs<T, TC> m = a;                                                               \
+        const MarchGrid gr = march_grid(a.g, (int)sizeof(T), (RESTR) || (SRC) == MS_PROLONG); \
+        m.kz = gr.kz;                                                                         \
+        const dim3 grd(gr.bx, gr.by, gr.bz), blk(256);                                        \
+        if (gr.tx == 64)                                                                      \
+            NYL_LAUNCH((k_mg_march<T, TC, 64, SRC, NSW, RESN, RESTR, OUTER>), grd, blk, 0, s, m); \
+        else                                                                                  \
+            NYL_LAUNCH((k_mg_march<T, TC, 32, SRC, NSW, RESN, RESTR, OUTER>), grd, blk, 0, s, m); \
+    } while (0)
+
+template <typename T, typename TC>
+hipError_t launch_march_up(const MarchArgs<T, TC> &a, hipStream_t s) {
+    if (a.src == a.dst || !a.xc) return hipErrorInvalidValue;
+    MARCH_GO(T, TC, MS_PROLONG, 2, false, false, false);
+    return hipGetLastError();
+}
+
+template <typename T, typename TC>
+hipError_t launch_march_down(const MarchArgs<T, TC> &a, hipStream_t s) {
+    if (a.src == a.dst || !a.bc || !a.yc) return hipErrorInvalidValue;
+    MARCH_GO(T, TC, MS_FIELD, 1, false, true, false);
+    return hipGetLastError();
+}
+
+template <typename T, typename TC>
+hipError_t launch_march_restrict(const MarchArgs<T, TC> &a, hipStream_t s) {
+    if (!a.bc || !a.yc) return hipErrorInvalidValue;
+    MARCH_GO(T, TC, MS_FIELD, 0, false, true, false);
+    return hipGetLastError();
+}
+
+template <typename T, typename TC>
+hipError_t launch_march_pre(const MarchArgs<T, TC> &a, hipStream_t s) {
+    if (a.src == a.dst || (!a.src && a.partials)) return hipErrorInvalidValue;
+    if (a.bc) {
+        if (!a.yc) return hipErrorInvalidValue;
+        if (!a.src) MARCH_GO(T, TC, MS_ZERO, 2, false, true, false);
+        else if (a.partials) MARCH_GO(T, TC, MS_FIELD, 2, true, true, false);
+        else MARCH_GO(T, TC, MS_FIELD, 2, false, true, false);
+        return hipGetLastError();
+    }
+    if (!a.src) MARCH_GO(T, TC, MS_ZERO, 2, false, false, false);
+    else if (a.partials) MARCH_GO(T, TC, MS_FIELD, 2, true, false, false);
+    else MARCH_GO(T, TC, MS_FIELD, 2, false, false, false);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_march_norm(const MarchArgs<T, T> &a, hipStream_t s) {
+    if (!a.partials) return hipErrorInvalidValue;
+    MARCH_GO(T, T, MS_FIELD, 0, true, false, false);
+    return hipGetLastError();
+}
+
+hipError_t launch_march_outer(const MarchArgs<double, double> &a, hipStream_t s) {
+    if (!a.partials || !a.rout) return hipErrorInvalidValue;
+    MARCH_GO(double, double, MS_FIELD, 0, true, false, true);
+    return hipGetLastError();
+}
+
+#define NYL_MARCH_INST(T, TC)                                                              \
+    template hipError_t launch_march_up<T, TC>(const MarchArgs<T, TC> &, hipStream_t);     \
+    template hipError_t launch_march_down<T, TC>(const MarchArgs<T, TC> &, hipStream_t);   \
+    template hipError_t launch_march_pre<T, TC>(const MarchArgs<T, TC> &, hipStream_t);    \
+    template hipError_t launch_march_restrict<T, TC>(const MarchArgs<T, TC> &, hipStream_t);
+NYL_MARCH_INST(double, double)
+NYL_MARCH_INST(float, float)
+NYL_MARCH_INST(float, double)
+template hipError_t launch_march_norm<double>(const MarchArgs<double, double> &, hipStream_t);
+template hipError_t launch_march_norm<float>(const MarchArgs<float, float> &, hipStream_t);
+
+}  // namespace nyl

@@ -217,21 +217,6 @@ hipError_t launch_mg_prolong(const Geo &gf, const Geo &gc, Tf *xf, const Tc *xc,
 // cell count, each thread sums a fixed set of cells in a fixed order and the
 // block trees are fixed, so a result does not change from run to run.
 
-#define RED_T 256
-
-// Fixed-order tree over the RED_T threads of a block; tid is the linear
-// thread index (blocks may be 2-D).
-__device__ __forceinline__ void block_sum_store(double v, double *out, int tid) {
-    __shared__ double sh[RED_T];
-    sh[tid] = v;
-    __syncthreads();
-    for (int s = RED_T / 2; s > 0; s >>= 1) {
-        if (tid < s) sh[tid] = sh[tid] + sh[tid + s];
-        __syncthreads();
-    }
-    if (tid == 0) *out = sh[0];
-}
-
 __device__ __forceinline__ void block_max_store(double v, double *out, int tid) {
     __shared__ double sh[RED_T];
     sh[tid] = v;
@@ -526,7 +511,7 @@ __global__ __launch_bounds__(256) void k_mg_restrict25(Geo g, Geo gc, const Tf *
     }
 }
 
-static inline int red_blocks(int64_t n) {
+int red_blocks(int64_t n) {
     int64_t b = (n + RED_T - 1) / RED_T;
     return (int)(b < NYL_RED_BLOCKS ? (b < 1 ? 1 : b) : NYL_RED_BLOCKS);
 }
@@ -582,7 +567,7 @@ hipError_t launch_norm2(const Geo &g, const T *v, double *partials, double *dev_
     const int64_t n = (int64_t)g.nx * g.ny * g.nz;
     const int nb = red_blocks(n);
     NYL_LAUNCH((k_norm2<T>), dim3(nb), dim3(RED_T), 0, s, n, v, partials);
-    (void)launch_final_sum(partials, nb, dev_out, s);
+    if (dev_out) (void)launch_final_sum(partials, nb, dev_out, s);
     return hipGetLastError();
 }
 
@@ -610,7 +595,7 @@ hipError_t launch_resnorm2(const Geo &g, const T *x, const T *b, const MGTabs &t
     const int64_t n = (int64_t)g.nx * g.ny * g.nz;
     const int nb = red_blocks(n);
     NYL_LAUNCH((k_resnorm2<T>), dim3(nb), dim3(RED_T), 0, s, g, x, b, tab, partials);
-    (void)launch_final_sum(partials, nb, dev_out, s);
+    if (dev_out) (void)launch_final_sum(partials, nb, dev_out, s);
     return hipGetLastError();
 }
 
@@ -751,16 +736,19 @@ bool outer_resid_fits(const Geo &g) {
 // x = x + e (the outer correction, in FP64)
 template <typename TI>
 __global__ __launch_bounds__(256) void k_add_correction(int64_t n, double *__restrict__ x,
-                                                        const TI *__restrict__ e) {
+                                                        const TI *__restrict__ e,
+                                                        const int *__restrict__ gate) {
+    if (gate && *gate) return;
     const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (q < n) x[q] = x[q] + (double)e[q];
 }
 
 template <typename TI>
-hipError_t launch_add_correction(const Geo &g, double *x, const TI *e, hipStream_t s) {
+hipError_t launch_add_correction(const Geo &g, double *x, const TI *e, const int *gate,
+                                 hipStream_t s) {
     const int64_t n = (int64_t)g.nx * g.ny * g.nz;
     NYL_LAUNCH((k_add_correction<TI>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
-                       n, x, e);
+                       n, x, e, gate);
     return hipGetLastError();
 }
 
@@ -779,14 +767,15 @@ __global__ __launch_bounds__(RED_T) void k_sum_sumsq(int64_t n, const double *__
     block_sum_store(a2, partials + nb + blockIdx.x, threadIdx.x);
 }
 
-hipError_t launch_sum_sumsq(const Geo &g, const double *v, double *partials, double *dev_out,
-                            hipStream_t s) {
+int sumsq_blocks(int64_t n) {
+    const int nb = red_blocks(n);
+    return nb > NYL_RED_BLOCKS / 2 ? NYL_RED_BLOCKS / 2 : nb;
+}
+
+hipError_t launch_sum_sumsq(const Geo &g, const double *v, double *partials, hipStream_t s) {
     const int64_t n = (int64_t)g.nx * g.ny * g.nz;
-    int nb = red_blocks(n);
-    if (nb > NYL_RED_BLOCKS / 2) nb = NYL_RED_BLOCKS / 2;
+    const int nb = sumsq_blocks(n);
     NYL_LAUNCH(k_sum_sumsq, dim3(nb), dim3(RED_T), 0, s, n, v, partials, nb);
-    (void)launch_final_sum(partials, nb, dev_out, s);
-    (void)launch_final_sum(partials + nb, nb, dev_out + 1, s);
     return hipGetLastError();
 }
 
@@ -1564,18 +1553,6 @@ __global__ __launch_bounds__(TAIL_T) void k_mg_tail(TailArgs a) {
     });
 }
 
-template <typename T, typename TC>
-hipError_t launch_mg_tail(const TailArgs &a, hipStream_t s) {
-    if (a.nlev > NYL_TAIL_MAXLEV || a.l0 < 0 || a.l0 > a.nlev - 2) return hipErrorInvalidValue;
-    TailArgs t = a;
-    if (tail_layout(t, sizeof(T), sizeof(TC)) > NYL_TAIL_LDS) return hipErrorInvalidValue;
-    NYL_LAUNCH((k_mg_tail<T, TC>), dim3(1), dim3(TAIL_T), 0, s, t);
-    return hipGetLastError();
-}
-template hipError_t launch_mg_tail<double, double>(const TailArgs &, hipStream_t);
-template hipError_t launch_mg_tail<float, double>(const TailArgs &, hipStream_t);
-template hipError_t launch_mg_tail<float, float>(const TailArgs &, hipStream_t);
-
 bool sweep25_fits(const Geo &g) {
     return g.nx % SW_TX == 0 && g.ny % SW_TY == 0 && g.nx >= SW_TX;
 }
@@ -1605,24 +1582,16 @@ int sweep25_blocks(const Geo &g) {
 template <typename T>
 hipError_t launch_mg_sweep25(const Geo &g, const T *src, T *dst, const T *b, double omega,
                              const MGTabs &tab, double *partials, double *dev_out,
-                             hipStream_t s, const Geo *gc, const T *xc, double *addx) {
+                             hipStream_t s) {
     const int kz = sweep25_kz(g, 1);
     dim3 grd(g.nx / SW_TX, g.ny / SW_TY, g.nz / kz), blk(SW_TX, 4);
-    const Geo gcv = gc ? *gc : g;
     if (partials) {
         NYL_LAUNCH((k_mg_sweep25<T, true, false, false>), grd, blk, 0, s, g, src, dst, b,
-                           omega, tab, kz, partials, gcv, xc, addx);
-        const int nb = grd.x * grd.y * grd.z;
-        (void)launch_final_sum(partials, nb, dev_out, s);
-    } else if (addx) {
-        NYL_LAUNCH((k_mg_sweep25<T, false, false, true>), grd, blk, 0, s, g, src, dst, b,
-                           omega, tab, kz, partials, gcv, xc, addx);
-    } else if (xc) {
-        NYL_LAUNCH((k_mg_sweep25<T, false, true, false>), grd, blk, 0, s, g, src, dst, b,
-                           omega, tab, kz, partials, gcv, xc, addx);
+                           omega, tab, kz, partials, g, (const T *)nullptr, (double *)nullptr);
+        (void)launch_final_sum(partials, (int)(grd.x * grd.y * grd.z), dev_out, s);
     } else {
-        NYL_LAUNCH((k_mg_sweep25<T, false, false, false>), grd, blk, 0, s, g, src, dst,
-                           b, omega, tab, kz, partials, gcv, xc, addx);
+        NYL_LAUNCH((k_mg_sweep25<T, false, false, false>), grd, blk, 0, s, g, src, dst, b,
+                           omega, tab, kz, partials, g, (const T *)nullptr, (double *)nullptr);
     }
     return hipGetLastError();
 }
@@ -1724,38 +1693,6 @@ bool outer25_fits(const Geo &g) {
     if (!sweep25_fits(g)) return false;
     const int64_t nb = (int64_t)(g.nx / SW_TX) * (g.ny / SW_TY) * (g.nz / outer25_kz(g));
     return nb <= NYL_RED_BLOCKS;
-}
-
-bool outer_bsq_fits(const Geo &g) {
-    if (!sweep25_fits(g)) return false;
-    const int64_t nb = (int64_t)(g.nx / SW_TX) * (g.ny / SW_TY) * (g.nz / outer25_kz(g));
-    return 2 * nb <= NYL_RED_BLOCKS;
-}
-
-template <typename TI>
-hipError_t launch_mg_outer_resid(const Geo &g, const double *x, const double *b, double shift,
-                                 TI *r, TI *y, double omega, const MGTabs &tab, double *partials,
-                                 double *dev_out, hipStream_t s, bool with_bsq) {
-    if (outer25_fits(g)) {
-        const int kz = outer25_kz(g);
-        const dim3 grd(g.nx / SW_TX, g.ny / SW_TY, g.nz / kz), blk(SW_TX, 4);
-        const int nb = grd.x * grd.y * grd.z;
-        if (with_bsq && 2 * nb > NYL_RED_BLOCKS) return hipErrorInvalidValue;
-        double *pb = with_bsq ? partials + nb : nullptr;
-        NYL_LAUNCH((k_mg_outer25<TI>), grd, blk, 0, s, g, x, b, shift, r, y, omega, tab,
-                           kz, partials, pb);
-        (void)launch_final_sum(partials, nb, dev_out, s);
-        if (with_bsq)
-            (void)launch_final_sum(pb, nb, dev_out + 1, s);
-        return hipGetLastError();
-    }
-    if (with_bsq) return hipErrorInvalidValue;
-    const dim3 grd = outer_grid(g);
-    NYL_LAUNCH((k_mg_outer_resid<TI>), grd, dim3(MG_BX, MG_BY, 1), 0, s, g, x, b, shift,
-                       r, y, omega, tab, partials);
-    const int nb = grd.x * grd.y * grd.z;
-    (void)launch_final_sum(partials, nb, dev_out, s);
-    return hipGetLastError();
 }
 
 // Prolongation with 2.5-D tiling: a block owns fine 64 x 8 cells (rows
@@ -2118,12 +2055,11 @@ __global__ __launch_bounds__(256) void k_mg_sweep2x25(Geo g, const T *__restrict
 #define S2T_RING1 (2 * S2T_MX + 2 * SW_TY)       // 148 cells
 #define S2T_RING2 (2 * S2T_LX + 2 * (SW_TY + 2))  // 156 cells
 template <typename T, bool ADDX, int PZ, bool RESNORM, bool ZSRC>
-__global__ __launch_bounds__(256) void k_mg_sweep2t(Geo g, const T *__restrict__ src,
-                                                    T *__restrict__ dst,
-                                                    const T *__restrict__ b, double omega,
-                                                    MGTabs tab, int kz,
-                                                    double *__restrict__ xo,
-                                                    double *__restrict__ partials) {
+__device__ __forceinline__ void sweep2t_pass(const Geo &g, const T *__restrict__ src,
+                                             T *__restrict__ dst, const T *__restrict__ b,
+                                             double omega, const MGTabs &tab, int kz,
+                                             double *__restrict__ xo,
+                                             double *__restrict__ partials) {
     __shared__ T sin_[2][S2T_LY][S2T_LX];
     __shared__ T smid[2][S2T_MY][S2T_MX];
     const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * SW_TX + tx;
@@ -2360,6 +2296,28 @@ __global__ __launch_bounds__(256) void k_mg_sweep2t(Geo g, const T *__restrict__
     }
 }
 
+template <typename T, bool ADDX, int PZ, bool RESNORM, bool ZSRC>
+__global__ __launch_bounds__(256) void k_mg_sweep2t(Geo g, const T *__restrict__ src,
+                                                    T *__restrict__ dst,
+                                                    const T *__restrict__ b, double omega,
+                                                    MGTabs tab, int kz,
+                                                    double *__restrict__ xo,
+                                                    double *__restrict__ partials) {
+    sweep2t_pass<T, ADDX, PZ, RESNORM, ZSRC>(g, src, dst, b, omega, tab, kz, xo, partials);
+}
+
+// the plain pass of a V-cycle's post-smoothing; when *gate is non-zero the
+// solve has stopped and dst stays as it is
+template <typename T, int PZ>
+__global__ __launch_bounds__(256) void k_mg_sweep2t_gated(Geo g, const T *__restrict__ src,
+                                                          T *__restrict__ dst,
+                                                          const T *__restrict__ b, double omega,
+                                                          MGTabs tab, int kz,
+                                                          const int *__restrict__ gate) {
+    if (*gate) return;
+    sweep2t_pass<T, false, PZ, false, false>(g, src, dst, b, omega, tab, kz, nullptr, nullptr);
+}
+
 // planes per block of the two-sweep pass: the longest march (at most 16
 // planes in FP32, 32 in FP64, dividing nz) that keeps at least 1024 blocks;
 // each block re-reads four input planes.  256^3 (k_mg_sweep2t): FP32 37.8 us
@@ -2371,46 +2329,36 @@ static int sweep2x_kz(const Geo &g, int es) {
     return kz;
 }
 
-// the two-sweep pass with register z-windows (k_mg_sweep2t) in place of
-// k_mg_sweep2x25
-#ifndef NYL_SWEEP2T
-#define NYL_SWEEP2T 1
-#endif
 template <typename T>
 hipError_t launch_mg_sweep2x25(const Geo &g, const T *src, T *dst, const T *b, double omega,
-                               const MGTabs &tab, hipStream_t s, double *addx,
-                               double *partials, double *dev_out) {
-    if (src == dst || (addx && partials) || (!src && (addx || partials)))
-        return hipErrorInvalidValue;
+                               const MGTabs &tab, hipStream_t s, double *partials,
+                               double *dev_out, const int *gate) {
+    if (src == dst || (!src && partials)) return hipErrorInvalidValue;
     const int kz = sweep2x_kz(g, (int)sizeof(T));
     dim3 grd(g.nx / SW_TX, g.ny / SW_TY, g.nz / kz), blk(SW_TX, 4);
-    if (NYL_SWEEP2T) {
-#define S2T_GO(A, Z, R)                                                                    \
-    NYL_LAUNCH((k_mg_sweep2t<T, A, Z, R, false>), grd, blk, 0, s, g, src, dst, b, omega, tab, \
-               kz, addx, partials)
-        if (!src) {   // from x = 0
-            if (g.pz)
-                NYL_LAUNCH((k_mg_sweep2t<T, false, 1, false, true>), grd, blk, 0, s, g, src, dst,
-                           b, omega, tab, kz, addx, partials);
-            else
-                NYL_LAUNCH((k_mg_sweep2t<T, false, 0, false, true>), grd, blk, 0, s, g, src, dst,
-                           b, omega, tab, kz, addx, partials);
-        } else if (partials) {
-            if (g.pz) S2T_GO(false, 1, true);
-            else S2T_GO(false, 0, true);
-            (void)launch_final_sum(partials, (int)(grd.x * grd.y * grd.z), dev_out, s);
-        } else if (addx) {
-            if (g.pz) S2T_GO(true, 1, false);
-            else S2T_GO(true, 0, false);
-        } else {
-            if (g.pz) S2T_GO(false, 1, false);
-            else S2T_GO(false, 0, false);
-        }
-#undef S2T_GO
-        return hipGetLastError();
+#define S2T_GO(Z, R, ZERO)                                                                 \
+    NYL_LAUNCH((k_mg_sweep2t<T, false, Z, R, ZERO>), grd, blk, 0, s, g, src, dst, b, omega, \
+               tab, kz, (double *)nullptr, partials)
+    if (gate) {
+        if (!src || partials) return hipErrorInvalidValue;
+        if (g.pz)
+            NYL_LAUNCH((k_mg_sweep2t_gated<T, 1>), grd, blk, 0, s, g, src, dst, b, omega, tab, kz,
+                       gate);
+        else
+            NYL_LAUNCH((k_mg_sweep2t_gated<T, 0>), grd, blk, 0, s, g, src, dst, b, omega, tab, kz,
+                       gate);
+    } else if (!src) {   // from x = 0
+        if (g.pz) S2T_GO(1, false, true);
+        else S2T_GO(0, false, true);
+    } else if (partials) {
+        if (g.pz) S2T_GO(1, true, false);
+        else S2T_GO(0, true, false);
+        if (dev_out) (void)launch_final_sum(partials, (int)(grd.x * grd.y * grd.z), dev_out, s);
+    } else {
+        if (g.pz) S2T_GO(1, false, false);
+        else S2T_GO(0, false, false);
     }
-    if (partials || !src) return hipErrorInvalidValue;   // these need k_mg_sweep2t
-    NYL_LAUNCH((k_mg_sweep2x25<T>), grd, blk, 0, s, g, src, dst, b, omega, tab, kz, addx);
+#undef S2T_GO
     return hipGetLastError();
 }
 
@@ -2420,10 +2368,10 @@ int sweep2x_blocks(const Geo &g, int es) {
 }
 template hipError_t launch_mg_sweep2x25<double>(const Geo &, const double *, double *,
                                                 const double *, double, const MGTabs &,
-                                                hipStream_t, double *, double *, double *);
+                                                hipStream_t, double *, double *, const int *);
 template hipError_t launch_mg_sweep2x25<float>(const Geo &, const float *, float *,
                                                const float *, double, const MGTabs &,
-                                               hipStream_t, double *, double *, double *);
+                                               hipStream_t, double *, double *, const int *);
 
 bool restrict25_fits(const Geo &g) {
     return sweep25_fits(g) && g.nz % 2 == 0;
@@ -2441,8 +2389,7 @@ hipError_t launch_mg_restrict25(const Geo &gf, const Geo &gc, const Tf *x, const
 
 #define NYL_MG_INST(T)                                                                          \
     template hipError_t launch_mg_sweep25<T>(const Geo &, const T *, T *, const T *, double,    \
-                                             const MGTabs &, double *, double *, hipStream_t,   \
-                                             const Geo *, const T *, double *);                 \
+                                             const MGTabs &, double *, double *, hipStream_t);  \
     template hipError_t launch_mg_prolong25<T, T>(const Geo &, const Geo &, T *, const T *,     \
                                                   const MGTabs &, hipStream_t, T *);            \
     template hipError_t launch_mg_restrict25<T, T>(const Geo &, const Geo &, const T *,         \
@@ -2496,11 +2443,7 @@ template hipError_t launch_mg_resid_restrict<float, double>(const Geo &, const G
                                                             hipStream_t, double *, double);
 template hipError_t launch_mg_prolong<float, double>(const Geo &, const Geo &, float *,
                                                      const double *, const MGTabs &, hipStream_t);
-template hipError_t launch_mg_outer_resid<float>(const Geo &, const double *, const double *,
-                                                 double, float *, float *, double,
-                                                 const MGTabs &, double *, double *, hipStream_t,
-                                                 bool);
 template hipError_t launch_add_correction<float>(const Geo &, double *, const float *,
-                                                 hipStream_t);
+                                                 const int *, hipStream_t);
 
 }  // namespace nyl

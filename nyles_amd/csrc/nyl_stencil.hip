@@ -951,13 +951,19 @@ static void launch_stage25_p(const Geo &g, const StageArgs<T> &a, int mode, hipS
 template <typename T>
 hipError_t launch_stage(const Geo &g, const StageArgs<T> &a, int mode, hipStream_t s) {
     if (mode < 0 || mode > 6) return hipErrorInvalidValue;
+#if NYL_STAGE25
     const bool t25 = s25_fits(g) && a.flags == 0;   // the 2.5-D form runs the LES only
-    switch (g.px + 2 * g.py + 4 * g.pz) {
-#define NYL_STAGE_CASE(c, X, Y, Z)                                                   \
-    case c:                                                                          \
+#define NYL_STAGE_GO(X, Y, Z)                                                        \
+    do {                                                                             \
         if (t25) launch_stage25_p<T, X, Y, Z>(g, a, mode, s);                        \
         else launch_stage_p<T, X, Y, Z>(g, a, mode, s);                              \
-        break;
+    } while (0)
+#else
+#define NYL_STAGE_GO(X, Y, Z) launch_stage_p<T, X, Y, Z>(g, a, mode, s)
+#endif
+    switch (g.px + 2 * g.py + 4 * g.pz) {
+#define NYL_STAGE_CASE(c, X, Y, Z)                                                   \
+    case c: NYL_STAGE_GO(X, Y, Z); break;
     NYL_STAGE_CASE(0, 0, 0, 0)
     NYL_STAGE_CASE(1, 1, 0, 0)
     NYL_STAGE_CASE(2, 0, 1, 0)
@@ -965,11 +971,9 @@ hipError_t launch_stage(const Geo &g, const StageArgs<T> &a, int mode, hipStream
     NYL_STAGE_CASE(4, 0, 0, 1)
     NYL_STAGE_CASE(5, 1, 0, 1)
     NYL_STAGE_CASE(6, 0, 1, 1)
-    default:
-        if (t25) launch_stage25_p<T, 1, 1, 1>(g, a, mode, s);
-        else launch_stage_p<T, 1, 1, 1>(g, a, mode, s);
-        break;
+    default: NYL_STAGE_GO(1, 1, 1); break;
 #undef NYL_STAGE_CASE
+#undef NYL_STAGE_GO
     }
     return hipGetLastError();
 }

@@ -65,9 +65,7 @@ class DeviceModel:
         self.workspace_bytes = nbytes.value
         with torch.cuda.device(self.device):
             self.ws = torch.empty(self.workspace_bytes, dtype=torch.uint8, device=self.device)
-            # a stream of its own (default priority): the library captures the
-            # coarse multigrid levels into a hipGraph, which the null stream
-            # does not allow
+            # a stream of its own (default priority)
             self.stream = torch.cuda.Stream(device=self.device)
         torch.cuda.current_stream(self.device).synchronize()   # ws allocated
         L.check(lib.nyl_set_stream(ctx, ctypes.c_void_p(self.stream.cuda_stream)))
@@ -179,7 +177,7 @@ class DeviceModel:
         L.check(self.lib.nyl_sync(self.ctx))
 
     def set_graphs(self, on):
-        """replay the coarse multigrid levels from a hipGraph (default) or not"""
+        """accepted and without effect (nyl_set_graphs)"""
         L.check(self.lib.nyl_set_graphs(self.ctx, int(bool(on))))
 
     def mg_levels(self):
