@@ -580,7 +580,7 @@ int pre_smooth(nyl_ctx *c, bool zero, int *np) {
             a.yc = F<TC>(c, q.y);
         }
         if (!zero) {
-            *np = march_grid(f.g, (int)sizeof(T), one).blocks();
+            *np = march_grid(f.g, march_resident(sizeof(T), MS_FIELD, 2, one), one).blocks();
             if (*np > NYL_RED_BLOCKS) {   // too wide for one partial sum per block
                 if constexpr (std::is_same<T, double>::value) {
                     LAUNCH(NYL_K_RESNORM, 2 * n,
@@ -611,7 +611,7 @@ int resid_norm(nyl_ctx *c, int *np) {
     const Level &f = c->lev[0];
     MarchArgs<T, T> a = march_args<T, T>(c, 0, f.x, f.y);
     a.partials = F<double>(c, c->partials);
-    *np = march_grid(f.g, (int)sizeof(T), false).blocks();
+    *np = march_grid(f.g, march_resident(sizeof(T), MS_FIELD, 0, false), false).blocks();
     if (*np > NYL_RED_BLOCKS) {
         *np = red_blocks((int64_t)cells(f.g));
         LAUNCH(NYL_K_RESNORM, 2 * cells(f.g) * sizeof(T),
@@ -636,7 +636,7 @@ void fill_stats(nyl_ctx *c, nyl_mg_stats *st, int nite, double res, double normb
 // mgfor tests the residual after every V-cycle (core/mgfor/solvers.f90:8-33).
 // Waiting for each test on the host left the GPU idle for 10 to 20 us per
 // V-cycle.  Here the tests run on the device (CtlArgs): the V-cycles that the
-// last solve at the same place of a step needed are enqueued without a wait,
+// last solves at the same place of a step needed are enqueued without a wait,
 // and one that follows the stopping test leaves the solution as it is (its
 // last pass is gated), so the result does not depend on the guess; the host
 // reads the sums of all tests once and takes the same decisions from them.
@@ -681,7 +681,28 @@ int ctl_read(nyl_ctx *c, double *normb, double *hist, int n) {
 // most tests between two reads
 constexpr int kMaxAhead = CTL_HIST - 8;
 
-int known(int pred, int other) { return pred >= 0 ? pred : other; }
+// The guess of a solve (or of an outer step of a mixed one): the fewer of the
+// V-cycles the last two at its place needed, those of the solves outside a
+// step where there was none, `other` where nothing is known.  One V-cycle too
+// many costs a V-cycle, one too few a host read, so the guess is low; `ends`:
+// the last one stopped at the guess, so that the test there is expected to be
+// the last and evaluates the norm alone.
+struct Guess {
+    int n;
+    bool ends;
+};
+Guess guess_of(const nyl_ctx *c, int site, int j, int other) {
+    const Pred *p = &c->pred[site][j];
+    if (p->last < 0) p = &c->pred[0][j];
+    if (p->last < 0) return {other, false};
+    const int n = p->before >= 0 ? std::min(p->last, p->before) : p->last;
+    return {n, n > 0 && p->last == n};
+}
+void set_guess(nyl_ctx *c, int site, int j, int n) {
+    Pred &p = c->pred[site][j];
+    p.before = p.last;
+    p.last = n;
+}
 
 // core/mgfor/solvers.f90:8-33 with normresidual (core/mgfor/operators.f90:81-96)
 int mg_solve_fp64(nyl_ctx *c, nyl_mg_stats *st, int site) {
@@ -694,7 +715,8 @@ int mg_solve_fp64(nyl_ctx *c, nyl_mg_stats *st, int site) {
     HIPCHK(launch_ctl(ctl_args(c, CTL_NORMB, red_blocks((int64_t)cells(f.g))), c->stream));
     double normb = 0.0, res = 0.0, hist[CTL_HIST];
     int done = 0;    // V-cycles enqueued
-    int guess = known(c->pred[site][0], known(c->pred[0][0], 0));
+    const Guess gs = guess_of(c, site, 0, 0);
+    int guess = gs.n;
     bool pre = false;   // the sweeps (and test) of V-cycle done + 1 are enqueued
     for (;;) {
         const int first = done;   // V-cycles before the first test of this round
@@ -718,7 +740,7 @@ int mg_solve_fp64(nyl_ctx *c, nyl_mg_stats *st, int site) {
             // the test after the last V-cycle: the norm alone where the solve
             // is expected to stop, else with the next V-cycle's sweeps
             int np = 0;
-            const bool ends = first == 0 && done > 0;
+            const bool ends = first == 0 && gs.ends;
             if (ends) rc = resid_norm<double>(c, &np);
             else rc = pre_smooth(c, false, &np);
             if (rc) return rc;
@@ -745,7 +767,7 @@ int mg_solve_fp64(nyl_ctx *c, nyl_mg_stats *st, int site) {
         if (done >= maxite) break;
         guess = done + 1;
     }
-    c->pred[site][0] = done;
+    set_guess(c, site, 0, done);
     fill_stats(c, st, done, res, normb);
     return NYL_OK;
 }
@@ -796,7 +818,7 @@ int mg_solve_mixed(nyl_ctx *c, nyl_mg_stats *st, int site) {
         a.shift = &ctl->shift;
         LAUNCH(NYL_K_RESNORM, (2 * sizeof(double) + sizeof(float)) * ncell,
                launch_march_outer(a, c->stream));
-        CtlArgs t = ctl_args(c, CTL_OUTER, march_grid(f.g, sizeof(double), false).blocks());
+        CtlArgs t = ctl_args(c, CTL_OUTER, march_grid(f.g, march_resident(8, MS_FIELD, 0, false), false).blocks());
         t.slot = slot;
         if (publish) ctl_publish(c, t, slot + 1);
         HIPCHK(launch_ctl(t, c->stream));
@@ -811,8 +833,7 @@ int mg_solve_mixed(nyl_ctx *c, nyl_mg_stats *st, int site) {
     auto relative = [&](double s) { return normb > 0.0 ? s / normb : 0.0; };
     // the first outer residual is read with the first outer step's tests,
     // unless the solve is expected to stop at it
-    const int g0 = known(c->pred[site][0], known(c->pred[0][0], 1));
-    bool have_res = g0 == 0;
+    bool have_res = guess_of(c, site, 0, 1).n == 0;
     if ((rc = outer(0, have_res))) return rc;
     if (have_res) {
         if ((rc = ctl_read(c, &normb, hist, 1))) return rc;
@@ -822,13 +843,11 @@ int mg_solve_mixed(nyl_ctx *c, nyl_mg_stats *st, int site) {
     bool at_max = false;
     for (int j = 0;; j++) {
         if (have_res && (res < tol || at_max)) {
-            if (j < kPredOuter) c->pred[site][j] = 0;
+            if (j < kPredOuter) set_guess(c, site, j, 0);
             break;
         }
-        const int jp = std::min(j, kPredOuter - 1);
-        int guess = known(c->pred[site][jp], known(c->pred[0][jp], 1));
-        if (guess < 1) guess = 1;
-        const bool sure = c->pred[site][jp] > 0 || c->pred[0][jp] > 0;
+        const Guess gs = guess_of(c, site, std::min(j, kPredOuter - 1), 1);
+        const int guess = std::max(gs.n, 1);
         int k = 0;            // V-cycles of this inner loop enqueued
         bool open = true;     // the inner loop has not stopped
         bool pre = false;     // the sweeps (and test) of V-cycle k + 1 are enqueued
@@ -858,7 +877,7 @@ int mg_solve_mixed(nyl_ctx *c, nyl_mg_stats *st, int site) {
                 k++;
             }
             const bool max_now = nite + k >= maxite;
-            const bool ends = max_now || (first && sure);   // expected to stop here
+            const bool ends = max_now || (first && gs.ends);   // expected to stop here
             if (!max_now) {
                 int np = 0;
                 if (ends) rc = resid_norm<float>(c, &np);
@@ -905,12 +924,12 @@ int mg_solve_mixed(nyl_ctx *c, nyl_mg_stats *st, int site) {
             first = false;
         }
         if (k == 0) {   // the first outer residual was below the tolerance
-            c->pred[site][0] = 0;
+            set_guess(c, site, 0, 0);
             break;
         }
         nite += k;
         at_max = nite >= maxite;
-        if (j < kPredOuter) c->pred[site][j] = k;
+        if (j < kPredOuter) set_guess(c, site, j, k);
         if (!added) {
             if ((rc = add(nullptr)) || (rc = outer(0, true))) return rc;
             if ((rc = ctl_read(c, &normb, hist, 1))) return rc;
@@ -1206,7 +1225,7 @@ int nyl_ctx_create(const nyl_desc *desc, nyl_ctx **out) {
     build_layout(c);
     c->t0 = cycle_first(c);
     for (int q = 0; q < kSites; q++)
-        for (int j = 0; j < kPredOuter; j++) c->pred[q][j] = -1;
+        for (int j = 0; j < kPredOuter; j++) c->pred[q][j] = {-1, -1};
     c->stream = nullptr;
     *out = c;
     return NYL_OK;

@@ -9,6 +9,9 @@ namespace nyl {
 
 constexpr int kMaxLevels = 32;
 constexpr int kSites = 4, kPredOuter = 8;
+struct Pred {
+    int last, before;
+};
 constexpr int kHostCtl = 16;   // doubles of host_out before the solve's results
 
 struct Level {
@@ -49,10 +52,10 @@ struct nyl_ctx {
     double *host_dev;        // host_out as the device addresses it
     uint32_t pub_seq;        // last published result sequence number
     int total_cycles;
-    // V-cycles the last solves needed, by the place of the solve in a step
-    // (0: outside a step) and, in mixed precision, by outer step: how many
-    // the next one enqueues before it reads their tests (-1: not known yet)
-    int pred[nyl::kSites][nyl::kPredOuter];
+    // V-cycles the last two solves needed, by the place of the solve in a step
+    // (0: outside a step) and, in mixed precision, by outer step (-1: not
+    // known yet): the fewer of them are enqueued before their tests are read
+    nyl::Pred pred[nyl::kSites][nyl::kPredOuter];
     int t0;                  // first level of the single-workgroup cycle (nlev: none)
     nyl::CycleArgs cyc;
     nyl::CycleEnt cyc_ent[CYC_ENT];

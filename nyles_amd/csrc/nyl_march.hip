@@ -420,23 +420,26 @@ __global__ __launch_bounds__(256) void k_mg_march(MarchArgs<T, TC> a) {
 }
 
 // Tile width and march length of a level.  The width (64 or 32 columns, rows
-// to match) is the one that pads the level less; the march is the longest
-// that still gives the chip `want` blocks (each block evaluates R extra
-// planes, so long marches save work and short ones latency), and at least
-// long enough to keep within the partial sums of a residual norm.
-MarchGrid march_grid(const Geo &g, int es, bool even) {
-    auto up = [](int n, int t) { return (n + t - 1) / t; };
+// to match) is the one that pads the level less.  The march is the shortest
+// whose blocks are all resident at once (res per CU): a second round of
+// blocks waits for the first and repeats its prologue, a longer march leaves
+// SIMDs idle.  Measured (us, planes per block: time): prolongation and two
+// sweeps FP32 256^3 16: 66, 32: 57, 64: 83; 256x256x512 32: 126, 64: 119;
+// FP64 256^3 32: 120, 64: 113; 96^3 2: 23, 4: 16, 8: 19; two sweeps FP64
+// 96^3 2: 17, 4: 13, 8: 15.
+MarchGrid march_grid(const Geo &g, int res, bool even) {
+    auto up = [](int64_t n, int64_t t) { return (int)((n + t - 1) / t); };
     MarchGrid m;
     const int64_t a64 = (int64_t)up(g.nx, 64) * up(g.ny, 8), a32 = (int64_t)up(g.nx, 32) * up(g.ny, 16);
     m.tx = a32 < a64 ? 32 : 64;
     m.bx = up(g.nx, m.tx);
     m.by = up(g.ny, 512 / m.tx);
     const int64_t cols = (int64_t)m.bx * m.by;
-    const int64_t want = 1024;
-    int kz = es == 4 ? 16 : 32;
-    const int least = even ? 2 : 1;
-    while (kz > least && cols * up(g.nz, kz) < want) kz >>= 1;
-    while (cols * up(g.nz, kz) > NYL_RED_BLOCKS && kz < g.nz) kz <<= 1;
+    int64_t bz = 256 * (int64_t)res / cols;
+    if (bz < 1) bz = 1;
+    int kz = up(g.nz, bz);
+    if (even && (kz & 1)) kz++;
+    if (kz < 2) kz = 2;
     m.kz = kz;
     m.bz = up(g.nz, kz);
     return m;
@@ -445,7 +448,8 @@ MarchGrid march_grid(const Geo &g, int es, bool even) {
 #define MARCH_GO(T, TC, SRC, NSW, RESN, RESTR, OUTER)                                          \
     do {                                                                                      \
         MarchArgs<T, TC> m = a;                                                               \
-        const MarchGrid gr = march_grid(a.g, (int)sizeof(T), (RESTR) || (SRC) == MS_PROLONG); \
+        const MarchGrid gr = march_grid(a.g, march_resident(sizeof(T), SRC, NSW, RESTR),      \
+                                        (RESTR) || (SRC) == MS_PROLONG);                      \
         m.kz = gr.kz;                                                                         \
         const dim3 grd(gr.bx, gr.by, gr.bz), blk(256);                                        \
         if (gr.tx == 64)                                                                      \
