@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "nyl_ctx.h"
+#include "nyl_march.h"
 
 using namespace nyl;
 
@@ -33,8 +34,7 @@ uint64_t al256(uint64_t v) { return (v + 255) & ~uint64_t(255); }
 
 // one launch of a plan
 enum LKind {
-    L_STAGE, L_DIV, L_CORR, L_DIAG, L_SWEEP, L_RESTR, L_PROL, L_RED, L_OUTER, L_FINAL,
-    L_ACC, L_COARSE
+    L_STAGE, L_DIV, L_CORR, L_DIAG, L_SWEEP, L_RED, L_MARCH, L_CYCLE, L_FINAL, L_ACC, L_COARSE
 };
 enum LType { T_D, T_F, T_FD };   // double, float, float fine over double coarse
 
@@ -45,7 +45,8 @@ struct Launch {
     int nitems;
     int64_t nblk;
     int arg;            // mode / kind / what / periodicity
-    int arg2;           // stage: periodicity class
+    int arg2;           // stage: periodicity class; march: skip members that have stopped
+    uint64_t off2;      // march: the item of each block
 };
 
 }  // namespace
@@ -65,7 +66,7 @@ struct nyl_batch {
     MGTabs tabs;
     // device control arrays (offsets)
     uint64_t o_normb, o_res, o_shift, o_tol, o_nite, o_maxite, o_active, o_any, o_dt, o_acc;
-    BMG mg;
+    BMG mg = {};
     // plans
     std::vector<Launch> pre[2][3], vcyc, post[2];
     std::vector<char> blob;     // host image of the item tables
@@ -104,6 +105,7 @@ Launch add_table(nyl_batch *b, LKind kind, LType type, const std::vector<I> &ite
     L.nblk = nblk;
     L.arg = arg;
     L.arg2 = arg2;
+    L.off2 = 0;
     b->blob.resize(L.off + sizeof(I) * items.size());
     memcpy(b->blob.data() + L.off, items.data(), sizeof(I) * items.size());
     return L;
@@ -182,9 +184,157 @@ Launch final_table(nyl_batch *b, const std::vector<int> &nparts, int kind) {
 // partials buffer (kind 2 stores two sets)
 constexpr int64_t kRedCap = NYL_RED_BLOCKS / 2;
 
+bool b_lev64(const nyl_batch *b, int q, int l) { return lev64(b->m[q], l); }
+
+// Levels of a member between the finest and its single-workgroup cycle (or
+// its coarsest level) run the marches; their corrections end in y, as that of
+// the cycle's first level; a coarsest level's in x.
+bool marched(const nyl_ctx *c, int l) { return l < std::min(c->t0, c->nlev - 1); }
+uint64_t correction(const nyl_ctx *c, int l) {
+    return l == c->nlev - 1 ? c->lev[l].x : c->lev[l].y;
+}
+
+// Planes per block of a member's level: its own, whatever the batch, so that
+// the block sums of its residual norms are.  Short marches for small levels
+// (a batch has blocks enough only when its members do).
+int march_kz(const Geo &g) {
+    int kz = gcells(g) < (1 << 18) ? 4 : 8;
+    const int64_t cols = (int64_t)((g.nx + 31) / 32) * ((g.ny + 15) / 16);
+    while (cols * ((g.nz + kz - 1) / kz) > NYL_RED_BLOCKS && kz < g.nz) kz *= 2;
+    return kz;
+}
+int64_t march_blocks(const Geo &g) {
+    const int kz = march_kz(g);
+    return (int64_t)((g.nx + 31) / 32) * ((g.ny + 15) / 16) * ((g.nz + kz - 1) / kz);
+}
+
+// which members a pass of level 0 covers: up to 1M cells the sweeps and the
+// restriction run as one pass, above that as two (see pre_smooth in
+// nyl_api.hip)
+enum Size { kAny, kSmall, kLarge };
+bool of_size(const nyl_ctx *c, Size s) {
+    const bool small = gcells(c->lev[0].g) <= (1 << 20);
+    return s == kAny || small == (s == kSmall);
+}
+
+// one pass (kind) over level l of the members whose levels l and l + 1 have
+// the types T and TC
+template <typename T, typename TC>
+void level_pass_t(nyl_batch *b, int l, MarchKind kind, LType type, std::vector<Launch> &out,
+                  bool gated, Size size) {
+    std::vector<MarchItem<T, TC>> v;
+    std::vector<uint16_t> map;
+    const bool f64 = std::is_same<T, double>::value, c64 = std::is_same<TC, double>::value;
+    int64_t nb = 0;
+    for (int q = 0; q < b->n; q++) {
+        nyl_ctx *c = b->m[q];
+        if (!of_size(c, size)) continue;
+        if (kind != MK_OUTER) {
+            if (l + 1 >= c->nlev || b_lev64(b, q, l) != f64 || b_lev64(b, q, l + 1) != c64) continue;
+            if (l > 0 && !marched(c, l)) continue;
+        }
+        const Level &f = c->lev[l], &k = c->lev[l + 1 < c->nlev ? l + 1 : l];
+        MarchItem<T, TC> it = {};
+        MarchArgs<T, TC> &a = it.a;
+        a.g = f.g;
+        a.gc = k.g;
+        a.kz = march_kz(f.g);
+        a.omega = c->d.mg_omega;
+        a.partials = F<double>(c, c->partials);
+        it.bx = (f.g.nx + 31) / 32;
+        it.by = (f.g.ny + 15) / 16;
+        it.h.g = f.g;
+        it.h.member = q;
+        it.h.nblk = (int)march_blocks(f.g);
+        it.h.start = nb;
+        nb += it.h.nblk;
+        if (kind == MK_OUTER) {
+            a.src = F<T>(c, c->mgx);
+            a.b = F<T>(c, c->mgb);
+            a.rout = F<float>(c, f.b);
+            a.shift = b->mg.shift ? b->mg.shift + q : nullptr;
+        } else {
+            T *x = F<T>(c, f.x), *y = F<T>(c, f.y);
+            a.b = F<T>(c, f.b);
+            a.bc = F<TC>(c, k.b);
+            a.yc = F<TC>(c, k.y);
+            a.xc = F<TC>(c, correction(c, l + 1));
+            switch (kind) {
+            case MK_UP: case MK_UP_ADD:
+                // level 0: both pre-sweeps are in y
+                a.src = l > 0 ? x : y;
+                a.dst = l > 0 ? y : x;
+                a.xadd = kind == MK_UP_ADD ? F<double>(c, c->mgx) : nullptr;
+                break;
+            case MK_DOWN: a.src = y; a.dst = x; break;
+            case MK_RESTRICT: a.src = y; break;
+            default: a.src = x; a.dst = y; break;   // level 0's pre-smoothing
+            }
+        }
+        map.insert(map.end(), it.h.nblk, (uint16_t)v.size());
+        v.push_back(it);
+    }
+    if (v.empty()) return;
+    Launch L = add_table(b, L_MARCH, type, v, nb, kind, gated);
+    L.off2 = al256(b->blob.size());
+    b->blob.resize(L.off2 + sizeof(uint16_t) * map.size());
+    memcpy(b->blob.data() + L.off2, map.data(), sizeof(uint16_t) * map.size());
+    out.push_back(L);
+}
+
+void level_pass(nyl_batch *b, int l, MarchKind kind, std::vector<Launch> &out, bool gated,
+                Size size = kAny) {
+    if (kind != MK_UP_ADD) level_pass_t<double, double>(b, l, kind, T_D, out, gated, size);
+    if (kind == MK_OUTER) return;
+    level_pass_t<float, float>(b, l, kind, T_F, out, gated, size);
+    level_pass_t<float, double>(b, l, kind, T_FD, out, gated, size);
+}
+
+// the cycles of the members whose cycle starts on a level of type T
+template <typename T>
+void cycle_launch(nyl_batch *b, std::vector<Launch> &out) {
+    std::vector<CycleItem<T>> v;
+    int most = 0;
+    for (int q = 0; q < b->n; q++) {
+        nyl_ctx *c = b->m[q];
+        if (c->t0 >= c->nlev || b_lev64(b, q, c->t0) != std::is_same<T, double>::value) continue;
+        const Level &f = c->lev[c->t0];
+        CycleItem<T> it = {};
+        it.member = q;
+        it.a = c->cyc;
+        it.b = F<T>(c, f.b);
+        it.y = F<T>(c, f.y);
+        it.x = F<T>(c, f.x);
+        most = std::max(most, c->cyc.n0);
+        v.push_back(it);
+    }
+    if (!v.empty())
+        out.push_back(add_table(b, L_CYCLE, std::is_same<T, double>::value ? T_D : T_F, v,
+                                (int64_t)v.size(), most));
+}
+
+// The residual test of every member (gated: those that have not stopped).
+// FP64: the norm comes with both pre-smoothing sweeps of the next V-cycle
+// into y and their restriction (unused when it stops the solve); mixed: the
+// FP64 outer residual, which is the next V-cycle's right-hand side.
+void test_launches(nyl_batch *b, std::vector<Launch> &out, bool gated) {
+    if (b->mixed) {
+        level_pass(b, 0, MK_OUTER, out, gated);
+    } else {
+        level_pass(b, 0, MK_PRE_RESTRICT, out, gated, kSmall);
+        level_pass(b, 0, MK_PRE, out, gated, kLarge);
+        level_pass(b, 0, MK_RESTRICT, out, gated, kLarge);
+    }
+}
+std::vector<int> test_blocks(const nyl_batch *b) {
+    std::vector<int> np(b->n);
+    for (int q = 0; q < b->n; q++) np[q] = (int)march_blocks(b->m[q]->lev[0].g);
+    return np;
+}
+
 template <typename T>
 void build_pre(nyl_batch *b, int p, int st, std::vector<Launch> &out) {
-    if (st == 1) out.push_back(Launch{L_ACC, T_D, 0, 0, 0, 0, 0});   // zero the V-cycle counts
+    if (st == 1) out.push_back(Launch{L_ACC, T_D, 0, 0, 0, 0, 0, 0});   // zero the V-cycle counts
     build_stage<T>(b, p, st, out);
     // divergence of the new state into the FP64 right-hand side
     {
@@ -204,99 +354,44 @@ void build_pre(nyl_batch *b, int p, int st, std::vector<Launch> &out) {
         out.push_back(add_table(b, L_DIV, b->mixed ? T_F : T_D, v, nb));
     }
     std::vector<int> np(b->n);
-    if (!b->mixed) {
-        // normb = |b|^2, then the residual of the warm-started x
-        std::vector<RedItem<double>> v0, v1;
-        int64_t nb0 = 0, nb1 = 0;
-        for (int q = 0; q < b->n; q++) {
-            nyl_ctx *c = b->m[q];
-            RedItem<double> it;
-            it.h = head(c->lev[0].g, q, gcells(c->lev[0].g), nb0, kRedCap);
-            it.v = F<double>(c, c->lev[0].b);
-            it.b = nullptr;
-            it.partials = F<double>(c, c->partials);
-            np[q] = it.h.nblk;
-            v0.push_back(it);
-            it.h = head(c->lev[0].g, q, gcells(c->lev[0].g), nb1, kRedCap);
-            it.v = F<double>(c, c->lev[0].x);
-            it.b = F<double>(c, c->lev[0].b);
-            v1.push_back(it);
-        }
-        out.push_back(add_table(b, L_RED, T_D, v0, nb0, 0));
-        out.push_back(final_table(b, np, NYL_FIN_NORMB));
-        out.push_back(add_table(b, L_RED, T_D, v1, nb1, 1));
-        out.push_back(final_table(b, np, NYL_FIN_INIT));
-    } else {
-        // sum and sum of squares of b (mean removal, normb), then the FP64
-        // outer residual of x
-        std::vector<RedItem<double>> v0;
-        std::vector<OuterItem> v1;
-        int64_t nb0 = 0, nb1 = 0;
-        std::vector<int> np1(b->n);
-        for (int q = 0; q < b->n; q++) {
-            nyl_ctx *c = b->m[q];
-            RedItem<double> it;
-            it.h = head(c->lev[0].g, q, gcells(c->lev[0].g), nb0, kRedCap);
-            it.v = F<double>(c, c->mgb);
-            it.b = nullptr;
-            it.partials = F<double>(c, c->partials);
-            np[q] = it.h.nblk;
-            v0.push_back(it);
-            OuterItem o;
-            o.h = head(c->lev[0].g, q, gcells(c->lev[0].g), nb1, kRedCap);
-            o.x = F<double>(c, c->mgx); o.b = F<double>(c, c->mgb);
-            o.r = F<float>(c, c->lev[0].b); o.y = F<float>(c, c->lev[0].y);
-            o.omega = c->d.mg_omega;
-            o.partials = F<double>(c, c->partials);
-            np1[q] = o.h.nblk;
-            v1.push_back(o);
-        }
-        out.push_back(add_table(b, L_RED, T_D, v0, nb0, 2));
-        out.push_back(final_table(b, np, NYL_FIN_SHIFT));
-        out.push_back(add_table(b, L_OUTER, T_D, v1, nb1));
-        out.push_back(final_table(b, np1, NYL_FIN_INIT));
+    // FP64: normb = |b|^2; mixed: sum and sum of squares of b (mean removal,
+    // normb)
+    std::vector<RedItem> v;
+    int64_t nb = 0;
+    for (int q = 0; q < b->n; q++) {
+        nyl_ctx *c = b->m[q];
+        RedItem it;
+        it.h = head(c->lev[0].g, q, gcells(c->lev[0].g), nb, kRedCap);
+        it.v = F<double>(c, c->mgb);
+        it.partials = F<double>(c, c->partials);
+        np[q] = it.h.nblk;
+        v.push_back(it);
     }
+    out.push_back(add_table(b, L_RED, T_D, v, nb, b->mixed ? 2 : 0));
+    out.push_back(final_table(b, np, b->mixed ? NYL_FIN_SHIFT : NYL_FIN_NORMB));
+    // then the residual of the warm-started x
+    test_launches(b, out, false);
+    out.push_back(final_table(b, test_blocks(b), NYL_FIN_INIT));
 }
 
-// Level element types of member q: FP64 batch: all double; mixed: FP32
-// except the coarsest level.
-bool b_lev64(const nyl_batch *b, int q, int l) { return lev64(b->m[q], l); }
-
-// the sweeps x -> y (first) and/or y -> x (second) of level l for members
-// whose level l has the type T and that have more than `below` levels below l
-template <typename T>
-void sweep_launch(nyl_batch *b, int l, bool first, bool second, bool t64,
-                  std::vector<Launch> &out, bool skip_first_l0, int below = 0,
-                  bool addx_l0 = false) {
-    for (int pass = 0; pass < 2; pass++) {
-        if ((pass == 0 && !first) || (pass == 1 && !second)) continue;
-        std::vector<SweepItem<T>> v;
-        int64_t nb = 0;
-        for (int q = 0; q < b->n; q++) {
-            nyl_ctx *c = b->m[q];
-            if (l + below >= c->nlev || b_lev64(b, q, l) != t64) continue;
-            if (pass == 0 && l == 0 && skip_first_l0) continue;
-            if (c->exact && l == c->nlev - 1) continue;   // solved directly
-            const Level &f = c->lev[l];
-            SweepItem<T> it;
-            it.h = head(f.g, q, gcells(f.g), nb);
-            it.src = F<T>(c, pass == 0 ? f.x : f.y);
-            it.dst = F<T>(c, pass == 0 ? f.y : f.x);
-            it.b = F<T>(c, f.b);
-            it.omega = c->d.mg_omega;
-            // the mixed solve's last sweep of a V-cycle adds its result to x
-            it.xo = (addx_l0 && pass == 1 && l == 0) ? F<double>(c, c->mgx) : nullptr;
-            v.push_back(it);
-        }
-        if (!v.empty()) out.push_back(add_table(b, L_SWEEP, t64 ? T_D : T_F, v, nb));
+// the second sweep (y -> x) of a coarsest level l that is neither in its
+// member's cycle nor solved directly
+void coarse_sweep(nyl_batch *b, int l, std::vector<Launch> &out) {
+    std::vector<SweepItem> v;
+    int64_t nb = 0;
+    for (int q = 0; q < b->n; q++) {
+        nyl_ctx *c = b->m[q];
+        if (l != c->nlev - 1 || c->exact || c->t0 < c->nlev) continue;
+        const Level &f = c->lev[l];
+        SweepItem it;
+        it.h = head(f.g, q, gcells(f.g), nb);
+        it.src = F<double>(c, f.y);
+        it.dst = F<double>(c, f.x);
+        it.b = F<double>(c, f.b);
+        it.omega = c->d.mg_omega;
+        v.push_back(it);
     }
-}
-
-void smooth_launches(nyl_batch *b, int l, std::vector<Launch> &out, bool skip_first_l0) {
-    sweep_launch<double>(b, l, true, false, true, out, skip_first_l0);
-    sweep_launch<float>(b, l, true, false, false, out, skip_first_l0);
-    sweep_launch<double>(b, l, false, true, true, out, skip_first_l0);
-    sweep_launch<float>(b, l, false, true, false, out, skip_first_l0);
+    if (!v.empty()) out.push_back(add_table(b, L_SWEEP, T_D, v, nb));
 }
 
 // the direct solve of the members whose coarsest level is l and has an odd
@@ -307,7 +402,7 @@ void coarse_launches(nyl_batch *b, int l, std::vector<Launch> &out) {
         int64_t nb = 0;
         for (int q = 0; q < b->n; q++) {
             nyl_ctx *c = b->m[q];
-            if (!c->exact || l != c->nlev - 1) continue;
+            if (!c->exact || l != c->nlev - 1 || c->t0 < c->nlev) continue;
             const Level &f = c->lev[l];
             CoarseItem it;
             it.h.g = f.g;
@@ -326,97 +421,26 @@ void coarse_launches(nyl_batch *b, int l, std::vector<Launch> &out) {
     }
 }
 
-template <typename Tf, typename Tc>
-void restrict_launch(nyl_batch *b, int l, LType type, std::vector<Launch> &out) {
-    std::vector<RestrItem<Tf, Tc>> v;
-    int64_t nb = 0;
-    const bool f64 = std::is_same<Tf, double>::value, c64 = std::is_same<Tc, double>::value;
-    for (int q = 0; q < b->n; q++) {
-        nyl_ctx *c = b->m[q];
-        if (l + 1 >= c->nlev || b_lev64(b, q, l) != f64 || b_lev64(b, q, l + 1) != c64) continue;
-        const Level &f = c->lev[l], &k = c->lev[l + 1];
-        RestrItem<Tf, Tc> it;
-        it.h = head(f.g, q, gcells(k.g), nb);
-        it.gc = k.g;
-        it.x = F<Tf>(c, f.x); it.b = F<Tf>(c, f.b);
-        it.bc = F<Tc>(c, k.b); it.xc = F<Tc>(c, k.x);
-        v.push_back(it);
-    }
-    if (!v.empty()) out.push_back(add_table(b, L_RESTR, type, v, nb));
-}
-
-template <typename Tf, typename Tc>
-void prolong_launch(nyl_batch *b, int l, LType type, std::vector<Launch> &out) {
-    std::vector<ProlItem<Tf, Tc>> v;
-    int64_t nb = 0;
-    const bool f64 = std::is_same<Tf, double>::value, c64 = std::is_same<Tc, double>::value;
-    for (int q = 0; q < b->n; q++) {
-        nyl_ctx *c = b->m[q];
-        if (l + 1 >= c->nlev || b_lev64(b, q, l) != f64 || b_lev64(b, q, l + 1) != c64) continue;
-        const Level &f = c->lev[l], &k = c->lev[l + 1];
-        ProlItem<Tf, Tc> it;
-        it.h = head(f.g, q, gcells(f.g), nb);
-        it.gc = k.g;
-        it.xf = F<Tf>(c, f.x); it.xc = F<Tc>(c, k.x);
-        v.push_back(it);
-    }
-    if (!v.empty()) out.push_back(add_table(b, L_PROL, type, v, nb));
-}
-
 // one V-cycle of every active member (core/mgfor/solvers.f90:35-55) and the
-// stop rule after it
+// stop rule after it.  FP64: both pre-smoothing sweeps and the restriction of
+// level 0 ran with the test before it; mixed: they start from e = 0.
 void build_vcycle(nyl_batch *b, std::vector<Launch> &out) {
-    const bool skip = b->mixed != 0;   // mixed: the first level-1 sweep comes from the outer residual
-    for (int l = 0; l < b->lmax; l++) {
-        smooth_launches(b, l, out, skip);
+    if (b->mixed) {
+        level_pass(b, 0, MK_ZERO_RESTRICT, out, true, kSmall);
+        level_pass(b, 0, MK_ZERO, out, true, kLarge);
+        level_pass(b, 0, MK_RESTRICT, out, true, kLarge);
+    }
+    for (int l = 1; l < b->lmax; l++) level_pass(b, l, MK_DOWN, out, true);
+    cycle_launch<double>(b, out);
+    cycle_launch<float>(b, out);
+    for (int l = 1; l < b->lmax; l++) {
+        coarse_sweep(b, l, out);
         coarse_launches(b, l, out);
-        restrict_launch<double, double>(b, l, T_D, out);
-        restrict_launch<float, float>(b, l, T_F, out);
-        restrict_launch<float, double>(b, l, T_FD, out);
     }
-    for (int l = b->lmax - 2; l >= 0; l--) {
-        prolong_launch<double, double>(b, l, T_D, out);
-        prolong_launch<float, float>(b, l, T_F, out);
-        prolong_launch<float, double>(b, l, T_FD, out);
-        // post-smoothing of the members that have a level below l
-        sweep_launch<double>(b, l, true, false, true, out, false, 1);
-        sweep_launch<float>(b, l, true, false, false, out, false, 1);
-        sweep_launch<double>(b, l, false, true, true, out, false, 1);
-        sweep_launch<float>(b, l, false, true, false, out, false, 1, b->mixed != 0);
-    }
-    std::vector<int> np(b->n);
-    if (!b->mixed) {
-        std::vector<RedItem<double>> v;
-        int64_t nb = 0;
-        for (int q = 0; q < b->n; q++) {
-            nyl_ctx *c = b->m[q];
-            RedItem<double> it;
-            it.h = head(c->lev[0].g, q, gcells(c->lev[0].g), nb, kRedCap);
-            it.v = F<double>(c, c->lev[0].x);
-            it.b = F<double>(c, c->lev[0].b);
-            it.partials = F<double>(c, c->partials);
-            np[q] = it.h.nblk;
-            v.push_back(it);
-        }
-        out.push_back(add_table(b, L_RED, T_D, v, nb, 1, 1));   // gated by active
-    } else {
-        // x += e was done by the last level-1 sweep (its result added to x)
-        std::vector<OuterItem> vo;
-        int64_t nbo = 0;
-        for (int q = 0; q < b->n; q++) {
-            nyl_ctx *c = b->m[q];
-            OuterItem o;
-            o.h = head(c->lev[0].g, q, gcells(c->lev[0].g), nbo, kRedCap);
-            o.x = F<double>(c, c->mgx); o.b = F<double>(c, c->mgb);
-            o.r = F<float>(c, c->lev[0].b); o.y = F<float>(c, c->lev[0].y);
-            o.omega = c->d.mg_omega;
-            o.partials = F<double>(c, c->partials);
-            np[q] = o.h.nblk;
-            vo.push_back(o);
-        }
-        out.push_back(add_table(b, L_OUTER, T_D, vo, nbo, 0, 1));   // gated by active
-    }
-    out.push_back(final_table(b, np, NYL_FIN_STEP));
+    for (int l = b->lmax - 2; l >= 1; l--) level_pass(b, l, MK_UP, out, true);
+    level_pass(b, 0, b->mixed ? MK_UP_ADD : MK_UP, out, true);
+    test_launches(b, out, true);
+    out.push_back(final_table(b, test_blocks(b), NYL_FIN_STEP));
 }
 
 template <typename T>
@@ -448,7 +472,7 @@ void build_post(nyl_batch *b, int p, std::vector<Launch> &out) {
     const LType t = b->mixed ? T_F : T_D;
     out.push_back(add_table(b, L_CORR, t, vc, nbc));
     out.push_back(add_table(b, L_DIAG, t, vd, nbd, 6));
-    out.push_back(Launch{L_ACC, T_D, 0, 0, 0, 1, 0});   // add this stage's V-cycles
+    out.push_back(Launch{L_ACC, T_D, 0, 0, 0, 1, 0, 0});   // add this stage's V-cycles
 }
 
 void destroy_graphs(nyl_batch *b) {
@@ -504,28 +528,27 @@ int run_launch(nyl_batch *b, const Launch &L) {
         else BCHK(launch_b_diag<double>((const DiagItem<double> *)tab, L.nitems, L.nblk, L.arg, s));
         break;
     case L_SWEEP:
-        if (L.type == T_F) BCHK(launch_b_sweep<float>((const SweepItem<float> *)tab, L.nitems, L.nblk, b->tabs, act, s));
-        else BCHK(launch_b_sweep<double>((const SweepItem<double> *)tab, L.nitems, L.nblk, b->tabs, act, s));
-        break;
-    case L_RESTR:
-        if (L.type == T_F) BCHK(launch_b_restrict<float, float>((const RestrItem<float, float> *)tab, L.nitems, L.nblk, b->tabs, act, s));
-        else if (L.type == T_FD) BCHK(launch_b_restrict<float, double>((const RestrItem<float, double> *)tab, L.nitems, L.nblk, b->tabs, act, s));
-        else BCHK(launch_b_restrict<double, double>((const RestrItem<double, double> *)tab, L.nitems, L.nblk, b->tabs, act, s));
-        break;
-    case L_PROL:
-        if (L.type == T_F) BCHK(launch_b_prolong<float, float>((const ProlItem<float, float> *)tab, L.nitems, L.nblk, b->tabs, act, s));
-        else if (L.type == T_FD) BCHK(launch_b_prolong<float, double>((const ProlItem<float, double> *)tab, L.nitems, L.nblk, b->tabs, act, s));
-        else BCHK(launch_b_prolong<double, double>((const ProlItem<double, double> *)tab, L.nitems, L.nblk, b->tabs, act, s));
+        BCHK(launch_b_sweep((const SweepItem *)tab, L.nitems, L.nblk, b->tabs, act, s));
         break;
     case L_RED:
-        // the initial reductions run for every member, the V-cycle's (arg2) for active ones
-        BCHK(launch_b_reduce<double>((const RedItem<double> *)tab, L.nitems, L.nblk, L.arg,
-                                     b->tabs, L.arg2 ? act : nullptr, s));
+        BCHK(launch_b_reduce((const RedItem *)tab, L.nitems, L.nblk, L.arg, s));
         break;
-    case L_OUTER:
-        // the initial residual runs for every member, the V-cycle's (arg2) for active ones
-        BCHK(launch_b_outer_resid((const OuterItem *)tab, L.nitems, L.nblk, b->mg, b->tabs,
-                                  L.arg2 ? act : nullptr, s));
+    case L_MARCH: {
+        // the initial residual runs for every member
+        const int *gate = L.arg2 ? act : nullptr;
+        const uint16_t *map = (const uint16_t *)(b->ws + tables_off(b) + L.off2);
+        const MarchKind kind = (MarchKind)L.arg;
+        if (L.type == T_F)
+            BCHK((launch_b_march<float, float>((const MarchItem<float, float> *)tab, map, L.nblk, kind, b->tabs, gate, s)));
+        else if (L.type == T_FD)
+            BCHK((launch_b_march<float, double>((const MarchItem<float, double> *)tab, map, L.nblk, kind, b->tabs, gate, s)));
+        else
+            BCHK((launch_b_march<double, double>((const MarchItem<double, double> *)tab, map, L.nblk, kind, b->tabs, gate, s)));
+        break;
+    }
+    case L_CYCLE:
+        if (L.type == T_F) BCHK(launch_b_cycle<float>((const CycleItem<float> *)tab, L.nitems, L.arg, act, s));
+        else BCHK(launch_b_cycle<double>((const CycleItem<double> *)tab, L.nitems, L.arg, act, s));
         break;
     case L_FINAL:
         BCHK(launch_b_final((const FinalItem *)tab, L.nitems, L.arg, b->mg, s));
@@ -743,6 +766,9 @@ int nyl_batch_bind_workspace(nyl_batch *b, void *dptr, uint64_t bytes) {
     mg.nite = (int *)(b->ws + b->o_nite); mg.maxite = (int *)(b->ws + b->o_maxite);
     mg.active = (int *)(b->ws + b->o_active); mg.any = (int *)(b->ws + b->o_any);
     mg.acc = (int *)(b->ws + b->o_acc);
+    // the tables hold addresses in this workspace
+    if (b->mixed) build_plans<float>(b);
+    else build_plans<double>(b);
     std::vector<char> ctl(tables_off(b), 0);
     for (int q = 0; q < n; q++) {
         ((double *)(ctl.data() + b->o_tol))[q] = b->m[q]->d.mg_tol;

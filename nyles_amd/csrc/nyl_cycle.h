@@ -105,4 +105,17 @@ template <typename T>
 hipError_t launch_mg_cycle(const CycleArgs &a, const T *b, T *y, T *x, const CtlArgs *fin,
                            hipStream_t s);
 
+// one member's cycle in a batch (a.bytes and a.n0 as for the single launch)
+template <typename T>
+struct CycleItem {
+    int member;
+    CycleArgs a;
+    const T *b;
+    T *y, *x;
+};
+// most: the largest a.n0 of the items
+template <typename T>
+hipError_t launch_b_cycle(const CycleItem<T> *items, int n, int most, const int *active,
+                          hipStream_t s);
+
 }  // namespace nyl

@@ -406,6 +406,34 @@ __global__ __launch_bounds__(CYC_T) void k_mg_cycle(CycleArgs a, const T *gb, T 
     cycle_body<T, R>(a, gb, gy, gx, reinterpret_cast<char *>(lds), slev, ent, tb, threadIdx.x);
 }
 
+// the cycles of a batch's members, one workgroup each
+template <typename T, int R>
+__global__ __launch_bounds__(CYC_T) void k_b_cycle(const CycleItem<T> *__restrict__ items,
+                                                   const int *__restrict__ active) {
+    __shared__ double lds[CYC_LDS / sizeof(double)];
+    __shared__ uint32_t slev[CYC_MAXLEV * sizeof(CycleLevel) / 4];
+    __shared__ CycleEnt ent[CYC_ENT];
+    __shared__ double tb[32];
+    const CycleItem<T> &it = items[blockIdx.x];
+    if (!active[it.member]) return;
+    cycle_body<T, R>(it.a, it.b, it.y, it.x, reinterpret_cast<char *>(lds), slev, ent, tb,
+                     threadIdx.x);
+}
+
+template <typename T>
+hipError_t launch_b_cycle(const CycleItem<T> *items, int n, int most, const int *active,
+                          hipStream_t s) {
+    const dim3 grd(n), blk(CYC_T);
+    if (most <= CYC_T) NYL_LAUNCH((k_b_cycle<T, 1>), grd, blk, 0, s, items, active);
+    else if (most <= 2 * CYC_T) NYL_LAUNCH((k_b_cycle<T, 2>), grd, blk, 0, s, items, active);
+    else NYL_LAUNCH((k_b_cycle<T, CYC_R>), grd, blk, 0, s, items, active);
+    return hipGetLastError();
+}
+template hipError_t launch_b_cycle<double>(const CycleItem<double> *, int, int, const int *,
+                                           hipStream_t);
+template hipError_t launch_b_cycle<float>(const CycleItem<float> *, int, int, const int *,
+                                          hipStream_t);
+
 bool cycle_layout(CycleArgs &a, CycleEnt *ent, const Geo *lev, int l0, int nlev, int es,
                   bool exact, double omega, const MGTabs &tab) {
     a = CycleArgs{};

@@ -299,17 +299,10 @@ template <typename T> struct StageItem { BHead h; StageArgs<T> a; };
 template <typename T> struct DivItem { BHead h; DivArgs<T, double> a; };
 template <typename T> struct CorrItem { BHead h; CorrectArgs<T, double> a; };
 template <typename T> struct DiagItem { BHead h; DiagArgs<T> a; };
-// xo non-null: the sweep result is added to xo (FP64) instead of stored in dst
-template <typename T> struct SweepItem { BHead h; const T *src; T *dst; const T *b; double omega;
-                                         double *xo; };
-template <typename Tf, typename Tc>
-struct RestrItem { BHead h; Geo gc; const Tf *x; const Tf *b; Tc *bc; Tc *xc; };
-template <typename Tf, typename Tc>
-struct ProlItem { BHead h; Geo gc; Tf *xf; const Tc *xc; };
-// per-member partial sums: v (norm2 / sum and sum of squares) or x, b (residual)
-template <typename T> struct RedItem { BHead h; const T *v; const T *b; double *partials; };
-struct OuterItem { BHead h; const double *x; const double *b; float *r; float *y; double omega;
-                   double *partials; };
+// one sweep of a coarsest level
+struct SweepItem { BHead h; const double *src; double *dst; const double *b; double omega; };
+// per-member partial sums of v
+struct RedItem { BHead h; const double *v; double *partials; };
 // h.nblk = nz (passes 0, 2) or ny (pass 1) of the member's coarsest level
 struct CoarseItem { BHead h; CoarseArgs a; };
 
@@ -351,23 +344,11 @@ template <typename T>
 hipError_t launch_b_correct(const CorrItem<T> *items, int n, int64_t nblk, hipStream_t s);
 template <typename T>
 hipError_t launch_b_diag(const DiagItem<T> *items, int n, int64_t nblk, int what, hipStream_t s);
-template <typename T>
-hipError_t launch_b_sweep(const SweepItem<T> *items, int n, int64_t nblk, const MGTabs &tab,
+hipError_t launch_b_sweep(const SweepItem *items, int n, int64_t nblk, const MGTabs &tab,
                           const int *active, hipStream_t s);
-template <typename Tf, typename Tc>
-hipError_t launch_b_restrict(const RestrItem<Tf, Tc> *items, int n, int64_t nblk,
-                             const MGTabs &tab, const int *active, hipStream_t s);
-template <typename Tf, typename Tc>
-hipError_t launch_b_prolong(const ProlItem<Tf, Tc> *items, int n, int64_t nblk,
-                            const MGTabs &tab, const int *active, hipStream_t s);
-// kind 0: sum v^2; 1: sum of squared residuals of (v = x, b); 2: sum v and sum v^2
-// (second set of partials at partials + nblk of the member)
-template <typename T>
-hipError_t launch_b_reduce(const RedItem<T> *items, int n, int64_t nblk, int kind,
-                           const MGTabs &tab, const int *active, hipStream_t s);
-// active null: every member (the initial residual of a solve)
-hipError_t launch_b_outer_resid(const OuterItem *items, int n, int64_t nblk, const BMG &mg,
-                                const MGTabs &tab, const int *active, hipStream_t s);
+// kind 0: sum v^2; 2: sum v and sum v^2 (second set of partials at partials +
+// nblk of the member)
+hipError_t launch_b_reduce(const RedItem *items, int n, int64_t nblk, int kind, hipStream_t s);
 hipError_t launch_b_final(const FinalItem *items, int n, int kind, const BMG &mg, hipStream_t s);
 hipError_t launch_b_coarse(const CoarseItem *items, int n, int64_t nblk, int pass,
                            const int *active, hipStream_t s);

@@ -24,9 +24,26 @@ struct MarchArgs {
     double *partials;       // one per block: sum of the input's squared residuals
     float *rout;            // outer residual: r of the input, in the inner precision
     const double *shift;    // outer residual: subtracted from b (null: 0)
+    double *xadd;           // MK_UP_ADD: the result is added to xadd instead of stored in dst
     const int *gate;        // the pass does nothing when *gate != 0 (null: always runs)
     int kz;                 // planes per block
 };
+
+// One member's share of a batched pass (tiles of 32 x 16 columns): a.kz is
+// the member's own, so its block sums do not depend on the batch.
+template <typename T, typename TC>
+struct MarchItem {
+    BHead h;
+    int bx, by;
+    MarchArgs<T, TC> a;
+};
+enum MarchKind {
+    MK_UP, MK_UP_ADD, MK_DOWN, MK_RESTRICT, MK_PRE, MK_PRE_RESTRICT, MK_ZERO, MK_ZERO_RESTRICT, MK_OUTER
+};
+// map: the item of each block
+template <typename T, typename TC>
+hipError_t launch_b_march(const MarchItem<T, TC> *items, const uint16_t *map, int64_t nblk,
+                          MarchKind kind, const MGTabs &tab, const int *active, hipStream_t s);
 
 // Blocks of a pass over a level, and their march length.  even: the march
 // works on plane pairs (restriction or prolongation).

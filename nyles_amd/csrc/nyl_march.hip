@@ -33,8 +33,10 @@ __device__ __forceinline__ int wrap_any(int m, int n) {
 // Every value is the per-cell kernel's expression (sweep_cell, residual_at,
 // restrict_cell, prolong_term) in its order, so the results are bitwise those
 // of the separate launches.
-template <typename T, typename TC, int TX, int SRC, int NSW, bool RESN, bool RESTR, bool OUTER>
-__global__ __launch_bounds__(256) void k_mg_march(MarchArgs<T, TC> a) {
+template <typename T, typename TC, int TX, int SRC, int NSW, bool RESN, bool RESTR, bool OUTER,
+          bool XADD = false>
+__device__ __forceinline__ void march_body(const MarchArgs<T, TC> &a, const MGTabs &tab,
+                                           const Blk3 &bk, int nb) {
     constexpr int TY = 512 / TX;
     constexpr int R = RESTR ? NSW + 1 : (NSW > 0 ? NSW : 1);
     constexpr int NP = 2 + R;                       // own cells, then one per ring
@@ -51,16 +53,18 @@ __global__ __launch_bounds__(256) void k_mg_march(MarchArgs<T, TC> a) {
     __shared__ T s2[LDS2 ? 2 * W2 * H2 : 1];
     __shared__ T sc[SRC == MS_PROLONG ? 3 * NC : 1];
     __shared__ T sid[8], spc[8];
-    if (a.gate && *a.gate) return;
+    __shared__ TC sidc[8];
     const Geo &g = a.g, &gc = a.gc;
     const int tid = threadIdx.x, tx = tid % TX, ty = tid / TX;
-    const Blk3 bk = xcd_block();
     const int i0 = bk.x * TX, j0 = bk.y * TY, k0 = bk.z * a.kz;
     const int nz = g.nz, k1 = k0 + a.kz < nz ? k0 + a.kz : nz;
     const bool pz = g.pz != 0;
     const T om = T(a.omega), cff1 = T(1.0 - a.omega);
-    if (tid < 7) sid[tid] = T(a.tab.idiag[tid]);
-    if (tid < 8) spc[tid] = T(a.tab.pcoef[tid]);
+    if (tid < 7) {
+        sid[tid] = T(tab.idiag[tid]);
+        sidc[tid] = TC(tab.idiag[tid]);
+    }
+    if (tid < 8) spc[tid] = T(tab.pcoef[tid]);
 
     // positions: in-plane offset, domain test, in-plane neighbour count, place
     // in the stage-0 plane; own cells: also whether the cell is stored
@@ -329,8 +333,11 @@ __global__ __launch_bounds__(256) void k_mg_march(MarchArgs<T, TC> a) {
                         K2[q] = (z1 && in[q]) ? v : T(0);
                         P2[place(q, 2)] = K2[q];
                     }
-                    if (q < 2 && m >= k0 && m < k1 && st[q])
-                        a.dst[(int64_t)m * g.sz + off[q]] = v;
+                    if (q < 2 && m >= k0 && m < k1 && st[q]) {
+                        const int64_t c = (int64_t)m * g.sz + off[q];
+                        if (XADD) a.xadd[c] = a.xadd[c] + (double)v;
+                        else a.dst[c] = v;
+                    }
                 }
             }
         }
@@ -366,7 +373,7 @@ __global__ __launch_bounds__(256) void k_mg_march(MarchArgs<T, TC> a) {
                         a.bc[cc] = bv;
                         // the coarse level's first sweep from x = 0
                         const TC omc = TC(a.omega), c1 = TC(1.0 - a.omega);
-                        a.yc[cc] = c1 * TC(0) + omc * (TC(0) - bv) * TC(a.tab.idiag[nw]);
+                        a.yc[cc] = c1 * TC(0) + omc * (TC(0) - bv) * sidc[nw];
                     }
                 }
             }
@@ -414,9 +421,33 @@ __global__ __launch_bounds__(256) void k_mg_march(MarchArgs<T, TC> a) {
     }
     if (RESN) {
         __syncthreads();
-        const int nb = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
         block_sum_store(acc, a.partials + nb, tid);
     }
+}
+
+template <typename T, typename TC, int TX, int SRC, int NSW, bool RESN, bool RESTR, bool OUTER>
+__global__ __launch_bounds__(256) void k_mg_march(MarchArgs<T, TC> a, MGTabs tab) {
+    if (a.gate && *a.gate) return;
+    march_body<T, TC, TX, SRC, NSW, RESN, RESTR, OUTER>(
+        a, tab, xcd_block(), blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
+}
+
+// The pass over one level of every member of a batch: block b works for item
+// map[b], on its block number b - start (x fastest, then y, then z).
+template <typename T, typename TC, int SRC, int NSW, bool RESN, bool RESTR, bool OUTER, bool XADD>
+__global__ __launch_bounds__(256) void k_b_march(const MarchItem<T, TC> *__restrict__ items,
+                                                 const uint16_t *__restrict__ map, MGTabs tab,
+                                                 const int *__restrict__ active) {
+    const MarchItem<T, TC> &it = items[map[blockIdx.x]];
+    if (active && !active[it.h.member]) return;
+    const MarchArgs<T, TC> a = it.a;
+    const int lb = (int)((int64_t)blockIdx.x - it.h.start);
+    Blk3 bk;
+    bk.x = lb % it.bx;
+    const int t = lb / it.bx;
+    bk.y = t % it.by;
+    bk.z = t / it.by;
+    march_body<T, TC, 32, SRC, NSW, RESN, RESTR, OUTER, XADD>(a, tab, bk, lb);
 }
 
 // Tile width and march length of a level.  The width (64 or 32 columns, rows
@@ -453,9 +484,11 @@ MarchGrid march_grid(const Geo &g, int res, bool even) {
         m.kz = gr.kz;                                                                         \
         const dim3 grd(gr.bx, gr.by, gr.bz), blk(256);                                        \
         if (gr.tx == 64)                                                                      \
-            NYL_LAUNCH((k_mg_march<T, TC, 64, SRC, NSW, RESN, RESTR, OUTER>), grd, blk, 0, s, m); \
+            NYL_LAUNCH((k_mg_march<T, TC, 64, SRC, NSW, RESN, RESTR, OUTER>), grd, blk, 0, s, m, \
+                       a.tab);                                                                \
         else                                                                                  \
-            NYL_LAUNCH((k_mg_march<T, TC, 32, SRC, NSW, RESN, RESTR, OUTER>), grd, blk, 0, s, m); \
+            NYL_LAUNCH((k_mg_march<T, TC, 32, SRC, NSW, RESN, RESTR, OUTER>), grd, blk, 0, s, m, \
+                       a.tab);                                                                \
     } while (0)
 
 template <typename T, typename TC>
@@ -507,6 +540,47 @@ hipError_t launch_march_outer(const MarchArgs<double, double> &a, hipStream_t s)
     MARCH_GO(double, double, MS_FIELD, 0, true, false, true);
     return hipGetLastError();
 }
+
+template <typename T, typename TC>
+hipError_t launch_b_march(const MarchItem<T, TC> *items, const uint16_t *map, int64_t nblk,
+                          MarchKind kind, const MGTabs &tab, const int *active, hipStream_t s) {
+    const dim3 grd((unsigned)nblk), blk(256);
+#define B_GO(SRC, NSW, RESN, RESTR)                                                      \
+    NYL_LAUNCH((k_b_march<T, TC, SRC, NSW, RESN, RESTR, false, false>), grd, blk, 0, s, items, \
+               map, tab, active)
+    switch (kind) {
+    case MK_UP: B_GO(MS_PROLONG, 2, false, false); break;
+    case MK_UP_ADD:
+        if constexpr (sizeof(T) == 4)
+            NYL_LAUNCH((k_b_march<T, TC, MS_PROLONG, 2, false, false, false, true>), grd, blk, 0,
+                       s, items, map, tab, active);
+        else return hipErrorInvalidValue;
+        break;
+    case MK_DOWN: B_GO(MS_FIELD, 1, false, true); break;
+    case MK_RESTRICT: B_GO(MS_FIELD, 0, false, true); break;
+    case MK_PRE: B_GO(MS_FIELD, 2, true, false); break;
+    case MK_PRE_RESTRICT: B_GO(MS_FIELD, 2, true, true); break;
+    case MK_ZERO: B_GO(MS_ZERO, 2, false, false); break;
+    case MK_ZERO_RESTRICT: B_GO(MS_ZERO, 2, false, true); break;
+    case MK_OUTER:
+        if constexpr (sizeof(T) == 8)
+            NYL_LAUNCH((k_b_march<T, TC, MS_FIELD, 0, true, false, true, false>), grd, blk, 0, s, items,
+                       map, tab, active);
+        else return hipErrorInvalidValue;
+        break;
+    }
+#undef B_GO
+    return hipGetLastError();
+}
+template hipError_t launch_b_march<double, double>(const MarchItem<double, double> *,
+                                                   const uint16_t *, int64_t, MarchKind,
+                                                   const MGTabs &, const int *, hipStream_t);
+template hipError_t launch_b_march<float, float>(const MarchItem<float, float> *,
+                                                 const uint16_t *, int64_t, MarchKind,
+                                                 const MGTabs &, const int *, hipStream_t);
+template hipError_t launch_b_march<float, double>(const MarchItem<float, double> *,
+                                                  const uint16_t *, int64_t, MarchKind,
+                                                  const MGTabs &, const int *, hipStream_t);
 
 #define NYL_MARCH_INST(T, TC)                                                              \
     template hipError_t launch_march_up<T, TC>(const MarchArgs<T, TC> &, hipStream_t);     \

@@ -848,92 +848,38 @@ hipError_t launch_kesum(const Geo &g, const T *u, const T *v, const T *w, double
 // blocks of members whose solve has stopped).
 #define BT NYL_BATCH_TPB
 
-template <typename T>
-__global__ __launch_bounds__(BT) void k_b_sweep(const SweepItem<T> *__restrict__ items, int n,
+__global__ __launch_bounds__(BT) void k_b_sweep(const SweepItem *__restrict__ items, int n,
                                                 MGTabs tab, const int *__restrict__ active) {
-    const SweepItem<T> &it = find_item(items, n, blockIdx.x);
+    const SweepItem &it = find_item(items, n, blockIdx.x);
     if (active && !active[it.h.member]) return;
     int i, j, k;
     if (!cell_of(it.h.g, ((int64_t)blockIdx.x - it.h.start) * BT + threadIdx.x, i, j, k)) return;
     const int64_t c = (int64_t)k * it.h.g.sz + (int64_t)j * it.h.g.sy + i;
-    const T v = sweep_value<T>(it.h.g, it.src, it.b, it.omega, tab, i, j, k, c);
-    if (it.xo) it.xo[c] = it.xo[c] + (double)v;   // the mixed solve's x += e, e not stored
-    else it.dst[c] = v;
+    it.dst[c] = sweep_value<double>(it.h.g, it.src, it.b, it.omega, tab, i, j, k, c);
 }
 
-template <typename T>
-hipError_t launch_b_sweep(const SweepItem<T> *items, int n, int64_t nblk, const MGTabs &tab,
+hipError_t launch_b_sweep(const SweepItem *items, int n, int64_t nblk, const MGTabs &tab,
                           const int *active, hipStream_t s) {
-    NYL_LAUNCH((k_b_sweep<T>), dim3((unsigned)nblk), BT, 0, s, items, n, tab, active);
-    return hipGetLastError();
-}
-
-// flattened over the coarse cells
-template <typename Tf, typename Tc>
-__global__ __launch_bounds__(BT) void k_b_restrict(const RestrItem<Tf, Tc> *__restrict__ items,
-                                                   int n, MGTabs tab,
-                                                   const int *__restrict__ active) {
-    const RestrItem<Tf, Tc> &it = find_item(items, n, blockIdx.x);
-    if (active && !active[it.h.member]) return;
-    int i, j, k;
-    if (!cell_of(it.gc, ((int64_t)blockIdx.x - it.h.start) * BT + threadIdx.x, i, j, k)) return;
-    restrict_cell<Tf, Tc>(it.h.g, it.gc, it.x, it.b, it.bc, it.xc, tab, i, j, k);
-}
-
-template <typename Tf, typename Tc>
-hipError_t launch_b_restrict(const RestrItem<Tf, Tc> *items, int n, int64_t nblk,
-                             const MGTabs &tab, const int *active, hipStream_t s) {
-    NYL_LAUNCH((k_b_restrict<Tf, Tc>), dim3((unsigned)nblk), BT, 0, s, items, n, tab,
-                       active);
-    return hipGetLastError();
-}
-
-template <typename Tf, typename Tc>
-__global__ __launch_bounds__(BT) void k_b_prolong(const ProlItem<Tf, Tc> *__restrict__ items,
-                                                  int n, MGTabs tab,
-                                                  const int *__restrict__ active) {
-    const ProlItem<Tf, Tc> &it = find_item(items, n, blockIdx.x);
-    if (active && !active[it.h.member]) return;
-    int i, j, k;
-    if (!cell_of(it.h.g, ((int64_t)blockIdx.x - it.h.start) * BT + threadIdx.x, i, j, k)) return;
-    const int64_t c = (int64_t)k * it.h.g.sz + (int64_t)j * it.h.g.sy + i;
-    it.xf[c] = it.xf[c] + prolong_term<Tf, Tc>(it.gc, it.xc, tab, i, j, k);
-}
-
-template <typename Tf, typename Tc>
-hipError_t launch_b_prolong(const ProlItem<Tf, Tc> *items, int n, int64_t nblk,
-                            const MGTabs &tab, const int *active, hipStream_t s) {
-    NYL_LAUNCH((k_b_prolong<Tf, Tc>), dim3((unsigned)nblk), BT, 0, s, items, n, tab,
-                       active);
+    NYL_LAUNCH(k_b_sweep, dim3((unsigned)nblk), BT, 0, s, items, n, tab, active);
     return hipGetLastError();
 }
 
 // Per-member partial sums: each member owns h.nblk blocks that stride over
 // its cells, so its partials (and their order) do not depend on the batch.
-template <typename T, int KIND>
-__global__ __launch_bounds__(BT) void k_b_reduce(const RedItem<T> *__restrict__ items, int n,
-                                                 MGTabs tab, const int *__restrict__ active) {
-    const RedItem<T> &it = find_item(items, n, blockIdx.x);
-    if (active && !active[it.h.member]) return;
+template <int KIND>
+__global__ __launch_bounds__(BT) void k_b_reduce(const RedItem *__restrict__ items, int n) {
+    const RedItem &it = find_item(items, n, blockIdx.x);
     const Geo &g = it.h.g;
     const int64_t nc = (int64_t)g.nx * g.ny * g.nz;
     const int64_t lb = (int64_t)blockIdx.x - it.h.start;
     double a1 = 0.0, a2 = 0.0;
     for (int64_t q = lb * BT + threadIdx.x; q < nc; q += (int64_t)it.h.nblk * BT) {
-        if (KIND == 1) {
-            const int i = (int)(q % g.nx);
-            const int64_t t = q / g.nx;
-            const double r = (double)residual_at<T>(g, it.v, it.b, i, (int)(t % g.ny),
-                                                    (int)(t / g.ny), tab);
-            a1 = a1 + r * r;
+        const double x = it.v[q];
+        if (KIND == 2) {
+            a1 = a1 + x;
+            a2 = a2 + x * x;
         } else {
-            const double x = (double)it.v[q];
-            if (KIND == 2) {
-                a1 = a1 + x;
-                a2 = a2 + x * x;
-            } else {
-                a1 = a1 + x * x;
-            }
+            a1 = a1 + x * x;
         }
     }
     block_sum_store(a1, it.partials + lb, threadIdx.x);
@@ -943,47 +889,10 @@ __global__ __launch_bounds__(BT) void k_b_reduce(const RedItem<T> *__restrict__ 
     }
 }
 
-template <typename T>
-hipError_t launch_b_reduce(const RedItem<T> *items, int n, int64_t nblk, int kind,
-                           const MGTabs &tab, const int *active, hipStream_t s) {
+hipError_t launch_b_reduce(const RedItem *items, int n, int64_t nblk, int kind, hipStream_t s) {
     const dim3 grd((unsigned)nblk);
-    if (kind == 0) NYL_LAUNCH((k_b_reduce<T, 0>), grd, BT, 0, s, items, n, tab, active);
-    else if (kind == 1) NYL_LAUNCH((k_b_reduce<T, 1>), grd, BT, 0, s, items, n, tab, active);
-    else NYL_LAUNCH((k_b_reduce<T, 2>), grd, BT, 0, s, items, n, tab, active);
-    return hipGetLastError();
-}
-
-// the outer FP64 residual of the mixed solve (k_mg_outer_resid per member)
-__global__ __launch_bounds__(BT) void k_b_outer_resid(const OuterItem *__restrict__ items, int n,
-                                                      BMG mg, MGTabs tab,
-                                                      const int *__restrict__ active) {
-    const OuterItem &it = find_item(items, n, blockIdx.x);
-    if (active && !active[it.h.member]) return;
-    const Geo &g = it.h.g;
-    const int64_t nc = (int64_t)g.nx * g.ny * g.nz;
-    const int64_t lb = (int64_t)blockIdx.x - it.h.start;
-    const double shift = mg.shift[it.h.member];
-    const float om = float(it.omega), cff1 = float(1.0 - it.omega);
-    double acc = 0.0;
-    for (int64_t q = lb * BT + threadIdx.x; q < nc; q += (int64_t)it.h.nblk * BT) {
-        const int i = (int)(q % g.nx);
-        const int64_t t = q / g.nx;
-        const int j = (int)(t % g.ny), k = (int)(t / g.ny);
-        const Nbrs<double> nb = neighbours<double>(g, it.x, i, j, k, q);
-        const double r = (it.b[q] - shift) + tab.diag[nb.nwet] * it.x[q]
-                       - (nb.xm + nb.xp + nb.ym + nb.yp + nb.zm + nb.zp);
-        acc = acc + r * r;
-        const float rf = float(r);
-        it.r[q] = rf;
-        it.y[q] = cff1 * 0.0f + om * (0.0f - rf) * float(tab.idiag[nb.nwet]);
-    }
-    block_sum_store(acc, it.partials + lb, threadIdx.x);
-}
-
-hipError_t launch_b_outer_resid(const OuterItem *items, int n, int64_t nblk, const BMG &mg,
-                                const MGTabs &tab, const int *active, hipStream_t s) {
-    NYL_LAUNCH(k_b_outer_resid, dim3((unsigned)nblk), BT, 0, s, items, n, mg, tab,
-                       active);
+    if (kind == 0) NYL_LAUNCH((k_b_reduce<0>), grd, BT, 0, s, items, n);
+    else NYL_LAUNCH((k_b_reduce<2>), grd, BT, 0, s, items, n);
     return hipGetLastError();
 }
 
@@ -2413,24 +2322,6 @@ hipError_t launch_mg_restrict25(const Geo &gf, const Geo &gc, const Tf *x, const
 NYL_MG_INST(double)
 NYL_MG_INST(float)
 #undef NYL_MG_INST
-
-#define NYL_B_MG_INST(T)                                                                         \
-    template hipError_t launch_b_sweep<T>(const SweepItem<T> *, int, int64_t, const MGTabs &,   \
-                                          const int *, hipStream_t);                            \
-    template hipError_t launch_b_restrict<T, T>(const RestrItem<T, T> *, int, int64_t,          \
-                                                const MGTabs &, const int *, hipStream_t);      \
-    template hipError_t launch_b_prolong<T, T>(const ProlItem<T, T> *, int, int64_t,            \
-                                               const MGTabs &, const int *, hipStream_t);       \
-    template hipError_t launch_b_reduce<T>(const RedItem<T> *, int, int64_t, int,               \
-                                           const MGTabs &, const int *, hipStream_t);
-NYL_B_MG_INST(double)
-NYL_B_MG_INST(float)
-#undef NYL_B_MG_INST
-template hipError_t launch_b_restrict<float, double>(const RestrItem<float, double> *, int,
-                                                     int64_t, const MGTabs &, const int *,
-                                                     hipStream_t);
-template hipError_t launch_b_prolong<float, double>(const ProlItem<float, double> *, int, int64_t,
-                                                    const MGTabs &, const int *, hipStream_t);
 
 template hipError_t launch_resnorm2<double>(const Geo &, const double *, const double *,
                                             const MGTabs &, double *, double *, hipStream_t);

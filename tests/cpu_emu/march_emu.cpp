@@ -47,22 +47,22 @@ int check(int nx, int ny, int nz, int px, int py, int pz, int kz, bool halves) {
         std::vector<double> p1(nblk, 0.0), p2(nblk, 0.0);
         a.src = x.data(); a.dst = z.data();
         run_blocks(grd, dim3(256), [&]() {
-            k_mg_march<T, TC, TX, MS_FIELD, 2, false, false, false>(a); }, true);
+            k_mg_march<T, TC, TX, MS_FIELD, 2, false, false, false>(a, tab); }, true);
         bad += ndiff(z, y2);
         z.assign(nf, T(7));
         a.partials = p1.data();
         run_blocks(grd, dim3(256), [&]() {
-            k_mg_march<T, TC, TX, MS_FIELD, 2, true, false, false>(a); }, true);
+            k_mg_march<T, TC, TX, MS_FIELD, 2, true, false, false>(a, tab); }, true);
         bad += ndiff(z, y2) + norm_of(p1);
         a.partials = p2.data();
         run_blocks(grd, dim3(256), [&]() {
-            k_mg_march<T, TC, TX, MS_FIELD, 0, true, false, false>(a); }, true);
+            k_mg_march<T, TC, TX, MS_FIELD, 0, true, false, false>(a, tab); }, true);
         bad += ndiff(p1, p2);
         const std::vector<T> zero(nf, T(0));
         const auto s2 = sweep(g, sweep(g, zero, b, tab), b, tab);
         a.src = nullptr;
         run_blocks(grd, dim3(256), [&]() {
-            k_mg_march<T, TC, TX, MS_ZERO, 2, false, false, false>(a); }, true);
+            k_mg_march<T, TC, TX, MS_ZERO, 2, false, false, false>(a, tab); }, true);
         bad += ndiff(z, s2);
     }
     if (halves) {
@@ -74,7 +74,7 @@ int check(int nx, int ny, int nz, int px, int py, int pz, int kz, bool halves) {
                                        yc1.data(), 0.9); }, false);
         a.src = x.data(); a.dst = z.data(); a.bc = bc2.data(); a.yc = yc2.data();
         run_blocks(grd, dim3(256), [&]() {
-            k_mg_march<T, TC, TX, MS_FIELD, 1, false, true, false>(a); }, true);
+            k_mg_march<T, TC, TX, MS_FIELD, 1, false, true, false>(a, tab); }, true);
         bad += ndiff(z, y1) + ndiff(bc1, bc2) + ndiff(yc1, yc2);
         run_blocks(mg_grid(g), dim3(MG_BX, MG_BY, 1), [&]() {
             k_mg_prolong<T, TC>(g, gc, xp.data(), xc.data(), tab); }, false);
@@ -82,14 +82,14 @@ int check(int nx, int ny, int nz, int px, int py, int pz, int kz, bool halves) {
         z.assign(nf, T(7));
         a.xc = xc.data();
         run_blocks(grd, dim3(256), [&]() {
-            k_mg_march<T, TC, TX, MS_PROLONG, 2, false, false, false>(a); }, true);
+            k_mg_march<T, TC, TX, MS_PROLONG, 2, false, false, false>(a, tab); }, true);
         bad += ndiff(z, u2);
         // the restriction alone, and in the pass of the two sweeps (from a
         // field with its residual norm, from zero)
         bc2.assign(nc, TC(5)); yc2.assign(nc, TC(6));
         a.src = y1.data();
         run_blocks(grd, dim3(256), [&]() {
-            k_mg_march<T, TC, TX, MS_FIELD, 0, false, true, false>(a); }, true);
+            k_mg_march<T, TC, TX, MS_FIELD, 0, false, true, false>(a, tab); }, true);
         bad += ndiff(bc1, bc2) + ndiff(yc1, yc2);
         for (int zero = 0; zero < 2; zero++) {
             const std::vector<T> o(nf, T(0));
@@ -102,8 +102,8 @@ int check(int nx, int ny, int nz, int px, int py, int pz, int kz, bool halves) {
             a.src = zero ? nullptr : x.data();
             a.partials = p3.data();
             run_blocks(grd, dim3(256), [&]() {
-                if (zero) k_mg_march<T, TC, TX, MS_ZERO, 2, false, true, false>(a);
-                else k_mg_march<T, TC, TX, MS_FIELD, 2, true, true, false>(a); }, true);
+                if (zero) k_mg_march<T, TC, TX, MS_ZERO, 2, false, true, false>(a, tab);
+                else k_mg_march<T, TC, TX, MS_FIELD, 2, true, true, false>(a, tab); }, true);
             bad += ndiff(z, t2) + ndiff(bc1, bc2) + ndiff(yc1, yc2) + (!zero && norm_of(p3));
         }
         a.src = x.data();
@@ -113,7 +113,7 @@ int check(int nx, int ny, int nz, int px, int py, int pz, int kz, bool halves) {
         a.gate = &one;
         a.src = y1.data();
         run_blocks(grd, dim3(256), [&]() {
-            k_mg_march<T, TC, TX, MS_PROLONG, 2, false, false, false>(a); }, true);
+            k_mg_march<T, TC, TX, MS_PROLONG, 2, false, false, false>(a, tab); }, true);
         bad += ndiff(z, z0);
     }
     if (sizeof(T) == 8 && sizeof(TC) == 8) {   // the mixed solve's FP64 residual
@@ -129,7 +129,7 @@ int check(int nx, int ny, int nz, int px, int py, int pz, int kz, bool halves) {
             k_mg_outer_resid<float>(g, xd.data(), bd.data(), shift, r1.data(), yd.data(), 0.9, tab,
                                     p1.data()); }, true);
         run_blocks(grd, dim3(256), [&]() {
-            k_mg_march<double, double, TX, MS_FIELD, 0, true, false, true>(o); }, true);
+            k_mg_march<double, double, TX, MS_FIELD, 0, true, false, true>(o, tab); }, true);
         double s1 = 0, s2 = 0;
         for (double v : p1) s1 += v;
         for (double v : p2) s2 += v;
