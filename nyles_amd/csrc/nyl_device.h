@@ -120,32 +120,74 @@ __device__ __forceinline__ float weno5_f32(float qmm, float qm, float q0, float 
     return fmaf(w1, qi1, fmaf(w2, qi2, w3 * qi3)) * __builtin_amdgcn_rcpf(w1 + w2 + w3);
 }
 
-// core/weno.f90:25-54
+// a/b by the instructions the compiler's FP64 division runs on its scaled
+// operands -- reciprocal, two Newton steps, quotient, residual -- without
+// v_div_scale, v_div_fmas and v_div_fixup, which issue at a quarter of the
+// FP64 rate and, for operands whose quotient, reciprocal and residual stay
+// normal, leave every operand as it is: the same double.  The caller holds b
+// in [2^-54, 2^190], and a = +0 or |a| in [2^-900, 2^320].
+__device__ __forceinline__ double div_mid(double a, double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    double r = __builtin_amdgcn_rcp(b);
+#else
+    double r = 1.0 / b;
+#endif
+    r = fma(r, fma(-b, r, 1.0), r);
+    r = fma(r, fma(-b, r, 1.0), r);
+    const double q = a * r;
+    return fma(fma(-b, q, a), r, q);
+}
+
+// core/weno.f90:25-54.  FP64: the operations of the reference in its order.
+// Products by 2, 4 and 1/4 are exact and share an fma with the sum that
+// follows (a quarter of a subnormal square would round, and is lost against
+// eps and in the REAL(4) tau5 either way).  Issue-bound: 110 instructions, 23
+// of them at a quarter of the rate, before; 95 and 4 with div_mid.  Its range:
+// the sum of the beta and |q0| below 2^126 bounds the differences, so every
+// value (2^127), tau5 (2^127) and the weights (2^184); inf and NaN fail it.
 template <typename T>
 __device__ __forceinline__ T weno5(T qmm, T qm, T q0, T qp, T qpp) {
-    if constexpr (sizeof(T) == 4) return weno5_f32(qmm, qm, q0, qp, qpp);
-    const T eps = T(1e-16f);
-    const T c13 = T(1.0f / 3.0f), c76 = T(7.0f / 6.0f), c116 = T(11.0f / 6.0f);
-    const T c16 = T(1.0f / 6.0f), c56 = T(5.0f / 6.0f);
-    const T k1 = T(13.0f / 12.0f), k2 = T(0.25);
+    if constexpr (sizeof(T) == 4) {
+        return weno5_f32(qmm, qm, q0, qp, qpp);
+    } else {
+        const T eps = T(1e-16f);
+        const T c13 = T(1.0f / 3.0f), c76 = T(7.0f / 6.0f), c116 = T(11.0f / 6.0f);
+        const T c16 = T(1.0f / 6.0f), c56 = T(5.0f / 6.0f);
+        const T k1 = T(13.0f / 12.0f), k2 = T(0.25);
 
-    T qi1 = c13 * qmm - c76 * qm + c116 * q0;
-    T qi2 = -(c16 * qm) + c56 * q0 + c13 * qp;
-    T qi3 = c13 * q0 + c56 * qp - c16 * qpp;
+        const T qi1 = c13 * qmm - c76 * qm + c116 * q0;
+        const T qi2 = -(c16 * qm) + c56 * q0 + c13 * qp;
+        const T qi3 = c13 * q0 + c56 * qp - c16 * qpp;
 
-    T t1 = qmm - T(2) * qm + q0, t2 = qmm - T(4) * qm + T(3) * q0;
-    T beta1 = k1 * (t1 * t1) + k2 * (t2 * t2);
-    T t3 = qm - T(2) * q0 + qp, t4 = qm - qp;
-    T beta2 = k1 * (t3 * t3) + k2 * (t4 * t4);
-    T t5 = q0 - T(2) * qp + qpp, t6 = T(3) * q0 - T(4) * qp + qpp;
-    T beta3 = k1 * (t5 * t5) + k2 * (t6 * t6);
+        const T t1 = fma(T(-2), qm, qmm) + q0, t2 = fma(T(-4), qm, qmm) + T(3) * q0;
+        const T beta1 = fma(k2, t2 * t2, k1 * (t1 * t1));
+        const T t3 = fma(T(-2), q0, qm) + qp, t4 = qm - qp;
+        const T beta2 = fma(k2, t4 * t4, k1 * (t3 * t3));
+        const T t5 = fma(T(-2), qp, q0) + qpp, t6 = fma(T(-4), qp, T(3) * q0) + qpp;
+        const T beta3 = fma(k2, t6 * t6, k1 * (t5 * t5));
 
-    T tau5 = T((float)fabs(beta1 - beta3));
+        const T tau5 = T((float)fabs(beta1 - beta3));
+        const T b1 = beta1 + eps, b2 = beta2 + eps, b3 = beta3 + eps;
 
-    T w1 = (T(1) + wdiv(tau5, beta1 + eps));
-    T w2 = T(6) * (T(1) + wdiv(tau5, beta2 + eps));
-    T w3 = T(3) * (T(1) + wdiv(tau5, beta3 + eps));
-    return wdiv(w1 * qi1 + w2 * qi2 + w3 * qi3, w1 + w2 + w3);
+        const bool mid = b1 + b2 + b3 + fabs(q0) < T(0x1p126);
+        T d1, d2, d3;
+        if (mid) {
+            d1 = div_mid(tau5, b1);
+            d2 = div_mid(tau5, b2);
+            d3 = div_mid(tau5, b3);
+        } else {
+            d1 = tau5 / b1;
+            d2 = tau5 / b2;
+            d3 = tau5 / b3;
+        }
+        const T w1 = (T(1) + d1);
+        const T w2 = T(6) * (T(1) + d2);
+        const T w3 = T(3) * (T(1) + d3);
+        const T num = w1 * qi1 + w2 * qi2 + w3 * qi3, den = w1 + w2 + w3;
+        // a zero keeps its sign, and a tiny sum its scaling, in the full division
+        if (mid && fabs(num) >= T(0x1p-900)) return div_mid(num, den);
+        return num / den;
+    }
 }
 
 // Flux at line position f (0-based) of core/weno.f90:106-153 flux1d, for a
@@ -189,6 +231,30 @@ __device__ __forceinline__ T face_flux(int f, int n, T u, const QF &q) {
     else if (kind == 1) w = a0;
     else return T(0);
     return u * w;
+}
+
+// face_flux with the values at -2..3 from the face given (held in registers):
+// the closures read the same stencils -- the five upwind values, the middle
+// three of them, the middle one -- so the five are selected once, one WENO5 is
+// evaluated for every lane, and the lanes (or planes) at the ends of a wall
+// line replace its result.  face_flux's values, operations and results.
+template <typename T>
+struct Stencil6 {
+    T m2, m1, z0, p1, p2, p3;
+};
+template <typename T, int PER>
+__device__ __forceinline__ T face_of(int f, int n, T u, const Stencil6<T> &w) {
+    const bool pos = u > T(0);
+    const T a0 = pos ? w.m2 : w.p3, a1 = pos ? w.m1 : w.p2, a2 = pos ? w.z0 : w.p1;
+    const T a3 = pos ? w.p1 : w.z0, a4 = pos ? w.p2 : w.m1;
+    T r = weno5<T>(a0, a1, a2, a3, a4);
+    if (!PER && (f < 2 || f > n - 4)) {
+        if (f == n - 1) return T(0);
+        const int lo = pos ? 2 : 1, hi = pos ? n - 3 : n - 4;   // WENO5 between these
+        if (f == lo - 1 || f == hi + 1) r = weno3<T>(a1, a2, a3);
+        else if (f < lo || f > hi) r = a2;
+    }
+    return u * r;
 }
 
 // face_flux with the stencil given relative to the face: qr(d) = q(f + d),

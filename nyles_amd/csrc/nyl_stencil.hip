@@ -1,79 +1,13 @@
-// nyl_stencil.hip -- explicit right-hand side, RK3 stage update and the
-// diagnostic stencils of the Nyles time step on gfx950.
+// nyl_stencil.hip -- the diagnostic stencils, passive tracers and ensemble
+// forms of the Nyles time step on gfx950 (the stage kernels: nyl_stage.h).
 //
 // Every FP64 instantiation reproduces the reference's arithmetic operation
 // by operation (the library is compiled with -ffp-contract=off), so its
 // results are bit-identical to the oracle's.
-#include "nyl_internal.h"
+#include "nyl_stage.h"
 #include <initializer_list>
 
 namespace nyl {
-
-#define NYL_BX 64
-#define NYL_BY 4
-
-// Minimum waves per SIMD for the stage kernel (caps its registers).
-#ifndef NYL_STAGE_WAVES
-#define NYL_STAGE_WAVES 1
-#endif
-// Sequencing of the flux evaluations of the stage kernel.  Its stencil loads
-// are invariant (const __restrict__), so the compiler is free to issue the
-// loads of all twelve reconstructions before any arithmetic, which needs
-// ~180 registers and leaves 2 waves per SIMD.  STAGE_SEQ(idx, dep) passes
-// the line index of the next evaluation through an empty asm that also takes
-// the previous evaluation's result: the next loads cannot be issued before
-// that result exists, each reconstruction holds only its own operands and
-// occupancy hides the load latency.  No instruction is emitted.
-#ifndef NYL_STAGE_SEQ
-#define NYL_STAGE_SEQ 1
-#endif
-// block order of the stage kernel: XCD y slabs marched in z (1) or z slabs (0)
-#ifndef NYL_STAGE_YSLAB
-#define NYL_STAGE_YSLAB 1
-#endif
-#if NYL_STAGE_SEQ
-#define STAGE_SEQ(idx, dep) asm volatile("" : "+v"(idx) : "v"(dep))
-#else
-#define STAGE_SEQ(idx, dep) ((void)0)
-#endif
-// the sequencing points between the two faces of one tracer axis (off: the
-// two reconstructions of an axis overlap; FP32 stage 6 % faster)
-#ifndef NYL_STAGE_SEQ_FACES
-#define NYL_STAGE_SEQ_FACES 0
-#endif
-// the sequencing points between the vortex-force terms in FP32: every
-// term (1), every second term (2) or none (0: FP32 stage 579 -> 533 us; the
-// FP32 operands are half the registers, so the overlap fits)
-#ifndef NYL_STAGE_SEQ_VF32
-#define NYL_STAGE_SEQ_VF32 0
-#endif
-// and in FP64 (0: FP64 stage modes 1 and 3 1214 -> 1152 us, mode 2 unchanged)
-#ifndef NYL_STAGE_SEQ_VF64
-#define NYL_STAGE_SEQ_VF64 0
-#endif
-#define STAGE_SEQ_V(idx, dep, odd)                                             \
-    do {                                                                       \
-        if constexpr ((sizeof(T) == 8 && (NYL_STAGE_SEQ_VF64 == 1 ||           \
-                                          (NYL_STAGE_SEQ_VF64 == 2 && (odd)))) || \
-                      (sizeof(T) == 4 && (NYL_STAGE_SEQ_VF32 == 1 ||           \
-                                          (NYL_STAGE_SEQ_VF32 == 2 && (odd)))))  \
-            STAGE_SEQ(idx, dep);                                               \
-    } while (0)
-// the sequencing points between the tracer axes: kept for FP64 (overlapping
-// them made the FP64 stage 2 % slower), dropped for FP32 (2 % faster)
-#define STAGE_SEQ_A(idx, dep)                      \
-    do {                                           \
-        if constexpr (sizeof(T) == 8) STAGE_SEQ(idx, dep); \
-    } while (0)
-#if NYL_STAGE_SEQ_FACES
-#define STAGE_SEQ_F(idx, dep) STAGE_SEQ(idx, dep)
-#else
-#define STAGE_SEQ_F(idx, dep) ((void)0)
-#endif
-
-static inline dim3 cell_grid(const Geo &g) {
-    return dim3((g.nx + NYL_BX - 1) / NYL_BX, (g.ny + NYL_BY - 1) / NYL_BY, g.nz);
-}
 
 // The per-cell diagnostic kernels (div, correct, diag): each thread takes
 // NYL_CELL_KZ consecutive planes of its column (when nz is a multiple), in
@@ -94,451 +28,6 @@ static inline dim3 cell_grid_kz(const Geo &g) {
 #define CELL_BLOCK() xcd_block()
 #endif
 
-// Stage-kernel loads and stores at a 32-bit byte offset from the field's
-// base pointer (the base is uniform, so the load takes it from scalar
-// registers and the offset as one 32-bit register: no 64-bit address
-// arithmetic per load).  A field is below 4 GiB (checked at context
-// creation); offsets wrap modulo 2^32 to the right address.
-template <typename T>
-__device__ __forceinline__ T ldb(const T *__restrict__ p, uint32_t boff) {
-    return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(p) + boff);
-}
-template <typename T>
-__device__ __forceinline__ void stb(T *__restrict__ p, uint32_t boff, T v) {
-    *reinterpret_cast<T *>(reinterpret_cast<char *>(p) + boff) = v;
-}
-template <typename T>
-__device__ __forceinline__ void stb_stream(T *__restrict__ p, uint32_t boff, T v) {
-    store_stream(reinterpret_cast<T *>(reinterpret_cast<char *>(p) + boff), v);
-}
-
-// Vortex-force flux of one term at a cell (core/fortran_vortex_force.f90
-// WENO branch, :66-81 and :145-159): the vorticity component `om` is
-// upwinded along axis d with the contravariant velocity U_d = ud*cu
-// averaged along the target axis e (UU) and then along d (u1d).  `based` is
-// the index of the cell's line start along d, `sd` the stride of d, `md` the
-// cell's position on that line, `oe` the offset to the e+1 neighbour.  U is
-// recomputed from the covariant u with the product U_from_u stores
-// (core/cov_to_contra.py:15-17), so it is the same double.
-template <typename T, int pd>
-__device__ __forceinline__ T vf_flux(const T *__restrict__ ud, T cu, const T *__restrict__ om,
-                                     int64_t based, int64_t sd, int md, int nd, int64_t oe) {
-    // 32-bit byte offsets from the field bases (a field is below 4 GiB)
-    constexpr uint32_t ES = sizeof(T);
-    const uint32_t bb = (uint32_t)based * ES, sb = (uint32_t)sd * ES, eb = (uint32_t)oe * ES;
-    auto UU = [&](int m) -> T {
-        const uint32_t p = bb + (uint32_t)m * sb;
-        return T(0.5) * (ldb(ud, p) * cu + ldb(ud, p + eb) * cu);
-    };
-    T uu_prev;
-    if (!pd && md == 0) uu_prev = T(0);   // UU_0 = 0. at the line start
-    else uu_prev = UU(pd ? wrapi(md - 1, nd) : md - 1);
-    const T u1d = T(0.5) * (uu_prev + UU(md));
-    auto q = [&](int m) -> T {            // q(1) = 0., q(k) = vort(k-1)
-        if (pd) return ldb(om, bb + (uint32_t)wrapi(m - 1, nd) * sb);
-        if (m == 0) return T(0);
-        return ldb(om, bb + (uint32_t)(m - 1) * sb);
-    };
-    return face_flux<T, pd>(md, nd, u1d, q);
-}
-
-// Tracer flux divergence along one axis (core/fortran_upwind.f90:77-81):
-// d = d + flux(m-1) - flux(m), or d - flux(1) at a wall start.
-// U_d = ud*cu as in vf_flux.
-template <typename T, int pd>
-__device__ __forceinline__ T tracer_axis(T d, const T *__restrict__ q_arr,
-                                         const T *__restrict__ ud, T cu, int64_t based,
-                                         int64_t sd, int md, int nd) {
-    // 32-bit byte offsets from the field bases (a field is below 4 GiB)
-    constexpr uint32_t ES = sizeof(T);
-    uint32_t bb = (uint32_t)based * ES;
-    const uint32_t sb = (uint32_t)sd * ES;
-    auto q = [&](int m) -> T { return ldb(q_arr, bb + (uint32_t)(pd ? wrapi(m, nd) : m) * sb); };
-    const T fr = face_flux<T, pd>(md, nd, ldb(ud, bb + (uint32_t)md * sb) * cu, q);
-    STAGE_SEQ_F(bb, fr);
-    if (!pd && md == 0) return d - fr;
-    const int ml = pd ? wrapi(md - 1, nd) : md - 1;
-    const T fl = face_flux<T, pd>(ml, nd, ldb(ud, bb + (uint32_t)ml * sb) * cu, q);
-    return (d + fl) - fr;
-}
-
-// ---------------------------------------------------------------------------
-// The reference's linear upwind branches (linear=.false. in its build:
-// core/fortran_upwind.f90:30, core/fortran_vortex_force.f90:28,104), odd
-// orders 1, 3, 5.  REAL(4) literals widened; sums left to right as written.
-
-// Reconstruction at line position j of the values q(.) (a functor over
-// positions, wrapped on a periodic axis): RIGHT = false the left-biased qp,
-// true the right-biased qm.  On a wall line the order drops near the ends:
-// tracer flavour (core/interpolate_tracer.f90:45-80) first order at 0 and
-// n-1, third at 1 and n-2; vortex-force flavour (core/interpolate.f90:35-79)
-// qp(-1) = 0, first order at 0 and n-2 (and qm at n-1), third at 1 and n-3.
-template <typename T, bool VF, bool RIGHT, typename QF>
-__device__ __forceinline__ T lin_rec(const QF &q, int j, int n, int order, bool per) {
-    const T c1 = T(-(1.0f / 6.0f)), c2 = T(5.0f / 6.0f), c3 = T(2.0f / 6.0f);
-    const T b1 = T(2.0f / 60.0f), b2 = T(-(13.0f / 60.0f)), b3 = T(47.0f / 60.0f);
-    const T b4 = T(27.0f / 60.0f), b5 = T(-(3.0f / 60.0f));
-    int ord = order;
-    if (!per) {
-        if (VF && !RIGHT && j < 0) return T(0);
-        const int last1 = VF ? n - 2 : n - 1;          // first order at 0 and here
-        if (j <= 0 || j >= last1) ord = 1;
-        else if (order == 5 && (j == 1 || j == last1 - 1)) ord = 3;
-    }
-    if (ord == 1) return q(j);
-    if (ord == 3) {
-        if (RIGHT) return c3 * q(j - 1) + c2 * q(j) + c1 * q(j + 1);
-        return c1 * q(j - 1) + c2 * q(j) + c3 * q(j + 1);
-    }
-    if (RIGHT) return b5 * q(j - 2) + b4 * q(j - 1) + b3 * q(j) + b2 * q(j + 1) + b1 * q(j + 2);
-    return b1 * q(j - 2) + b2 * q(j - 1) + b3 * q(j) + b4 * q(j + 1) + b5 * q(j + 2);
-}
-
-// core/fortran_upwind.f90:34-67: d = (d + fx(m-1)) - fx(m), the face flux
-// fx(i) = up(i)*qp(i) + um(i)*qm(i+1) with up/um = 0.5*(U -+ |U|), no flux
-// through the ends of a wall line.  U_d = ud*cu as in tracer_axis.
-template <typename T, int PD>
-__device__ __forceinline__ T lin_tracer_axis(T d, const T *__restrict__ q_arr,
-                                             const T *__restrict__ ud, T cu, int64_t based,
-                                             int64_t sd, int m, int n, int order) {
-    auto pos = [&](int p) -> int64_t { return based + (int64_t)(PD ? wrapi(p, n) : p) * sd; };
-    auto q = [&](int p) -> T { return q_arr[pos(p)]; };
-    auto face = [&](int i) -> T {
-        const T ui = ud[pos(i)] * cu, au = fabs(ui);
-        const T up = T(0.5) * (ui + au), um = T(0.5) * (ui - au);
-        return up * lin_rec<T, false, false>(q, i, n, order, PD != 0)
-             + um * lin_rec<T, false, true>(q, i + 1, n, order, PD != 0);
-    };
-    const T fxm = (PD || m > 0) ? face(m - 1) : T(0);
-    const T fx = (PD || m < n - 1) ? face(m) : T(0);
-    return (d + fxm) - fx;
-}
-
-// core/fortran_vortex_force.f90:43-65 (SIGN < 0, direc) and :121-144
-// (SIGN > 0, flip): res = (res -+ qp(md-1)*up) -+ qm(md)*um, where the
-// vorticity is not shifted (vU(k) = vort(k)) and up/um split U_interp, the
-// WENO branch's u1d (UU averaged along e, then along d from UU_0 = 0).
-template <typename T, int PD, int SIGN>
-__device__ __forceinline__ T vf_lin(T res, const T *__restrict__ ud, T cu,
-                                    const T *__restrict__ om, int64_t based, int64_t sd, int md,
-                                    int nd, int64_t oe, int order) {
-    auto pos = [&](int p) -> int64_t { return based + (int64_t)(PD ? wrapi(p, nd) : p) * sd; };
-    auto UU = [&](int m) -> T {
-        const int64_t p = pos(m);
-        return T(0.5) * (ud[p] * cu + ud[p + oe] * cu);
-    };
-    const T uu_prev = (!PD && md == 0) ? T(0) : UU(md - 1);
-    const T ui = T(0.5) * (uu_prev + UU(md)), au = fabs(ui);
-    const T up = T(0.5) * (ui + au), um = T(0.5) * (ui - au);
-    auto v = [&](int p) -> T { return om[pos(p)]; };
-    const T a = lin_rec<T, true, false>(v, md - 1, nd, order, PD != 0) * up;
-    const T b = lin_rec<T, true, true>(v, md, nd, order, PD != 0) * um;
-    if (SIGN < 0) return (res - a) - b;
-    return (res + a) + b;
-}
-
-// Periodic axes: the byte offsets of the cells -3..+3 away along the axis
-// (wrapped), computed once per cell; every stencil load of that axis is then
-// at cb + off[..].  The loads and the arithmetic are those of the general
-// path (face_flux's interior stencil), so the results are the same.
-struct PerLine {
-    int m3, m2, m1, z, p1, p2, p3;   // byte offsets of the cells -3..+3 away
-};
-
-__device__ __forceinline__ PerLine per_line(int m, int n, int stride) {
-    PerLine L;
-    L.m3 = (wrapi(m - 3, n) - m) * stride;
-    L.m2 = (wrapi(m - 2, n) - m) * stride;
-    L.m1 = (wrapi(m - 1, n) - m) * stride;
-    L.z = 0;
-    L.p1 = (wrapi(m + 1, n) - m) * stride;
-    L.p2 = (wrapi(m + 2, n) - m) * stride;
-    L.p3 = (wrapi(m + 3, n) - m) * stride;
-    return L;
-}
-
-// offset of relative position d (-3..3; a constant at every call site, so
-// the offsets stay in registers)
-__device__ __forceinline__ int lo(const PerLine &L, int d) {
-    switch (d) {
-    case -3: return L.m3;
-    case -2: return L.m2;
-    case -1: return L.m1;
-    case 0: return L.z;
-    case 1: return L.p1;
-    case 2: return L.p2;
-    default: return L.p3;
-    }
-}
-
-// u times the WENO5 reconstruction at the face between relative positions r
-// and r + 1, upwinded by the sign of u; the value at relative position p is
-// q[c + lo(L, p + qs)] (qs = -1: the vortex force's q(k) = vort(k-1)).
-template <typename T>
-__device__ __forceinline__ T per_face(T u, const T *__restrict__ q, uint32_t cb, const PerLine &L,
-                                      int r, int qs) {
-    const uint32_t om2 = cb + lo(L, r - 2 + qs), om1 = cb + lo(L, r - 1 + qs);
-    const uint32_t o0 = cb + lo(L, r + qs), op1 = cb + lo(L, r + 1 + qs);
-    const uint32_t op2 = cb + lo(L, r + 2 + qs), op3 = cb + lo(L, r + 3 + qs);
-    // upwind stencil: offsets selected, then one set of five loads
-    const bool pos = u > T(0);
-    const uint32_t s0 = pos ? om2 : op3, s1 = pos ? om1 : op2, s2 = pos ? o0 : op1;
-    const uint32_t s3 = pos ? op1 : o0, s4 = pos ? op2 : om1;
-    return u * weno5<T>(ldb(q, s0), ldb(q, s1), ldb(q, s2), ldb(q, s3), ldb(q, s4));
-}
-
-// tracer_axis on a periodic axis (cb: the cell's byte offset)
-template <typename T>
-__device__ __forceinline__ T tracer_axis_per(T d, const T *__restrict__ q, const T *__restrict__ ud,
-                                             T cu, uint32_t cb, const PerLine &L) {
-    const T fr = per_face<T>(ldb(ud, cb) * cu, q, cb, L, 0, 0);
-    STAGE_SEQ_F(cb, fr);
-    const T fl = per_face<T>(ldb(ud, cb + L.m1) * cu, q, cb, L, -1, 0);
-    STAGE_SEQ(cb, fl);
-    return (d + fl) - fr;
-}
-
-// vf_flux on a periodic axis (cb, oe: byte offsets)
-template <typename T>
-__device__ __forceinline__ T vf_flux_per(const T *__restrict__ ud, T cu, const T *__restrict__ om,
-                                         uint32_t cb, const PerLine &L, uint32_t oe) {
-    auto UU = [&](uint32_t p) -> T { return T(0.5) * (ldb(ud, p) * cu + ldb(ud, p + oe) * cu); };
-    const T uu_prev = UU(cb + L.m1);
-    const T u1d = T(0.5) * (uu_prev + UU(cb));
-    return per_face<T>(u1d, om, cb, L, 0, -1);
-}
-
-// One direction of core/fortran_dissipation.f90:2-34 add_laplacian at a
-// cell: d + coef*(fx - fxm), fx = f(m+1) - f(m), fxm = f(m) - f(m-1); on a
-// wall axis fxm = 0 at the first cell and fx = 0 at the last (no flux
-// through the ends of the line).  om, op: byte offsets of the m-1 and m+1
-// neighbours (wrapped on a periodic axis).
-template <typename T, int P>
-__device__ __forceinline__ T lap_axis(T d, const T *__restrict__ f, uint32_t cb, int m, int n,
-                                      int32_t om, int32_t op, T coef) {
-    const T c0 = ldb(f, cb);
-    const T fx = (P || m < n - 1) ? ldb(f, cb + (uint32_t)op) - c0 : T(0);
-    const T fxm = (P || m > 0) ? c0 - ldb(f, cb + (uint32_t)om) : T(0);
-    return d + coef * (fx - fxm);
-}
-
-// add_viscosity (core/viscosity.py:3-9) for the three components of a cell:
-// for each component, the x, y and z directions in that order
-template <typename T, int PX, int PY, int PZ>
-__device__ __forceinline__ void viscosity_cell(const Geo &g, const StageArgs<T> &a, uint32_t cb,
-                                               int i, int j, int k, T &du, T &dv, T &dw) {
-    constexpr int ES = (int)sizeof(T);
-    const int32_t sx = ES, sy = (int32_t)g.sy * ES, sz = (int32_t)g.sz * ES;
-    const int32_t oxm = PX ? (wrapi(i - 1, g.nx) - i) * sx : -sx;
-    const int32_t oxp = PX ? (wrapi(i + 1, g.nx) - i) * sx : sx;
-    const int32_t oym = PY ? (wrapi(j - 1, g.ny) - j) * sy : -sy;
-    const int32_t oyp = PY ? (wrapi(j + 1, g.ny) - j) * sy : sy;
-    const int32_t ozm = PZ ? (wrapi(k - 1, g.nz) - k) * sz : -sz;
-    const int32_t ozp = PZ ? (wrapi(k + 1, g.nz) - k) * sz : sz;
-    const T cx = T(a.vcx), cy = T(a.vcy), cz = T(a.vcz);
-    auto lap3 = [&](T d, const T *__restrict__ f) -> T {
-        d = lap_axis<T, PX>(d, f, cb, i, g.nx, oxm, oxp, cx);
-        d = lap_axis<T, PY>(d, f, cb, j, g.ny, oym, oyp, cy);
-        return lap_axis<T, PZ>(d, f, cb, k, g.nz, ozm, ozp, cz);
-    };
-    du = lap3(du, a.u);
-    dv = lap3(dv, a.v);
-    dw = lap3(dw, a.w);
-}
-
-// Fused LES.rhs (core/model_les.py:129-144) + RK3_SSP stage update
-// (core/timescheme.py:199-220) for one cell.
-template <typename T, int MODE, int PX, int PY, int PZ>
-__device__ __forceinline__ void stage_cell(const Geo &g, const StageArgs<T> &a, int i, int j,
-                                           int k) {
-    const int64_t c = (int64_t)k * g.sz + (int64_t)j * g.sy + i;
-    constexpr int ES = (int)sizeof(T);
-    const uint32_t cb = (uint32_t)c * (uint32_t)ES;   // the cell's byte offset
-    PerLine Lx, Ly, Lz;
-    if constexpr (PX != 0) Lx = per_line(i, g.nx, ES);
-    if constexpr (PY != 0) Ly = per_line(j, g.ny, (int)g.sy * ES);
-    if constexpr (PZ != 0) Lz = per_line(k, g.nz, (int)g.sz * ES);
-
-    // model variants (tendencies-only mode): the linear model has no vortex
-    // force (core/model_les.py:135-136), Euler3d neither advects b
-    // (core/model_les_euler.py:131) nor adds buoyancy (core/bernoulli.py:26-32)
-    const bool vf = MODE != 0 || !(a.flags & NYL_SF_NO_VF);
-    const bool with_b = MODE != 0 || !(a.flags & NYL_SF_NO_B);
-    // the reference's linear upwind branches (tendencies-only mode)
-    const bool lin_a = MODE == 0 && a.upw_a != 0;
-    const bool lin_vf = MODE == 0 && a.upw_vf != 0;
-
-    // tracer b: rhstrac, directions i, j, k (core/tracer.py:63-72)
-    const T cx = T(a.idx2), cy = T(a.idy2), cz = T(a.idz2);
-    T db = T(0);
-    int64_t bx = c - i, by = c - (int64_t)j * g.sy, bz = c - (int64_t)k * g.sz;
-    uint32_t cs = cb;
-    if (with_b && lin_a) {
-        db = lin_tracer_axis<T, PX>(db, a.b, a.u, cx, bx, 1, i, g.nx, a.upw_a);
-        db = lin_tracer_axis<T, PY>(db, a.b, a.v, cy, by, g.sy, j, g.ny, a.upw_a);
-        db = lin_tracer_axis<T, PZ>(db, a.b, a.w, cz, bz, g.sz, k, g.nz, a.upw_a);
-    } else if (with_b) {
-        if constexpr (PX != 0) db = tracer_axis_per<T>(db, a.b, a.u, cx, cs, Lx);
-        else db = tracer_axis<T, 0>(db, a.b, a.u, cx, bx, 1, i, g.nx);
-        STAGE_SEQ_A(by, db);
-        STAGE_SEQ_A(cs, db);
-        if constexpr (PY != 0) db = tracer_axis_per<T>(db, a.b, a.v, cy, cs, Ly);
-        else db = tracer_axis<T, 0>(db, a.b, a.v, cy, by, g.sy, j, g.ny);
-        STAGE_SEQ_A(bz, db);
-        STAGE_SEQ_A(cs, db);
-        if constexpr (PZ != 0) db = tracer_axis_per<T>(db, a.b, a.w, cz, cs, Lz);
-        else db = tracer_axis<T, 0>(db, a.b, a.w, cz, bz, g.sz, k, g.nz);
-        STAGE_SEQ(bx, db);
-        STAGE_SEQ(cs, db);
-    }
-
-    // vortex force, triplets 'ikj', 'jik', 'kji' (core/vortex_force.py:69-81)
-    const int64_t oex = PX ? (int64_t)(wrapi(i + 1, g.nx) - i) : 1;
-    const int64_t oey = PY ? (int64_t)(wrapi(j + 1, g.ny) - j) * g.sy : g.sy;
-    const int64_t oez = PZ ? (int64_t)(wrapi(k + 1, g.nz) - k) * g.sz : g.sz;
-    const uint32_t bex = (uint32_t)oex * (uint32_t)ES, bey = (uint32_t)oey * (uint32_t)ES;
-    const uint32_t bez = (uint32_t)oez * (uint32_t)ES;
-    const bool ex = PX || i < g.nx - 1;   // loops stop at n-1 on a wall axis
-    const bool ey = PY || j < g.ny - 1;
-    const bool ez = PZ || k < g.nz - 1;
-    T du = T(0), dv = T(0), dw = T(0);
-    if (vf && lin_vf) {
-        // the six terms in the order below, with the linear branch
-        const int o = a.upw_vf;
-        if (ey) dv = vf_lin<T, PX, -1>(dv, a.u, cx, a.oz, bx, 1, i, g.nx, oey, o);
-        if (ex) du = vf_lin<T, PY, +1>(du, a.v, cy, a.oz, by, g.sy, j, g.ny, oex, o);
-        if (ez) dw = vf_lin<T, PY, -1>(dw, a.v, cy, a.ox, by, g.sy, j, g.ny, oez, o);
-        if (ey) dv = vf_lin<T, PZ, +1>(dv, a.w, cz, a.ox, bz, g.sz, k, g.nz, oey, o);
-        if (ex) du = vf_lin<T, PZ, -1>(du, a.w, cz, a.oy, bz, g.sz, k, g.nz, oex, o);
-        if (ez) dw = vf_lin<T, PX, +1>(dw, a.u, cx, a.oy, bx, 1, i, g.nx, oez, o);
-    } else if (vf) {
-    // direc(U_i, vor_k, du_j)
-    if (ey) {
-        if constexpr (PX != 0) dv = dv - vf_flux_per<T>(a.u, cx, a.oz, cs, Lx, bey);
-        else dv = dv - vf_flux<T, 0>(a.u, cx, a.oz, bx, 1, i, g.nx, oey);
-    }
-    STAGE_SEQ_V(by, dv, 0);
-    STAGE_SEQ_V(cs, dv, 0);
-    // flip (U_j, vor_k, du_i)
-    if (ex) {
-        if constexpr (PY != 0) du = du + vf_flux_per<T>(a.v, cy, a.oz, cs, Ly, bex);
-        else du = du + vf_flux<T, 0>(a.v, cy, a.oz, by, g.sy, j, g.ny, oex);
-    }
-    STAGE_SEQ_V(by, du, 1);
-    STAGE_SEQ_V(cs, du, 1);
-    // direc(U_j, vor_i, du_k)
-    if (ez) {
-        if constexpr (PY != 0) dw = dw - vf_flux_per<T>(a.v, cy, a.ox, cs, Ly, bez);
-        else dw = dw - vf_flux<T, 0>(a.v, cy, a.ox, by, g.sy, j, g.ny, oez);
-    }
-    STAGE_SEQ_V(bz, dw, 0);
-    STAGE_SEQ_V(cs, dw, 0);
-    // flip (U_k, vor_i, du_j)
-    if (ey) {
-        if constexpr (PZ != 0) dv = dv + vf_flux_per<T>(a.w, cz, a.ox, cs, Lz, bey);
-        else dv = dv + vf_flux<T, 0>(a.w, cz, a.ox, bz, g.sz, k, g.nz, oey);
-    }
-    STAGE_SEQ_V(bz, dv, 1);
-    STAGE_SEQ_V(cs, dv, 1);
-    // direc(U_k, vor_j, du_i)
-    if (ex) {
-        if constexpr (PZ != 0) du = du - vf_flux_per<T>(a.w, cz, a.oy, cs, Lz, bex);
-        else du = du - vf_flux<T, 0>(a.w, cz, a.oy, bz, g.sz, k, g.nz, oex);
-    }
-    STAGE_SEQ_V(bx, du, 0);
-    STAGE_SEQ_V(cs, du, 0);
-    // flip (U_i, vor_j, du_k)
-    if (ez) {
-        if constexpr (PX != 0) dw = dw + vf_flux_per<T>(a.u, cx, a.oy, cs, Lx, bez);
-        else dw = dw + vf_flux<T, 0>(a.u, cx, a.oy, bx, 1, i, g.nx, oez);
-    }
-    }
-
-    // bernoulli (core/bernoulli.py:14-23, core/fortran_bernoulli.f90:2-58)
-    const T kec = ldb(a.ke, cb);
-    if (ex) du = du - (ldb(a.ke, cb + bex) - kec);
-    if (ey) dv = dv - (ldb(a.ke, cb + bey) - kec);
-    if (ez) {
-        const T cff = T(0.5 * a.dz);
-        if (with_b) dw = dw - (ldb(a.ke, cb + bez) - kec) + cff * (ldb(a.b, cb + bez) + ldb(a.b, cb));
-        else dw = dw - (ldb(a.ke, cb + bez) - kec);
-    }
-    // viscosity at the last stage (core/model_les.py:140-141)
-    if (a.visc) viscosity_cell<T, PX, PY, PZ>(g, a, cb, i, j, k, du, dv, dw);
-
-    if (MODE == 0 || MODE == 1 || MODE == 2) {   // read at a later RK stage
-        stb_stream(a.tb, cb, db); stb_stream(a.tu, cb, du);
-        stb_stream(a.tv, cb, dv); stb_stream(a.tw, cb, dw);
-    }
-    const T cc = T(a.c);
-    if (MODE == 1) {            // s += dt*ds0
-        stb(a.bn, cb, ldb(a.b, cb) + cc * db);
-        stb(a.un, cb, ldb(a.u, cb) + cc * du);
-        stb(a.vn, cb, ldb(a.v, cb) + cc * dv);
-        stb(a.wn, cb, ldb(a.w, cb) + cc * dw);
-    } else if (MODE == 2) {     // s += (dt/4.)*(ds1-3*ds0)
-        stb(a.bn, cb, ldb(a.b, cb) + cc * (db - T(3) * ldb(a.d0b, cb)));
-        stb(a.un, cb, ldb(a.u, cb) + cc * (du - T(3) * ldb(a.d0u, cb)));
-        stb(a.vn, cb, ldb(a.v, cb) + cc * (dv - T(3) * ldb(a.d0v, cb)));
-        stb(a.wn, cb, ldb(a.w, cb) + cc * (dw - T(3) * ldb(a.d0w, cb)));
-    } else if (MODE == 3) {     // s += (dt/12.)*(8*ds2-ds0-ds1)
-        stb(a.bn, cb, ldb(a.b, cb) + cc * ((T(8) * db - ldb(a.d0b, cb)) - ldb(a.d1b, cb)));
-        stb(a.un, cb, ldb(a.u, cb) + cc * ((T(8) * du - ldb(a.d0u, cb)) - ldb(a.d1u, cb)));
-        stb(a.vn, cb, ldb(a.v, cb) + cc * ((T(8) * dv - ldb(a.d0v, cb)) - ldb(a.d1v, cb)));
-        stb(a.wn, cb, ldb(a.w, cb) + cc * ((T(8) * dw - ldb(a.d0w, cb)) - ldb(a.d1w, cb)));
-    } else if (MODE == 4) {     // LFAM3 predictor (core/timescheme.py:144-162)
-        // s = sb + (2.*dt)*ds; s = (1./12.)*(5.*s+8.*sn-sb); sb = sn
-        const T c2 = T(a.c2), c12 = T(1. / 12.);
-        T sb, t1;
-        sb = ldb(a.sbb, cb); t1 = sb + c2 * db; stb(a.bn, cb, c12 * (T(5) * t1 + T(8) * ldb(a.b, cb) - sb)); stb(a.sbb, cb, ldb(a.b, cb));
-        sb = ldb(a.sbu, cb); t1 = sb + c2 * du; stb(a.un, cb, c12 * (T(5) * t1 + T(8) * ldb(a.u, cb) - sb)); stb(a.sbu, cb, ldb(a.u, cb));
-        sb = ldb(a.sbv, cb); t1 = sb + c2 * dv; stb(a.vn, cb, c12 * (T(5) * t1 + T(8) * ldb(a.v, cb) - sb)); stb(a.sbv, cb, ldb(a.v, cb));
-        sb = ldb(a.sbw, cb); t1 = sb + c2 * dw; stb(a.wn, cb, c12 * (T(5) * t1 + T(8) * ldb(a.w, cb) - sb)); stb(a.sbw, cb, ldb(a.w, cb));
-    } else if (MODE == 5) {     // LFAM3 corrector: s = sn + dt*ds (core/timescheme.py:170-175)
-        stb(a.bn, cb, ldb(a.bn, cb) + cc * db);
-        stb(a.un, cb, ldb(a.un, cb) + cc * du);
-        stb(a.vn, cb, ldb(a.vn, cb) + cc * dv);
-        stb(a.wn, cb, ldb(a.wn, cb) + cc * dw);
-    } else if (MODE == 6) {     // first LFAM3 step: sn = s; sb = s; s += dt*ds (:352-364)
-        stb(a.sbb, cb, ldb(a.b, cb)); stb(a.sbu, cb, ldb(a.u, cb)); stb(a.sbv, cb, ldb(a.v, cb)); stb(a.sbw, cb, ldb(a.w, cb));
-        stb(a.bn, cb, ldb(a.b, cb) + cc * db);
-        stb(a.un, cb, ldb(a.u, cb) + cc * du);
-        stb(a.vn, cb, ldb(a.v, cb) + cc * dv);
-        stb(a.wn, cb, ldb(a.w, cb) + cc * dw);
-    }
-}
-
-template <typename T, int MODE, int PX, int PY, int PZ>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NYL_STAGE_WAVES)))
-void k_stage(Geo g, StageArgs<T> a) {
-#if NYL_STAGE_YSLAB
-    const Blk3 bk = xcd_block_yslab();
-#else
-    const Blk3 bk = xcd_block();
-#endif
-    const int i = bk.x * NYL_BX + threadIdx.x;
-    const int j = bk.y * NYL_BY + threadIdx.y;
-    const int k = bk.z;
-    if (i >= g.nx || j >= g.ny) return;
-    stage_cell<T, MODE, PX, PY, PZ>(g, a, i, j, k);
-}
-
-template <typename T, int PX, int PY, int PZ>
-static void launch_stage_p(const Geo &g, const StageArgs<T> &a, int mode, hipStream_t s) {
-    dim3 blk(NYL_BX, NYL_BY, 1), grd = cell_grid(g);
-    switch (mode) {
-    case 0: NYL_LAUNCH((k_stage<T, 0, PX, PY, PZ>), grd, blk, 0, s, g, a); break;
-    case 1: NYL_LAUNCH((k_stage<T, 1, PX, PY, PZ>), grd, blk, 0, s, g, a); break;
-    case 2: NYL_LAUNCH((k_stage<T, 2, PX, PY, PZ>), grd, blk, 0, s, g, a); break;
-    case 3: NYL_LAUNCH((k_stage<T, 3, PX, PY, PZ>), grd, blk, 0, s, g, a); break;
-    case 4: NYL_LAUNCH((k_stage<T, 4, PX, PY, PZ>), grd, blk, 0, s, g, a); break;
-    case 5: NYL_LAUNCH((k_stage<T, 5, PX, PY, PZ>), grd, blk, 0, s, g, a); break;
-    case 6: NYL_LAUNCH((k_stage<T, 6, PX, PY, PZ>), grd, blk, 0, s, g, a); break;
-    default: break;
-    }
-}
-
-
 // ---------------------------------------------------------------------------
 // The stage kernel as a 2.5-D march (k_stage25).  A block owns a tile of
 // S25_TX x S25_TY columns and walks a range of z planes.  Per plane:
@@ -555,18 +44,14 @@ static void launch_stage_p(const Geo &g, const StageArgs<T> &a, int mode, hipStr
 //    velocities of terms 4 and 5 are carried to the next plane.
 // Per cell that is about 9.5 reconstructions instead of 12, and no stencil
 // value is gathered from L1/L2.  Every value is the per-cell kernel's
-// expression in the same order (stage_cell, vf_flux, tracer_axis), so the
-// results are the same bits (checked on the CPU against k_stage).
+// expression in the same order (stage_cells), so the results are the same
+// bits (checked on the CPU against k_stage).  Nothing launches it: its
+// registers leave 3 waves per SIMD between the barriers (1.7 ms against 1.0
+// for k_stage_flat, FP64 256^3); it stays as an independent form of the
+// stage to check k_stage against.
 #define S25_TX 64
 #define S25_TY 4
 #define S25_NT (S25_TX * S25_TY)
-#ifndef NYL_STAGE25
-#define NYL_STAGE25 0
-#endif
-// planes per block (the grid needs many blocks to fill the chip)
-#ifndef NYL_S25_BLOCKS
-#define NYL_S25_BLOCKS 4096
-#endif
 
 constexpr int S25_BW = S25_TX + 6, S25_BH = S25_TY + 6;
 constexpr int S25_W1 = S25_TX + 1, S25_H1 = S25_TY + 1;
@@ -918,66 +403,6 @@ __global__ __launch_bounds__(S25_NT) void k_stage25(Geo g, StageArgs<T> a, int k
     }
 }
 
-static inline int s25_kz(const Geo &g) {
-    const int64_t tiles = (int64_t)((g.nx + S25_TX - 1) / S25_TX) * ((g.ny + S25_TY - 1) / S25_TY);
-    int64_t chunks = (NYL_S25_BLOCKS + tiles - 1) / tiles;
-    if (chunks > g.nz) chunks = g.nz;
-    if (chunks < 1) chunks = 1;
-    int kz = (int)((g.nz + chunks - 1) / chunks);
-    return kz < 1 ? 1 : kz;
-}
-
-// the 2.5-D form needs a full-width tile row (narrower grids keep the
-// per-cell kernel)
-static inline bool s25_fits(const Geo &g) { return NYL_STAGE25 && g.nx >= S25_TX; }
-
-template <typename T, int PX, int PY, int PZ>
-static void launch_stage25_p(const Geo &g, const StageArgs<T> &a, int mode, hipStream_t s) {
-    const int kz = s25_kz(g);
-    dim3 blk(S25_NT), grd((g.nx + S25_TX - 1) / S25_TX, (g.ny + S25_TY - 1) / S25_TY,
-                          (g.nz + kz - 1) / kz);
-    switch (mode) {
-    case 0: NYL_LAUNCH((k_stage25<T, 0, PX, PY, PZ>), grd, blk, 0, s, g, a, kz); break;
-    case 1: NYL_LAUNCH((k_stage25<T, 1, PX, PY, PZ>), grd, blk, 0, s, g, a, kz); break;
-    case 2: NYL_LAUNCH((k_stage25<T, 2, PX, PY, PZ>), grd, blk, 0, s, g, a, kz); break;
-    case 3: NYL_LAUNCH((k_stage25<T, 3, PX, PY, PZ>), grd, blk, 0, s, g, a, kz); break;
-    case 4: NYL_LAUNCH((k_stage25<T, 4, PX, PY, PZ>), grd, blk, 0, s, g, a, kz); break;
-    case 5: NYL_LAUNCH((k_stage25<T, 5, PX, PY, PZ>), grd, blk, 0, s, g, a, kz); break;
-    case 6: NYL_LAUNCH((k_stage25<T, 6, PX, PY, PZ>), grd, blk, 0, s, g, a, kz); break;
-    default: break;
-    }
-}
-
-template <typename T>
-hipError_t launch_stage(const Geo &g, const StageArgs<T> &a, int mode, hipStream_t s) {
-    if (mode < 0 || mode > 6) return hipErrorInvalidValue;
-#if NYL_STAGE25
-    const bool t25 = s25_fits(g) && a.flags == 0;   // the 2.5-D form runs the LES only
-#define NYL_STAGE_GO(X, Y, Z)                                                        \
-    do {                                                                             \
-        if (t25) launch_stage25_p<T, X, Y, Z>(g, a, mode, s);                        \
-        else launch_stage_p<T, X, Y, Z>(g, a, mode, s);                              \
-    } while (0)
-#else
-#define NYL_STAGE_GO(X, Y, Z) launch_stage_p<T, X, Y, Z>(g, a, mode, s)
-#endif
-    switch (g.px + 2 * g.py + 4 * g.pz) {
-#define NYL_STAGE_CASE(c, X, Y, Z)                                                   \
-    case c: NYL_STAGE_GO(X, Y, Z); break;
-    NYL_STAGE_CASE(0, 0, 0, 0)
-    NYL_STAGE_CASE(1, 1, 0, 0)
-    NYL_STAGE_CASE(2, 0, 1, 0)
-    NYL_STAGE_CASE(3, 1, 1, 0)
-    NYL_STAGE_CASE(4, 0, 0, 1)
-    NYL_STAGE_CASE(5, 1, 0, 1)
-    NYL_STAGE_CASE(6, 0, 1, 1)
-    default: NYL_STAGE_GO(1, 1, 1); break;
-#undef NYL_STAGE_CASE
-#undef NYL_STAGE_GO
-    }
-    return hipGetLastError();
-}
-
 // ---------------------------------------------------------------------------
 // Passive tracers: the b part of stage_cell for another scalar, with the
 // stage update of the mode (same expressions as b's).
@@ -995,15 +420,14 @@ __device__ __forceinline__ void tracer_cell(const Geo &g, const TracerArgs<T> &a
         dq = lin_tracer_axis<T, PY>(dq, a.q, a.v, cy, by, g.sy, j, g.ny, a.upw);
         dq = lin_tracer_axis<T, PZ>(dq, a.q, a.w, cz, bz, g.sz, k, g.nz, a.upw);
     } else {
-        if constexpr (PX != 0)
-            dq = tracer_axis_per<T>(dq, a.q, a.u, cx, cb, per_line(i, g.nx, ES));
-        else dq = tracer_axis<T, 0>(dq, a.q, a.u, cx, bx, 1, i, g.nx);
-        if constexpr (PY != 0)
-            dq = tracer_axis_per<T>(dq, a.q, a.v, cy, cb, per_line(j, g.ny, (int)g.sy * ES));
-        else dq = tracer_axis<T, 0>(dq, a.q, a.v, cy, by, g.sy, j, g.ny);
-        if constexpr (PZ != 0)
-            dq = tracer_axis_per<T>(dq, a.q, a.w, cz, cb, per_line(k, g.nz, (int)g.sz * ES));
-        else dq = tracer_axis<T, 0>(dq, a.q, a.w, cz, bz, g.sz, k, g.nz);
+        const LineX<1> Lx = linex_of<1, PX>(i, g.nx, ES);
+        const Line<int32_t> Ly = line_of<PY, int32_t>(j, g.ny, (int32_t)(g.sy * ES));
+        const Line<int32_t> Lz = line_of<PZ, int32_t>(k, g.nz, (int32_t)(g.sz * ES));
+        Vec<T, 1> d = {};
+        tracer_x<1, PX>(d, a.q, a.u, cx, cb, Lx, i, g.nx);
+        tracer_yz<1, PY>(d, a.q, a.v, cy, cb, Ly, j, g.ny);
+        tracer_yz<1, PZ>(d, a.q, a.w, cz, cb, Lz, k, g.nz);
+        dq = d.v[0];
     }
 
     if (MODE == 0 || MODE == 1 || MODE == 2) stb(a.tout, cb, dq);
@@ -1604,7 +1028,7 @@ __global__ __launch_bounds__(TPB) void k_b_stage(const StageItem<T> *__restrict_
         StageArgs<T> a = it.a;
         const double d = dt[it.h.member];
         a.c = MODE == 1 ? d : (MODE == 2 ? d / 4. : d / 12.);
-        stage_cell<T, MODE, PX, PY, PZ>(it.h.g, a, i, j, k);
+        stage_cells<T, 1, MODE, PX, PY, PZ, MODE == 0, int32_t, int32_t>(it.h.g, a, i, j, k);
     }
 }
 
@@ -1709,8 +1133,6 @@ NYL_B_STENCIL_INST(double)
 NYL_B_STENCIL_INST(float)
 #undef NYL_B_STENCIL_INST
 
-template hipError_t launch_stage<double>(const Geo &, const StageArgs<double> &, int, hipStream_t);
-template hipError_t launch_stage<float>(const Geo &, const StageArgs<float> &, int, hipStream_t);
 template hipError_t launch_tracer_stage<double>(const Geo &, const TracerArgs<double> &, int,
                                                 hipStream_t);
 template hipError_t launch_tracer_stage<float>(const Geo &, const TracerArgs<float> &, int,
