@@ -537,13 +537,24 @@ int coarse_levels(nyl_ctx *c, const CtlArgs *fin) {
     return NYL_OK;
 }
 
+// Level 0's pre-smoothing as one march with the restriction in it (x, b read
+// and y written once), or as the tiled two-sweep pass and the tiled
+// restriction (y and b read once more).  One march: levels that do not tile,
+// FP64 from 4M cells, and FP32 whose three fields exceed the 256 MB cache.
+// us of pre-smoothing + restriction + post-smoothing, two passes / one: FP64
+// 256^3 270 / 253, 128x128x256 75 / 71, 128^3 45.7 / 48.1; FP32 256x256x512
+// 323 / 279, 256x256x384 210 / 207, 320x256x256 163 / 181, 256^3 131 / 135;
+// not tiled (two marches / one) FP64 160^3 78 / 72, 96^3 36 / 35, FP32
+// 200x120x56 39.3 / 38.1, 240^3 125 / 124.
+bool pre_tiled(const nyl_ctx *c) {
+    const double n = cells(c->lev[0].g);
+    return tiled_level(c, 0) &&
+           (lev64(c, 0) ? n < (1 << 22) : 3.0 * n * sizeof(float) <= 256.0 * (1 << 20));
+}
+
 // Both pre-smoothing sweeps of level 0 into its y and the restriction into
 // level 1.  zero: from a zero solution; else from x, with the block sums of
 // its residual norm in the partials (their number in *np).
-// A level that does not tile runs the march; up to 1M cells with the
-// restriction in the same pass (96^3 FP64: 19.4 us against 12.9 + 7.0), above
-// that its wider rings cost more than the second pass reads (192x128x96: 39
-// against 20.7 + 11.6).
 int pre_smooth(nyl_ctx *c, bool zero, int *np) {
     const Level &f = c->lev[0], &q = c->lev[1];
     const double om = c->d.mg_omega, n = cells(f.g) * elem(c, 0);
@@ -552,7 +563,7 @@ int pre_smooth(nyl_ctx *c, bool zero, int *np) {
         using T = decltype(t);
         using TC = decltype(tc);
         if constexpr (std::is_same<T, TC>::value) {
-            if (tiled_level(c, 0)) {
+            if (pre_tiled(c)) {
                 if (zero) {
                     // (not in the fine-level class of the roofline: it reads one field)
                     LAUNCH(NYL_K_MG_SWEEP2, 2 * n,
@@ -572,15 +583,12 @@ int pre_smooth(nyl_ctx *c, bool zero, int *np) {
             }
         }
         MarchArgs<T, TC> a = march_args<T, TC>(c, 0, f.x, f.y);
-        const bool one = cells(f.g) <= (1 << 20);
         if (zero) a.src = nullptr;
         else a.partials = part;
-        if (one) {
-            a.bc = F<TC>(c, q.b);
-            a.yc = F<TC>(c, q.y);
-        }
+        a.bc = F<TC>(c, q.b);
+        a.yc = F<TC>(c, q.y);
         if (!zero) {
-            *np = march_grid(f.g, march_resident(sizeof(T), MS_FIELD, 2, one), one).blocks();
+            *np = march_grid(f.g, march_resident(sizeof(T), MS_FIELD, 2, true), true).blocks();
             if (*np > NYL_RED_BLOCKS) {   // too wide for one partial sum per block
                 if constexpr (std::is_same<T, double>::value) {
                     LAUNCH(NYL_K_RESNORM, 2 * n,
@@ -593,14 +601,9 @@ int pre_smooth(nyl_ctx *c, bool zero, int *np) {
                 }
             }
         }
-        LAUNCH(NYL_K_MG_SWEEP2 | (zero ? 0 : kFineLevel), (zero ? 2 : 3) * n,
+        LAUNCH(NYL_K_MG_SWEEP2 | (zero ? 0 : kFineLevel),
+               (zero ? 2 : 3) * n + 2 * cells(q.g) * sizeof(TC),
                (launch_march_pre<T, TC>(a, c->stream)));
-        if (!one) {
-            MarchArgs<T, TC> r = march_args<T, TC>(c, 0, f.y, f.x);
-            r.bc = F<TC>(c, q.b);
-            r.yc = F<TC>(c, q.y);
-            LAUNCH(NYL_K_MG_RESTRICT, 2.25 * n, (launch_march_restrict<T, TC>(r, c->stream)));
-        }
         return NYL_OK;
     });
 }

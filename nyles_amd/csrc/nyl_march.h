@@ -68,13 +68,10 @@ hipError_t launch_march_up(const MarchArgs<T, TC> &a, hipStream_t s);
 // one sweep src -> dst, then residual and restriction of dst into bc and yc
 template <typename T, typename TC>
 hipError_t launch_march_down(const MarchArgs<T, TC> &a, hipStream_t s);
-// two sweeps src (null: zero) -> dst; partials non-null: the residual norm of
-// src; bc, yc non-null: also the residual and restriction of dst
+// two sweeps src (null: zero) -> dst, then residual and restriction of dst
+// into bc and yc; partials non-null: also the residual norm of src
 template <typename T, typename TC>
 hipError_t launch_march_pre(const MarchArgs<T, TC> &a, hipStream_t s);
-// residual and restriction of src into bc and yc
-template <typename T, typename TC>
-hipError_t launch_march_restrict(const MarchArgs<T, TC> &a, hipStream_t s);
 // the residual norm of src alone
 template <typename T>
 hipError_t launch_march_norm(const MarchArgs<T, T> &a, hipStream_t s);

@@ -506,25 +506,11 @@ hipError_t launch_march_down(const MarchArgs<T, TC> &a, hipStream_t s) {
 }
 
 template <typename T, typename TC>
-hipError_t launch_march_restrict(const MarchArgs<T, TC> &a, hipStream_t s) {
-    if (!a.bc || !a.yc) return hipErrorInvalidValue;
-    MARCH_GO(T, TC, MS_FIELD, 0, false, true, false);
-    return hipGetLastError();
-}
-
-template <typename T, typename TC>
 hipError_t launch_march_pre(const MarchArgs<T, TC> &a, hipStream_t s) {
-    if (a.src == a.dst || (!a.src && a.partials)) return hipErrorInvalidValue;
-    if (a.bc) {
-        if (!a.yc) return hipErrorInvalidValue;
-        if (!a.src) MARCH_GO(T, TC, MS_ZERO, 2, false, true, false);
-        else if (a.partials) MARCH_GO(T, TC, MS_FIELD, 2, true, true, false);
-        else MARCH_GO(T, TC, MS_FIELD, 2, false, true, false);
-        return hipGetLastError();
-    }
-    if (!a.src) MARCH_GO(T, TC, MS_ZERO, 2, false, false, false);
-    else if (a.partials) MARCH_GO(T, TC, MS_FIELD, 2, true, false, false);
-    else MARCH_GO(T, TC, MS_FIELD, 2, false, false, false);
+    if (a.src == a.dst || (!a.src && a.partials) || !a.bc || !a.yc) return hipErrorInvalidValue;
+    if (!a.src) MARCH_GO(T, TC, MS_ZERO, 2, false, true, false);
+    else if (a.partials) MARCH_GO(T, TC, MS_FIELD, 2, true, true, false);
+    else MARCH_GO(T, TC, MS_FIELD, 2, false, true, false);
     return hipGetLastError();
 }
 
@@ -585,8 +571,7 @@ template hipError_t launch_b_march<float, double>(const MarchItem<float, double>
 #define NYL_MARCH_INST(T, TC)                                                              \
     template hipError_t launch_march_up<T, TC>(const MarchArgs<T, TC> &, hipStream_t);     \
     template hipError_t launch_march_down<T, TC>(const MarchArgs<T, TC> &, hipStream_t);   \
-    template hipError_t launch_march_pre<T, TC>(const MarchArgs<T, TC> &, hipStream_t);    \
-    template hipError_t launch_march_restrict<T, TC>(const MarchArgs<T, TC> &, hipStream_t);
+    template hipError_t launch_march_pre<T, TC>(const MarchArgs<T, TC> &, hipStream_t);
 NYL_MARCH_INST(double, double)
 NYL_MARCH_INST(float, float)
 NYL_MARCH_INST(float, double)
