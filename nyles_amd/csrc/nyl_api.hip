@@ -1035,9 +1035,10 @@ double stage_words(int mode) {
     }
 }
 
-// mode st of the stage kernel; slot >= 0 also writes the tendencies there
+// mode st of the stage kernel (mode tst of the passive tracers'); slot >= 0
+// also writes the tendencies there
 template <typename T>
-int stage_t(nyl_ctx *c, int st, int slot, double coef, double coef2, bool last) {
+int stage_t(nyl_ctx *c, int st, int tst, int slot, double coef, double coef2, bool last) {
     StageArgs<T> a = stage_args<T>(c);
     if (slot >= 0) set_tendency_out<T>(c, a, slot);
     a.c = coef;
@@ -1050,7 +1051,7 @@ int stage_t(nyl_ctx *c, int st, int slot, double coef, double coef2, bool last) 
     }
     if (c->d.model == NYL_MODEL_LINEAR) a.flags |= NYL_SF_NO_VF;
     if (c->d.model == NYL_MODEL_EULER) a.flags |= NYL_SF_NO_B;
-    const double words = stage_words(st);
+    const double words = stage_words(st) + (st == 3 && slot == 2 ? 4 : 0);
     LAUNCH(NYL_K_STAGE, words * cells(c->g) * sizeof(T), launch_stage<T>(c->g, a, st, c->stream));
     // passive tracers: the same right-hand side and update, one launch each;
     // Euler3d advects none of them (zero tendencies)
@@ -1072,17 +1073,18 @@ int stage_t(nyl_ctx *c, int st, int slot, double coef, double coef2, bool last) 
         ta.c = coef;
         ta.c2 = coef2;
         ta.upw = c->d.upwind_a;
-        LAUNCH(NYL_K_STAGE, (words / 4.0) * cells(c->g) * sizeof(T),
-               launch_tracer_stage<T>(c->g, ta, st, c->stream));
+        LAUNCH(NYL_K_STAGE, (stage_words(tst) / 4.0) * cells(c->g) * sizeof(T),
+               launch_tracer_stage<T>(c->g, ta, tst, c->stream));
     }
     return NYL_OK;
 }
 
 // the stage combination of mode st from the stored tendencies of every
-// prognostic field (b, u, v, w, tracers): slot 0 for modes 1 and 4..6, slots
-// 0..1 for mode 2 and 0..2 for mode 3
+// prognostic field (b, u, v, w unless only the tracers are asked for;
+// tracers): slot 0 for modes 1 and 4..6, slots 0..1 for mode 2 and 0..2 for
+// mode 3
 template <typename T>
-int update_t(nyl_ctx *c, int st, double coef, double coef2) {
+int update_t(nyl_ctx *c, int st, double coef, double coef2, bool tracers_only = false) {
     const int s = c->cur, t = 1 - c->cur;
     auto one = [&](uint64_t cur, uint64_t nxt, uint64_t d0, uint64_t d1, uint64_t d2,
                    uint64_t sb) -> int {
@@ -1099,7 +1101,7 @@ int update_t(nyl_ctx *c, int st, double coef, double coef2) {
         return NYL_OK;
     };
     int rc;
-    for (int f = 0; f < 4; f++)
+    for (int f = 0; f < 4 && !tracers_only; f++)
         if ((rc = one(c->state[s][f], c->state[t][f], c->ds[0][f], c->ds[1][f], c->ds[2][f],
                       c->sb[f])))
             return rc;
@@ -1116,21 +1118,24 @@ int stage(nyl_ctx *c, int st, double coef, double coef2, bool last) {
     int rc;
     if (c->d.model != NYL_MODEL_LES || c->d.upwind_a || c->d.upwind_vf) {
         // model variants and the linear upwind branches: the tendencies
-        // into the slot the stage combination
-        // reads last (0 for modes 1 and 4..6, 1 for mode 2, 2 for mode 3),
-        // then the combination
+        // into the slot the stage combination reads last (0 for modes 1 and
+        // 4..6, 1 for mode 2, 2 for mode 3), then the combination; the stages
+        // of RK3 combine b, u, v, w in the stage kernel (256x128x64 FP32,
+        // order 5: 91 us and four updates of 7 became 50..59 us)
         const int slot = st == 2 ? 1 : (st == 3 ? 2 : 0);
-        rc = c->mixed ? stage_t<float>(c, 0, slot, 0.0, 0.0, last)
-                      : stage_t<double>(c, 0, slot, 0.0, 0.0, last);
+        const bool one = st <= 3;
+        rc = c->mixed ? stage_t<float>(c, one ? st : 0, 0, slot, coef, coef2, last)
+                      : stage_t<double>(c, one ? st : 0, 0, slot, coef, coef2, last);
         if (rc) return rc;
-        rc = c->mixed ? update_t<float>(c, st, coef, coef2) : update_t<double>(c, st, coef, coef2);
+        rc = c->mixed ? update_t<float>(c, st, coef, coef2, one)
+                      : update_t<double>(c, st, coef, coef2, one);
         if (rc) return rc;
         if (st != 5) c->cur = 1 - c->cur;
         return NYL_OK;
     }
     const int slot = (st == 1 || st == 2) ? st - 1 : -1;
-    rc = c->mixed ? stage_t<float>(c, st, slot, coef, coef2, last)
-                  : stage_t<double>(c, st, slot, coef, coef2, last);
+    rc = c->mixed ? stage_t<float>(c, st, st, slot, coef, coef2, last)
+                  : stage_t<double>(c, st, st, slot, coef, coef2, last);
     if (rc) return rc;
     if (st != 5) c->cur = 1 - c->cur;
     return NYL_OK;
@@ -1348,8 +1353,8 @@ int nyl_rhs(nyl_ctx *c, int slot, int last) {
     int rc = check_ready(c);
     if (rc) return rc;
     if (slot < 0 || slot > 2) return fail(NYL_E_ARG, "slot must be 0..2");
-    return c->mixed ? stage_t<float>(c, 0, slot, 0.0, 0.0, last != 0)
-                    : stage_t<double>(c, 0, slot, 0.0, 0.0, last != 0);
+    return c->mixed ? stage_t<float>(c, 0, 0, slot, 0.0, 0.0, last != 0)
+                    : stage_t<double>(c, 0, 0, slot, 0.0, 0.0, last != 0);
 }
 
 int nyl_stage_update(nyl_ctx *c, int mode, double coef, double coef2) {

@@ -50,12 +50,12 @@ struct StageArgs {
     // vc_d = viscosity * ids2[d] (core/viscosity.py:3-9)
     double vcx, vcy, vcz;
     int visc;
-    // model variant, mode 0 only (the variants run tendencies + update):
-    // bit 0 no vortex force (linear model), bit 1 no advection of b and no
+    // model variant, modes 0..3 only (the variants' other stages run
+    // tendencies + update): bit 0 no vortex force (linear model), bit 1 no advection of b and no
     // buoyancy (Euler3d)
     int flags;
     // linear upwind orders (1, 3, 5) of the tracer advection and of the
-    // vortex force, mode 0 only; 0: WENO (the branch the reference runs)
+    // vortex force, modes 0..3 only; 0: WENO (the branch the reference runs)
     int upw_a, upw_vf;
 };
 #define NYL_SF_NO_VF 1
@@ -66,6 +66,18 @@ struct StageArgs {
 // 6: Euler step that also copies the state into the LFAM3 'before' state
 template <typename T>
 hipError_t launch_stage(const Geo &g, const StageArgs<T> &a, int mode, hipStream_t s);
+// the kernels of launch_stage for non-zero flags or orders (modes 0..3, which
+// store the tendencies too)
+template <typename T>
+hipError_t launch_stage_lin(const Geo &g, const StageArgs<T> &a, int mode, hipStream_t s);
+template <>
+hipError_t launch_stage<double>(const Geo &, const StageArgs<double> &, int, hipStream_t);
+template <>
+hipError_t launch_stage<float>(const Geo &, const StageArgs<float> &, int, hipStream_t);
+template <>
+hipError_t launch_stage_lin<double>(const Geo &, const StageArgs<double> &, int, hipStream_t);
+template <>
+hipError_t launch_stage_lin<float>(const Geo &, const StageArgs<float> &, int, hipStream_t);
 
 // One passive tracer (core/model_les.py:36-43): its flux divergence with the
 // current U (core/tracer.py:59-72, as for b) and the stage update of the

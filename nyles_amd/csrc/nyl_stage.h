@@ -57,74 +57,46 @@ __device__ __forceinline__ void stb_stream(T *__restrict__ p, uint32_t boff, T v
 // core/fortran_upwind.f90:30, core/fortran_vortex_force.f90:28,104), odd
 // orders 1, 3, 5.  REAL(4) literals widened; sums left to right as written.
 
-// Reconstruction at line position j of the values q(.) (a functor over
-// positions, wrapped on a periodic axis): RIGHT = false the left-biased qp,
-// true the right-biased qm.  On a wall line the order drops near the ends:
-// tracer flavour (core/interpolate_tracer.f90:45-80) first order at 0 and
-// n-1, third at 1 and n-2; vortex-force flavour (core/interpolate.f90:35-79)
-// qp(-1) = 0, first order at 0 and n-2 (and qm at n-1), third at 1 and n-3.
-template <typename T, bool VF, bool RIGHT, typename QF>
-__device__ __forceinline__ T lin_rec(const QF &q, int j, int n, int order, bool per) {
+// The order at line position j of the left-biased (qp) or, RIGHT, the
+// right-biased (qm) reconstruction; 0: the value is zero.  On a wall line it
+// drops near the ends: tracer flavour (core/interpolate_tracer.f90:45-80)
+// first order at 0 and n-1, third at 1 and n-2; vortex-force flavour
+// (core/interpolate.f90:35-79) qp(-1) = 0, first order at 0 and n-2 (and qm
+// at n-1), third at 1 and n-3.
+template <bool VF, bool RIGHT>
+__device__ __forceinline__ int lin_order(int j, int n, int order, bool per) {
+    if (per) return order;
+    if (VF && !RIGHT && j < 0) return 0;
+    const int last1 = VF ? n - 2 : n - 1;          // first order at 0 and here
+    if (j <= 0 || j >= last1) return 1;
+    return order == 5 && (j == 1 || j == last1 - 1) ? 3 : order;
+}
+// The reconstruction of that order from the values at j-2 .. j+2.
+template <typename T, bool RIGHT>
+__device__ __forceinline__ T lin_value(int ord, T q0, T q1, T q2, T q3, T q4) {
     const T c1 = T(-(1.0f / 6.0f)), c2 = T(5.0f / 6.0f), c3 = T(2.0f / 6.0f);
     const T b1 = T(2.0f / 60.0f), b2 = T(-(13.0f / 60.0f)), b3 = T(47.0f / 60.0f);
     const T b4 = T(27.0f / 60.0f), b5 = T(-(3.0f / 60.0f));
-    int ord = order;
-    if (!per) {
-        if (VF && !RIGHT && j < 0) return T(0);
-        const int last1 = VF ? n - 2 : n - 1;          // first order at 0 and here
-        if (j <= 0 || j >= last1) ord = 1;
-        else if (order == 5 && (j == 1 || j == last1 - 1)) ord = 3;
-    }
-    if (ord == 1) return q(j);
+    if (ord == 0) return T(0);
+    if (ord == 1) return q2;
     if (ord == 3) {
-        if (RIGHT) return c3 * q(j - 1) + c2 * q(j) + c1 * q(j + 1);
-        return c1 * q(j - 1) + c2 * q(j) + c3 * q(j + 1);
+        if (RIGHT) return c3 * q1 + c2 * q2 + c1 * q3;
+        return c1 * q1 + c2 * q2 + c3 * q3;
     }
-    if (RIGHT) return b5 * q(j - 2) + b4 * q(j - 1) + b3 * q(j) + b2 * q(j + 1) + b1 * q(j + 2);
-    return b1 * q(j - 2) + b2 * q(j - 1) + b3 * q(j) + b4 * q(j + 1) + b5 * q(j + 2);
+    if (RIGHT) return b5 * q0 + b4 * q1 + b3 * q2 + b2 * q3 + b1 * q4;
+    return b1 * q0 + b2 * q1 + b3 * q2 + b4 * q3 + b5 * q4;
 }
-
-// core/fortran_upwind.f90:34-67: d = (d + fx(m-1)) - fx(m), the face flux
-// fx(i) = up(i)*qp(i) + um(i)*qm(i+1) with up/um = 0.5*(U -+ |U|), no flux
-// through the ends of a wall line.  U_d = ud*cu as in tracer_axis.
-template <typename T, int PD>
-__device__ __forceinline__ T lin_tracer_axis(T d, const T *__restrict__ q_arr,
-                                             const T *__restrict__ ud, T cu, int64_t based,
-                                             int64_t sd, int m, int n, int order) {
-    auto pos = [&](int p) -> int64_t { return based + (int64_t)(PD ? wrapi(p, n) : p) * sd; };
-    auto q = [&](int p) -> T { return q_arr[pos(p)]; };
-    auto face = [&](int i) -> T {
-        const T ui = ud[pos(i)] * cu, au = fabs(ui);
-        const T up = T(0.5) * (ui + au), um = T(0.5) * (ui - au);
-        return up * lin_rec<T, false, false>(q, i, n, order, PD != 0)
-             + um * lin_rec<T, false, true>(q, i + 1, n, order, PD != 0);
-    };
-    const T fxm = (PD || m > 0) ? face(m - 1) : T(0);
-    const T fx = (PD || m < n - 1) ? face(m) : T(0);
-    return (d + fxm) - fx;
-}
-
-// core/fortran_vortex_force.f90:43-65 (SIGN < 0, direc) and :121-144
-// (SIGN > 0, flip): res = (res -+ qp(md-1)*up) -+ qm(md)*um, where the
-// vorticity is not shifted (vU(k) = vort(k)) and up/um split U_interp, the
-// WENO branch's u1d (UU averaged along e, then along d from UU_0 = 0).
-template <typename T, int PD, int SIGN>
-__device__ __forceinline__ T vf_lin(T res, const T *__restrict__ ud, T cu,
-                                    const T *__restrict__ om, int64_t based, int64_t sd, int md,
-                                    int nd, int64_t oe, int order) {
-    auto pos = [&](int p) -> int64_t { return based + (int64_t)(PD ? wrapi(p, nd) : p) * sd; };
-    auto UU = [&](int m) -> T {
-        const int64_t p = pos(m);
-        return T(0.5) * (ud[p] * cu + ud[p + oe] * cu);
-    };
-    const T uu_prev = (!PD && md == 0) ? T(0) : UU(md - 1);
-    const T ui = T(0.5) * (uu_prev + UU(md)), au = fabs(ui);
-    const T up = T(0.5) * (ui + au), um = T(0.5) * (ui - au);
-    auto v = [&](int p) -> T { return om[pos(p)]; };
-    const T a = lin_rec<T, true, false>(v, md - 1, nd, order, PD != 0) * up;
-    const T b = lin_rec<T, true, true>(v, md, nd, order, PD != 0) * um;
-    if (SIGN < 0) return (res - a) - b;
-    return (res + a) + b;
+// The two upwind contributions at a face from its six values: the left-biased
+// reconstruction at line position j times up and the right-biased one at
+// j + 1 times um, up/um = 0.5*(U -+ |U|).
+template <typename T, bool VF, int PER>
+__device__ __forceinline__ void lin_parts(T u, const Stencil6<T> &w, int j, int n, int order, T &a,
+                                          T &b) {
+    const T au = fabs(u), up = T(0.5) * (u + au), um = T(0.5) * (u - au);
+    a = up * lin_value<T, false>(lin_order<VF, false>(j, n, order, PER != 0), w.m2, w.m1, w.z0,
+                                 w.p1, w.p2);
+    b = um * lin_value<T, true>(lin_order<VF, true>(j + 1, n, order, PER != 0), w.m1, w.z0, w.p1,
+                                w.p2, w.p3);
 }
 
 // Byte offsets of the cells -3..+3 away along an axis, wrapped on a periodic
@@ -256,14 +228,32 @@ __device__ __forceinline__ void load_next(T (&r)[N + 1], const T *__restrict__ f
 // five selected in registers: a wavefront with both directions in it then
 // reads whole lines once (selected addresses scatter it over two sets).
 //
-// Tracer flux divergence along x of N cells (core/fortran_upwind.f90:77-81):
-// d = d + flux(m-1) - flux(m), or d - flux(1) at a wall start; the N + 1
-// faces are evaluated once.  U_d = ud*cu, recomputed from the covariant
-// velocity with the product U_from_u stores (core/cov_to_contra.py:15-17).
-template <int N, int PER, typename T>
+// The tracer flux at line position m, and its divergence d + flux(m-1) -
+// flux(m) with no flux through the ends of a wall line.  WENO
+// (core/fortran_upwind.f90:77-81), or, order = 1, 3, 5 (LIN), the linear
+// branch (:34-67): fx(i) = up(i)*qp(i) + um(i)*qm(i+1).
+template <typename T, int PER, bool LIN>
+__device__ __forceinline__ T tracer_flux(int m, int n, T u, const Stencil6<T> &w, int order) {
+    if (LIN && order != 0) {
+        if (!PER && m == n - 1) return T(0);
+        T a, b;
+        lin_parts<T, false, PER>(u, w, m, n, order, a, b);
+        return a + b;
+    }
+    return face_of<T, PER>(m, n, u, w);
+}
+template <typename T, int PER, bool LIN>
+__device__ __forceinline__ T tracer_div(T d, T fl, T fr, int m, int order) {
+    if (!PER && m == 0) return LIN && order != 0 ? (d + T(0)) - fr : d - fr;
+    return (d + fl) - fr;
+}
+// Along x, N cells: the N + 1 faces are evaluated once.  U_d = ud*cu,
+// recomputed from the covariant velocity with the product U_from_u stores
+// (core/cov_to_contra.py:15-17).
+template <int N, int PER, bool LIN, typename T>
 __device__ __forceinline__ void tracer_x(Vec<T, N> &d, const T *__restrict__ q,
                                          const T *__restrict__ ud, T cu, uint32_t cb,
-                                         const LineX<N> &L, int i, int nx) {
+                                         const LineX<N> &L, int i, int nx, int order) {
     T r[N + 8], u[N + 1], fl[N + 1];
     load_row<N, true>(r, q, cb, L);
     load_next<N, true>(u, ud, cb, L, (int32_t)0);
@@ -271,17 +261,17 @@ __device__ __forceinline__ void tracer_x(Vec<T, N> &d, const T *__restrict__ q,
     for (int f = 0; f <= N; f++) {
         const int m = i + f - 1;
         const Stencil6<T> w = {r[f + 1], r[f + 2], r[f + 3], r[f + 4], r[f + 5], r[f + 6]};
-        fl[f] = face_of<T, PER>(PER ? 0 : m, nx, u[f] * cu, w);
+        fl[f] = tracer_flux<T, PER, LIN>(PER ? 0 : m, nx, u[f] * cu, w, order);
     }
 #pragma unroll
     for (int c = 0; c < N; c++)
-        d.v[c] = (!PER && i + c == 0) ? d.v[c] - fl[c + 1] : (d.v[c] + fl[c]) - fl[c + 1];
+        d.v[c] = tracer_div<T, PER, LIN>(d.v[c], fl[c], fl[c + 1], i + c, order);
 }
 // ... and along y or z (line position m of n)
-template <int N, int PER, typename T, typename O>
+template <int N, int PER, bool LIN, typename T, typename O>
 __device__ __forceinline__ void tracer_yz(Vec<T, N> &d, const T *__restrict__ q,
                                           const T *__restrict__ ud, T cu, uint32_t cb,
-                                          const Line<O> &L, int m, int n) {
+                                          const Line<O> &L, int m, int n, int order) {
     const Vec<T, N> m3 = ldv<N>(q, cb, L.m3), m2 = ldv<N>(q, cb, L.m2), m1 = ldv<N>(q, cb, L.m1);
     const Vec<T, N> z0 = ldv<N>(q, cb), p1 = ldv<N>(q, cb, L.p1), p2 = ldv<N>(q, cb, L.p2);
     const Vec<T, N> p3 = ldv<N>(q, cb, L.p3), u1 = ldv<N>(ud, cb), u0 = ldv<N>(ud, cb, L.m1);
@@ -289,25 +279,40 @@ __device__ __forceinline__ void tracer_yz(Vec<T, N> &d, const T *__restrict__ q,
     for (int c = 0; c < N; c++) {
         const Stencil6<T> hi = {m2.v[c], m1.v[c], z0.v[c], p1.v[c], p2.v[c], p3.v[c]};
         const Stencil6<T> lo = {m3.v[c], m2.v[c], m1.v[c], z0.v[c], p1.v[c], p2.v[c]};
-        const T fr = face_of<T, PER>(m, n, u1.v[c] * cu, hi);
-        if (!PER && m == 0) {
-            d.v[c] = d.v[c] - fr;
-        } else {
-            const T fl = face_of<T, PER>(m - 1, n, u0.v[c] * cu, lo);
-            d.v[c] = (d.v[c] + fl) - fr;
-        }
+        const T fr = tracer_flux<T, PER, LIN>(m, n, u1.v[c] * cu, hi, order);
+        T fl = T(0);
+        if (PER || m > 0) fl = tracer_flux<T, PER, LIN>(m - 1, n, u0.v[c] * cu, lo, order);
+        d.v[c] = tracer_div<T, PER, LIN>(d.v[c], fl, fr, m, order);
     }
 }
 
-// Vortex-force flux of one term at N cells (core/fortran_vortex_force.f90
-// WENO branch, :66-81 and :145-159): the vorticity component `om` is
-// upwinded along axis d with the contravariant velocity U_d = ud*cu
-// averaged along the target axis e (UU, UU_0 = 0. at the line start) and then
-// along d (u1d); q(1) = 0., q(k) = vort(k-1).  Along x, averaged with the
-// cells at offset oe:
-template <int N, int PER, typename T, typename E>
-__device__ __forceinline__ Vec<T, N> vf_x(const T *__restrict__ ud, T cu, const T *__restrict__ om,
-                                          uint32_t cb, const LineX<N> &L, int i, int nx, E oe) {
+// One term of the vortex force at N cells, d -+ its flux: the vorticity
+// component `om` is upwinded along axis d with the contravariant velocity
+// U_d = ud*cu averaged along the target axis e (UU, UU_0 = 0. at the line
+// start) and then along d (u1d).  WENO (core/fortran_vortex_force.f90:66-81,
+// 145-159): q(1) = 0., q(k) = vort(k-1).  Linear (order != 0; :43-65 direc,
+// :121-144 flip): (d -+ qp(md-1)*up) -+ qm(md)*um, where the vorticity is not
+// shifted -- the same six values.
+template <typename T, int PER, int SIGN, bool LIN>
+__device__ __forceinline__ T vf_term(T d, int m, int n, T u1d, Stencil6<T> &w, int order) {
+    if (LIN && order != 0) {
+        T a, b;
+        lin_parts<T, true, PER>(u1d, w, m - 1, n, order, a, b);
+        return SIGN < 0 ? (d - a) - b : (d + a) + b;
+    }
+    if (!PER) {   // line position 0
+        if (m == 0) w.z0 = T(0);
+        else if (m == 1) w.m1 = T(0);
+        else if (m == 2) w.m2 = T(0);
+    }
+    const T f = face_of<T, PER>(m, n, u1d, w);
+    return SIGN < 0 ? d - f : d + f;
+}
+// Along x, averaged with the cells at offset oe:
+template <int N, int PER, int SIGN, bool LIN, typename T, typename E>
+__device__ __forceinline__ void vf_x(Vec<T, N> &d, const T *__restrict__ ud, T cu,
+                                     const T *__restrict__ om, uint32_t cb, const LineX<N> &L,
+                                     int i, int nx, E oe, int order) {
     T a[N + 1], b[N + 1], r[N + 8];
     load_next<N, true>(a, ud, cb, L, (int32_t)0);
     load_next<N, true>(b, ud, cb, L, oe);
@@ -316,60 +321,48 @@ __device__ __forceinline__ Vec<T, N> vf_x(const T *__restrict__ ud, T cu, const 
 #pragma unroll
     for (int c = 0; c <= N; c++) uu[c] = T(0.5) * (a[c] * cu + b[c] * cu);
     if (!PER && i == 0) uu[0] = T(0);
-    Vec<T, N> o;
 #pragma unroll
     for (int c = 0; c < N; c++) {
         Stencil6<T> w = {r[c + 1], r[c + 2], r[c + 3], r[c + 4], r[c + 5], r[c + 6]};
-        if (!PER) {   // line position 0
-            if (i + c == 0) w.z0 = T(0);
-            else if (i + c == 1) w.m1 = T(0);
-            else if (i + c == 2) w.m2 = T(0);
-        }
-        o.v[c] = face_of<T, PER>(i + c, nx, T(0.5) * (uu[c] + uu[c + 1]), w);
+        d.v[c] = vf_term<T, PER, SIGN, LIN>(d.v[c], i + c, nx, T(0.5) * (uu[c] + uu[c + 1]), w,
+                                            order);
     }
-    return o;
 }
-// along y or z (line position m of n): the velocities at the cells, at the
-// line position before (both given with their averages, uu and up)
-template <int N, int PER, typename T, typename O>
-__device__ __forceinline__ Vec<T, N> vf_line(const T (&uu)[N], const T (&up)[N],
-                                             const T *__restrict__ om, uint32_t cb,
-                                             const Line<O> &L, int m, int n) {
+// along y or z (line position m of n): uu and up, the averaged velocities at
+// the cells and at the line position before
+template <int N, int PER, int SIGN, bool LIN, typename T, typename O>
+__device__ __forceinline__ void vf_line(Vec<T, N> &d, const T (&uu)[N], const T (&up)[N],
+                                        const T *__restrict__ om, uint32_t cb, const Line<O> &L,
+                                        int m, int n, int order) {
     const Vec<T, N> m3 = ldv<N>(om, cb, L.m3), m2 = ldv<N>(om, cb, L.m2), m1 = ldv<N>(om, cb, L.m1);
     const Vec<T, N> z0 = ldv<N>(om, cb), p1 = ldv<N>(om, cb, L.p1), p2 = ldv<N>(om, cb, L.p2);
-    Vec<T, N> o;
 #pragma unroll
     for (int c = 0; c < N; c++) {
         Stencil6<T> w = {m3.v[c], m2.v[c], m1.v[c], z0.v[c], p1.v[c], p2.v[c]};
-        T uprev = up[c];
-        if (!PER) {
-            if (m == 0) { w.z0 = T(0); uprev = T(0); }
-            else if (m == 1) w.m1 = T(0);
-            else if (m == 2) w.m2 = T(0);
-        }
-        o.v[c] = face_of<T, PER>(m, n, T(0.5) * (uprev + uu[c]), w);
+        const T uprev = !PER && m == 0 ? T(0) : up[c];
+        d.v[c] = vf_term<T, PER, SIGN, LIN>(d.v[c], m, n, T(0.5) * (uprev + uu[c]), w, order);
     }
-    return o;
 }
 // averaged with the cells at offset oe (y or z)
-template <int N, int PER, typename T, typename O, typename E>
-__device__ __forceinline__ Vec<T, N> vf_yz(const T *__restrict__ ud, T cu, const T *__restrict__ om,
-                                           uint32_t cb, const Line<O> &L, int m, int n, E oe) {
+template <int N, int PER, int SIGN, bool LIN, typename T, typename O, typename E>
+__device__ __forceinline__ void vf_yz(Vec<T, N> &d, const T *__restrict__ ud, T cu,
+                                      const T *__restrict__ om, uint32_t cb, const Line<O> &L,
+                                      int m, int n, E oe, int order) {
     const Vec<T, N> a = ldv<N>(ud, cb), b = ldv<N>(ud, cb, oe);
-    const Vec<T, N> c = ldv<N>(ud, cb, L.m1), d = ldv2<N>(ud, cb, L.m1, oe);
+    const Vec<T, N> c = ldv<N>(ud, cb, L.m1), e = ldv2<N>(ud, cb, L.m1, oe);
     T uu[N], up[N];
 #pragma unroll
     for (int q = 0; q < N; q++) {
         uu[q] = T(0.5) * (a.v[q] * cu + b.v[q] * cu);
-        up[q] = T(0.5) * (c.v[q] * cu + d.v[q] * cu);
+        up[q] = T(0.5) * (c.v[q] * cu + e.v[q] * cu);
     }
-    return vf_line<N, PER, T>(uu, up, om, cb, L, m, n);
+    vf_line<N, PER, SIGN, LIN>(d, uu, up, om, cb, L, m, n, order);
 }
 // averaged with the next cells in x
-template <int N, int PER, typename T, typename O>
-__device__ __forceinline__ Vec<T, N> vf_yz_x(const T *__restrict__ ud, T cu,
-                                             const T *__restrict__ om, uint32_t cb,
-                                             const Line<O> &L, const LineX<N> &Lx, int m, int n) {
+template <int N, int PER, int SIGN, bool LIN, typename T, typename O>
+__device__ __forceinline__ void vf_yz_x(Vec<T, N> &d, const T *__restrict__ ud, T cu,
+                                        const T *__restrict__ om, uint32_t cb, const Line<O> &L,
+                                        const LineX<N> &Lx, int m, int n, int order) {
     T a[N + 1], c[N + 1], uu[N], up[N];
     load_next<N, false>(a, ud, cb, Lx, (int32_t)0);
     load_next<N, false>(c, ud, cb, Lx, L.m1);
@@ -378,7 +371,7 @@ __device__ __forceinline__ Vec<T, N> vf_yz_x(const T *__restrict__ ud, T cu,
         uu[q] = T(0.5) * (a[q] * cu + a[q + 1] * cu);
         up[q] = T(0.5) * (c[q] * cu + c[q + 1] * cu);
     }
-    return vf_line<N, PER, T>(uu, up, om, cb, L, m, n);
+    vf_line<N, PER, SIGN, LIN>(d, uu, up, om, cb, L, m, n, order);
 }
 
 // One direction of core/fortran_dissipation.f90:2-34 add_laplacian at a
@@ -422,12 +415,13 @@ __device__ __forceinline__ void viscosity_cell(const Geo &g, const StageArgs<T> 
 // The stage combination of one field at N cells (core/timescheme.py): its
 // tendency d, the current and next state, the tendency slots and the LFAM3
 // 'before' state.
-template <int N, int MODE, typename T>
+template <int N, int MODE, bool LIN, typename T>
 __device__ __forceinline__ void stage_out(const StageArgs<T> &a, uint32_t cb, const Vec<T, N> &d,
                                           const T *__restrict__ now, T *__restrict__ next,
                                           T *__restrict__ tend, const T *__restrict__ d0,
                                           const T *__restrict__ d1, T *__restrict__ before) {
-    if (MODE == 0 || MODE == 1 || MODE == 2) stv<N, true>(tend, cb, d);   // read at a later stage
+    // read at a later stage; the model variants keep them at every stage
+    if (MODE == 0 || MODE == 1 || MODE == 2 || LIN) stv<N, true>(tend, cb, d);
     if (MODE == 0) return;
     const T cc = T(a.c);
     const Vec<T, N> s = ldv<N>((MODE == 5 ? (const T *)next : now), cb);
@@ -455,8 +449,7 @@ __device__ __forceinline__ void stage_out(const StageArgs<T> &a, uint32_t cb, co
 // Fused LES.rhs (core/model_les.py:129-144) + stage update
 // (core/timescheme.py:199-220, LFAM3 :144-175 and :352-364) for N cells of a
 // row.  LIN: with the model variants and the reference's linear upwind
-// branches (tendencies-only mode).  Y, Z: the types of the offsets along
-// those axes.
+// branches.  Y, Z: the types of the offsets along those axes.
 template <typename T, int N, int MODE, int PX, int PY, int PZ, bool LIN, typename Y, typename Z>
 __device__ __forceinline__ void stage_cells(const Geo &g, const StageArgs<T> &a, int i, int j,
                                             int k) {
@@ -479,57 +472,31 @@ __device__ __forceinline__ void stage_cells(const Geo &g, const StageArgs<T> &a,
     const T cx = T(a.idx2), cy = T(a.idy2), cz = T(a.idz2);
     Vec<T, N> db = {}, du = {}, dv = {}, dw = {};
     uint32_t cs = cb;
-    const int64_t bx = cell - i, by = cell - (int64_t)j * g.sy, bz = cell - (int64_t)k * g.sz;
-    if (LIN && with_b && a.upw_a != 0) {
-        T d = T(0);
-        d = lin_tracer_axis<T, PX>(d, a.b, a.u, cx, bx, 1, i, g.nx, a.upw_a);
-        d = lin_tracer_axis<T, PY>(d, a.b, a.v, cy, by, g.sy, j, g.ny, a.upw_a);
-        db.v[0] = lin_tracer_axis<T, PZ>(d, a.b, a.w, cz, bz, g.sz, k, g.nz, a.upw_a);
-    } else if (with_b) {
-        tracer_x<N, PX>(db, a.b, a.u, cx, cs, Lx, i, g.nx);
+    const int oa = LIN ? a.upw_a : 0, ov = LIN ? a.upw_vf : 0;
+    if (with_b) {
+        tracer_x<N, PX, LIN>(db, a.b, a.u, cx, cs, Lx, i, g.nx, oa);
         if constexpr (N < 4) STAGE_SEQ(cs, db.v[0]);   // N = 4: overlapped, 3 % faster
-        tracer_yz<N, PY>(db, a.b, a.v, cy, cs, Ly, j, g.ny);
+        tracer_yz<N, PY, LIN>(db, a.b, a.v, cy, cs, Ly, j, g.ny, oa);
         if constexpr (N < 4) STAGE_SEQ(cs, db.v[0]);
-        tracer_yz<N, PZ>(db, a.b, a.w, cz, cs, Lz, k, g.nz);
+        tracer_yz<N, PZ, LIN>(db, a.b, a.w, cz, cs, Lz, k, g.nz, oa);
         STAGE_SEQ(cs, db.v[0]);
     }
 
-    // vortex force, triplets 'ikj', 'jik', 'kji' (core/vortex_force.py:69-81)
-    auto add = [](Vec<T, N> &d, const Vec<T, N> &f) {
-#pragma unroll
-        for (int q = 0; q < N; q++) d.v[q] = d.v[q] + f.v[q];
-    };
-    auto sub = [](Vec<T, N> &d, const Vec<T, N> &f) {
-#pragma unroll
-        for (int q = 0; q < N; q++) d.v[q] = d.v[q] - f.v[q];
-    };
-    if (LIN && vf && a.upw_vf != 0) {
-        // the six terms in the order below, with the linear branch
-        const int o = a.upw_vf;
-        const bool ex = PX || i < g.nx - 1;
-        const int64_t ocx = (int64_t)Lx.after() / ES;
-        const int64_t ocy = (int64_t)Ly.p1 / ES, ocz = (int64_t)Lz.p1 / ES;
-        T *const u = &du.v[0], *const v = &dv.v[0], *const w = &dw.v[0];
-        if (ey) *v = vf_lin<T, PX, -1>(*v, a.u, cx, a.oz, bx, 1, i, g.nx, ocy, o);
-        if (ex) *u = vf_lin<T, PY, +1>(*u, a.v, cy, a.oz, by, g.sy, j, g.ny, ocx, o);
-        if (ez) *w = vf_lin<T, PY, -1>(*w, a.v, cy, a.ox, by, g.sy, j, g.ny, ocz, o);
-        if (ey) *v = vf_lin<T, PZ, +1>(*v, a.w, cz, a.ox, bz, g.sz, k, g.nz, ocy, o);
-        if (ex) *u = vf_lin<T, PZ, -1>(*u, a.w, cz, a.oy, bz, g.sz, k, g.nz, ocx, o);
-        if (ez) *w = vf_lin<T, PX, +1>(*w, a.u, cx, a.oy, bx, 1, i, g.nx, ocz, o);
-    } else if (vf) {
-        // direc(U_i, vor_k, du_j), flip(U_j, vor_k, du_i), direc(U_j, vor_i, du_k),
-        // flip(U_k, vor_i, du_j), direc(U_k, vor_j, du_i), flip(U_i, vor_j, du_k)
-        if (ey) sub(dv, vf_x<N, PX>(a.u, cx, a.oz, cs, Lx, i, g.nx, Ly.p1));
+    // vortex force, triplets 'ikj', 'jik', 'kji' (core/vortex_force.py:69-81):
+    // direc(U_i, vor_k, du_j), flip(U_j, vor_k, du_i), direc(U_j, vor_i, du_k),
+    // flip(U_k, vor_i, du_j), direc(U_k, vor_j, du_i), flip(U_i, vor_j, du_k)
+    if (vf) {
+        if (ey) vf_x<N, PX, -1, LIN>(dv, a.u, cx, a.oz, cs, Lx, i, g.nx, Ly.p1, ov);
         STAGE_SEQ(cs, dv.v[0]);
-        add(du, vf_yz_x<N, PY>(a.v, cy, a.oz, cs, Ly, Lx, j, g.ny));
+        vf_yz_x<N, PY, +1, LIN>(du, a.v, cy, a.oz, cs, Ly, Lx, j, g.ny, ov);
         STAGE_SEQ(cs, du.v[0]);
-        if (ez) sub(dw, vf_yz<N, PY>(a.v, cy, a.ox, cs, Ly, j, g.ny, Lz.p1));
+        if (ez) vf_yz<N, PY, -1, LIN>(dw, a.v, cy, a.ox, cs, Ly, j, g.ny, Lz.p1, ov);
         STAGE_SEQ(cs, dw.v[0]);
-        if (ey) add(dv, vf_yz<N, PZ>(a.w, cz, a.ox, cs, Lz, k, g.nz, Ly.p1));
+        if (ey) vf_yz<N, PZ, +1, LIN>(dv, a.w, cz, a.ox, cs, Lz, k, g.nz, Ly.p1, ov);
         STAGE_SEQ(cs, dv.v[0]);
-        sub(du, vf_yz_x<N, PZ>(a.w, cz, a.oy, cs, Lz, Lx, k, g.nz));
+        vf_yz_x<N, PZ, -1, LIN>(du, a.w, cz, a.oy, cs, Lz, Lx, k, g.nz, ov);
         STAGE_SEQ(cs, du.v[0]);
-        if (ez) add(dw, vf_x<N, PX>(a.u, cx, a.oy, cs, Lx, i, g.nx, Lz.p1));
+        if (ez) vf_x<N, PX, +1, LIN>(dw, a.u, cx, a.oy, cs, Lx, i, g.nx, Lz.p1, ov);
     }
 
     // bernoulli (core/bernoulli.py:14-23, core/fortran_bernoulli.f90:2-58)
@@ -564,10 +531,10 @@ __device__ __forceinline__ void stage_cells(const Geo &g, const StageArgs<T> &a,
             viscosity_cell<T, PX, PY, PZ>(g, a, cb + (uint32_t)(q * ES), i + q, j, k, du.v[q],
                                           dv.v[q], dw.v[q]);
     }
-    stage_out<N, MODE>(a, cb, db, a.b, a.bn, a.tb, a.d0b, a.d1b, a.sbb);
-    stage_out<N, MODE>(a, cb, du, a.u, a.un, a.tu, a.d0u, a.d1u, a.sbu);
-    stage_out<N, MODE>(a, cb, dv, a.v, a.vn, a.tv, a.d0v, a.d1v, a.sbv);
-    stage_out<N, MODE>(a, cb, dw, a.w, a.wn, a.tw, a.d0w, a.d1w, a.sbw);
+    stage_out<N, MODE, LIN>(a, cb, db, a.b, a.bn, a.tb, a.d0b, a.d1b, a.sbb);
+    stage_out<N, MODE, LIN>(a, cb, du, a.u, a.un, a.tu, a.d0u, a.d1u, a.sbu);
+    stage_out<N, MODE, LIN>(a, cb, dv, a.v, a.vn, a.tv, a.d0v, a.d1v, a.sbv);
+    stage_out<N, MODE, LIN>(a, cb, dw, a.w, a.wn, a.tw, a.d0w, a.d1w, a.sbw);
 }
 
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -576,8 +543,7 @@ __device__ __forceinline__ void stage_cells(const Geo &g, const StageArgs<T> &a,
 #define WAVE_UNIFORM(x) (x)
 #endif
 
-// One cell per thread, 64 x 4 x 1 blocks: the tendencies with the model
-// variants and the linear branches, and the LFAM3 start.
+// One cell per thread, 64 x 4 x 1 blocks: the first LFAM3 step.
 template <typename T, int MODE, int PX, int PY, int PZ>
 __global__ __launch_bounds__(256) void k_stage(Geo g, StageArgs<T> a) {
     const Blk3 bk = xcd_block_yslab();
@@ -585,7 +551,7 @@ __global__ __launch_bounds__(256) void k_stage(Geo g, StageArgs<T> a) {
     const int j = WAVE_UNIFORM((int)(bk.y * NYL_BY + threadIdx.y));
     const int k = bk.z;
     if (i >= g.nx || j >= g.ny) return;
-    stage_cells<T, 1, MODE, PX, PY, PZ, MODE == 0, int64_t, int64_t>(g, a, i, j, k);
+    stage_cells<T, 1, MODE, PX, PY, PZ, false, int64_t, int64_t>(g, a, i, j, k);
 }
 
 // N cells per thread, the N-groups of a plane numbered along its rows: no lane
@@ -601,7 +567,7 @@ __global__ __launch_bounds__(256) void k_stage(Geo g, StageArgs<T> a) {
 // periodic 1161 -> 970, 160x96x128 162 -> 112, 96^3 87 -> 57; FP32 256^3
 // 510 -> 440, walls 256x128x64 106 -> 58, 200x120x56 72 -> 42.
 #define STAGE_NT 256
-template <typename T, int N, int MODE, int PX, int PY, int PZ>
+template <typename T, int N, int MODE, int PX, int PY, int PZ, bool LIN = false>
 __global__ __launch_bounds__(STAGE_NT) void k_stage_flat(Geo g, StageArgs<T> a, int lw) {
     const Blk3 bk = xcd_block_yslab();
     const int nxg = g.nx / N;
@@ -616,10 +582,10 @@ __global__ __launch_bounds__(STAGE_NT) void k_stage_flat(Geo g, StageArgs<T> a, 
         if (i >= nxg) return;
     }
     if (j >= g.ny) return;
-    stage_cells<T, N, MODE, PX, PY, PZ, false, int32_t, int64_t>(g, a, i * N, j, bk.z);
+    stage_cells<T, N, MODE, PX, PY, PZ, LIN, int32_t, int64_t>(g, a, i * N, j, bk.z);
 }
 
-template <typename T, int N, int MODE, int PX, int PY, int PZ>
+template <typename T, int N, int MODE, int PX, int PY, int PZ, bool LIN>
 static void stage_flat_go(const Geo &g, const StageArgs<T> &a, hipStream_t s) {
     const int nxg = g.nx / N;
     // FP64 in whole tiles of 8 pairs (one line of L2) x 32 rows: the rows that
@@ -629,7 +595,7 @@ static void stage_flat_go(const Geo &g, const StageArgs<T> &a, hipStream_t s) {
     const int rows = STAGE_NT >> lw;
     const dim3 grd = lw ? dim3(nxg >> lw, g.ny / rows, g.nz)
                         : dim3(1, (unsigned)(((int64_t)nxg * g.ny + STAGE_NT - 1) / STAGE_NT), g.nz);
-    NYL_LAUNCH((k_stage_flat<T, N, MODE, PX, PY, PZ>), grd, STAGE_NT, 0, s, g, a, lw);
+    NYL_LAUNCH((k_stage_flat<T, N, MODE, PX, PY, PZ, LIN>), grd, STAGE_NT, 0, s, g, a, lw);
 }
 
 // Cells per thread.  16 bytes where the row divides into such groups (an FP64
@@ -644,45 +610,54 @@ static inline bool stage_wide(const Geo &g) {
     return g.nx % N == 0 && (int64_t)g.nx * g.ny * g.nz >= (sizeof(T) == 8 ? 1 << 18 : 3 << 19);
 }
 
-template <typename T, int MODE, int PX, int PY, int PZ>
+template <typename T, int MODE, int PX, int PY, int PZ, bool LIN = false>
 static void stage_go(const Geo &g, const StageArgs<T> &a, hipStream_t s) {
-    if (stage_wide<T>(g)) stage_flat_go<T, 16 / (int)sizeof(T), MODE, PX, PY, PZ>(g, a, s);
-    else stage_flat_go<T, 1, MODE, PX, PY, PZ>(g, a, s);
+    if (stage_wide<T>(g)) stage_flat_go<T, 16 / (int)sizeof(T), MODE, PX, PY, PZ, LIN>(g, a, s);
+    else stage_flat_go<T, 1, MODE, PX, PY, PZ, LIN>(g, a, s);
 }
 
 template <typename T, int PX, int PY, int PZ>
-static void launch_stage_p(const Geo &g, const StageArgs<T> &a, int mode, hipStream_t s) {
-    const dim3 blk(NYL_BX, NYL_BY, 1);
+static hipError_t stage_les(const Geo &g, const StageArgs<T> &a, int mode, hipStream_t s) {
     switch (mode) {
-    case 0:
-        if (a.flags || a.upw_a || a.upw_vf) NYL_LAUNCH((k_stage<T, 0, PX, PY, PZ>), cell_grid(g), blk, 0, s, g, a);
-        else stage_go<T, 0, PX, PY, PZ>(g, a, s);
-        break;
+    case 0: stage_go<T, 0, PX, PY, PZ>(g, a, s); break;
     case 1: stage_go<T, 1, PX, PY, PZ>(g, a, s); break;
     case 2: stage_go<T, 2, PX, PY, PZ>(g, a, s); break;
     case 3: stage_go<T, 3, PX, PY, PZ>(g, a, s); break;
     case 4: stage_go<T, 4, PX, PY, PZ>(g, a, s); break;
     case 5: stage_go<T, 5, PX, PY, PZ>(g, a, s); break;
-    // the first step of a run only
-    case 6: NYL_LAUNCH((k_stage<T, 6, PX, PY, PZ>), cell_grid(g), blk, 0, s, g, a); break;
-    default: break;
-    }
-}
-
-template <typename T>
-hipError_t launch_stage(const Geo &g, const StageArgs<T> &a, int mode, hipStream_t s) {
-    if (mode < 0 || mode > 6) return hipErrorInvalidValue;
-    switch (g.px + 2 * g.py + 4 * g.pz) {
-    case 0: launch_stage_p<T, 0, 0, 0>(g, a, mode, s); break;
-    case 1: launch_stage_p<T, 1, 0, 0>(g, a, mode, s); break;
-    case 2: launch_stage_p<T, 0, 1, 0>(g, a, mode, s); break;
-    case 3: launch_stage_p<T, 1, 1, 0>(g, a, mode, s); break;
-    case 4: launch_stage_p<T, 0, 0, 1>(g, a, mode, s); break;
-    case 5: launch_stage_p<T, 1, 0, 1>(g, a, mode, s); break;
-    case 6: launch_stage_p<T, 0, 1, 1>(g, a, mode, s); break;
-    default: launch_stage_p<T, 1, 1, 1>(g, a, mode, s); break;
+    case 6:   // the first step of a run only
+        NYL_LAUNCH((k_stage<T, 6, PX, PY, PZ>), cell_grid(g), dim3(NYL_BX, NYL_BY, 1), 0, s, g, a);
+        break;
+    default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
+
+// the model variants and the linear branches: the tendencies, or an RK3 stage
+// with its tendencies stored too
+template <typename T, int PX, int PY, int PZ>
+static hipError_t stage_lin(const Geo &g, const StageArgs<T> &a, int mode, hipStream_t s) {
+    switch (mode) {
+    case 0: stage_go<T, 0, PX, PY, PZ, true>(g, a, s); break;
+    case 1: stage_go<T, 1, PX, PY, PZ, true>(g, a, s); break;
+    case 2: stage_go<T, 2, PX, PY, PZ, true>(g, a, s); break;
+    case 3: stage_go<T, 3, PX, PY, PZ, true>(g, a, s); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+// fn<T, PX, PY, PZ>(g, a, mode, s) for the geometry's periodic axes
+#define NYL_STAGE_GEO(fn, T)                              \
+    switch (g.px + 2 * g.py + 4 * g.pz) {                 \
+    case 0: return fn<T, 0, 0, 0>(g, a, mode, s);         \
+    case 1: return fn<T, 1, 0, 0>(g, a, mode, s);         \
+    case 2: return fn<T, 0, 1, 0>(g, a, mode, s);         \
+    case 3: return fn<T, 1, 1, 0>(g, a, mode, s);         \
+    case 4: return fn<T, 0, 0, 1>(g, a, mode, s);         \
+    case 5: return fn<T, 1, 0, 1>(g, a, mode, s);         \
+    case 6: return fn<T, 0, 1, 1>(g, a, mode, s);         \
+    default: return fn<T, 1, 1, 1>(g, a, mode, s);        \
+    }
 
 }  // namespace nyl

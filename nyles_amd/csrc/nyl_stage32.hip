@@ -4,6 +4,10 @@
 
 namespace nyl {
 
-template hipError_t launch_stage<float>(const Geo &, const StageArgs<float> &, int, hipStream_t);
+template <>
+hipError_t launch_stage<float>(const Geo &g, const StageArgs<float> &a, int mode, hipStream_t s) {
+    if (a.flags || a.upw_a || a.upw_vf) return launch_stage_lin<float>(g, a, mode, s);
+    NYL_STAGE_GEO(stage_les, float)
+}
 
 }  // namespace nyl

@@ -4,6 +4,10 @@
 
 namespace nyl {
 
-template hipError_t launch_stage<double>(const Geo &, const StageArgs<double> &, int, hipStream_t);
+template <>
+hipError_t launch_stage<double>(const Geo &g, const StageArgs<double> &a, int mode, hipStream_t s) {
+    if (a.flags || a.upw_a || a.upw_vf) return launch_stage_lin<double>(g, a, mode, s);
+    NYL_STAGE_GEO(stage_les, double)
+}
 
 }  // namespace nyl

@@ -413,23 +413,16 @@ __device__ __forceinline__ void tracer_cell(const Geo &g, const TracerArgs<T> &a
     constexpr int ES = (int)sizeof(T);
     const uint32_t cb = (uint32_t)c * (uint32_t)ES;
     const T cx = T(a.idx2), cy = T(a.idy2), cz = T(a.idz2);
-    T dq = T(0);
-    const int64_t bx = c - i, by = c - (int64_t)j * g.sy, bz = c - (int64_t)k * g.sz;
-    if (MODE == 0 && a.upw != 0) {   // the linear upwind branch (tendencies-only mode)
-        dq = lin_tracer_axis<T, PX>(dq, a.q, a.u, cx, bx, 1, i, g.nx, a.upw);
-        dq = lin_tracer_axis<T, PY>(dq, a.q, a.v, cy, by, g.sy, j, g.ny, a.upw);
-        dq = lin_tracer_axis<T, PZ>(dq, a.q, a.w, cz, bz, g.sz, k, g.nz, a.upw);
-    } else {
-        const LineX<1> Lx = linex_of<1, PX>(i, g.nx, ES);
-        const Line<int32_t> Ly = line_of<PY, int32_t>(j, g.ny, (int32_t)(g.sy * ES));
-        const Line<int32_t> Lz = line_of<PZ, int32_t>(k, g.nz, (int32_t)(g.sz * ES));
-        Vec<T, 1> d = {};
-        tracer_x<1, PX>(d, a.q, a.u, cx, cb, Lx, i, g.nx);
-        tracer_yz<1, PY>(d, a.q, a.v, cy, cb, Ly, j, g.ny);
-        tracer_yz<1, PZ>(d, a.q, a.w, cz, cb, Lz, k, g.nz);
-        dq = d.v[0];
-    }
-
+    constexpr bool LIN = MODE == 0;   // the linear upwind branch too
+    const int oa = LIN ? a.upw : 0;
+    const LineX<1> Lx = linex_of<1, PX>(i, g.nx, ES);
+    const Line<int32_t> Ly = line_of<PY, int32_t>(j, g.ny, (int32_t)(g.sy * ES));
+    const Line<int32_t> Lz = line_of<PZ, int32_t>(k, g.nz, (int32_t)(g.sz * ES));
+    Vec<T, 1> d = {};
+    tracer_x<1, PX, LIN>(d, a.q, a.u, cx, cb, Lx, i, g.nx, oa);
+    tracer_yz<1, PY, LIN>(d, a.q, a.v, cy, cb, Ly, j, g.ny, oa);
+    tracer_yz<1, PZ, LIN>(d, a.q, a.w, cz, cb, Lz, k, g.nz, oa);
+    const T dq = d.v[0];
     if (MODE == 0 || MODE == 1 || MODE == 2) stb(a.tout, cb, dq);
     const T cc = T(a.c);
     if (MODE == 1) {
@@ -1028,7 +1021,7 @@ __global__ __launch_bounds__(TPB) void k_b_stage(const StageItem<T> *__restrict_
         StageArgs<T> a = it.a;
         const double d = dt[it.h.member];
         a.c = MODE == 1 ? d : (MODE == 2 ? d / 4. : d / 12.);
-        stage_cells<T, 1, MODE, PX, PY, PZ, MODE == 0, int32_t, int32_t>(it.h.g, a, i, j, k);
+        stage_cells<T, 1, MODE, PX, PY, PZ, false, int32_t, int32_t>(it.h.g, a, i, j, k);
     }
 }
 

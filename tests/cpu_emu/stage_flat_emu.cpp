@@ -1,7 +1,8 @@
 // Stage kernel with one or 16 bytes of cells per thread (k_stage_flat)
 // against the per-cell kernel (k_stage), bit for bit: every mode and
 // periodicity, rows of one group to several tiles, planes that leave a block
-// partly filled, the smallest wall axes (8 cells).  And the FP64 WENO5 with
+// partly filled, the smallest wall axes (8 cells); with the model variants
+// and the linear branches, 16 bytes of cells against one.  And the FP64 WENO5 with
 // its short division against the reference's expression, over magnitudes
 // that leave the short division's range (zeros, subnormals, overflow, inf,
 // NaN).
@@ -77,6 +78,23 @@ int check_mode(const Geo &g, StageArgs<T> a1, StageArgs<T> a2, std::vector<std::
     return b;
 }
 
+// the linear branches and the model variants: N cells per thread against one
+template <typename T, int N, int MODE, int PX, int PY, int PZ>
+int check_lin(const Geo &g, StageArgs<T> a1, StageArgs<T> a2, std::vector<std::vector<T>> &o1,
+              std::vector<std::vector<T>> &o2, int k) {
+    const int orders[][3] = {{1, 1, 0}, {3, 5, 0}, {5, 3, 0}, {5, 0, NYL_SF_NO_B}, {0, 0, NYL_SF_NO_VF}};
+    const int *o = orders[k];
+    for (StageArgs<T> *a : {&a1, &a2}) { a->upw_a = o[0]; a->upw_vf = o[1]; a->flags = o[2]; }
+    auto grd = [&](int n) { return dim3(1, (g.nx / n * g.ny + STAGE_NT - 1) / STAGE_NT, g.nz); };
+    run_blocks(grd(1), dim3(STAGE_NT, 1, 1),
+               [&]() { k_stage_flat<T, 1, MODE, PX, PY, PZ, true>(g, a1, 0); }, false);
+    run_blocks(grd(N), dim3(STAGE_NT, 1, 1),
+               [&]() { k_stage_flat<T, N, MODE, PX, PY, PZ, true>(g, a2, 0); }, false);
+    int b = 0;
+    for (int f = 0; f < 12; f++) b += ndiff(o1[f], o2[f]);
+    return b;
+}
+
 template <typename T, int N, int PX, int PY, int PZ>
 int check(int nx, int ny, int nz, int lw, int visc) {
     const Geo g = mk(nx, ny, nz, PX, PY, PZ);
@@ -87,7 +105,8 @@ int check(int nx, int ny, int nz, int lw, int visc) {
     for (int f = 1; f <= 3; f++)   // exact zeros: the u > 0 / u <= 0 split
         for (size_t q = 0; q < n; q += 7) in[f][q] = T(0);
     int bad = 0;
-    for (int mode = 0; mode <= 5; mode++) {
+    for (int run = 0; run <= 5 + (N > 1 && PX == PY ? 10 : 0); run++) {
+        const int mode = run <= 5 ? run : (run <= 10 ? 1 : 3);
         std::vector<std::vector<T>> o1(12), o2;
         for (int f = 0; f < 12; f++) o1[f] = f < 4 ? in[11 + f] : (f < 8 ? std::vector<T>(n, T(5)) : in[15 + f - 8]);
         o2 = o1;
@@ -108,7 +127,11 @@ int check(int nx, int ny, int nz, int lw, int visc) {
         };
         const StageArgs<T> a1 = args(o1), a2 = args(o2);
         int b = 0;
-        switch (mode) {
+        if (run > 5) {
+            if constexpr (N > 1 && PX == PY)
+                b = run > 10 ? check_lin<T, N, 3, PX, PY, PZ>(g, a1, a2, o1, o2, run - 11)
+                             : check_lin<T, N, 1, PX, PY, PZ>(g, a1, a2, o1, o2, run - 6);
+        } else switch (mode) {
         case 0: b = check_mode<T, N, 0, PX, PY, PZ>(g, a1, a2, o1, o2, lw); break;
         case 1: b = check_mode<T, N, 1, PX, PY, PZ>(g, a1, a2, o1, o2, lw); break;
         case 2: b = check_mode<T, N, 2, PX, PY, PZ>(g, a1, a2, o1, o2, lw); break;
@@ -116,7 +139,7 @@ int check(int nx, int ny, int nz, int lw, int visc) {
         case 4: b = check_mode<T, N, 4, PX, PY, PZ>(g, a1, a2, o1, o2, lw); break;
         default: b = check_mode<T, N, 5, PX, PY, PZ>(g, a1, a2, o1, o2, lw); break;
         }
-        if (b) printf("  mode %d: %d mismatches\n", mode, b);
+        if (b) printf("  run %d mode %d: %d mismatches\n", run, mode, b);
         bad += b;
     }
     printf("stage_flat<%s, %d> %dx%dx%d p=%d%d%d lw=%d visc=%d: %d mismatches\n",
