@@ -34,7 +34,7 @@ __device__ __forceinline__ int wrap_any(int m, int n) {
 // restrict_cell, prolong_term) in its order, so the results are bitwise those
 // of the separate launches.
 template <typename T, typename TC, int TX, int SRC, int NSW, bool RESN, bool RESTR, bool OUTER,
-          bool XADD = false>
+          bool XADD = false, bool LONG = false>
 __device__ __forceinline__ void march_body(const MarchArgs<T, TC> &a, const MGTabs &tab,
                                            const Blk3 &bk, int nb) {
     constexpr int TY = 512 / TX;
@@ -182,11 +182,11 @@ __device__ __forceinline__ void march_body(const MarchArgs<T, TC> &a, const MGTa
     };
     // stage-0 values of plane m from the raw loads; PROLONG: lo, hi the planar
     // sums of the coarse planes around it (lo the lower one), par the parity of m
-    auto enter = [&](auto par, int m, const T (&v)[NP], const T (&lo)[NP], const T (&hi)[NP],
-                     T (&out)[NP]) {
-        constexpr bool odd = decltype(par)::value != 0;
-        const bool zi = zin(m);
-        const bool mz = SRC == MS_PROLONG && czin(odd ? (m >> 1) + 1 : (m >> 1) - 1);
+    auto enter = [&](auto par, auto inner, int m, const T (&v)[NP], const T (&lo)[NP],
+                     const T (&hi)[NP], T (&out)[NP]) {
+        constexpr bool odd = decltype(par)::value != 0, FAST = decltype(inner)::value;
+        const bool zi = FAST || zin(m);
+        const bool mz = FAST || (SRC == MS_PROLONG && czin(odd ? (m >> 1) + 1 : (m >> 1) - 1));
 #pragma unroll
         for (int p = 0; p < NP; p++) {
             T t = v[p];
@@ -201,6 +201,8 @@ __device__ __forceinline__ void march_body(const MarchArgs<T, TC> &a, const MGTa
     };
     using Even = std::integral_constant<int, 0>;
     using Odd = std::integral_constant<int, 1>;
+    using Edge = std::false_type;
+    using Inner = std::true_type;
 
     const int p0 = k0 - (R - 1), p1 = k1 - 1 + (R - 1);
     // windows: stage 0 planes p-1, p, p+1; stage 1 planes p-2, p-1, p; stage 2
@@ -235,15 +237,15 @@ __device__ __forceinline__ void march_body(const MarchArgs<T, TC> &a, const MGTa
             planar(0, Am);
             planar(1, A0);
             planar(2, A1);
-            enter(Even(), p0 - 1, x0, Am, A0, I0);
-            enter(Odd(), p0, x1, A0, A1, I1);
-            enter(Even(), p0 + 1, x2, A0, A1, I2);
+            enter(Even(), Edge(), p0 - 1, x0, Am, A0, I0);
+            enter(Odd(), Edge(), p0, x1, A0, A1, I1);
+            enter(Even(), Edge(), p0 + 1, x2, A0, A1, I2);
             ldc(kc + 2);
             __syncthreads();   // slot 0 is written again in the first step
         } else if (SRC == MS_FIELD) {
-            enter(Even(), p0 - 1, x0, A0, A1, I0);
-            enter(Even(), p0, x1, A0, A1, I1);
-            enter(Even(), p0 + 1, x2, A0, A1, I2);
+            enter(Even(), Edge(), p0 - 1, x0, A0, A1, I0);
+            enter(Even(), Edge(), p0, x1, A0, A1, I1);
+            enter(Even(), Edge(), p0 + 1, x2, A0, A1, I2);
         }
     }
     int qx = pl(p0 + 3, nz, pz), qb = pl(p0 + 2, nz, pz);
@@ -263,8 +265,13 @@ __device__ __forceinline__ void march_body(const MarchArgs<T, TC> &a, const MGTa
     // One step; ph alternates 0, 1 from the first one.  The march of a
     // restriction or prolongation starts on an even plane k0, so there ph = 0
     // is an odd p of a prolongation (p0 = k0 - 1) and an even residual plane.
-    auto step = [&](auto ph, int p, T (&xu)[NP], T (&xn)[NP], T (&bu)[NB], T (&bn)[NB]) {
+    // inner: a step whose planes all have both z neighbours and are all the
+    // block's own, so that nothing depends on z (the march is latency-bound:
+    // two waves per SIMD, and a branch per position and stage costs as much as
+    // its arithmetic).
+    auto step = [&](auto ph, auto inner, int p, T (&xu)[NP], T (&xn)[NP], T (&bu)[NB], T (&bn)[NB]) {
         constexpr int A = decltype(ph)::value, B = 1 - A;   // slots of planes p, p - 1
+        constexpr bool FAST = decltype(inner)::value;
         constexpr bool pair = SRC == MS_PROLONG && A == 0;  // a new coarse plane this step
         if (SRC != MS_ZERO) {
             T *P = s0 + A * (W0 * H0);
@@ -276,13 +283,16 @@ __device__ __forceinline__ void march_body(const MarchArgs<T, TC> &a, const MGTa
             putc((p + 3) >> 1, 0);
             if (p + 2 <= p1 + 1) ldc(((p + 3) >> 1) + 1);
         }
-        if (p + 3 <= p1 + 1) ldx(qx, xn);
-        if (p + 2 <= p1) ldb(qb, bn);
+        // (always issued, past the end from the last plane again: behind a
+        // condition the compiler waits for the loads of this step where it
+        // needs those of the one before)
+        ldx(qx, xn);
+        ldb(qb, bn);
         __syncthreads();
         // residual of the input, and stage 1 of plane p
         const T *P0 = s0 + A * (W0 * H0);
-        const bool z0 = zin(p);
-        const int n0 = nzw(p);
+        const bool z0 = FAST || zin(p);
+        const int n0 = FAST ? 2 : nzw(p);
         T *P1 = s1 + A * (W1 * H1);
 #pragma unroll
         for (int q = 0; q < (NSW > 0 ? N1 : 2); q++) {
@@ -292,7 +302,7 @@ __device__ __forceinline__ void march_body(const MarchArgs<T, TC> &a, const MGTa
                 const T own[2] = {I1[0], I1[1]};
                 S = six(P0, 0, q, own, I0[q], I2[q]);
             }
-            if (RESN && q < 2 && p >= k0 && p < k1 && st[q]) {
+            if (RESN && q < 2 && (FAST || (p >= k0 && p < k1)) && st[q]) {
                 const T d = T(nxy[q] + n0);
                 if constexpr (OUTER) {
                     const double rr = (B0[q] - shift) + d * I1[q] - S;
@@ -305,21 +315,21 @@ __device__ __forceinline__ void march_body(const MarchArgs<T, TC> &a, const MGTa
             }
             if constexpr (NSW > 0) {
                 T id = id2[q];
-                if (n0 != 2) id = sid[nxy[q] + n0];
+                if (!FAST && n0 != 2) id = sid[nxy[q] + n0];
                 const T v = cff1 * I1[q] + om * (S - B0[q]) * id;
                 M2[q] = (z0 && in[q]) ? v : T(0);
                 if (LDS1) P1[place(q, 1)] = M2[q];
-                if (NSW == 1 && q < 2 && p >= k0 && p < k1 && st[q])
+                if (NSW == 1 && q < 2 && (FAST || (p >= k0 && p < k1)) && st[q])
                     a.dst[(int64_t)p * g.sz + off[q]] = M2[q];
             }
         }
         // stage 2 of plane p - 1
         const int m = p - 1;
         const T *Q1 = s1 + B * (W1 * H1);
-        const int n1 = nzw(m);
-        const bool z1 = zin(m);
+        const int n1 = FAST ? 2 : nzw(m);
+        const bool z1 = FAST || zin(m);
         if constexpr (NSW == 2) {
-            if (m >= p0 && m >= k0 - (R - 2)) {
+            if (FAST || (m >= p0 && m >= k0 - (R - 2))) {
                 T *P2 = s2 + B * (W2 * H2);
 #pragma unroll
                 for (int q = 0; q < N2; q++) {
@@ -327,13 +337,13 @@ __device__ __forceinline__ void march_body(const MarchArgs<T, TC> &a, const MGTa
                     const T own[2] = {M1[0], M1[1]};
                     const T S = six(Q1, 1, q, own, M0[q], M2[q]);
                     T id = id2[q];
-                    if (n1 != 2) id = sid[nxy[q] + n1];
+                    if (!FAST && n1 != 2) id = sid[nxy[q] + n1];
                     const T v = cff1 * M1[q] + om * (S - B1[q]) * id;
                     if (RESTR) {
                         K2[q] = (z1 && in[q]) ? v : T(0);
                         P2[place(q, 2)] = K2[q];
                     }
-                    if (q < 2 && m >= k0 && m < k1 && st[q]) {
+                    if (q < 2 && (FAST || (m >= k0 && m < k1)) && st[q]) {
                         const int64_t c = (int64_t)m * g.sz + off[q];
                         if (XADD) a.xadd[c] = a.xadd[c] + (double)v;
                         else a.dst[c] = v;
@@ -344,9 +354,9 @@ __device__ __forceinline__ void march_body(const MarchArgs<T, TC> &a, const MGTa
         // residual of the last stage and its restriction
         if constexpr (RESTR) {
             const int k = p - NSW;
-            if (k >= k0 && k < k1) {
+            if (FAST || (k >= k0 && k < k1)) {
                 const T *Q = NSW == 2 ? s2 + A * (W2 * H2) : (NSW == 1 ? Q1 : P0);
-                const int nk = nzw(k);
+                const int nk = FAST ? 2 : nzw(k);
                 T r[2];
 #pragma unroll
                 for (int q = 0; q < 2; q++) {
@@ -387,7 +397,7 @@ __device__ __forceinline__ void march_body(const MarchArgs<T, TC> &a, const MGTa
         T In[NP];
         // (p + 2 is odd in the steps that bring a coarse plane)
         if (SRC != MS_ZERO)
-            enter(std::integral_constant<int, B>(), p + 2, xu, A0, A1, In);
+            enter(std::integral_constant<int, B>(), inner, p + 2, xu, A0, A1, In);
 #pragma unroll
         for (int q = 0; q < NP; q++) {
             I0[q] = I1[q];
@@ -412,12 +422,22 @@ __device__ __forceinline__ void march_body(const MarchArgs<T, TC> &a, const MGTa
             B1[q] = B0[q];
             B0[q] = bu[q];
         }
-        qx = next(qx, p + 3, nz, pz);
-        qb = next(qb, p + 2, nz, pz);
+        if (p + 3 <= p1) qx = next(qx, p + 3, nz, pz);
+        if (p + 2 < p1) qb = next(qb, p + 2, nz, pz);
+    };
+    auto inside = [&](int p) {
+        return p - 2 >= k0 && p < k1 && (pz || (p > 2 && p + 3 < nz));
     };
     for (int p = p0; p <= p1; p += 2) {
-        step(Even(), p, xa, xb, ba, bb);
-        if (p + 1 <= p1) step(Odd(), p + 1, xb, xa, bb, ba);
+        if constexpr (LONG) {
+            if (inside(p) && inside(p + 1)) {
+                step(Even(), Inner(), p, xa, xb, ba, bb);
+                step(Odd(), Inner(), p + 1, xb, xa, bb, ba);
+                continue;
+            }
+        }
+        step(Even(), Edge(), p, xa, xb, ba, bb);
+        if (p + 1 <= p1) step(Odd(), Edge(), p + 1, xb, xa, bb, ba);
     }
     if (RESN) {
         __syncthreads();
@@ -425,10 +445,24 @@ __device__ __forceinline__ void march_body(const MarchArgs<T, TC> &a, const MGTa
     }
 }
 
-template <typename T, typename TC, int TX, int SRC, int NSW, bool RESN, bool RESTR, bool OUTER>
-__global__ __launch_bounds__(256) void k_mg_march(MarchArgs<T, TC> a, MGTabs tab) {
+// LONG: with the steps inside the march as a path of its own, and the
+// registers held to the residency that march_grid counts on.  For marches of
+// 16 planes or more with sweeps: pre-smoothing with restriction + post-
+// smoothing FP64 256^3 252 -> 238 us, FP32 256^3 136 -> 126, 256x256x512
+// 279 -> 271; in short marches the second copy of the code costs more than
+// its few steps gain (96^3: 35.5 -> 36.6).
+template <typename T, int SRC, int NSW, bool RESTR, bool LONG>
+constexpr int march_waves() {
+    return LONG ? march_resident(sizeof(T), SRC, NSW, RESTR) : 1;
+}
+constexpr int MARCH_LONG = 16;
+
+template <typename T, typename TC, int TX, int SRC, int NSW, bool RESN, bool RESTR, bool OUTER,
+          bool LONG = false>
+__global__ __launch_bounds__(256, (march_waves<T, SRC, NSW, RESTR, LONG>())) void k_mg_march(
+    MarchArgs<T, TC> a, MGTabs tab) {
     if (a.gate && *a.gate) return;
-    march_body<T, TC, TX, SRC, NSW, RESN, RESTR, OUTER>(
+    march_body<T, TC, TX, SRC, NSW, RESN, RESTR, OUTER, false, LONG>(
         a, tab, xcd_block(), blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
 }
 
@@ -483,9 +517,16 @@ MarchGrid march_grid(const Geo &g, int res, bool even) {
                                         (RESTR) || (SRC) == MS_PROLONG);                      \
         m.kz = gr.kz;                                                                         \
         const dim3 grd(gr.bx, gr.by, gr.bz), blk(256);                                        \
-        if (gr.tx == 64)                                                                      \
+        const bool lng = (NSW) > 0 && gr.kz >= MARCH_LONG;                                    \
+        if (gr.tx == 64 && lng)                                                               \
+            NYL_LAUNCH((k_mg_march<T, TC, 64, SRC, NSW, RESN, RESTR, OUTER, (NSW) != 0>), grd, blk, 0, \
+                       s, m, a.tab);                                                          \
+        else if (gr.tx == 64)                                                                 \
             NYL_LAUNCH((k_mg_march<T, TC, 64, SRC, NSW, RESN, RESTR, OUTER>), grd, blk, 0, s, m, \
                        a.tab);                                                                \
+        else if (lng)                                                                         \
+            NYL_LAUNCH((k_mg_march<T, TC, 32, SRC, NSW, RESN, RESTR, OUTER, (NSW) != 0>), grd, blk, 0, \
+                       s, m, a.tab);                                                          \
         else                                                                                  \
             NYL_LAUNCH((k_mg_march<T, TC, 32, SRC, NSW, RESN, RESTR, OUTER>), grd, blk, 0, s, m, \
                        a.tab);                                                                \

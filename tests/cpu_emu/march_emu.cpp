@@ -15,7 +15,8 @@ static std::vector<T> sweep(const Geo &g, const std::vector<T> &x, const std::ve
     return y;
 }
 
-template <typename T, typename TC, int TX>
+// LONG: with the steps inside the march as a path of its own
+template <typename T, typename TC, int TX, bool LONG = false>
 int check(int nx, int ny, int nz, int px, int py, int pz, int kz, bool halves) {
     const Geo g = mk(nx, ny, nz, px, py, pz), gc = mk(nx / 2, ny / 2, nz / 2, px, py, pz);
     const MGTabs tab = mktab();
@@ -47,12 +48,12 @@ int check(int nx, int ny, int nz, int px, int py, int pz, int kz, bool halves) {
         std::vector<double> p1(nblk, 0.0), p2(nblk, 0.0);
         a.src = x.data(); a.dst = z.data();
         run_blocks(grd, dim3(256), [&]() {
-            k_mg_march<T, TC, TX, MS_FIELD, 2, false, false, false>(a, tab); }, true);
+            k_mg_march<T, TC, TX, MS_FIELD, 2, false, false, false, LONG>(a, tab); }, true);
         bad += ndiff(z, y2);
         z.assign(nf, T(7));
         a.partials = p1.data();
         run_blocks(grd, dim3(256), [&]() {
-            k_mg_march<T, TC, TX, MS_FIELD, 2, true, false, false>(a, tab); }, true);
+            k_mg_march<T, TC, TX, MS_FIELD, 2, true, false, false, LONG>(a, tab); }, true);
         bad += ndiff(z, y2) + norm_of(p1);
         a.partials = p2.data();
         run_blocks(grd, dim3(256), [&]() {
@@ -62,7 +63,7 @@ int check(int nx, int ny, int nz, int px, int py, int pz, int kz, bool halves) {
         const auto s2 = sweep(g, sweep(g, zero, b, tab), b, tab);
         a.src = nullptr;
         run_blocks(grd, dim3(256), [&]() {
-            k_mg_march<T, TC, TX, MS_ZERO, 2, false, false, false>(a, tab); }, true);
+            k_mg_march<T, TC, TX, MS_ZERO, 2, false, false, false, LONG>(a, tab); }, true);
         bad += ndiff(z, s2);
     }
     if (halves) {
@@ -74,7 +75,7 @@ int check(int nx, int ny, int nz, int px, int py, int pz, int kz, bool halves) {
                                        yc1.data(), 0.9); }, false);
         a.src = x.data(); a.dst = z.data(); a.bc = bc2.data(); a.yc = yc2.data();
         run_blocks(grd, dim3(256), [&]() {
-            k_mg_march<T, TC, TX, MS_FIELD, 1, false, true, false>(a, tab); }, true);
+            k_mg_march<T, TC, TX, MS_FIELD, 1, false, true, false, LONG>(a, tab); }, true);
         bad += ndiff(z, y1) + ndiff(bc1, bc2) + ndiff(yc1, yc2);
         run_blocks(mg_grid(g), dim3(MG_BX, MG_BY, 1), [&]() {
             k_mg_prolong<T, TC>(g, gc, xp.data(), xc.data(), tab); }, false);
@@ -82,7 +83,7 @@ int check(int nx, int ny, int nz, int px, int py, int pz, int kz, bool halves) {
         z.assign(nf, T(7));
         a.xc = xc.data();
         run_blocks(grd, dim3(256), [&]() {
-            k_mg_march<T, TC, TX, MS_PROLONG, 2, false, false, false>(a, tab); }, true);
+            k_mg_march<T, TC, TX, MS_PROLONG, 2, false, false, false, LONG>(a, tab); }, true);
         bad += ndiff(z, u2);
         // the restriction alone, and in the pass of the two sweeps (from a
         // field with its residual norm, from zero)
@@ -102,8 +103,8 @@ int check(int nx, int ny, int nz, int px, int py, int pz, int kz, bool halves) {
             a.src = zero ? nullptr : x.data();
             a.partials = p3.data();
             run_blocks(grd, dim3(256), [&]() {
-                if (zero) k_mg_march<T, TC, TX, MS_ZERO, 2, false, true, false>(a, tab);
-                else k_mg_march<T, TC, TX, MS_FIELD, 2, true, true, false>(a, tab); }, true);
+                if (zero) k_mg_march<T, TC, TX, MS_ZERO, 2, false, true, false, LONG>(a, tab);
+                else k_mg_march<T, TC, TX, MS_FIELD, 2, true, true, false, LONG>(a, tab); }, true);
             bad += ndiff(z, t2) + ndiff(bc1, bc2) + ndiff(yc1, yc2) + (!zero && norm_of(p3));
         }
         a.src = x.data();
@@ -113,7 +114,7 @@ int check(int nx, int ny, int nz, int px, int py, int pz, int kz, bool halves) {
         a.gate = &one;
         a.src = y1.data();
         run_blocks(grd, dim3(256), [&]() {
-            k_mg_march<T, TC, TX, MS_PROLONG, 2, false, false, false>(a, tab); }, true);
+            k_mg_march<T, TC, TX, MS_PROLONG, 2, false, false, false, LONG>(a, tab); }, true);
         bad += ndiff(z, z0);
     }
     if (sizeof(T) == 8 && sizeof(TC) == 8) {   // the mixed solve's FP64 residual
@@ -148,6 +149,10 @@ int main() {
         fails += check<float, float, 32>(40, 18, 10, px, py, pz, 4, true);
         fails += check<float, double, 32>(6, 10, 14, px, py, pz, 8, true);
         fails += check<float, float, 64>(2, 2, 2, px, py, pz, 2, true);
+        if (p == 0 || p == 7) {   // one march; one with a short rest
+            fails += check<double, double, 64, true>(34, 10, 16, px, py, pz, 16, true);
+            fails += check<float, float, 32, true>(6, 10, 22, px, py, pz, 16, true);
+        }
         if (p == 0 || p == 7) {
             fails += check<double, double, 64>(64, 8, 8, px, py, pz, 8, true);
             fails += check<float, float, 64>(130, 24, 4, px, py, pz, 2, true);
