@@ -13,6 +13,8 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <vector>
 
 #include "nyl_ctx.h"
@@ -65,13 +67,16 @@ struct nyl_batch {
     hipStream_t stream = nullptr;
     MGTabs tabs;
     // device control arrays (offsets)
-    uint64_t o_normb, o_res, o_shift, o_tol, o_nite, o_maxite, o_active, o_any, o_dt, o_acc;
+    uint64_t o_normb, o_res, o_shift, o_tol, o_nite, o_maxite, o_active, o_dt, o_acc;
     BMG mg = {};
     // plans
     std::vector<Launch> pre[2][3], vcyc, post[2];
     std::vector<char> blob;     // host image of the item tables
     hipGraphExec_t g_pre[2][3] = {}, g_vcyc = nullptr, g_post[2] = {};
-    int *host_any = nullptr;    // pinned: members still iterating, most V-cycles so far
+    int *host_any = nullptr;    // coherent: members still iterating, most V-cycles so far,
+                                // and the sequence number of the launch that wrote them
+    int *dev_any = nullptr;     // its device address
+    uint32_t any_seq = 0;
     int vcap[3] = {0, 0, 0};    // V-cycles launched without a poll, per RK stage
     double *host_dt = nullptr;  // pinned, n
     void *host_stats = nullptr; // pinned: nite_acc (int n), res (double n), normb (double n)
@@ -587,11 +592,23 @@ int run_plan(nyl_batch *b, std::vector<Launch> &plan, hipGraphExec_t *g) {
     return NYL_OK;
 }
 
+// the active count and V-cycle maximum in host_any, polled (a copy and a
+// stream synchronisation left the GPU idle for 30..50 us each)
 int read_any(nyl_batch *b, int *any) {
-    BCHK(hipMemcpyAsync(b->host_any, b->mg.any, 2 * sizeof(int), hipMemcpyDeviceToHost,
-                        b->stream));
-    BCHK(hipStreamSynchronize(b->stream));
-    *any = b->host_any[0];
+    const uint32_t seq = ++b->any_seq;
+    BCHK(launch_b_count(b->n, b->mg, b->dev_any, (uint32_t *)(b->dev_any + 2), seq, b->stream));
+    volatile uint32_t *flag = (volatile uint32_t *)(b->host_any + 2);
+    const auto t0 = std::chrono::steady_clock::now();
+    for (uint64_t it = 1; *flag != seq; it++) {
+        if ((it & 1023) == 0 &&
+            std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(50)) {
+            BCHK(hipStreamSynchronize(b->stream));
+            if (*flag != seq) return set_error(NYL_E_HIP, "active count of the batch not published");
+            break;
+        }
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
+    *any = ((volatile int *)b->host_any)[0];
     return NYL_OK;
 }
 
@@ -715,7 +732,7 @@ int nyl_batch_create(nyl_ctx *const *members, int32_t n, nyl_batch **out) {
     b->o_normb = take(8 * n); b->o_res = take(8 * n); b->o_shift = take(8 * n);
     b->o_tol = take(8 * n); b->o_dt = take(8 * n);
     b->o_nite = take(4 * n); b->o_maxite = take(4 * n); b->o_active = take(4 * n);
-    b->o_any = take(8); b->o_acc = take(4 * n);
+    b->o_acc = take(4 * n);
     if (b->mixed) build_plans<float>(b);
     else build_plans<double>(b);
     b->ws_bytes = tables_off(b) + al256(b->blob.size()) + tune_bytes(b);
@@ -753,7 +770,11 @@ int nyl_batch_bind_workspace(nyl_batch *b, void *dptr, uint64_t bytes) {
     if (((uintptr_t)dptr) & 255) return set_error(NYL_E_ARG, "workspace must be 256-byte aligned");
     const int n = b->n;
     if (!b->host_any) {
-        BCHK(hipHostMalloc((void **)&b->host_any, 2 * sizeof(int), 0));
+        BCHK(hipHostMalloc((void **)&b->host_any, 4 * sizeof(int),
+                           hipHostMallocMapped | hipHostMallocCoherent));
+        BCHK(hipHostGetDevicePointer((void **)&b->dev_any, b->host_any, 0));
+        ((volatile int *)b->host_any)[2] = 0;
+        b->any_seq = 0;
         BCHK(hipHostMalloc((void **)&b->host_dt, sizeof(double) * n, 0));
         BCHK(hipHostMalloc(&b->host_stats, (sizeof(int) + 2 * sizeof(double)) * n, 0));
     }
@@ -764,7 +785,7 @@ int nyl_batch_bind_workspace(nyl_batch *b, void *dptr, uint64_t bytes) {
     mg.shift = (double *)(b->ws + b->o_shift); mg.tol = (double *)(b->ws + b->o_tol);
     mg.dt = (const double *)(b->ws + b->o_dt);
     mg.nite = (int *)(b->ws + b->o_nite); mg.maxite = (int *)(b->ws + b->o_maxite);
-    mg.active = (int *)(b->ws + b->o_active); mg.any = (int *)(b->ws + b->o_any);
+    mg.active = (int *)(b->ws + b->o_active);
     mg.acc = (int *)(b->ws + b->o_acc);
     // the tables hold addresses in this workspace
     if (b->mixed) build_plans<float>(b);

@@ -322,7 +322,7 @@ struct CoarseItem { BHead h; CoarseArgs a; };
 // (core/mgfor/solvers.f90:17-30) evaluated per member on the device.
 struct BMG {
     double *normb, *res, *shift, *tol;
-    int *nite, *maxite, *active, *any;
+    int *nite, *maxite, *active;
     int *acc;              // V-cycles summed over the stages of a step
     const double *dt;
 };
@@ -362,6 +362,8 @@ hipError_t launch_b_sweep(const SweepItem *items, int n, int64_t nblk, const MGT
 // nblk of the member)
 hipError_t launch_b_reduce(const RedItem *items, int n, int64_t nblk, int kind, hipStream_t s);
 hipError_t launch_b_final(const FinalItem *items, int n, int kind, const BMG &mg, hipStream_t s);
+hipError_t launch_b_count(int n, const BMG &mg, int *out, uint32_t *flag, uint32_t seq,
+                          hipStream_t s);
 hipError_t launch_b_coarse(const CoarseItem *items, int n, int64_t nblk, int pass,
                            const int *active, hipStream_t s);
 // mode 0: acc = 0; mode 1: acc += nite

@@ -946,9 +946,12 @@ __global__ __launch_bounds__(RED_T) void k_b_final(const FinalItem *__restrict__
     }
 }
 
-// mg.any[0] = number of members still iterating, mg.any[1] = the most
-// V-cycles any member has run in the current solve
-__global__ __launch_bounds__(RED_T) void k_b_count(int n, BMG mg) {
+// out[0] = number of members still iterating, out[1] = the most V-cycles any
+// member has run in the current solve; out is coherent host memory, whose
+// flag takes seq once they are there.  Launched where the host reads them,
+// not in every V-cycle (4 us each).
+__global__ __launch_bounds__(RED_T) void k_b_count(int n, BMG mg, int *out, uint32_t *flag,
+                                                   uint32_t seq) {
     __shared__ double tot, most;
     double acc = 0.0, mx = 0.0;
     for (int q = threadIdx.x; q < n; q += RED_T) {
@@ -960,9 +963,17 @@ __global__ __launch_bounds__(RED_T) void k_b_count(int n, BMG mg) {
     block_max_store(mx, &most, threadIdx.x);
     __syncthreads();
     if (threadIdx.x == 0) {
-        mg.any[0] = (int)tot;
-        mg.any[1] = (int)most;
+        out[0] = (int)tot;
+        out[1] = (int)most;
+        __threadfence_system();
+        __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
+}
+
+hipError_t launch_b_count(int n, const BMG &mg, int *out, uint32_t *flag, uint32_t seq,
+                          hipStream_t s) {
+    NYL_LAUNCH(k_b_count, dim3(1), RED_T, 0, s, n, mg, out, flag, seq);
+    return hipGetLastError();
 }
 
 hipError_t launch_b_final(const FinalItem *items, int n, int kind, const BMG &mg, hipStream_t s) {
@@ -972,8 +983,6 @@ hipError_t launch_b_final(const FinalItem *items, int n, int kind, const BMG &mg
     case NYL_FIN_STEP: NYL_LAUNCH((k_b_final<NYL_FIN_STEP>), dim3(n), RED_T, 0, s, items, mg); break;
     default: NYL_LAUNCH((k_b_final<NYL_FIN_SHIFT>), dim3(n), RED_T, 0, s, items, mg); break;
     }
-    if (kind == NYL_FIN_INIT || kind == NYL_FIN_STEP)
-        NYL_LAUNCH(k_b_count, dim3(1), RED_T, 0, s, n, mg);
     return hipGetLastError();
 }
 
