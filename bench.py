@@ -25,10 +25,11 @@ both precisions.
 Prints ONE JSON line.  ``roofline`` prices the dominant kernel of the
 headline path, the two-sweep damped-Jacobi smoothing pass on the finest
 multigrid level (k_mg_sweep2t: both pre-smoothing sweeps with the residual
-norm of the convergence test, or both post-smoothing sweeps; the kernel with
-the largest time per step): achieved = its algorithmic HBM bytes per launch
-(each input field read once, each output written once: 12 bytes per cell in
-FP32 for two sweeps) divided by its mean launch time, both measured with HIP
+norm of the convergence test; k_mg_march: the prolongation and both
+post-smoothing sweeps; together the largest time per step): achieved = their
+algorithmic HBM bytes per launch (each input field read once, each output
+written once: 12 bytes per cell in FP32 for two sweeps, and the coarse level
+of the prolongation) divided by their mean launch time, both measured with HIP
 events on the library's stream over the timed steps.  ``cpu_baseline`` times the
 FP64 CPU oracle (C restatement of the reference kernels + numpy
 orchestration, OpenMP) on a bounded sample of the same workload.
@@ -437,7 +438,7 @@ def stage_report(dev, dt, precision, n, steps=2):
         return None
     us = ms / nl * 1e3
     gbs = by / nl / (us * 1e-6) / 1e9
-    return {"kernel": "k_stage (RK3 modes 1-3)", "launches": nl, "mean_launch_us": round(us, 2),
+    return {"kernel": "k_stage_flat (RK3 modes 1-3)", "launches": nl, "mean_launch_us": round(us, 2),
             "alg_bytes_per_launch": by / nl, "achieved": round(gbs, 2), "unit": "GB/s",
             "hbm_frac": round(gbs / HBM_PEAK_GBS, 4),
             "valu_issue_frac": measured_valu(precision, n)}

@@ -474,7 +474,8 @@ int level_up(nyl_ctx *c, int l, const int *gate = nullptr) {
         MarchArgs<T, TC> a = march_args<T, TC>(c, l, l > 0 ? f.x : f.y, l > 0 ? f.y : f.x);
         a.xc = F<TC>(c, qx);
         a.gate = gate;
-        LAUNCH(NYL_K_MG_PROLONG, 3 * n + cells(q.g) * sizeof(TC),
+        LAUNCH(l == 0 ? (NYL_K_MG_SWEEP2 | kFineLevel) : NYL_K_MG_PROLONG,
+               3 * n + cells(q.g) * sizeof(TC),
                (launch_march_up<T, TC>(a, c->stream)));
         return NYL_OK;
     });
