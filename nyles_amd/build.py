@@ -18,8 +18,8 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libnyles_hip.so")
 OBJDIR = os.path.join(HERE, "_build")
 SOURCES = ["nyl_stage64.hip", "nyl_stage32.hip", "nyl_stagelin64.hip", "nyl_stagelin32.hip",
-           "nyl_stencil.hip", "nyl_api.hip", "nyl_mg.hip", "nyl_march.hip", "nyl_cycle.hip",
-           "nyl_batch.hip", "nyl_coarse.hip", "nyl_noalloc.hip", "nyl_mgfor.hip"]
+           "nyl_stencil.hip", "nyl_tracer.hip", "nyl_api.hip", "nyl_mg.hip", "nyl_march.hip",
+           "nyl_cycle.hip", "nyl_batch.hip", "nyl_coarse.hip", "nyl_noalloc.hip", "nyl_mgfor.hip"]
 ARCH = os.environ.get("NYL_OFFLOAD_ARCH", "gfx950")
 
 FLAGS = [

@@ -412,18 +412,18 @@ __device__ __forceinline__ void viscosity_cell(const Geo &g, const StageArgs<T> 
     dw = lap3(dw, a.w);
 }
 
-// The stage combination of one field at N cells (core/timescheme.py): its
-// tendency d, the current and next state, the tendency slots and the LFAM3
+// The stage combination of one field at N cells (core/timescheme.py) with the
+// coefficients c and (LFAM3 predictor) c2: its tendency d, the current and next state, the tendency slots and the LFAM3
 // 'before' state.
 template <int N, int MODE, bool LIN, typename T>
-__device__ __forceinline__ void stage_out(const StageArgs<T> &a, uint32_t cb, const Vec<T, N> &d,
+__device__ __forceinline__ void stage_out(double c, double c2, uint32_t cb, const Vec<T, N> &d,
                                           const T *__restrict__ now, T *__restrict__ next,
                                           T *__restrict__ tend, const T *__restrict__ d0,
                                           const T *__restrict__ d1, T *__restrict__ before) {
     // read at a later stage; the model variants keep them at every stage
     if (MODE == 0 || MODE == 1 || MODE == 2 || LIN) stv<N, true>(tend, cb, d);
     if (MODE == 0) return;
-    const T cc = T(a.c);
+    const T cc = T(c);
     const Vec<T, N> s = ldv<N>((MODE == 5 ? (const T *)next : now), cb);
     Vec<T, N> o, e0, e1;
     if (MODE == 2 || MODE == 3) e0 = ldv<N>(d0, cb);
@@ -438,7 +438,7 @@ __device__ __forceinline__ void stage_out(const StageArgs<T> &a, uint32_t cb, co
         } else if (MODE == 3) {                      // s += (dt/12.)*(8*ds2-ds0-ds1)
             o.v[q] = s.v[q] + cc * ((T(8) * d.v[q] - e0.v[q]) - e1.v[q]);
         } else {   // LFAM3 predictor: s = sb + (2.*dt)*ds; s = (1./12.)*(5.*s+8.*sn-sb); sb = sn
-            const T t1 = e0.v[q] + T(a.c2) * d.v[q];
+            const T t1 = e0.v[q] + T(c2) * d.v[q];
             o.v[q] = T(1. / 12.) * (T(5) * t1 + T(8) * s.v[q] - e0.v[q]);
         }
     }
@@ -531,10 +531,10 @@ __device__ __forceinline__ void stage_cells(const Geo &g, const StageArgs<T> &a,
             viscosity_cell<T, PX, PY, PZ>(g, a, cb + (uint32_t)(q * ES), i + q, j, k, du.v[q],
                                           dv.v[q], dw.v[q]);
     }
-    stage_out<N, MODE, LIN>(a, cb, db, a.b, a.bn, a.tb, a.d0b, a.d1b, a.sbb);
-    stage_out<N, MODE, LIN>(a, cb, du, a.u, a.un, a.tu, a.d0u, a.d1u, a.sbu);
-    stage_out<N, MODE, LIN>(a, cb, dv, a.v, a.vn, a.tv, a.d0v, a.d1v, a.sbv);
-    stage_out<N, MODE, LIN>(a, cb, dw, a.w, a.wn, a.tw, a.d0w, a.d1w, a.sbw);
+    stage_out<N, MODE, LIN>(a.c, a.c2, cb, db, a.b, a.bn, a.tb, a.d0b, a.d1b, a.sbb);
+    stage_out<N, MODE, LIN>(a.c, a.c2, cb, du, a.u, a.un, a.tu, a.d0u, a.d1u, a.sbu);
+    stage_out<N, MODE, LIN>(a.c, a.c2, cb, dv, a.v, a.vn, a.tv, a.d0v, a.d1v, a.sbv);
+    stage_out<N, MODE, LIN>(a.c, a.c2, cb, dw, a.w, a.wn, a.tw, a.d0w, a.d1w, a.sbw);
 }
 
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -561,8 +561,9 @@ __global__ __launch_bounds__(256) void k_stage(Geo g, StageArgs<T> a) {
 // What bounds it.  FP64: a load of 8 bytes per lane passes L1 at 32 B/clk, of
 // 16 bytes at 64 B/clk; with one cell per thread the kernel sat at 80 % of
 // that rate, with two at 43 %, and the N + 1 x faces of the group are shared.
-// Now VALU issue (85 %) at the clock FP64 runs at (1.95 GHz).  FP32: VALU
-// issue (93 %); four cells share x faces and address arithmetic.
+// Now the VALU (busy 85 %) at the clock FP64 runs at (1.95 GHz).  FP32: the
+// VALU (busy 93 % with one cell per thread); four cells share x faces and
+// address arithmetic (944 -> 771 instructions per 64 cells).
 // us per call, one cell per thread in 64-wide rows -> now: FP64 256^3
 // periodic 1161 -> 970, 160x96x128 162 -> 112, 96^3 87 -> 57; FP32 256^3
 // 510 -> 440, walls 256x128x64 106 -> 58, 200x120x56 72 -> 42.

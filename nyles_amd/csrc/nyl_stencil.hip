@@ -1,5 +1,5 @@
-// nyl_stencil.hip -- the diagnostic stencils, passive tracers and ensemble
-// forms of the Nyles time step on gfx950 (the stage kernels: nyl_stage.h).
+// nyl_stencil.hip -- the diagnostic stencils, reductions and ensemble forms of
+// the Nyles time step on gfx950 (the stage kernels: nyl_stage.h).
 //
 // Every FP64 instantiation reproduces the reference's arithmetic operation
 // by operation (the library is compiled with -ffp-contract=off), so its
@@ -403,88 +403,7 @@ __global__ __launch_bounds__(S25_NT) void k_stage25(Geo g, StageArgs<T> a, int k
     }
 }
 
-// ---------------------------------------------------------------------------
-// Passive tracers: the b part of stage_cell for another scalar, with the
-// stage update of the mode (same expressions as b's).
-template <typename T, int MODE, int PX, int PY, int PZ>
-__device__ __forceinline__ void tracer_cell(const Geo &g, const TracerArgs<T> &a, int i, int j,
-                                            int k) {
-    const int64_t c = (int64_t)k * g.sz + (int64_t)j * g.sy + i;
-    constexpr int ES = (int)sizeof(T);
-    const uint32_t cb = (uint32_t)c * (uint32_t)ES;
-    const T cx = T(a.idx2), cy = T(a.idy2), cz = T(a.idz2);
-    constexpr bool LIN = MODE == 0;   // the linear upwind branch too
-    const int oa = LIN ? a.upw : 0;
-    const LineX<1> Lx = linex_of<1, PX>(i, g.nx, ES);
-    const Line<int32_t> Ly = line_of<PY, int32_t>(j, g.ny, (int32_t)(g.sy * ES));
-    const Line<int32_t> Lz = line_of<PZ, int32_t>(k, g.nz, (int32_t)(g.sz * ES));
-    Vec<T, 1> d = {};
-    tracer_x<1, PX, LIN>(d, a.q, a.u, cx, cb, Lx, i, g.nx, oa);
-    tracer_yz<1, PY, LIN>(d, a.q, a.v, cy, cb, Ly, j, g.ny, oa);
-    tracer_yz<1, PZ, LIN>(d, a.q, a.w, cz, cb, Lz, k, g.nz, oa);
-    const T dq = d.v[0];
-    if (MODE == 0 || MODE == 1 || MODE == 2) stb(a.tout, cb, dq);
-    const T cc = T(a.c);
-    if (MODE == 1) {
-        stb(a.qn, cb, ldb(a.q, cb) + cc * dq);
-    } else if (MODE == 2) {
-        stb(a.qn, cb, ldb(a.q, cb) + cc * (dq - T(3) * ldb(a.d0, cb)));
-    } else if (MODE == 3) {
-        stb(a.qn, cb, ldb(a.q, cb) + cc * ((T(8) * dq - ldb(a.d0, cb)) - ldb(a.d1, cb)));
-    } else if (MODE == 4) {
-        const T c2 = T(a.c2), c12 = T(1. / 12.);
-        const T sb = ldb(a.sb, cb), t1 = sb + c2 * dq;
-        stb(a.qn, cb, c12 * (T(5) * t1 + T(8) * ldb(a.q, cb) - sb));
-        stb(a.sb, cb, ldb(a.q, cb));
-    } else if (MODE == 5) {
-        stb(a.qn, cb, ldb(a.qn, cb) + cc * dq);
-    } else if (MODE == 6) {
-        stb(a.sb, cb, ldb(a.q, cb));
-        stb(a.qn, cb, ldb(a.q, cb) + cc * dq);
-    }
-}
-
-template <typename T, int MODE, int PX, int PY, int PZ>
-__global__ __launch_bounds__(256) void k_tracer_stage(Geo g, TracerArgs<T> a) {
-    const Blk3 bk = xcd_block();
-    const int i = bk.x * NYL_BX + threadIdx.x;
-    const int j = bk.y * NYL_BY + threadIdx.y;
-    if (i >= g.nx || j >= g.ny) return;
-    tracer_cell<T, MODE, PX, PY, PZ>(g, a, i, j, bk.z);
-}
-
-template <typename T, int PX, int PY, int PZ>
-static void launch_tracer_p(const Geo &g, const TracerArgs<T> &a, int mode, hipStream_t s) {
-    dim3 blk(NYL_BX, NYL_BY, 1), grd = cell_grid(g);
-    switch (mode) {
-    case 0: NYL_LAUNCH((k_tracer_stage<T, 0, PX, PY, PZ>), grd, blk, 0, s, g, a); break;
-    case 1: NYL_LAUNCH((k_tracer_stage<T, 1, PX, PY, PZ>), grd, blk, 0, s, g, a); break;
-    case 2: NYL_LAUNCH((k_tracer_stage<T, 2, PX, PY, PZ>), grd, blk, 0, s, g, a); break;
-    case 3: NYL_LAUNCH((k_tracer_stage<T, 3, PX, PY, PZ>), grd, blk, 0, s, g, a); break;
-    case 4: NYL_LAUNCH((k_tracer_stage<T, 4, PX, PY, PZ>), grd, blk, 0, s, g, a); break;
-    case 5: NYL_LAUNCH((k_tracer_stage<T, 5, PX, PY, PZ>), grd, blk, 0, s, g, a); break;
-    case 6: NYL_LAUNCH((k_tracer_stage<T, 6, PX, PY, PZ>), grd, blk, 0, s, g, a); break;
-    default: break;
-    }
-}
-
-template <typename T>
-hipError_t launch_tracer_stage(const Geo &g, const TracerArgs<T> &a, int mode, hipStream_t s) {
-    if (mode < 0 || mode > 6) return hipErrorInvalidValue;
-    switch (g.px + 2 * g.py + 4 * g.pz) {
-    case 0: launch_tracer_p<T, 0, 0, 0>(g, a, mode, s); break;
-    case 1: launch_tracer_p<T, 1, 0, 0>(g, a, mode, s); break;
-    case 2: launch_tracer_p<T, 0, 1, 0>(g, a, mode, s); break;
-    case 3: launch_tracer_p<T, 1, 1, 0>(g, a, mode, s); break;
-    case 4: launch_tracer_p<T, 0, 0, 1>(g, a, mode, s); break;
-    case 5: launch_tracer_p<T, 1, 0, 1>(g, a, mode, s); break;
-    case 6: launch_tracer_p<T, 0, 1, 1>(g, a, mode, s); break;
-    default: launch_tracer_p<T, 1, 1, 1>(g, a, mode, s); break;
-    }
-    return hipGetLastError();
-}
-
-// The stage combinations of stage_cell with the tendency read from memory
+// The stage combinations of the stage kernel with the tendency read from memory
 template <typename T, int MODE>
 __global__ __launch_bounds__(256) void k_update(int64_t n, UpdateArgs<T> a) {
     const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -1126,10 +1045,6 @@ NYL_B_STENCIL_INST(double)
 NYL_B_STENCIL_INST(float)
 #undef NYL_B_STENCIL_INST
 
-template hipError_t launch_tracer_stage<double>(const Geo &, const TracerArgs<double> &, int,
-                                                hipStream_t);
-template hipError_t launch_tracer_stage<float>(const Geo &, const TracerArgs<float> &, int,
-                                               hipStream_t);
 template hipError_t launch_update<double>(int64_t, const UpdateArgs<double> &, int, hipStream_t);
 template hipError_t launch_update<float>(int64_t, const UpdateArgs<float> &, int, hipStream_t);
 template hipError_t launch_diag<double>(const Geo &, const DiagArgs<double> &, int, hipStream_t);

@@ -47,3 +47,32 @@ def test_rhs_forms_match_the_oracle(shape, geometry, scale):
         bad = cmp.mismatches(dev.download(ids[k]), orc.interior(want[k]))
         assert bad == 0, "d%s: %d elements differ" % (k, bad)
     dev.close()
+
+
+@pytest.mark.parametrize("scheme", ["rk3", "lfam3"])
+@pytest.mark.parametrize("geometry", ["closed", "perio_xy"])
+def test_tracers_in_pairs_match_the_oracle(scheme, geometry):
+    """two steps with passive tracers on a grid that takes two cells per thread"""
+    import compare as cmp
+    print("case tracer pairs", scheme, geometry, flush=True)
+    orc, dev = cmp.make_pair(64, 64, 64, geometry, n_tracers=2)
+    st = cmp.random_state(orc, seed=19, amp_u=3e-3)
+    rng = np.random.default_rng(20)
+    for q in range(2):
+        st["t%d" % q] = rng.standard_normal(st["b"].shape)
+    cmp.load_state(orc, dev, st)
+    orc.diagnose_var()
+    dev.diagnose()
+    for n in range(2):
+        dt = orc.compute_dt(cfl=0.5, dt_max=0.1)
+        if scheme == "rk3":
+            orc.rk3_ssp(dt)
+            dev.step_rk3(dt)
+        else:
+            orc.lfam3(dt)
+            dev.step_lfam3(dt)
+    want, got = cmp.oracle_fields(orc), cmp.device_fields(dev)
+    for k in want:
+        bad = cmp.mismatches(got[k], want[k])
+        assert bad == 0, "%s: %d elements differ" % (k, bad)
+    dev.close()
