@@ -143,7 +143,10 @@ void build_layout(nyl_ctx *c) {
         c->mgx = c->lev[0].x;
         c->mgb = c->lev[0].b;
     }
-    c->partials = take(NYL_RED_BLOCKS * sizeof(double));
+    // block sums: of the reductions (capped), and of the batched march over
+    // level 0, which has one per block
+    c->partials = take(std::max<uint64_t>(NYL_RED_BLOCKS, b_march_blocks(c->lev[0].g)) *
+                       sizeof(double));
     c->result = take(8 * sizeof(double));
     c->ctl = take(sizeof(MGCtl));
     c->ent = take(sizeof(c->cyc_ent));

@@ -199,20 +199,6 @@ uint64_t correction(const nyl_ctx *c, int l) {
     return l == c->nlev - 1 ? c->lev[l].x : c->lev[l].y;
 }
 
-// Planes per block of a member's level: its own, whatever the batch, so that
-// the block sums of its residual norms are.  Short marches for small levels
-// (a batch has blocks enough only when its members do).
-int march_kz(const Geo &g) {
-    int kz = gcells(g) < (1 << 18) ? 4 : 8;
-    const int64_t cols = (int64_t)((g.nx + 31) / 32) * ((g.ny + 15) / 16);
-    while (cols * ((g.nz + kz - 1) / kz) > NYL_RED_BLOCKS && kz < g.nz) kz *= 2;
-    return kz;
-}
-int64_t march_blocks(const Geo &g) {
-    const int kz = march_kz(g);
-    return (int64_t)((g.nx + 31) / 32) * ((g.ny + 15) / 16) * ((g.nz + kz - 1) / kz);
-}
-
 // which members a pass of level 0 covers: up to 1M cells the sweeps and the
 // restriction run as one pass, above that as two (see pre_smooth in
 // nyl_api.hip)
@@ -243,14 +229,14 @@ void level_pass_t(nyl_batch *b, int l, MarchKind kind, LType type, std::vector<L
         MarchArgs<T, TC> &a = it.a;
         a.g = f.g;
         a.gc = k.g;
-        a.kz = march_kz(f.g);
+        a.kz = b_march_kz(f.g);
         a.omega = c->d.mg_omega;
         a.partials = F<double>(c, c->partials);
         it.bx = (f.g.nx + 31) / 32;
         it.by = (f.g.ny + 15) / 16;
         it.h.g = f.g;
         it.h.member = q;
-        it.h.nblk = (int)march_blocks(f.g);
+        it.h.nblk = (int)b_march_blocks(f.g);
         it.h.start = nb;
         nb += it.h.nblk;
         if (kind == MK_OUTER) {
@@ -333,7 +319,7 @@ void test_launches(nyl_batch *b, std::vector<Launch> &out, bool gated) {
 }
 std::vector<int> test_blocks(const nyl_batch *b) {
     std::vector<int> np(b->n);
-    for (int q = 0; q < b->n; q++) np[q] = (int)march_blocks(b->m[q]->lev[0].g);
+    for (int q = 0; q < b->n; q++) np[q] = (int)b_march_blocks(b->m[q]->lev[0].g);
     return np;
 }
 

@@ -40,6 +40,14 @@ struct MarchItem {
 enum MarchKind {
     MK_UP, MK_UP_ADD, MK_DOWN, MK_RESTRICT, MK_PRE, MK_PRE_RESTRICT, MK_ZERO, MK_ZERO_RESTRICT, MK_OUTER
 };
+// Planes per block of a member's level, and the blocks of a pass over it: the
+// member's own, whatever the batch, so that the block sums of its residual
+// norms are.  Short marches for small levels (a batch has blocks enough only
+// when its members do), longer ones where the blocks exceed NYL_RED_BLOCKS.
+// A level of more than NYL_RED_BLOCKS tiles has more blocks than that all the
+// same: the partials of a context have room for them (build_layout).
+int b_march_kz(const Geo &g);
+int64_t b_march_blocks(const Geo &g);
 // map: the item of each block
 template <typename T, typename TC>
 hipError_t launch_b_march(const MarchItem<T, TC> *items, const uint16_t *map, int64_t nblk,

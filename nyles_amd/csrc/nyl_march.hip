@@ -568,6 +568,21 @@ hipError_t launch_march_outer(const MarchArgs<double, double> &a, hipStream_t s)
     return hipGetLastError();
 }
 
+static int64_t b_march_tiles(const Geo &g) {
+    return (int64_t)((g.nx + 31) / 32) * ((g.ny + 15) / 16);
+}
+
+int b_march_kz(const Geo &g) {
+    int kz = (int64_t)g.nx * g.ny * g.nz < (1 << 18) ? 4 : 8;
+    while (b_march_tiles(g) * ((g.nz + kz - 1) / kz) > NYL_RED_BLOCKS && kz < g.nz) kz *= 2;
+    return kz;
+}
+
+int64_t b_march_blocks(const Geo &g) {
+    const int kz = b_march_kz(g);
+    return b_march_tiles(g) * ((g.nz + kz - 1) / kz);
+}
+
 template <typename T, typename TC>
 hipError_t launch_b_march(const MarchItem<T, TC> *items, const uint16_t *map, int64_t nblk,
                           MarchKind kind, const MGTabs &tab, const int *active, hipStream_t s) {
