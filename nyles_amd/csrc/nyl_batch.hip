@@ -214,7 +214,7 @@ template <typename T, typename TC>
 void level_pass_t(nyl_batch *b, int l, MarchKind kind, LType type, std::vector<Launch> &out,
                   bool gated, Size size) {
     std::vector<MarchItem<T, TC>> v;
-    std::vector<uint16_t> map;
+    std::vector<uint32_t> map;
     const bool f64 = std::is_same<T, double>::value, c64 = std::is_same<TC, double>::value;
     int64_t nb = 0;
     for (int q = 0; q < b->n; q++) {
@@ -262,14 +262,14 @@ void level_pass_t(nyl_batch *b, int l, MarchKind kind, LType type, std::vector<L
             default: a.src = x; a.dst = y; break;   // level 0's pre-smoothing
             }
         }
-        map.insert(map.end(), it.h.nblk, (uint16_t)v.size());
+        map.insert(map.end(), it.h.nblk, (uint32_t)v.size());
         v.push_back(it);
     }
     if (v.empty()) return;
     Launch L = add_table(b, L_MARCH, type, v, nb, kind, gated);
     L.off2 = al256(b->blob.size());
-    b->blob.resize(L.off2 + sizeof(uint16_t) * map.size());
-    memcpy(b->blob.data() + L.off2, map.data(), sizeof(uint16_t) * map.size());
+    b->blob.resize(L.off2 + sizeof(uint32_t) * map.size());
+    memcpy(b->blob.data() + L.off2, map.data(), sizeof(uint32_t) * map.size());
     out.push_back(L);
 }
 
@@ -527,7 +527,7 @@ int run_launch(nyl_batch *b, const Launch &L) {
     case L_MARCH: {
         // the initial residual runs for every member
         const int *gate = L.arg2 ? act : nullptr;
-        const uint16_t *map = (const uint16_t *)(b->ws + tables_off(b) + L.off2);
+        const uint32_t *map = (const uint32_t *)(b->ws + tables_off(b) + L.off2);
         const MarchKind kind = (MarchKind)L.arg;
         if (L.type == T_F)
             BCHK((launch_b_march<float, float>((const MarchItem<float, float> *)tab, map, L.nblk, kind, b->tabs, gate, s)));

@@ -48,9 +48,9 @@ enum MarchKind {
 // same: the partials of a context have room for them (build_layout).
 int b_march_kz(const Geo &g);
 int64_t b_march_blocks(const Geo &g);
-// map: the item of each block
+// map: the item of each block (32 bits: a batch may have any number of members)
 template <typename T, typename TC>
-hipError_t launch_b_march(const MarchItem<T, TC> *items, const uint16_t *map, int64_t nblk,
+hipError_t launch_b_march(const MarchItem<T, TC> *items, const uint32_t *map, int64_t nblk,
                           MarchKind kind, const MGTabs &tab, const int *active, hipStream_t s);
 
 // Blocks of a pass over a level, and their march length.  even: the march

@@ -470,7 +470,7 @@ __global__ __launch_bounds__(256, (march_waves<T, SRC, NSW, RESTR, LONG>())) voi
 // map[b], on its block number b - start (x fastest, then y, then z).
 template <typename T, typename TC, int SRC, int NSW, bool RESN, bool RESTR, bool OUTER, bool XADD>
 __global__ __launch_bounds__(256) void k_b_march(const MarchItem<T, TC> *__restrict__ items,
-                                                 const uint16_t *__restrict__ map, MGTabs tab,
+                                                 const uint32_t *__restrict__ map, MGTabs tab,
                                                  const int *__restrict__ active) {
     const MarchItem<T, TC> &it = items[map[blockIdx.x]];
     if (active && !active[it.h.member]) return;
@@ -584,7 +584,7 @@ int64_t b_march_blocks(const Geo &g) {
 }
 
 template <typename T, typename TC>
-hipError_t launch_b_march(const MarchItem<T, TC> *items, const uint16_t *map, int64_t nblk,
+hipError_t launch_b_march(const MarchItem<T, TC> *items, const uint32_t *map, int64_t nblk,
                           MarchKind kind, const MGTabs &tab, const int *active, hipStream_t s) {
     const dim3 grd((unsigned)nblk), blk(256);
 #define B_GO(SRC, NSW, RESN, RESTR)                                                      \
@@ -615,13 +615,13 @@ hipError_t launch_b_march(const MarchItem<T, TC> *items, const uint16_t *map, in
     return hipGetLastError();
 }
 template hipError_t launch_b_march<double, double>(const MarchItem<double, double> *,
-                                                   const uint16_t *, int64_t, MarchKind,
+                                                   const uint32_t *, int64_t, MarchKind,
                                                    const MGTabs &, const int *, hipStream_t);
 template hipError_t launch_b_march<float, float>(const MarchItem<float, float> *,
-                                                 const uint16_t *, int64_t, MarchKind,
+                                                 const uint32_t *, int64_t, MarchKind,
                                                  const MGTabs &, const int *, hipStream_t);
 template hipError_t launch_b_march<float, double>(const MarchItem<float, double> *,
-                                                  const uint16_t *, int64_t, MarchKind,
+                                                  const uint32_t *, int64_t, MarchKind,
                                                   const MGTabs &, const int *, hipStream_t);
 
 #define NYL_MARCH_INST(T, TC)                                                              \
