@@ -556,6 +556,31 @@ bool pre_tiled(const nyl_ctx *c) {
            (lev64(c, 0) ? n < (1 << 22) : 3.0 * n * sizeof(float) <= 256.0 * (1 << 20));
 }
 
+// The block sums of level 0's residual norm: those of the pre-smoothing pass
+// with a norm.  The norm alone (resid_norm) sums the same cells in the same
+// order, so a test gives the same bits whichever of the two the guess of a
+// solve chose.  capped: more blocks than partial sums, k_resnorm2 instead.
+struct NormForm {
+    MarchGrid grid;
+    bool tiled, capped;
+    int np;
+};
+NormForm norm_form(const nyl_ctx *c) {
+    const Geo &g = c->lev[0].g;
+    const int es = lev64(c, 0) ? 8 : 4;
+    NormForm f = {};
+    f.tiled = pre_tiled(c);
+    if (f.tiled) {
+        const int kz = sweep2x_kz(g, es);
+        f.grid = {64, g.nx / 64, g.ny / 8, g.nz / kz, kz};
+    } else {
+        f.grid = march_pre_grid(g, es);
+    }
+    f.capped = f.grid.blocks() > NYL_RED_BLOCKS;
+    f.np = f.capped ? red_blocks((int64_t)cells(g)) : f.grid.blocks();
+    return f;
+}
+
 // Both pre-smoothing sweeps of level 0 into its y and the restriction into
 // level 1.  zero: from a zero solution; else from x, with the block sums of
 // its residual norm in the partials (their number in *np).
@@ -563,11 +588,13 @@ int pre_smooth(nyl_ctx *c, bool zero, int *np) {
     const Level &f = c->lev[0], &q = c->lev[1];
     const double om = c->d.mg_omega, n = cells(f.g) * elem(c, 0);
     double *part = F<double>(c, c->partials);
+    const NormForm nf = norm_form(c);
+    if (!zero) *np = nf.np;
     return with_types(c, 0, [&](auto t, auto tc) -> int {
         using T = decltype(t);
         using TC = decltype(tc);
         if constexpr (std::is_same<T, TC>::value) {
-            if (pre_tiled(c)) {
+            if (nf.tiled) {
                 if (zero) {
                     // (not in the fine-level class of the roofline: it reads one field)
                     LAUNCH(NYL_K_MG_SWEEP2, 2 * n,
@@ -577,7 +604,6 @@ int pre_smooth(nyl_ctx *c, bool zero, int *np) {
                     LAUNCH(NYL_K_MG_SWEEP2 | kFineLevel, 3 * n,
                            launch_mg_sweep2x25<T>(f.g, F<T>(c, f.x), F<T>(c, f.y), F<T>(c, f.b),
                                                   om, c->tabs, c->stream, part));
-                    *np = sweep2x_blocks(f.g, (int)sizeof(T));
                 }
                 LAUNCH(NYL_K_MG_RESTRICT, 2.25 * n,
                        launch_mg_restrict25<T, T>(f.g, q.g, F<T>(c, f.y), F<T>(c, f.b),
@@ -591,18 +617,13 @@ int pre_smooth(nyl_ctx *c, bool zero, int *np) {
         else a.partials = part;
         a.bc = F<TC>(c, q.b);
         a.yc = F<TC>(c, q.y);
-        if (!zero) {
-            *np = march_grid(f.g, march_resident(sizeof(T), MS_FIELD, 2, true), true).blocks();
-            if (*np > NYL_RED_BLOCKS) {   // too wide for one partial sum per block
-                if constexpr (std::is_same<T, double>::value) {
-                    LAUNCH(NYL_K_RESNORM, 2 * n,
-                           launch_resnorm2<double>(f.g, a.src, a.b, c->tabs, part, nullptr,
-                                                   c->stream));
-                    *np = red_blocks((int64_t)cells(f.g));
-                    a.partials = nullptr;
-                } else {
-                    return fail(NYL_E_SIZE, "level 1 is too wide for the residual norm");
-                }
+        if (!zero && nf.capped) {
+            if constexpr (std::is_same<T, double>::value) {
+                LAUNCH(NYL_K_RESNORM, 2 * n,
+                       launch_resnorm2<double>(f.g, a.src, a.b, c->tabs, part, nullptr, c->stream));
+                a.partials = nullptr;
+            } else {
+                return fail(NYL_E_SIZE, "level 1 is too wide for the residual norm");
             }
         }
         LAUNCH(NYL_K_MG_SWEEP2 | (zero ? 0 : kFineLevel),
@@ -618,14 +639,14 @@ int resid_norm(nyl_ctx *c, int *np) {
     const Level &f = c->lev[0];
     MarchArgs<T, T> a = march_args<T, T>(c, 0, f.x, f.y);
     a.partials = F<double>(c, c->partials);
-    *np = march_grid(f.g, march_resident(sizeof(T), MS_FIELD, 0, false), false).blocks();
-    if (*np > NYL_RED_BLOCKS) {
-        *np = red_blocks((int64_t)cells(f.g));
+    const NormForm nf = norm_form(c);
+    *np = nf.np;
+    if (nf.capped)
         LAUNCH(NYL_K_RESNORM, 2 * cells(f.g) * sizeof(T),
                launch_resnorm2<T>(f.g, a.src, a.b, c->tabs, a.partials, nullptr, c->stream));
-        return NYL_OK;
-    }
-    LAUNCH(NYL_K_RESNORM, 2 * cells(f.g) * sizeof(T), launch_march_norm<T>(a, c->stream));
+    else
+        LAUNCH(NYL_K_RESNORM, 2 * cells(f.g) * sizeof(T),
+               launch_march_norm<T>(a, nf.grid, nf.tiled, c->stream));
     return NYL_OK;
 }
 
@@ -645,7 +666,8 @@ void fill_stats(nyl_ctx *c, nyl_mg_stats *st, int nite, double res, double normb
 // V-cycle.  Here the tests run on the device (CtlArgs): the V-cycles that the
 // last solves at the same place of a step needed are enqueued without a wait,
 // and one that follows the stopping test leaves the solution as it is (its
-// last pass is gated), so the result does not depend on the guess; the host
+// last pass is gated).  Both forms of a test sum the same cells in the same
+// order (norm_form), so the result does not depend on the guess; the host
 // reads the sums of all tests once and takes the same decisions from them.
 // When the guess was too low, V-cycles follow one at a time.
 

@@ -279,6 +279,7 @@ template <typename T>
 hipError_t launch_mg_sweep2x25(const Geo &g, const T *src, T *dst, const T *b, double omega,
                                const MGTabs &tab, hipStream_t s, double *partials = nullptr,
                                double *dev_out = nullptr, const int *gate = nullptr);
+int sweep2x_kz(const Geo &g, int es);       // planes per block
 int sweep2x_blocks(const Geo &g, int es);
 template <typename Tf, typename Tc>
 hipError_t launch_mg_restrict25(const Geo &gf, const Geo &gc, const Tf *x, const Tf *b, Tc *bc,

@@ -80,9 +80,14 @@ hipError_t launch_march_down(const MarchArgs<T, TC> &a, hipStream_t s);
 // into bc and yc; partials non-null: also the residual norm of src
 template <typename T, typename TC>
 hipError_t launch_march_pre(const MarchArgs<T, TC> &a, hipStream_t s);
-// the residual norm of src alone
+// its blocks (es bytes per value)
+MarchGrid march_pre_grid(const Geo &g, int es);
+// the residual norm of src alone, block sums over the cells of gr's blocks;
+// strips: in the order of k_mg_sweep2t's (tiles of 64 x 8), else of
+// launch_march_pre's
 template <typename T>
-hipError_t launch_march_norm(const MarchArgs<T, T> &a, hipStream_t s);
+hipError_t launch_march_norm(const MarchArgs<T, T> &a, const MarchGrid &gr, bool strips,
+                             hipStream_t s);
 // the mixed solve's FP64 residual (b - shift) - A src: its norm, and its
 // values in FP32 into rout
 hipError_t launch_march_outer(const MarchArgs<double, double> &a, hipStream_t s);

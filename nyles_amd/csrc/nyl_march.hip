@@ -33,10 +33,13 @@ __device__ __forceinline__ int wrap_any(int m, int n) {
 // Every value is the per-cell kernel's expression (sweep_cell, residual_at,
 // restrict_cell, prolong_term) in its order, so the results are bitwise those
 // of the separate launches.
+// STRIPS (the norm alone): thread (tx, ty) owns rows ty and ty + TY/2, so that
+// its sum runs over the cells, in the order, of a thread of k_mg_sweep2t.
 template <typename T, typename TC, int TX, int SRC, int NSW, bool RESN, bool RESTR, bool OUTER,
-          bool XADD = false, bool LONG = false>
+          bool XADD = false, bool LONG = false, bool STRIPS = false>
 __device__ __forceinline__ void march_body(const MarchArgs<T, TC> &a, const MGTabs &tab,
                                            const Blk3 &bk, int nb) {
+    static_assert(!STRIPS || (SRC == MS_FIELD && NSW == 0 && RESN && !RESTR), "the norm alone");
     constexpr int TY = 512 / TX;
     constexpr int R = RESTR ? NSW + 1 : (NSW > 0 ? NSW : 1);
     constexpr int NP = 2 + R;                       // own cells, then one per ring
@@ -77,7 +80,7 @@ __device__ __forceinline__ void march_body(const MarchArgs<T, TC> &a, const MGTa
         has[p] = true;
         if (p < 2) {
             lx = tx + R;
-            ly = 2 * ty + p + R;
+            ly = (STRIPS ? ty + p * (TY / 2) : 2 * ty + p) + R;
         } else {
             const int q = p - 1, W = TX + 2 * q, H = TY + 2 * q;
             // rings 1 and 3 belong to the first threads, ring 2 to the last
@@ -253,12 +256,12 @@ __device__ __forceinline__ void march_body(const MarchArgs<T, TC> &a, const MGTa
     // place of position p in the plane of stage e
     auto place = [&](int p, int e) { return at[p] - e * (W0 + 1) - 2 * e * (ay[p] - e); };
     // sum of the x-, x+, y-, y+, z-, z+ neighbours of position p in the plane P
-    // of stage e; the two own cells are each other's y neighbours
+    // of stage e; the two own cells are each other's y neighbours (not in STRIPS)
     auto six = [&](const T *P, int e, int p, const T (&c)[2], T zm, T zp) -> T {
         const int q = place(p, e), W = W0 - 2 * e;
         const T xm = P[q - 1], xp = P[q + 1];
-        const T ym = p == 1 ? c[0] : P[q - W];
-        const T yp = p == 0 ? c[1] : P[q + W];
+        const T ym = !STRIPS && p == 1 ? c[0] : P[q - W];
+        const T yp = !STRIPS && p == 0 ? c[1] : P[q + W];
         return xm + xp + ym + yp + zm + zp;
     };
 
@@ -458,11 +461,11 @@ constexpr int march_waves() {
 constexpr int MARCH_LONG = 16;
 
 template <typename T, typename TC, int TX, int SRC, int NSW, bool RESN, bool RESTR, bool OUTER,
-          bool LONG = false>
+          bool LONG = false, bool STRIPS = false>
 __global__ __launch_bounds__(256, (march_waves<T, SRC, NSW, RESTR, LONG>())) void k_mg_march(
     MarchArgs<T, TC> a, MGTabs tab) {
     if (a.gate && *a.gate) return;
-    march_body<T, TC, TX, SRC, NSW, RESN, RESTR, OUTER, false, LONG>(
+    march_body<T, TC, TX, SRC, NSW, RESN, RESTR, OUTER, false, LONG, STRIPS>(
         a, tab, xcd_block(), blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
 }
 
@@ -555,10 +558,25 @@ hipError_t launch_march_pre(const MarchArgs<T, TC> &a, hipStream_t s) {
     return hipGetLastError();
 }
 
+MarchGrid march_pre_grid(const Geo &g, int es) {
+    return march_grid(g, march_resident(es, MS_FIELD, 2, true), true);
+}
+
 template <typename T>
-hipError_t launch_march_norm(const MarchArgs<T, T> &a, hipStream_t s) {
-    if (!a.partials) return hipErrorInvalidValue;
-    MARCH_GO(T, T, MS_FIELD, 0, true, false, false);
+hipError_t launch_march_norm(const MarchArgs<T, T> &a, const MarchGrid &gr, bool strips,
+                             hipStream_t s) {
+    if (!a.partials || (strips && (gr.tx != 64 || a.g.nx % 64 || a.g.ny % 8)))
+        return hipErrorInvalidValue;
+    MarchArgs<T, T> m = a;
+    m.kz = gr.kz;
+    const dim3 grd(gr.bx, gr.by, gr.bz), blk(256);
+    if (strips)
+        NYL_LAUNCH((k_mg_march<T, T, 64, MS_FIELD, 0, true, false, false, false, true>), grd, blk,
+                   0, s, m, a.tab);
+    else if (gr.tx == 64)
+        NYL_LAUNCH((k_mg_march<T, T, 64, MS_FIELD, 0, true, false, false>), grd, blk, 0, s, m, a.tab);
+    else
+        NYL_LAUNCH((k_mg_march<T, T, 32, MS_FIELD, 0, true, false, false>), grd, blk, 0, s, m, a.tab);
     return hipGetLastError();
 }
 
@@ -631,7 +649,9 @@ template hipError_t launch_b_march<float, double>(const MarchItem<float, double>
 NYL_MARCH_INST(double, double)
 NYL_MARCH_INST(float, float)
 NYL_MARCH_INST(float, double)
-template hipError_t launch_march_norm<double>(const MarchArgs<double, double> &, hipStream_t);
-template hipError_t launch_march_norm<float>(const MarchArgs<float, float> &, hipStream_t);
+template hipError_t launch_march_norm<double>(const MarchArgs<double, double> &, const MarchGrid &,
+                                              bool, hipStream_t);
+template hipError_t launch_march_norm<float>(const MarchArgs<float, float> &, const MarchGrid &,
+                                             bool, hipStream_t);
 
 }  // namespace nyl

@@ -2240,7 +2240,7 @@ __global__ __launch_bounds__(256) void k_mg_sweep2t_gated(Geo g, const T *__rest
 // planes in FP32, 32 in FP64, dividing nz) that keeps at least 1024 blocks;
 // each block re-reads four input planes.  256^3 (k_mg_sweep2t): FP32 37.8 us
 // at 16 planes (41.0 at 32), FP64 93.4 us at 32 (95.6 at 16).
-static int sweep2x_kz(const Geo &g, int es) {
+int sweep2x_kz(const Geo &g, int es) {
     const int64_t cols = (int64_t)(g.nx / SW_TX) * (g.ny / SW_TY);
     int kz = es == 4 ? 16 : 32;
     while (kz > 1 && (g.nz % kz != 0 || cols * (g.nz / kz) < 1024)) kz >>= 1;
