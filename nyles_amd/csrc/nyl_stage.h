@@ -568,13 +568,24 @@ __global__ __launch_bounds__(256) void k_stage(Geo g, StageArgs<T> a) {
 // periodic 1161 -> 970, 160x96x128 162 -> 112, 96^3 87 -> 57; FP32 256^3
 // 510 -> 440, walls 256x128x64 106 -> 58, 200x120x56 72 -> 42.
 #define STAGE_NT 256
+// The blocks of a plane of ngroup groups: along y, as xcd_block_yslab orders
+// them, and along x past the 65536 blocks that y takes (rows of 2M cells and
+// more); block_group is the first group of a block.
+static inline dim3 flat_grid(int64_t ngroup, int nz) {
+    const int64_t n = (ngroup + STAGE_NT - 1) / STAGE_NT, gx = (n + 65535) / 65536;
+    return dim3((unsigned)gx, (unsigned)((n + gx - 1) / gx), nz);
+}
+__device__ __forceinline__ uint32_t block_group(const Blk3 &bk) {
+    return ((uint32_t)bk.y * gridDim.x + bk.x) * STAGE_NT;
+}
+
 template <typename T, int N, int MODE, int PX, int PY, int PZ, bool LIN = false>
 __global__ __launch_bounds__(STAGE_NT) void k_stage_flat(Geo g, StageArgs<T> a, int lw) {
     const Blk3 bk = xcd_block_yslab();
     const int nxg = g.nx / N;
     int i, j;
     if (lw == 0) {
-        const uint32_t q = (uint32_t)bk.y * STAGE_NT + threadIdx.x;
+        const uint32_t q = block_group(bk) + threadIdx.x;
         j = (int)(q / (uint32_t)nxg);
         i = (int)(q - (uint32_t)j * (uint32_t)nxg);
     } else {
@@ -595,7 +606,7 @@ static void stage_flat_go(const Geo &g, const StageArgs<T> &a, hipStream_t s) {
     const int lw = (N == 2 && nxg % 8 == 0 && g.ny % 32 == 0) ? 3 : 0;
     const int rows = STAGE_NT >> lw;
     const dim3 grd = lw ? dim3(nxg >> lw, g.ny / rows, g.nz)
-                        : dim3(1, (unsigned)(((int64_t)nxg * g.ny + STAGE_NT - 1) / STAGE_NT), g.nz);
+                        : flat_grid((int64_t)nxg * g.ny, g.nz);
     NYL_LAUNCH((k_stage_flat<T, N, MODE, PX, PY, PZ, LIN>), grd, STAGE_NT, 0, s, g, a, lw);
 }
 

@@ -13,7 +13,7 @@ __global__ __launch_bounds__(STAGE_NT) void k_tracer_stage(Geo g, TracerArgs<T> 
     constexpr bool LIN = MODE == 0;   // the linear upwind branch too
     const Blk3 bk = xcd_block_yslab();
     const uint32_t nxg = (uint32_t)g.nx / N;
-    const uint32_t q = (uint32_t)bk.y * STAGE_NT + threadIdx.x;
+    const uint32_t q = block_group(bk) + threadIdx.x;
     const int j = (int)(q / nxg), i = (int)(q - (uint32_t)j * nxg) * N, k = bk.z;
     if (j >= g.ny) return;
     const uint32_t cb = (uint32_t)((int64_t)k * g.sz + (int64_t)j * g.sy + i) * (uint32_t)ES;
@@ -30,7 +30,7 @@ __global__ __launch_bounds__(STAGE_NT) void k_tracer_stage(Geo g, TracerArgs<T> 
 
 template <typename T, int N, int PX, int PY, int PZ>
 static void tracer_modes(const Geo &g, const TracerArgs<T> &a, int mode, hipStream_t s) {
-    const dim3 grd(1, (unsigned)(((int64_t)(g.nx / N) * g.ny + STAGE_NT - 1) / STAGE_NT), g.nz);
+    const dim3 grd = flat_grid((int64_t)(g.nx / N) * g.ny, g.nz);
 #define NYL_TRACER_MODE(M) \
     case M: NYL_LAUNCH((k_tracer_stage<T, N, M, PX, PY, PZ>), grd, STAGE_NT, 0, s, g, a); break;
     switch (mode) {

@@ -44,3 +44,7 @@ def run(exe):
 
 def test_batch_block_sums_stay_inside_their_partials(tmp_path):
     run(build(tmp_path, "batch_plan", without=("nyl_batch.hip",)))
+
+
+def test_stage_grids_stay_within_the_limits(tmp_path):
+    run(build(tmp_path, "stage_grids", without=("nyl_api.hip",)))
