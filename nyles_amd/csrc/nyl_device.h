@@ -125,7 +125,10 @@ __device__ __forceinline__ float weno5_f32(float qmm, float qm, float q0, float 
 // v_div_scale, v_div_fmas and v_div_fixup, which issue at a quarter of the
 // FP64 rate and, for operands whose quotient, reciprocal and residual stay
 // normal, leave every operand as it is: the same double.  The caller holds b
-// in [2^-54, 2^190], and a = +0 or |a| in [2^-900, 2^320].
+// in [2^-54, 2^190], and a = +0 or |a| in [NYL_DIV_LEAST, 2^320]: the least
+// quotient is 2^-990 (a subnormal one, from |a| near 2^-900, rounds wrongly
+// next to a tie).
+#define NYL_DIV_LEAST 0x1p-800
 __device__ __forceinline__ double div_mid(double a, double b) {
 #if defined(__HIP_DEVICE_COMPILE__)
     double r = __builtin_amdgcn_rcp(b);
@@ -185,7 +188,7 @@ __device__ __forceinline__ T weno5(T qmm, T qm, T q0, T qp, T qpp) {
         const T w3 = T(3) * (T(1) + d3);
         const T num = w1 * qi1 + w2 * qi2 + w3 * qi3, den = w1 + w2 + w3;
         // a zero keeps its sign, and a tiny sum its scaling, in the full division
-        if (mid && fabs(num) >= T(0x1p-900)) return div_mid(num, den);
+        if (mid && fabs(num) >= T(NYL_DIV_LEAST)) return div_mid(num, den);
         return num / den;
     }
 }

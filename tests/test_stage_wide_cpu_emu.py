@@ -1,5 +1,6 @@
-"""The stage and tracer kernels of wide planes on the CPU (no GPU), built for
-the host as in test_kernels_cpu_emu.py, with AddressSanitizer."""
+"""The stage and tracer kernels of wide planes, and the short FP64 division of
+the reconstructions over the whole range it is used on, on the CPU (no GPU),
+built for the host as in test_kernels_cpu_emu.py, with AddressSanitizer."""
 import os
 import shutil
 import subprocess
@@ -11,13 +12,14 @@ EMU = os.path.join(HERE, "cpu_emu")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 
 
-def test_wide_stage_forms_bitwise(tmp_path):
+@pytest.mark.parametrize("name", ["stage_wide_emu", "division_emu"])
+def test_wide_stage_forms_bitwise(name, tmp_path):
     gxx = shutil.which("g++")
     if gxx is None:
         pytest.skip("g++ is not available")
-    exe = str(tmp_path / "stage_wide_emu")
+    exe = str(tmp_path / name)
     build = [gxx, "-std=c++17", "-O1", "-fsanitize=address", "-fno-omit-frame-pointer",
-             "-I", EMU, "-I", INCLUDE, os.path.join(EMU, "stage_wide_emu.cpp"), "-lpthread",
+             "-I", EMU, "-I", INCLUDE, os.path.join(EMU, name + ".cpp"), "-lpthread",
              "-o", exe]
     subprocess.run(build, check=True, timeout=900)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=900)
