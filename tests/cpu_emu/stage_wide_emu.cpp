@@ -1,6 +1,7 @@
 // The stage and tracer kernels with the blocks of a plane along x and y (as
-// for planes of more than 65536 blocks) against the blocks along y alone, bit
-// for bit.
+// for planes of more than 65536 blocks) against the blocks along y alone, and
+// the tendencies and the second RK3 stage of the linear branches and model
+// variants with 16 bytes of cells per thread against one cell, bit for bit.
 #define NYL_STAGE_SEQ 0
 #include "../../nyles_amd/csrc/nyl_stage.h"
 #include "../../nyles_amd/csrc/nyl_tracer.hip"
@@ -62,8 +63,35 @@ int split(int nx, int ny, int nz, int gx) {
     return bad != 0;
 }
 
+template <typename T, int N, int MODE, int PX, int PY, int PZ>
+int lin(int nx, int ny, int nz) {
+    const int orders[][3] = {{1, 1, 0}, {3, 5, 0}, {5, 3, 0}, {5, 0, NYL_SF_NO_B}, {0, 0, NYL_SF_NO_VF}};
+    const Geo g = mk(nx, ny, nz, PX, PY, PZ);
+    int bad = 0;
+    for (auto &o : orders) {
+        Fields<T> f1(g, nx + ny), f2(g, nx + ny);
+        for (auto *f : {&f1, &f2}) { f->a.upw_a = o[0]; f->a.upw_vf = o[1]; f->a.flags = o[2]; }
+        auto grd = [&](int n) { return dim3(1, (nx / n * ny + STAGE_NT - 1) / STAGE_NT, nz); };
+        run_blocks(grd(1), dim3(STAGE_NT), [&]() {
+            k_stage_flat<T, 1, MODE, PX, PY, PZ, true>(g, f1.a, 0); }, false);
+        run_blocks(grd(N), dim3(STAGE_NT), [&]() {
+            k_stage_flat<T, N, MODE, PX, PY, PZ, true>(g, f2.a, 0); }, false);
+        for (int q = 0; q < 12; q++) bad += ndiff(f1.out[q], f2.out[q]);
+    }
+    printf("lin<%d, %d> mode %d %dx%dx%d p=%d%d%d: %d mismatches\n", (int)sizeof(T), N, MODE, nx, ny,
+           nz, PX, PY, PZ, bad);
+    return bad != 0;
+}
+
+template <int PX, int PY, int PZ>
+int lin_all() {
+    return lin<double, 2, 0, PX, PY, PZ>(8, 8, 8) + lin<double, 2, 2, PX, PY, PZ>(30, 9, 8) +
+           lin<float, 4, 0, PX, PY, PZ>(12, 9, 8) + lin<float, 4, 2, PX, PY, PZ>(8, 8, 8);
+}
+
 int main() {
-    int fails = 0;
+    int fails = lin_all<0, 0, 0>() + lin_all<1, 0, 0>() + lin_all<0, 1, 0>() + lin_all<0, 0, 1>() +
+                lin_all<1, 1, 1>();
     for (int gx : {2, 3}) {
         fails += split<double, 2, 0, 1, 0>(66, 40, 8, gx);
         fails += split<double, 1, 1, 0, 0>(33, 40, 8, gx);
