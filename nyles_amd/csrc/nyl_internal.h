@@ -194,17 +194,6 @@ hipError_t launch_mg_down(const Geo &gf, const Geo &gc, const Tf *y, const Tf *b
 template <typename Tf, typename Tc>
 hipError_t launch_mg_up(const Geo &gf, const Geo &gc, const Tf *x, const Tc *xc, const Tf *b,
                         Tf *y, double omega, const MGTabs &tab, hipStream_t s);
-// residual + restriction from a level of type Tf to the next of type Tc;
-// yc non-null: also the coarse level's first sweep from x = 0 into yc (coarse
-// x is then left as is, the second sweep overwrites it), else xc = 0
-template <typename Tf, typename Tc>
-hipError_t launch_mg_resid_restrict(const Geo &gf, const Geo &gc, const Tf *x, const Tf *b,
-                                    Tc *bc, Tc *xc, const MGTabs &tab, hipStream_t s,
-                                    Tc *yc = nullptr, double omega = 0.0);
-template <typename Tf, typename Tc>
-hipError_t launch_mg_prolong(const Geo &gf, const Geo &gc, Tf *xf, const Tc *xc,
-                             const MGTabs &tab, hipStream_t s);
-
 // whether the mixed solve takes a level-1 grid of this width
 bool outer_resid_fits(const Geo &g);
 // x += e, unless *gate is non-zero (gate null: always)

@@ -155,15 +155,6 @@ __device__ __forceinline__ void restrict_cell(const Geo &gf, const Geo &gc,
     else xc[cc] = Tc(0);
 }
 
-template <typename Tf, typename Tc>
-hipError_t launch_mg_resid_restrict(const Geo &gf, const Geo &gc, const Tf *x, const Tf *b,
-                                    Tc *bc, Tc *xc, const MGTabs &tab, hipStream_t s, Tc *yc,
-                                    double omega) {
-    NYL_LAUNCH((k_mg_resid_restrict<Tf, Tc>), mg_grid(gc), dim3(MG_BX, MG_BY, 1), 0, s,
-                       gf, gc, x, b, bc, xc, tab, yc, omega);
-    return hipGetLastError();
-}
-
 // fprolongation_centers3d (core/mgfor/basicoperators.f90:173-231) at one
 // fine cell: Pcoef*(3*b + a) with the (9,3,3,1) planar weights, b the
 // parent's coarse plane and a the coarse plane on the child's side.
@@ -202,14 +193,6 @@ __global__ __launch_bounds__(256) void k_mg_prolong(Geo gf, Geo gc, Tf *__restri
     if (i >= gf.nx || j >= gf.ny) return;
     const int64_t c = (int64_t)k * gf.sz + (int64_t)j * gf.sy + i;
     xf[c] = xf[c] + prolong_term<Tf, Tc>(gc, xc, tab, i, j, k);
-}
-
-template <typename Tf, typename Tc>
-hipError_t launch_mg_prolong(const Geo &gf, const Geo &gc, Tf *xf, const Tc *xc,
-                             const MGTabs &tab, hipStream_t s) {
-    NYL_LAUNCH((k_mg_prolong<Tf, Tc>), mg_grid(gf), dim3(MG_BX, MG_BY, 1), 0, s, gf, gc,
-                       xf, xc, tab);
-    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
@@ -1607,12 +1590,6 @@ static int outer25_kz(const Geo &g) {
     return kz;
 }
 
-bool outer25_fits(const Geo &g) {
-    if (!sweep25_fits(g)) return false;
-    const int64_t nb = (int64_t)(g.nx / SW_TX) * (g.ny / SW_TY) * (g.nz / outer25_kz(g));
-    return nb <= NYL_RED_BLOCKS;
-}
-
 // Prolongation with 2.5-D tiling: a block owns fine 64 x 8 cells (rows
 // j0 + ty + 4r of column i0 + tx) and marches up kz fine planes (kz even).
 // The coarse values its cells use (a 34 x 6 footprint per coarse plane,
@@ -2315,11 +2292,6 @@ hipError_t launch_mg_restrict25(const Geo &gf, const Geo &gc, const Tf *x, const
                                                    hipStream_t, T *, double);                   \
     template hipError_t launch_mg_sweep<T>(const Geo &, const T *, T *, const T *, double,      \
                                            const MGTabs &, hipStream_t);                        \
-    template hipError_t launch_mg_resid_restrict<T, T>(const Geo &, const Geo &, const T *,     \
-                                                       const T *, T *, T *, const MGTabs &,     \
-                                                       hipStream_t, T *, double);               \
-    template hipError_t launch_mg_prolong<T, T>(const Geo &, const Geo &, T *, const T *,       \
-                                                const MGTabs &, hipStream_t);                   \
     template hipError_t launch_norm2<T>(const Geo &, const T *, double *, double *, hipStream_t); \
     template hipError_t launch_maxu2<T>(const Geo &, const T *, const T *, const T *, double,   \
                                         double, double, double *, double *, hipStream_t);       \
@@ -2336,13 +2308,6 @@ template hipError_t launch_resnorm2<double>(const Geo &, const double *, const d
                                             const MGTabs &, double *, double *, hipStream_t);
 template hipError_t launch_resnorm2<float>(const Geo &, const float *, const float *,
                                            const MGTabs &, double *, double *, hipStream_t);
-// FP32 inner levels above an FP64 coarsest level
-template hipError_t launch_mg_resid_restrict<float, double>(const Geo &, const Geo &,
-                                                            const float *, const float *,
-                                                            double *, double *, const MGTabs &,
-                                                            hipStream_t, double *, double);
-template hipError_t launch_mg_prolong<float, double>(const Geo &, const Geo &, float *,
-                                                     const double *, const MGTabs &, hipStream_t);
 template hipError_t launch_add_correction<float>(const Geo &, double *, const float *,
                                                  const int *, hipStream_t);
 
