@@ -1,6 +1,6 @@
 // The residual norm alone (k_mg_march, STRIPS) against the norm that comes
 // with the tiled two-sweep pass (k_mg_sweep2t): the same block sums, bit for
-// bit, for every periodicity and march length.
+// bit, with walls and periodic axes, marches of one plane and of several.
 #include "../../nyles_amd/csrc/nyl_mg.hip"
 #include "../../nyles_amd/csrc/nyl_march.hip"
 #include "emu.h"
@@ -34,8 +34,8 @@ int check(int nx, int ny, int nz, int px, int py, int kz) {
 
 int main() {
     int fails = 0;
-    for (int p = 0; p < 4; p++)
-        for (int kz : {1, 2, 8}) {
+    for (int p : {0, 1, 3})
+        for (int kz : {1, 8}) {
             fails += check<double, 0>(128, 16, 8, p & 1, p >> 1, kz);
             fails += check<double, 1>(64, 8, 8, p & 1, p >> 1, kz);
             fails += check<float, 0>(64, 24, 8, p & 1, p >> 1, kz);
