@@ -152,9 +152,9 @@ int nyl_ctx_destroy(nyl_ctx *ctx);
 int nyl_workspace_bytes(const nyl_ctx *ctx, uint64_t *bytes);
 int nyl_bind_workspace(nyl_ctx *ctx, void *dptr, uint64_t bytes);
 int nyl_set_stream(nyl_ctx *ctx, void *hip_stream);
-/* Accepted and without effect: a solve enqueues its V-cycles ahead of the GPU
- * with no host read between them, so that nothing is gained by replaying part
- * of one from a hipGraph.  No counterpart in the reference. */
+/* Accepted and without effect: a solve enqueues the V-cycles it expects ahead
+ * of the GPU with no host read between them, so that nothing is gained by
+ * replaying part of one from a hipGraph.  No counterpart in the reference. */
 int nyl_set_graphs(nyl_ctx *ctx, int on);
 
 /* Byte offset, element count and dtype of a field in the workspace.  The

@@ -361,8 +361,11 @@ int cycle_first(nyl_ctx *c) {
     for (int l = c->nlev - 1; l >= 1; l--) {
         CycleArgs a;
         CycleEnt ent[CYC_ENT];
-        // a direct solve alone pays only while it is small: 25x15x7 takes 21 us
-        // in one workgroup, 13 us in its own three launches
+        // A direct solve alone pays only while it is small.  us per V-cycle of a
+        // two-level solve, in one workgroup / in its own three launches: 5^3
+        // 28.6 / 33.9, 9^3 31.5 / 35.1, 13x9x9 33.3 / 35.4, 15x15x7 36.6 / 37.3,
+        // 13^3 40.2 / 36.7, 25x15x7 46.7 / 40.2, 15^3 46.8 / 37.6.  The line is
+        // at one cell per thread; up to 1600 cells the two are 1 to 2 us apart.
         if (l == c->nlev - 1 && c->exact && cells(g[l]) > 1024) break;
         if (cells(g[l]) > CYC_CELLS ||
             !cycle_layout(a, ent, g, l, c->nlev, lev64(c, l) ? 8 : 4, c->exact != 0,

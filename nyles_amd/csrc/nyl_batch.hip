@@ -7,7 +7,9 @@
 // member's arithmetic does not depend on the batch it is in.  The multigrid
 // stop rule (core/mgfor/solvers.f90:17-30) is evaluated per member on the
 // device (k_b_final), members that have stopped skip the V-cycle kernels,
-// and the host only reads one counter per V-cycle.  Each plan (stage kernel
+// and the host reads the active count once per RK stage, after the V-cycles
+// that stage needed in the step before, and once more per V-cycle beyond
+// them.  Each plan (stage kernel
 // + divergence + initial norms, one V-cycle, correction + diagnostics) is a
 // fixed launch sequence and is captured once into a hipGraph.
 #include <string.h>

@@ -63,7 +63,7 @@ MarchGrid march_grid(const Geo &g, int res, bool even);
 // resident blocks per CU of a kind of pass, from its registers: es bytes per
 // value, src a MarchSrc, sweeps, restr: with a restriction
 constexpr int march_resident(int es, int src, int sweeps, bool restr) {
-    if (sweeps == 0) return es == 4 ? 8 : 6;
+    if (sweeps == 0) return 6;   // the FP64 outer residual
     if (src == MS_PROLONG) return es == 4 ? 4 : 2;
     if (sweeps == 2 && restr) return src == MS_ZERO ? (es == 4 ? 4 : 3) : (es == 4 ? 3 : 2);
     if (src == MS_ZERO) return es == 4 ? 8 : 6;

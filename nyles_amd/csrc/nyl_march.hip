@@ -453,7 +453,10 @@ __device__ __forceinline__ void march_body(const MarchArgs<T, TC> &a, const MGTa
 // 16 planes or more with sweeps: pre-smoothing with restriction + post-
 // smoothing FP64 256^3 252 -> 238 us, FP32 256^3 136 -> 126, 256x256x512
 // 279 -> 271; in short marches the second copy of the code costs more than
-// its few steps gain (96^3: 35.5 -> 36.6).
+// its few steps gain (96^3: 35.5 -> 36.6).  The limit costs a few spills: 6 of
+// the 128 registers of the FP32 prolongation march (28 bytes of scratch per
+// lane, 2 and 12 with 32 columns), 1 of the 256 of the FP64 pre-smoothing with
+// restriction and norm; the times above include them.
 template <typename T, int SRC, int NSW, bool RESTR, bool LONG>
 constexpr int march_waves() {
     return LONG ? march_resident(sizeof(T), SRC, NSW, RESTR) : 1;
