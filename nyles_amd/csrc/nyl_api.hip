@@ -562,7 +562,9 @@ bool pre_tiled(const nyl_ctx *c) {
 // The block sums of level 0's residual norm: those of the pre-smoothing pass
 // with a norm.  The norm alone (resid_norm) sums the same cells in the same
 // order, so a test gives the same bits whichever of the two the guess of a
-// solve chose.  capped: more blocks than partial sums, k_resnorm2 instead.
+// solve chose.  That fixes its blocks: at 256^3 it takes 59.4 us in FP64 where
+// blocks of its own choice took 53.1, and 27.8 in FP32 as before.  capped: more
+// blocks than partial sums, k_resnorm2 instead.
 struct NormForm {
     MarchGrid grid;
     bool tiled, capped;
