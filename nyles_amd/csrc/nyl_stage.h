@@ -568,16 +568,8 @@ __global__ __launch_bounds__(256) void k_stage(Geo g, StageArgs<T> a) {
 // periodic 1161 -> 970, 160x96x128 162 -> 112, 96^3 87 -> 57; FP32 256^3
 // 510 -> 440, walls 256x128x64 106 -> 58, 200x120x56 72 -> 42.
 #define STAGE_NT 256
-// The blocks of a plane of ngroup groups: along y, as xcd_block_yslab orders
-// them, and along x past the 65536 blocks that y takes (rows of 2M cells and
-// more); block_group is the first group of a block.
-static inline dim3 flat_grid(int64_t ngroup, int nz) {
-    const int64_t n = (ngroup + STAGE_NT - 1) / STAGE_NT, gx = (n + 65535) / 65536;
-    return dim3((unsigned)gx, (unsigned)((n + gx - 1) / gx), nz);
-}
-__device__ __forceinline__ uint32_t block_group(const Blk3 &bk) {
-    return ((uint32_t)bk.y * gridDim.x + bk.x) * STAGE_NT;
-}
+#define GRID_YZ 65536   // most blocks along y and z of a launch
+static inline int64_t flat_blocks(int64_t ngroup) { return (ngroup + STAGE_NT - 1) / STAGE_NT; }
 
 template <typename T, int N, int MODE, int PX, int PY, int PZ, bool LIN = false>
 __global__ __launch_bounds__(STAGE_NT) void k_stage_flat(Geo g, StageArgs<T> a, int lw) {
@@ -585,7 +577,7 @@ __global__ __launch_bounds__(STAGE_NT) void k_stage_flat(Geo g, StageArgs<T> a, 
     const int nxg = g.nx / N;
     int i, j;
     if (lw == 0) {
-        const uint32_t q = block_group(bk) + threadIdx.x;
+        const uint32_t q = (uint32_t)bk.y * STAGE_NT + threadIdx.x;
         j = (int)(q / (uint32_t)nxg);
         i = (int)(q - (uint32_t)j * (uint32_t)nxg);
     } else {
@@ -603,10 +595,13 @@ static void stage_flat_go(const Geo &g, const StageArgs<T> &a, hipStream_t s) {
     // FP64 in whole tiles of 8 pairs (one line of L2) x 32 rows: the rows that
     // neighbours in y share stay in L1, 256^3 1033 -> 978 us, 160x96x128
     // 114 -> 110; no gain in FP32, whose loads are half as long
-    const int lw = (N == 2 && nxg % 8 == 0 && g.ny % 32 == 0) ? 3 : 0;
-    const int rows = STAGE_NT >> lw;
-    const dim3 grd = lw ? dim3(nxg >> lw, g.ny / rows, g.nz)
-                        : flat_grid((int64_t)nxg * g.ny, g.nz);
+    // (lw = 3).  Planes of more groups than the blocks along y take (2M cells in
+    // a row): tiles of 64 x 4, whose blocks along x are not so limited (lw = 6).
+    const int64_t nb = flat_blocks((int64_t)nxg * g.ny);
+    const int lw = (N == 2 && nxg % 8 == 0 && g.ny % 32 == 0) ? 3 : (nb > GRID_YZ ? 6 : 0);
+    const int cols = 1 << lw, rows = STAGE_NT >> lw;
+    const dim3 grd = lw ? dim3((nxg + cols - 1) / cols, (g.ny + rows - 1) / rows, g.nz)
+                        : dim3(1, (unsigned)nb, g.nz);
     NYL_LAUNCH((k_stage_flat<T, N, MODE, PX, PY, PZ, LIN>), grd, STAGE_NT, 0, s, g, a, lw);
 }
 

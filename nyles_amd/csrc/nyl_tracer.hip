@@ -6,14 +6,15 @@ namespace nyl {
 
 // N cells per thread as in k_stage_flat, whose rule chooses N: the tracer of
 // 128x64x64 FP64 in a closed box took 23 us with one cell per thread in
-// 64-wide rows, 19.7 with two (bound by VALU issue, as the stage kernel).
+// 64-wide rows, 19.7 with two (bound by VALU issue, as the stage kernel).  The
+// blocks of a plane lie along y, and along x past the GRID_YZ that y takes.
 template <typename T, int N, int MODE, int PX, int PY, int PZ>
 __global__ __launch_bounds__(STAGE_NT) void k_tracer_stage(Geo g, TracerArgs<T> a) {
     constexpr int ES = (int)sizeof(T);
     constexpr bool LIN = MODE == 0;   // the linear upwind branch too
     const Blk3 bk = xcd_block_yslab();
     const uint32_t nxg = (uint32_t)g.nx / N;
-    const uint32_t q = block_group(bk) + threadIdx.x;
+    const uint32_t q = ((uint32_t)bk.y * gridDim.x + bk.x) * STAGE_NT + threadIdx.x;
     const int j = (int)(q / nxg), i = (int)(q - (uint32_t)j * nxg) * N, k = bk.z;
     if (j >= g.ny) return;
     const uint32_t cb = (uint32_t)((int64_t)k * g.sz + (int64_t)j * g.sy + i) * (uint32_t)ES;
@@ -30,7 +31,8 @@ __global__ __launch_bounds__(STAGE_NT) void k_tracer_stage(Geo g, TracerArgs<T> 
 
 template <typename T, int N, int PX, int PY, int PZ>
 static void tracer_modes(const Geo &g, const TracerArgs<T> &a, int mode, hipStream_t s) {
-    const dim3 grd = flat_grid((int64_t)(g.nx / N) * g.ny, g.nz);
+    const int64_t nb = flat_blocks((int64_t)(g.nx / N) * g.ny), bx = (nb + GRID_YZ - 1) / GRID_YZ;
+    const dim3 grd((unsigned)bx, (unsigned)((nb + bx - 1) / bx), g.nz);
 #define NYL_TRACER_MODE(M) \
     case M: NYL_LAUNCH((k_tracer_stage<T, N, M, PX, PY, PZ>), grd, STAGE_NT, 0, s, g, a); break;
     switch (mode) {

@@ -1,5 +1,6 @@
-// The stage and tracer kernels with the blocks of a plane along x and y (as
-// for planes of more than 65536 blocks) against the blocks along y alone, and
+// The stage and tracer kernels with the blocks of a plane as for planes of more
+// than 65536 blocks (the stage in tiles of 64 x 4 groups with partial ones, the
+// tracers' along x and y) against the blocks along y alone, and
 // the tendencies and the second RK3 stage of the linear branches and model
 // variants with 16 bytes of cells per thread against one cell, bit for bit.
 #define NYL_STAGE_SEQ 0
@@ -45,16 +46,16 @@ int split(int nx, int ny, int nz, int gx) {
     const unsigned nb = (nx / N * ny + STAGE_NT - 1) / STAGE_NT;
     Fields<T> f1(g, nx + ny), f2(g, nx + ny);
     const dim3 one(1, nb, nz), many(gx, (nb + gx - 1) / gx, nz);
-    auto stage = [&](dim3 grd, Fields<T> &f) {
-        run_blocks(grd, dim3(STAGE_NT), [&]() { k_stage_flat<T, N, 3, PX, PY, PZ>(g, f.a, 0); }, false);
+    auto stage = [&](dim3 grd, Fields<T> &f, int lw) {
+        run_blocks(grd, dim3(STAGE_NT), [&]() { k_stage_flat<T, N, 3, PX, PY, PZ>(g, f.a, lw); }, false);
     };
     auto tracer = [&](dim3 grd, Fields<T> &f) {
         const TracerArgs<T> t = f.tracer();
         run_blocks(grd, dim3(STAGE_NT), [&]() { k_tracer_stage<T, N, 2, PX, PY, PZ>(g, t); }, false);
     };
     int bad = 0;
-    stage(one, f1);
-    stage(many, f2);
+    stage(one, f1, 0);
+    stage(dim3((nx / N + 63) / 64, (ny + 3) / 4, nz), f2, 6);
     for (int q = 0; q < 12; q++) bad += ndiff(f1.out[q], f2.out[q]);
     tracer(one, f1);
     tracer(many, f2);
